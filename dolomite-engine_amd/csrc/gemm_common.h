@@ -1,0 +1,43 @@
+// Types shared by the grouped-GEMM kernels: the register-staged and DMA-staged tiles of grouped_gemm.hip and the
+// persistent kernel of persistent_gemm.hip.
+#pragma once
+
+#include "common.h"
+
+struct GemmArgs {
+  const void* in;
+  const void* w;
+  void* out;
+  const int32_t* sorted_scattered;
+  const int32_t* expert_offsets;
+  int L;        // rows of the sorted order
+  int K;        // contraction length
+  int N;        // output columns (SwiGLU: I, with 2N weight rows per expert)
+  int E;
+  int kdiv;     // gather divisor (top-k) for scattered inputs
+  int kshift;   // log2(kdiv) if kdiv is a power of two, else -1 (set by the persistent launch)
+  int n_tiles;  // column tiles per row tile
+  int gather;   // input row of sorted row i is sorted_scattered[i] / kdiv (else i)
+  int scatter;  // output row of sorted row i is sorted_scattered[i] (else i)
+  int remap;    // XCD-aware tile order
+  void* ws;     // persistent kernel: workspace for splitting the last round of tiles along K (or null)
+  void* pre;    // persistent SwiGLU kernel: (L, 2N) pre-activation output next to the activation (or null)
+  int out_nt;   // persistent kernel: store the output non-temporal (set in run_gemm)
+  // fp8 weights (register-staged kernel, W8 form): w holds e4m3fn bytes, row-major (E, rows, K) or in the streamed-tile
+  // layout of decode_fp8.hip; wscale (E, rows) fp32 is applied to the accumulators in the epilogue
+  const float* wscale;
+  int w_tiled;
+};
+
+// ---- persistent_gemm.hip ---------------------------------------------------------------------------------------------
+#define PERSIST_REMAP_INTERLEAVE 2
+#define PERSIST_REMAP_FIXED 4  // the caller chose the form (cfg 8 / 9): the host does not apply its own rule
+#define PERSIST_MAX_E 256
+#define PERSIST_WS_TILE_BYTES (256 * 256 * 4)
+
+enum { PG_PLAIN = 0, PG_SWIGLU = 1, PG_SWIGLU_KEEP = 2, PG_WEIGHT_KN = 3 };
+// K % 8 == 0 and N % 8 == 0, at most PERSIST_MAX_E experts, 16-byte aligned output
+bool mi_gemm_persistent_ok(const GemmArgs& a);
+// whether a contraction of length K can be cut along K (the only calls that use a workspace)
+bool mi_gemm_persistent_splits(int K);
+int mi_gemm_persistent(const GemmArgs& a, int dtype, int form, hipStream_t s);

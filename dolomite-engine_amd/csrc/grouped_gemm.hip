@@ -11,10 +11,8 @@
 //   grouped_gemm_kernel             register-staged tiles (any K that is a multiple of one 16-byte chunk; bf16, fp16
 //                                   and fp32): the design notes below
 //   grouped_gemm_dma_kernel         the same tile with the operands brought to LDS by DMA, one tile per workgroup
-//   grouped_gemm_persistent_kernel  one workgroup per CU walking a list of 256 x 256 tiles, two wave groups in
-//                                   ping-pong (large expert loads; its notes stand in front of it), with
-//   grouped_gemm_split_finish_kernel  for the tiles of a last round that were cut along K
 //   grouped_gemm_naive_kernel       one thread per output element, only on request (cfg 3)
+// Large expert loads run on the persistent kernel of persistent_gemm.hip.
 //
 // Design
 //   * One workgroup computes a BM x BN output tile of ONE expert.  The tile list is not built on the
@@ -31,7 +29,7 @@
 //     so the epilogue packs 4 results into one 8-byte store.
 //   * Two LDS stages: the global loads of K-tile i+1 are issued before the MFMAs of tile i and
 //     written to the other stage afterwards; one barrier per K-tile.
-#include "common.h"
+#include "gemm_common.h"
 
 #include <type_traits>
 
@@ -59,48 +57,6 @@ template <> struct Mfma32<float> {
     for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], c, 0, 0, 0);
     return c;
   }
-};
-
-// 16x16x32: half the flops per instruction and the same rate, but a quarter of the accumulator traffic
-// per flop.  Under the chip's power limit (random operands) it sustains about 30 % more throughput than
-// 32x32x16, so the persistent ping-pong kernel uses it.
-template <typename T> struct Mfma16;
-template <> struct Mfma16<bf16_t> {
-  typedef bf16x8 vec;
-  static __device__ __forceinline__ f32x4 run(vec a, vec b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mfma16<f16_t> {
-  typedef f16x8 vec;
-  static __device__ __forceinline__ f32x4 run(vec a, vec b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-
-struct GemmArgs {
-  const void* in;
-  const void* w;
-  void* out;
-  const int32_t* sorted_scattered;
-  const int32_t* expert_offsets;
-  int L;        // rows of the sorted order
-  int K;        // contraction length
-  int N;        // output columns (SwiGLU: I, with 2N weight rows per expert)
-  int E;
-  int kdiv;     // gather divisor (top-k) for scattered inputs
-  int kshift;   // log2(kdiv) if kdiv is a power of two, else -1 (set by launch_persistent)
-  int n_tiles;  // column tiles per row tile
-  int gather;   // input row of sorted row i is sorted_scattered[i] / kdiv (else i)
-  int scatter;  // output row of sorted row i is sorted_scattered[i] (else i)
-  int remap;    // XCD-aware tile order
-  void* ws;     // persistent kernel: workspace for splitting the last round of tiles along K (or null)
-  void* pre;    // persistent SwiGLU kernel: (L, 2N) pre-activation output next to the activation (or null)
-  int out_nt;   // persistent kernel: store the output non-temporal (set in run_gemm)
-  // fp8 weights (register-staged kernel, W8 form): w holds e4m3fn bytes, row-major (E, rows, K) or in the streamed-tile
-  // layout of decode_fp8.hip; wscale (E, rows) fp32 is applied to the accumulators in the epilogue
-  const float* wscale;
-  int w_tiled;
 };
 
 // 8 fp8 e4m3fn values (two dwords) -> 8 values of a 16-bit type (exact: e4m3 fits in either)
@@ -753,762 +709,6 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GemmArgs 
   }
 }
 
-// ------------------------------------------------------------------------------------------------
-// Persistent variant of the DMA kernel: one workgroup per CU walks a list of tiles and the 4-stage
-// LDS ring runs straight through the tile boundaries.
-//
-// A workgroup that handles one tile pays, per tile, for a launch, the tile lookup, the row-index
-// loads, an empty pipeline (three stages of DMA latency) and an epilogue during which nothing is in
-// flight; with K = 1536 that is as long as the MFMA work itself.  Here
-//   * the DMA for the first four K slices of tile i+1 is issued during the last four slices of tile i,
-//   * the lookup of tile i+2 comes from a per-expert table in LDS (no global loads) and its row-index
-//     loads are issued before the epilogue of tile i and consumed after it,
-//   * the epilogue stages each 32 x 64 block of results through a per-wave LDS scratch so that global
-//     stores are 16 bytes per lane and 128 contiguous bytes per row.
-// Tile order: workgroup b serves XCD b % 8 (hardware deals workgroup ids round-robin to the XCDs); the
-// XCD's contiguous tile range is dealt to its workgroups in turn, so at any moment the CUs of one XCD
-// work on neighbouring tiles (same expert weights, shared activation rows) out of one L2.
-//
-// The eight waves form two groups that alternate between a memory phase and a matrix phase (see pp_slice).  With
-// all waves in one phase and one barrier per K slice, the two waves of a SIMD stall together (barrier, LDS latency,
-// DMA issue) and the matrix pipe idles: measured on the 32768-token Granite-3B shape, about 65 % matrix-pipe
-// occupancy in cycles inside the K loop against about 80 % for the alternating form, with 32-wide as with 64-wide
-// K slices.  (With random operands the chip then lowers its clock to stay inside its power limit, so wall time
-// improves less than the cycle count.)
-// ------------------------------------------------------------------------------------------------
-
-#define PERSIST_MAX_E 256
-
-// Splitting the last round along K.  A workgroup's tiles all take the same time, so when the tiles of an XCD do not
-// fill its last round, the workgroups without a tile wait for one tile time.  With a workspace, the `rem` tiles of
-// that round are cut into `parts` = min(slots / rem, PERSIST_SPLIT_MAX) ranges of K slices, one per workgroup; a
-// part writes its fp32 accumulators to the workspace instead of running the epilogue, and a second, small launch
-// (grouped_gemm_split_finish_kernel) adds the parts of every split tile in part order and runs the epilogue, so
-// the result does not depend on timing.  A round is only split if that shortens it by at least
-// PERSIST_SPLIT_MIN_SAVED slices: the partial tiles' trip through memory and the second launch cost 40-80 us
-// (measured), about 100 slices' worth.
-#define PERSIST_SPLIT_MAX 4
-#define PERSIST_SPLIT_MIN_SAVED 120
-#define PERSIST_SPLIT_MIN_SLICES 32
-#define PERSIST_WS_TILE_BYTES (256 * 256 * 4)
-
-// whether a contraction of length K can be shortened by PERSIST_SPLIT_MIN_SAVED slices at all (launch_persistent
-// applies the same rule, plus one on the grid)
-static bool persistent_may_split(int K) {
-  const int nk = K / 32;
-  return nk - nk / PERSIST_SPLIT_MAX >= PERSIST_SPLIT_MIN_SAVED;
-}
-
-// Which tiles a workgroup runs.  Workgroup b sits on XCD b % 8 (the hardware deals workgroup ids round-robin to the
-// XCDs) in slot b / 8.  Two ways of dealing the band-ordered tile list to them:
-//   * contiguous (the default): XCD x owns the x-th eighth of the list and deals it to its slots in turn, so the
-//     CUs of an XCD work on neighbouring tiles out of one L2 and an XCD stays with its experts;
-//   * interleaved (PERSIST_REMAP_INTERLEAVE): round r of the whole chip is the tiles [r * grid, (r + 1) * grid), XCD
-//     x taking the x-th run of grid / 8 of them.  All XCDs then work on neighbouring tiles at the same time.  When
-//     an expert has more column tiles than a band is wide (intermediate size 14336: 112 column tiles, bands of 8),
-//     consecutive bands read the same activation rows, and the XCDs share them through the memory-side cache
-//     instead of each fetching them from HBM in its own time: Mixtral-shape layer 5.02 -> 4.73 ms.  With few
-//     column tiles (the band is the whole row) it changes little either way (-1.3 % on the Granite-1B shape,
-//     +1.1 % on the Granite-3B shape), so the host asks for it only from 8 column tiles on.
-// Either way the tiles that do not fill the last round can be cut along K (see PERSIST_SPLIT_MAX).
-#define PERSIST_REMAP_INTERLEAVE 2
-#define PERSIST_REMAP_FIXED 4  // the caller chose the form (cfg 8 / 9): the host does not apply its own rule
-
-struct SplitPlan {
-  int base, stride;  // tile of this workgroup in round i < full_rounds: base + i * stride
-  int full_rounds;   // rounds in which every slot has a tile
-  int rem;           // tiles of the last round, the first of them being rem_base
-  int rem_base;
-  int parts;         // K ranges each of them is cut into (1: not split)
-  int lslot;         // this workgroup's slot in the last round: part lslot / rem of tile rem_base + lslot % rem
-  int ws_base;       // first partial-tile slot of the last round's tiles in the workspace
-};
-
-// xcd / slot of the workgroup (slot < nslot); for the finishing kernel, slot is the tile of the last round it adds up
-__device__ __forceinline__ SplitPlan persist_split_plan(int total, int xcd, int slot, int nslot, int nk, bool have_ws,
-                                                        bool interleave) {
-  SplitPlan sp;
-  int cap;  // slots that share one last round
-  if (interleave) {
-    cap = nslot * 8;
-    sp.lslot = xcd * nslot + slot;
-    sp.base = sp.lslot;
-    sp.stride = cap;
-    sp.full_rounds = total / cap;
-    sp.rem = total - sp.full_rounds * cap;
-    sp.rem_base = sp.full_rounds * cap;
-    sp.ws_base = 0;
-  } else {
-    cap = nslot;
-    const int per = (total + 7) >> 3;
-    int n_x = total - xcd * per;
-    n_x = n_x < 0 ? 0 : (n_x < per ? n_x : per);
-    sp.lslot = slot;
-    sp.base = xcd * per + slot;
-    sp.stride = nslot;
-    sp.full_rounds = n_x / nslot;
-    sp.rem = n_x - sp.full_rounds * nslot;
-    sp.rem_base = xcd * per + sp.full_rounds * nslot;
-    sp.ws_base = xcd * nslot;
-  }
-  sp.parts = 1;
-  if (have_ws && sp.rem > 0) {
-    int p = cap / sp.rem;
-    if (p > PERSIST_SPLIT_MAX) p = PERSIST_SPLIT_MAX;
-    if (p >= 2 && nk / p >= PERSIST_SPLIT_MIN_SLICES && nk - nk / p >= PERSIST_SPLIT_MIN_SAVED) sp.parts = p;
-  }
-  return sp;
-}
-
-// etab[2e] = row tiles of experts 0..e, etab[2e+1] = offsets[e]; filled by the calling wave (all 64 lanes)
-template <int BM>
-__device__ __forceinline__ void persist_expert_table(const int32_t* __restrict__ off, int E, int* etab) {
-  const int lane = threadIdx.x & 63;
-  int carry = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    const int e = e0 + lane;
-    const int end = e < E ? off[e] : 0;
-    const int prev = (e < E && e > 0) ? off[e - 1] : 0;
-    const int t = e < E ? (end - prev + BM - 1) / BM : 0;
-    int incl = t;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    incl += carry;
-    if (e < E) {
-      etab[2 * e] = incl;
-      etab[2 * e + 1] = end;
-    }
-    carry = __shfl(incl, 63, 64);
-  }
-}
-
-// tile id -> coordinates, from the LDS table (wave-uniform result).  An expert's tiles are numbered band
-// by band: a band is up to 8 column tiles wide and runs over all of the expert's row tiles, row tile
-// slowest.  The 32 workgroups of an XCD, which take 32 consecutive tiles at a time, then cover about
-// 4 row tiles x 8 column tiles: 12 operand slabs for 32 tiles, and each weight slab is fetched once per
-// band instead of once per row tile (with many column tiles -- intermediate 14336 -- a plain row-major
-// order re-streams all of an expert's weights from HBM for every row tile).  Up to 8 column tiles the band
-// is the whole row, so that complete output rows are written at about the same time.
-template <int BM>
-__device__ __forceinline__ void persist_locate(const int* etab, int E, int n_tiles, int tile, TileCoord& tc) {
-  const int lane = threadIdx.x & 63;
-  const int tile_band = n_tiles < 8 ? n_tiles : 8;
-  const int q = tile / n_tiles;  // experts own contiguous tile ranges: (row tiles before) * n_tiles
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    const int e = e0 + lane;
-    const int incl = e < E ? etab[2 * e] : 0x7fffffff;
-    const uint64_t hit = __ballot(incl > q);
-    if (hit) {
-      const int ex = e0 + __ffsll((long long)hit) - 1;
-      const int first_tile = ex > 0 ? etab[2 * (ex - 1)] : 0;
-      const int prev = ex > 0 ? etab[2 * (ex - 1) + 1] : 0;
-      const int row_tiles = etab[2 * ex] - first_tile;
-      const int local = tile - first_tile * n_tiles;
-      const int band = local / (row_tiles * tile_band);
-      const int rem = local - band * row_tiles * tile_band;
-      const int left = n_tiles - band * tile_band;
-      const int width = left < tile_band ? left : tile_band;
-      const int mt = rem / width;
-      tc.expert = ex;
-      tc.nt = band * tile_band + rem - mt * width;
-      tc.row_begin = prev + mt * BM;
-      tc.row_end = etab[2 * ex + 1];
-      return;
-    }
-  }
-  tc.expert = 0; tc.nt = 0; tc.row_begin = 0; tc.row_end = 1;  // unreachable for a valid tile id
-}
-
-template <typename T, int BM, int BNW, int WM, int WN, bool GLU, bool WT = false, bool KEEP_PRE = false>
-__global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_persistent_kernel(GemmArgs a) {
-  // KEEP_PRE: the SwiGLU form that also writes the pre-activation (a.pre), for training
-  static_assert(!KEEP_PRE || GLU, "the pre-activation belongs to the SwiGLU form");
-  // WT: the expert weights are (K, N) row-major ("x @ W" with W as stored, the form both data gradients of the
-  // backward take).  A K slice of them is 32 rows of 512 bytes; it is staged as it lies in HBM and the fragments
-  // are read with the transposing LDS read (see read_frags).
-  static_assert(!WT || (!GLU && BNW == 256), "transposed-weight form");
-  constexpr int BK = 32;                     // K slice per ring stage = one 16x16x32 matrix instruction deep
-  constexpr int NSTAGE = 4;                  // ring of 128 KiB
-  constexpr int RPI = 16;                    // stage rows filled by one DMA instruction (1 KiB)
-  constexpr int LROW_SHIFT = 2;              // lane -> row within the instruction's rows
-  constexpr int NW = WM * WN;
-  constexpr int ROWS = BM + BNW;
-  constexpr int STAGE_BYTES = ROWS * BK * 2;
-  constexpr int RING_BYTES = NSTAGE * STAGE_BYTES;
-  // per-wave epilogue scratch: 32 rows x 64 columns, in the ring stage that is free at a tile boundary.  64 columns
-  // make every store a run of whole 128-byte lines per row (measured: 64-byte pieces write at 4.4-4.6 TB/s
-  // chip-wide, 128-byte ones at 5.0-5.3).
-  constexpr int EPI_COLS = 64;
-  constexpr int EPI_BYTES = 32 * EPI_COLS * 2;
-  constexpr int EPI_CPR = EPI_COLS / 8;      // 16-byte chunks per scratch row
-  constexpr int NLD = ROWS / RPI / NW;       // DMA instructions per wave per K slice
-  constexpr int NXLD = BM / RPI / NW;        // ... of which activation rows (the first NXLD)
-  constexpr int BN = GLU ? BNW / 2 : BNW;
-  constexpr int WTM = BM / WM, WTN = BNW / WN;
-  constexpr int MT = 16;                     // edge of one accumulator block (v_mfma_f32_16x16x32)
-  constexpr int MB = WTM / MT, NB = WTN / MT;
-  constexpr int OB = GLU ? NB / 2 : NB;      // output column blocks per wave
-  constexpr int EPI_MB = 32 / MT;            // accumulator row blocks per 32-row epilogue pass
-  constexpr int EPI_NB = EPI_COLS / MT;      // accumulator column blocks per epilogue pass
-  static_assert(BM % (16 * NW) == 0 && BNW % (16 * NW) == 0 && NW % 2 == 0, "tile/wave shape");
-  static_assert(OB % EPI_NB == 0 && MB % EPI_MB == 0, "epilogue pass shape");
-  static_assert((NSTAGE - 1) * NLD <= 63, "vmcnt range");
-  typedef typename Mfma16<T>::vec frag_t;
-  typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  // [ring][expert table: E x (tiles inclusive, row end)]
-  int* etab = reinterpret_cast<int*>(smem_raw + RING_BYTES);
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % WM, wn = wave / WM;
-
-  // ---- per-expert table: etab[2e] = row tiles of experts 0..e, etab[2e+1] = offsets[e] ---------------
-  if (wave == 0) persist_expert_table<BM>(a.expert_offsets, a.E, etab);
-  __syncthreads();
-  const int total = etab[2 * (a.E - 1)] * a.n_tiles;
-  const int xcd = blockIdx.x & 7, slot0 = blockIdx.x >> 3, nslot = gridDim.x >> 3;
-  const int nk = a.K / BK;  // >= NSTAGE (host-checked)
-  // full_rounds rounds in which every slot has a tile, then `rem` tiles, each cut into `parts` K ranges
-  const SplitPlan sp =
-      persist_split_plan(total, xcd, slot0, nslot, nk, a.ws != nullptr, (a.remap & PERSIST_REMAP_INTERLEAVE) != 0);
-  const int my_part = sp.parts > 1 ? sp.lslot / sp.rem : 0, my_rem_tile = sp.rem > 0 ? sp.lslot % sp.rem : 0;
-
-  // i-th tile of this workgroup, or -1
-  auto tile_of = [&](int i) -> int {
-    if (i < sp.full_rounds) return sp.base + i * sp.stride;
-    if (i > sp.full_rounds || sp.lslot >= sp.rem * sp.parts) return -1;
-    return sp.rem_base + my_rem_tile;
-  };
-  // K slices [k0, k0 + len) of the i-th item
-  auto item_k = [&](int i, int& k0, int& len) {
-    if (i == sp.full_rounds && sp.parts > 1) {
-      k0 = my_part * nk / sp.parts;
-      len = (my_part + 1) * nk / sp.parts - k0;
-    } else {
-      k0 = 0;
-      len = nk;
-    }
-  };
-  auto locate = [&](int tile, TileCoord& tc) { persist_locate<BM>(etab, a.E, a.n_tiles, tile, tc); };
-
-  // ---- DMA sources -----------------------------------------------------------------------------------
-  // A tile's sources are NLD 32-bit byte offsets per lane (activation rows relative to the input
-  // matrix, weight rows relative to the expert's weight matrix) plus the expert's scalar base; the K
-  // position is added on the scalar side, so a DMA instruction is "scalar base + lane offset".
-  constexpr int WROWS_MUL = GLU ? 2 : 1;
-  const unsigned char* __restrict__ xbase = static_cast<const unsigned char*>(a.in);
-  const unsigned char* __restrict__ wall = static_cast<const unsigned char*>(a.w);
-  const size_t expert_bytes = (size_t)WROWS_MUL * a.N * a.K * sizeof(T);
-  // logical 16-byte chunk this lane fetches so that it lands in its swizzled slot (see read_frags): row =
-  // 16*grp + lane/4, slot = lane%4, swizzle (row >> 1) & 3 -- the one that reads the 16 rows x 4 chunks of a
-  // fragment without bank conflicts (measured; (row >> 2) & 3 costs about 20 % of the LDS read rate there)
-  const int lchunk = (lane & 3) ^ ((lane >> 3) & 3);
-  struct TileSrc {
-    uint32_t off[NLD];
-    const unsigned char* wbase;
-  };
-  // sorted-order row of the activation rows this lane fetches (clamped into the tile's expert)
-  auto load_rows = [&](const TileCoord& tc, int (&raw)[NXLD]) {
-#pragma unroll
-    for (int j = 0; j < NXLD; ++j) {
-      int srow = tc.row_begin + (j * NW + wave) * RPI + (lane >> LROW_SHIFT);
-      if (srow > tc.row_end - 1) srow = tc.row_end - 1;  // tail rows re-read the last valid row; never stored
-      raw[j] = a.gather ? a.sorted_scattered[srow] : srow;
-    }
-  };
-  auto make_src = [&](const TileCoord& tc, const int (&raw)[NXLD], TileSrc& ts) {
-    ts.wbase = wall + (size_t)tc.expert * expert_bytes;
-#pragma unroll
-    for (int j = 0; j < NLD; ++j) {
-      if (j < NXLD) {
-        // (top-k is a power of two in every configuration of the reference: a shift instead of a division per lane
-        // and tile; launch_persistent sets kshift to -1 otherwise)
-        const int s = !a.gather ? raw[j] : (a.kshift >= 0 ? raw[j] >> a.kshift : raw[j] / a.kdiv);
-        ts.off[j] = ((uint32_t)s * (uint32_t)a.K + lchunk * 8) * (uint32_t)sizeof(T);
-      } else if constexpr (WT) {
-        // DMA instruction = two K rows of the slice; LDS piece lane % 32 of row krow holds the logical 16-byte
-        // piece whose 32-byte group is (piece / 2) ^ f(krow): the swizzle the transposing reads expect
-        const int krow = 2 * ((j - NXLD) * NW + wave) + (lane >> 5);
-        const int f = (krow & 3) | (((krow >> 3) & 3) << 2);
-        const int piece = lane & 31;
-        int col = tc.nt * BN + ((((piece >> 1) ^ f) & 15) << 4) + (piece & 1) * 8;
-        if (col > a.N - 8) col = a.N - 8;  // column tail re-reads the last piece of the row; never stored
-        ts.off[j] = ((uint32_t)krow * (uint32_t)a.N + col) * (uint32_t)sizeof(T);
-      } else {
-        const int wr = ((j - NXLD) * NW + wave) * RPI + (lane >> LROW_SHIFT);
-        int col, half = 0;
-        if (GLU) {
-          half = wr >= BN;
-          col = tc.nt * BN + (half ? wr - BN : wr);
-        } else {
-          col = tc.nt * BN + wr;
-        }
-        if (col > a.N - 1) col = a.N - 1;  // column tail re-reads the last weight row; never stored
-        ts.off[j] = ((uint32_t)(half * a.N + col) * (uint32_t)a.K + lchunk * 8) * (uint32_t)sizeof(T);
-      }
-    }
-  };
-  // slice kt of tile `cur`, or (from_next) of tile `next`, into ring stage `stage`
-  auto dma_slice = [&](const TileSrc& cur, const TileSrc& next, bool from_next, int kt, int stage) {
-    const size_t kbytes = (size_t)kt * BK * sizeof(T);
-    const unsigned char* xs = xbase + kbytes;
-    const unsigned char* ws = (from_next ? next.wbase : cur.wbase) + (WT ? kbytes * a.N : kbytes);
-    const uint32_t stage_lds = (uint32_t)(size_t)(lds_ptr_t)smem_raw + stage * STAGE_BYTES;
-    // activation rows fill stage rows [0, BM), weight rows [BM, BM + BNW)
-    auto grp = [&](int j) { return j < NXLD ? (j * NW + wave) : (BM / RPI + (j - NXLD) * NW + wave); };
-    if (from_next) {
-#pragma unroll
-      for (int j = 0; j < NLD; ++j) dma16_to_lds<1>(j < NXLD ? xs : ws, next.off[j], stage_lds + grp(j) * 1024);
-    } else {
-#pragma unroll
-      for (int j = 0; j < NLD; ++j) dma16_to_lds<0>(j < NXLD ? xs : ws, cur.off[j], stage_lds + grp(j) * 1024);
-    }
-  };
-
-  // ---- fragment reads ----------------------------------------------------------------------------------
-  // lane -> (row of its 16-row block, k chunk): the instruction takes k = 8 * (lane / 16) + [0, 8) of the slice
-  const int frow = lane % MT, fhalf = lane / MT;
-  const int fswz = (frow >> 1) & 3;
-  int frag_x_off[MB], frag_w_off[NB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) frag_x_off[mb] = (wm * WTM + mb * MT + frow) * (BK * 2);
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    int r;
-    if (GLU) {
-      constexpr int HB = NB / 2;
-      int h = nb >= HB;
-      r = h * BN + wn * (WTN / 2) + (h ? nb - HB : nb) * MT + frow;
-    } else {
-      r = wn * WTN + nb * MT + frow;
-    }
-    frag_w_off[nb] = (BM + r) * (BK * 2);
-  }
-  const int chunk_byte = (fhalf ^ fswz) * 16;
-  frag_t xf[MB], wf[NB];
-  // WT: ds_read_b64_tr_b16 transposes 4 rows x 16 columns across 16 lanes: lane i of the group supplies the
-  // address of (row i / 4, columns 4 (i % 4) ..) and receives column i of the four rows.  Lane group q reads rows
-  // 8q .. 8q + 3 and, 2 KiB further, 8q + 4 .. 8q + 7: together the 8 contraction values the matrix instruction
-  // wants from lane (column, q).
-  typedef short tr_s16x4 __attribute__((ext_vector_type(4)));
-  const int tr_i = lane & 15, tr_q = lane >> 4;
-  const uint32_t tr_base = (8 * tr_q + (tr_i >> 2)) * (BNW * 2) + ((((tr_i >> 2) | (tr_q << 2))) << 5) + (tr_i & 3) * 8;
-  const uint32_t lds_base = (uint32_t)(size_t)(lds_ptr_t)smem_raw;
-  auto read_frags = [&](int stage) {
-    const unsigned char* s = smem_raw + stage * STAGE_BYTES + chunk_byte;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      if constexpr (WT) {
-        typedef __attribute__((address_space(3))) tr_s16x4* tr_ptr_t;
-        const uint32_t addr = lds_base + stage * STAGE_BYTES + BM * BK * 2 + (tr_base ^ ((uint32_t)(wn * NB + nb) << 5));
-        const tr_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(size_t)addr);
-        const tr_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(size_t)(addr + 4 * BNW * 2));
-        wf[nb] = __builtin_bit_cast(frag_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-      } else {
-        wf[nb] = __builtin_bit_cast(frag_t, *reinterpret_cast<const u32x4*>(s + frag_w_off[nb]));
-      }
-    }
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-      xf[mb] = __builtin_bit_cast(frag_t, *reinterpret_cast<const u32x4*>(s + frag_x_off[mb]));
-  };
-
-  // accumulator block (nb, mb): register i of a lane is output column 16 * nb + 4 * fhalf + i (weight row) of
-  // token row 16 * mb + frow
-  f32x4 acc[NB][MB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[nb][mb][i] = 0.f;
-
-  // eight instructions in a row share the activation operand.  The first slice of a tile multiplies onto a zero
-  // operand instead of the accumulators (an inline constant of the instruction), so that the accumulators need not
-  // be cleared between tiles: 128 moves per wave and tile, issued when the matrix pipe has nothing else to do.
-  auto mfma_step = [&](auto first_tag) {
-    constexpr bool FIRST = decltype(first_tag)::value;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[nb][mb] = Mfma16<T>::run(wf[nb], xf[mb], FIRST ? zero : acc[nb][mb]);
-  };
-
-  int g = 0;  // running K-slice count; slice g lives in ring stage g % NSTAGE
-  // One K slice.  The waves with wn == 0 and those with
-  // wn == 1 -- one of each per SIMD -- run this same code one phase apart (see the tile loop): while one group
-  // issues its NB * MB matrix instructions back to back out of registers, the other reads its fragments of the
-  // slice from LDS and issues its share of the DMA for slice g + 3 into the stage both groups have finished
-  // reading.  Every phase ends in a workgroup barrier; at each barrier one group has just issued its last MFMA
-  // and the other has its operands in registers, so the matrix pipe of the SIMD never waits for LDS, DMA or the
-  // barrier itself.
-  auto pp_slice = [&](auto first_tag, const TileSrc& tcur, const TileSrc& tnext, bool from_next, int kload) {
-    const int cur = g & (NSTAGE - 1), fill = (g + NSTAGE - 1) & (NSTAGE - 1);
-    read_frags(cur);
-    dma_slice(tcur, tnext, from_next, kload, fill);
-    asm volatile("" ::: "memory");
-    // own DMA of slice g + 1 has landed (slices g + 2 and g + 3 stay in flight); fragments are in registers
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm((NSTAGE - 2) * NLD, 0));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    // (Signalling the second barrier a few matrix instructions early, so that they cover its release
-    // latency, measured slower: the group's next memory phase then starts late and becomes the long one.)
-    mfma_step(first_tag);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    ++g;
-  };
-
-  // ---- epilogue of one tile: acc -> (SwiGLU) -> LDS scratch -> 16-byte row-contiguous stores -----------
-  T* __restrict__ out = static_cast<T*>(a.out);
-  static_assert(NW * EPI_BYTES <= STAGE_BYTES, "epilogue scratch must fit the free ring stage");
-  constexpr int RPP = 64 / EPI_CPR;  // rows per read-back pass
-  static_assert(RPP == 8, "read-back row order below");
-  // Row of the 32-row block that read-back instruction `it` takes for this lane: instruction 0 the even rows of
-  // the first sixteen, instruction 1 the odd ones, then the second sixteen.  All rows of an instruction have the
-  // same parity, which is what lets the epilogue's writes use both 8-byte halves of a 16-byte chunk (see there).
-  auto rb_row = [&](int it) { return 16 * (it >> 1) + 2 * (lane / EPI_CPR) + (it & 1); };
-  constexpr int MP = MB / EPI_MB;    // 32-row passes over the wave's token rows
-  // Destination rows of everything this lane will store in a tile's epilogue.  With scattered output they are
-  // fetched one tile ahead (next to the gather indices of the tile after), so that the epilogue does not start
-  // with a memory latency.
-  struct OutRows {
-    int r[MP][32 / RPP];
-  };
-  auto load_out_rows = [&](const TileCoord& tc, OutRows& o) {
-    // (rows past the expert's end are never stored: with scattered output they read the index of its last row, so
-    // that the loads need no predicates)
-    const int row0 = tc.row_begin + wm * WTM;
-    if (a.scatter) {
-#pragma unroll
-      for (int mp = 0; mp < MP; ++mp)
-#pragma unroll
-        for (int it = 0; it < 32 / RPP; ++it) {
-          const int row = row0 + mp * 32 + rb_row(it);
-          o.r[mp][it] = a.sorted_scattered[row < tc.row_end ? row : tc.row_end - 1];
-        }
-    } else {
-#pragma unroll
-      for (int mp = 0; mp < MP; ++mp)
-#pragma unroll
-        for (int it = 0; it < 32 / RPP; ++it) o.r[mp][it] = row0 + mp * 32 + rb_row(it);
-    }
-  };
-  // INTERIOR: every row and column of the tile exists (all tiles but an expert's last row tile and a ragged last
-  // column tile), so the stores need no predicates; NT: non-temporal stores (see persistent_out_nt).  Both are
-  // compile-time forms of one body: the tile boundary is bound by instruction issue (no matrix work covers it),
-  // and a predicate, an exec-mask save / restore and a branch on the store's cache policy around each of a wave's
-  // 16 stores were a sixth of its instructions.
-  // WHAT: 0 the kernel's result (with SwiGLU: up * silu(gate)); 1 / 2 (SwiGLU kernel keeping the pre-activation):
-  // the up / the gate half of h, into a.pre.  KEEP: the result is formed from the ROUNDED halves, as the separate
-  // activation kernel forms it from the stored h (swiglu_forward_kernel).
-  auto epilogue_as = [&](auto what_tag, auto interior_tag, auto nt_tag, auto keep_tag, const TileCoord& tc,
-                         const OutRows& orows) {
-    constexpr int WHAT = decltype(what_tag)::value;
-    constexpr bool INTERIOR = decltype(interior_tag)::value;
-    constexpr bool NT = decltype(nt_tag)::value;
-    constexpr bool KEEP = decltype(keep_tag)::value;
-    constexpr int OBX = WHAT == 0 ? OB : NB / 2;  // output column blocks of this form
-    static_assert(OBX % EPI_NB == 0, "epilogue pass shape");
-    T* __restrict__ dst_base = WHAT == 0 ? out : static_cast<T*>(a.pre);
-    const int ld = WHAT == 0 ? a.N : 2 * a.N;
-    // the ring stage consumed last is free until the next tile's first memory phase refills it (the tile loop
-    // puts a barrier between this epilogue and that refill)
-    unsigned char* scratch = smem_raw + ((g + NSTAGE - 1) & (NSTAGE - 1)) * STAGE_BYTES + wave * EPI_BYTES;
-    // Scratch row r (128 bytes: the full width of the 32 banks) keeps its 16-byte chunks at slots chunk ^ swz(r),
-    // and odd rows keep the two 8-byte halves of every chunk swapped: the sixteen lanes that write together hold
-    // sixteen different rows and the same 8 bytes of each, and land in sixteen different bank pairs (with the chunk
-    // swizzle alone rows 2j and 2j + 1 collided on every write: 1000 conflict cycles per plain tile, now 500 --
-    // off the critical path either way, the layer's time did not move).
-    // The read-back takes rows of one parity per instruction and swaps the halves of the odd ones by naming.
-    auto swz = [](int r) { return (r >> 1) & 7; };
-    const auto& orow_of = orows.r;
-#pragma unroll
-    for (int mp = 0; mp < MP; ++mp) {
-#pragma unroll
-      for (int og = 0; og < OBX / EPI_NB; ++og) {
-        // write the 32 x EPI_COLS block: a lane holds, per accumulator block, token row frow and the four
-        // output columns 4 * fhalf + [0, 4)
-#pragma unroll
-        for (int mbb = 0; mbb < EPI_MB; ++mbb) {
-          const int mb = mp * EPI_MB + mbb;
-          const int srow = mbb * MT + frow;
-#pragma unroll
-          for (int ob = 0; ob < EPI_NB; ++ob) {
-            const int nb = og * EPI_NB + ob;
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              if (WHAT == 1) {
-                v[i] = acc[nb][mb][i];
-              } else if (WHAT == 2) {
-                v[i] = acc[nb + NB / 2][mb][i];
-              } else if (GLU) {
-                float up = acc[nb][mb][i];
-                float gt = acc[nb + NB / 2][mb][i];
-                if (KEEP) {
-                  up = Elt<T>::round(up);
-                  gt = Elt<T>::round(gt);
-                }
-                v[i] = up * gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
-              } else {
-                v[i] = acc[nb][mb][i];
-              }
-            }
-            const int colp = ob * MT + fhalf * 4;  // column inside the pass
-            const u32x2 p = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
-            *reinterpret_cast<u32x2*>(scratch + srow * (EPI_COLS * 2) + (((colp >> 3) ^ swz(srow)) * 16) +
-                                      (((colp >> 2) ^ srow) & 1) * 8) = p;
-          }
-        }
-        // read back: lane -> row rb_row(it), 16-byte chunk lane%EPI_CPR
-        const int cchunk = lane % EPI_CPR;
-        // column of the result (the predicate's), and of what this form writes
-        const int col = tc.nt * BN + (GLU ? wn * (WTN / 2) : wn * WTN) + og * EPI_COLS + cchunk * 8;
-        const int dcol = WHAT == 2 ? a.N + col : col;
-        // two reads at a time in front of their stores (one LDS latency for both): left alone, the compiler sinks
-        // each read into its store's predicated region and waits for it there; all four at once do not fit next
-        // to the accumulators
-        constexpr int RB = 2;
-        static_assert((32 / RPP) % RB == 0, "read-back batches");
-#pragma unroll
-        for (int it0 = 0; it0 < 32 / RPP; it0 += RB) {
-          __builtin_amdgcn_sched_barrier(0);  // (one batch's addresses and values live at a time)
-          u32x4 vals[RB];
-#pragma unroll
-          for (int j = 0; j < RB; ++j) {
-            const int r = rb_row(it0 + j);
-            const u32x4 v = *reinterpret_cast<const u32x4*>(scratch + r * (EPI_COLS * 2) + ((cchunk ^ swz(r)) * 16));
-            vals[j] = ((it0 + j) & 1) ? u32x4{v[2], v[3], v[0], v[1]} : v;
-          }
-#pragma unroll
-          for (int j = 0; j < RB; ++j) asm volatile("" : "+v"(vals[j]));
-#pragma unroll
-          for (int j = 0; j < RB; ++j) {
-            const int it = it0 + j;
-            const int r = rb_row(it);
-            const int row = tc.row_begin + wm * WTM + mp * 32 + r;
-            if (INTERIOR || (row < tc.row_end && col < a.N)) {
-              int orow = orow_of[mp][it];
-              asm volatile("" : "+v"(orow));  // (the address is formed here, not once per row and kept in registers)
-              u32x4* dst = reinterpret_cast<u32x4*>(dst_base + (size_t)orow * ld + dcol);
-              if constexpr (NT) __builtin_nontemporal_store(vals[j], dst);
-              else *dst = vals[j];
-            }
-          }
-        }
-      }
-    }
-  };
-  typedef std::integral_constant<int, 0> what_result;
-  typedef std::integral_constant<int, 1> what_up;
-  typedef std::integral_constant<int, 2> what_gate;
-  auto epilogue = [&](const TileCoord& tc, const OutRows& orows) {
-    const bool interior = tc.row_begin + BM <= tc.row_end && (tc.nt + 1) * BN <= a.N;
-    if constexpr (KEEP_PRE) {
-      {
-        // the activation and both halves of the pre-activation (plain stores: the backward reads them again)
-        if (interior) {
-          epilogue_as(what_result{}, std::true_type{}, std::false_type{}, std::true_type{}, tc, orows);
-          epilogue_as(what_up{}, std::true_type{}, std::false_type{}, std::true_type{}, tc, orows);
-          epilogue_as(what_gate{}, std::true_type{}, std::false_type{}, std::true_type{}, tc, orows);
-        } else {
-          epilogue_as(what_result{}, std::false_type{}, std::false_type{}, std::true_type{}, tc, orows);
-          epilogue_as(what_up{}, std::false_type{}, std::false_type{}, std::true_type{}, tc, orows);
-          epilogue_as(what_gate{}, std::false_type{}, std::false_type{}, std::true_type{}, tc, orows);
-        }
-        return;
-      }
-    }
-    if (interior) {
-      if (a.out_nt) epilogue_as(what_result{}, std::true_type{}, std::true_type{}, std::false_type{}, tc, orows);
-      else epilogue_as(what_result{}, std::true_type{}, std::false_type{}, std::false_type{}, tc, orows);
-    } else {
-      if (a.out_nt) epilogue_as(what_result{}, std::false_type{}, std::true_type{}, std::false_type{}, tc, orows);
-      else epilogue_as(what_result{}, std::false_type{}, std::false_type{}, std::false_type{}, tc, orows);
-    }
-  };
-
-  // ---- a part of a split tile: accumulators -> workspace (one partial tile per (XCD, slot), fp32) -----------------
-  // Vector j of thread t lies at [j][t]: every store instruction writes 8 KB in a row.  The address is a uniform
-  // base that moves from vector to vector plus one per-thread offset (the accumulators leave no registers for an
-  // address per vector).
-  auto store_part = [&]() {
-    constexpr size_t PART_VECS = (size_t)NB * MB * NW * 64;  // f32x4 per partial tile
-    unsigned t = tid;
-    asm volatile("" : "+v"(t));  // (keeps the offset from being computed ahead of the tile loop and held through it)
-    f32x4* base = static_cast<f32x4*>(a.ws) + ((size_t)sp.ws_base + (size_t)my_rem_tile * sp.parts + my_part) * PART_VECS;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) (base + (nb * MB + mb) * (NW * 64))[t] = acc[nb][mb];
-  };
-
-  // ---- tile loop -------------------------------------------------------------------------------------------
-  int t0 = tile_of(0);
-  if (t0 < 0) return;
-  TileCoord c0, c1;
-  locate(t0, c0);
-  int t1 = tile_of(1);
-  if (t1 >= 0) locate(t1, c1); else c1 = c0;
-  int k0_cur, nk_cur, k0_next, nk_next;
-  item_k(0, k0_cur, nk_cur);
-  if (t1 >= 0) item_k(1, k0_next, nk_next); else { k0_next = k0_cur; nk_next = nk_cur; }
-  TileSrc src_cur, src_next;
-  {
-    int raw0[NXLD], raw1[NXLD];
-    load_rows(c0, raw0);
-    load_rows(c1, raw1);
-    make_src(c0, raw0, src_cur);
-    make_src(c1, raw1, src_next);
-  }
-  OutRows out_cur, out_next;
-  load_out_rows(c0, out_cur);
-  __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
-  constexpr int AHEAD = NSTAGE - 1;  // slices in flight ahead of the one being consumed
-  static_assert(WN == 2, "two wave groups");
-#pragma unroll
-  for (int st = 0; st < AHEAD; ++st) dma_slice(src_cur, src_cur, false, k0_cur + st, st);
-  __builtin_amdgcn_s_waitcnt(waitcnt_imm((AHEAD - 1) * NLD, 0));
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-
-  for (int i = 0;; ++i) {
-    // the ring runs on into the next tile: the last AHEAD slices refill with its first AHEAD.
-    // group wn == 1 runs one phase behind group wn == 0 inside a tile; both leave the tile together
-    if (wn == 1) __builtin_amdgcn_s_barrier();
-    // (a tile or a part of one has at least NSTAGE slices: the first is never among the last AHEAD)
-    pp_slice(std::true_type{}, src_cur, src_next, false, k0_cur + AHEAD);
-    for (int kt = 1; kt < nk_cur; ++kt) {
-      const bool from_next = kt >= nk_cur - AHEAD;
-      pp_slice(std::false_type{}, src_cur, src_next, from_next,
-               from_next ? k0_next + kt + AHEAD - nk_cur : k0_cur + kt + AHEAD);
-    }
-    if (wn == 0) __builtin_amdgcn_s_barrier();
-    if (nk_cur != nk) {
-      // a part of a split tile, always a workgroup's last item: the finishing launch adds the parts up
-      store_part();
-      break;
-    }
-    const int t2 = tile_of(i + 2);
-    TileCoord c2 = c1;
-    if (t2 >= 0) locate(t2, c2);
-    int raw2[NXLD];
-    load_rows(c2, raw2);
-    load_out_rows(c1, out_next);
-    epilogue(c0, out_cur);
-    // every wave is done with its scratch before any wave's DMA of the next tile lands in that stage
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (t1 < 0) {
-      // The compiler folds this exit into the loop's back edge and then assumes, inside the slice loop, that
-      // the row-index loads above may still be in flight (nobody consumes them on this path): it would drain
-      // the DMA ring with vmcnt(0) at the top of every K slice.  Retiring them here keeps that path clean.
-      __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
-      break;
-    }
-    c0 = c1;
-    c1 = c2;
-    t1 = t2;
-    src_cur = src_next;
-    out_cur = out_next;
-    k0_cur = k0_next;
-    nk_cur = nk_next;
-    if (t2 >= 0) item_k(i + 2, k0_next, nk_next);  // else: the surplus DMA of the last item re-reads its own slices
-    make_src(c2, raw2, src_next);
-    // Retire every load the compiler knows about (row indices, epilogue traffic) here, once per tile:
-    // otherwise it re-checks them with vmcnt(0) inside the slice loop and drains the DMA ring there.
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
-  }
-  __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));  // surplus DMA must not outlive the workgroup's LDS
-}
-
-// The tiles the persistent kernel cut along K (see PERSIST_SPLIT_MAX): one workgroup per (XCD, tile of its last
-// round) recomputes the same plan, adds the tile's partial accumulators in part order and writes the tile the way
-// the persistent kernel's epilogue does (same arithmetic, same rounding; thread t holds what thread t of a part
-// held).  Workgroups whose tile does not exist or was not split return at once.
-template <typename T, int BM, int BNW, int WM, int WN, bool GLU>
-__global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_split_finish_kernel(GemmArgs a, int nslot) {
-  constexpr int NW = WM * WN;
-  constexpr int BN = GLU ? BNW / 2 : BNW;
-  constexpr int WTM = BM / WM, WTN = BNW / WN;
-  constexpr int MT = 16;
-  constexpr int MB = WTM / MT, NB = WTN / MT;
-  constexpr int OB = GLU ? NB / 2 : NB;
-  constexpr size_t PART_VECS = (size_t)NB * MB * NW * 64;
-  __shared__ int etab[2 * PERSIST_MAX_E];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave % WM, wn = wave / WM;
-  if (wave == 0) persist_expert_table<BM>(a.expert_offsets, a.E, etab);
-  __syncthreads();
-  const int total = etab[2 * (a.E - 1)] * a.n_tiles;
-  // contiguous: workgroup b adds up tile b / 8 of XCD b % 8's last round; interleaved: tile b of the chip's last round
-  const bool interleave = (a.remap & PERSIST_REMAP_INTERLEAVE) != 0;
-  const int xcd = interleave ? 0 : (int)(blockIdx.x & 7), j = interleave ? (int)blockIdx.x : (int)(blockIdx.x >> 3);
-  const SplitPlan sp = persist_split_plan(total, xcd, 0, nslot, a.K / 32, true, interleave);
-  if (sp.parts == 1 || j >= sp.rem) return;
-  TileCoord tc;
-  persist_locate<BM>(etab, a.E, a.n_tiles, sp.rem_base + j, tc);
-
-  // vector j of thread t of a part lies at [j][t]
-  const f32x4* part = static_cast<const f32x4*>(a.ws) + ((size_t)sp.ws_base + (size_t)j * sp.parts) * PART_VECS + tid;
-  f32x4 sum[NB][MB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) sum[nb][mb] = __builtin_nontemporal_load(part + (nb * MB + mb) * (NW * 64));
-  for (int p = 1; p < sp.parts; ++p) {
-    part += PART_VECS;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const f32x4 v = __builtin_nontemporal_load(part + (nb * MB + mb) * (NW * 64));
-#pragma unroll
-        for (int c = 0; c < 4; ++c) sum[nb][mb][c] += v[c];
-      }
-  }
-
-  // accumulator block (nb, mb): register i of a lane is output column 16 * nb + 4 * fhalf + i of the wave's
-  // columns, token row 16 * mb + frow of the wave's rows; with SwiGLU block nb + NB / 2 holds the gate of block nb
-  const int frow = lane % MT, fhalf = lane / MT;
-  T* __restrict__ out = static_cast<T*>(a.out);
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int row = tc.row_begin + wm * WTM + mb * MT + frow;
-    if (row >= tc.row_end) continue;
-    const int orow = a.scatter ? a.sorted_scattered[row] : row;
-#pragma unroll
-    for (int nb = 0; nb < OB; ++nb) {
-      const int col = tc.nt * BN + (GLU ? wn * (WTN / 2) : wn * WTN) + nb * MT + fhalf * 4;
-      if (col >= a.N) continue;
-      float v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (GLU) {
-          const float up = sum[nb][mb][i];
-          const float gt = sum[nb + NB / 2][mb][i];
-          v[i] = up * gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
-        } else {
-          v[i] = sum[nb][mb][i];
-        }
-      }
-      const u32x2 p2 = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
-      *reinterpret_cast<u32x2*>(out + (size_t)orow * a.N + col) = p2;
-    }
-  }
-}
-
 // ---- any-shape / any-dtype fallback (one thread per output element) ------------------------------
 // Used for fp32 and for shapes the tiled kernel does not take (K % 8 != 0, N % 4 != 0, unaligned
 // pointers).  Correct, not fast.
@@ -1586,38 +786,6 @@ static int launch_dma(GemmArgs a, hipStream_t s) {
   return mi_launch_status();
 }
 
-template <typename T, int BM, int BNW, int WM, int WN, bool GLU, bool WT = false, bool KEEP_PRE = false>
-static int launch_persistent(GemmArgs a, hipStream_t s) {
-  constexpr int BN = GLU ? BNW / 2 : BNW;
-  constexpr int NW = WM * WN;
-  static_assert(BM * BNW * 4 == PERSIST_WS_TILE_BYTES, "size of a partial tile in the workspace");
-  const size_t lds = 4ull * (BM + BNW) * 32 * sizeof(T) + (size_t)a.E * 8;
-  auto kern = grouped_gemm_persistent_kernel<T, BM, BNW, WM, WN, GLU, WT, KEEP_PRE>;
-  static std::atomic<uint64_t> lds_ok{0};  // the expert table makes lds vary with E: opt in to the most it can be
-  int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), MI_LDS_MAX_BYTES, lds_ok);
-  if (rc != MI_MOE_OK) return rc;
-  a.n_tiles = mi_ceil_div(a.N, BN);
-  a.kshift = -1;
-  if (a.kdiv > 0 && (a.kdiv & (a.kdiv - 1)) == 0)
-    for (a.kshift = 0; (1 << a.kshift) < a.kdiv;) ++a.kshift;
-  if (!(a.remap & PERSIST_REMAP_FIXED) && a.n_tiles >= 8) a.remap |= PERSIST_REMAP_INTERLEAVE;  // (see there)
-  int cus = 0;
-  if ((rc = mi_cu_count(&cus)) != MI_MOE_OK) return rc;
-  long max_tiles = ((long)a.L / BM + (a.E < a.L ? a.E : a.L)) * a.n_tiles;
-  long grid = cus < max_tiles ? cus : max_tiles;
-  grid = (grid + 7) / 8 * 8;
-  // no contraction length that a split could shorten by PERSIST_SPLIT_MIN_SAVED slices, or one slot per XCD
-  if (!persistent_may_split(a.K) || grid < 16 || a.pre != nullptr) a.ws = nullptr;  // (the finishing launch writes the result only)
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), lds, s, a);
-  if ((rc = mi_launch_status()) != MI_MOE_OK || a.ws == nullptr) return rc;
-  // the tiles that were cut: at most half of the slots of a round that was split hold tiles (rounded up: an odd
-  // number of slots per XCD)
-  const int nslot = (int)(grid / 8);
-  hipLaunchKernelGGL((grouped_gemm_split_finish_kernel<T, BM, BNW, WM, WN, GLU>), dim3(8u * (unsigned)((nslot + 1) / 2)),
-                     dim3(NW * 64), 0, s, a, nslot);
-  return mi_launch_status();
-}
-
 // fp8 expert weights on the register-staged tiles: out[orow(i)] = scale[e_i] * (in[irow(i)] @ Wq[e_i]^T), with SwiGLU
 // over the [up ; gate] halves when glu.  Called by decode_fp8.hip for batches beyond a few rows per expert (the
 // streaming kernels there read an expert's weights once per 16 of its rows).  Shapes: K % 16 == 0, N % 4 == 0,
@@ -1660,7 +828,7 @@ extern "C" size_t mi_moe_grouped_gemm_workspace_bytes(void) {
 }
 
 extern "C" int mi_moe_grouped_gemm_splits(int K, int dtype) {
-  return (dtype == MI_MOE_BF16 || dtype == MI_MOE_F16) && K > 0 && K % 32 == 0 && persistent_may_split(K);
+  return (dtype == MI_MOE_BF16 || dtype == MI_MOE_F16) && K > 0 && K % 8 == 0 && mi_gemm_persistent_splits(K);
 }
 
 static int check_ws(const void* ws, size_t ws_bytes) {
@@ -1668,10 +836,6 @@ static int check_ws(const void* ws, size_t ws_bytes) {
   const size_t need = mi_moe_grouped_gemm_workspace_bytes();
   if (need == 0 || ws_bytes < need) return MI_MOE_EWORKSPACE;
   return mi_aligned(ws, 16) ? MI_MOE_OK : MI_MOE_EALIGN;
-}
-
-static bool persistent_ok(const GemmArgs& a) {
-  return a.K % 32 == 0 && a.K >= 128 && a.N % 8 == 0 && a.E <= PERSIST_MAX_E && mi_aligned(a.out, 16);
 }
 
 template <typename T, bool GLU>
@@ -1686,7 +850,7 @@ static int launch_naive(GemmArgs a, hipStream_t s) {
 //   0 / 1 / 2  register-staged 256x256 / 128x128 / 32x256 (any K % 8 == 0)
 //   3          one thread per output element (any shape, any dtype)
 //   4          DMA-staged 128x128, one tile per workgroup (K % 32 == 0)
-//   7          persistent DMA-staged 256x256, 8 waves, 32-wide K slices, two wave groups in ping-pong
+//   7 / 8 / 9  persistent 256x256 tiles (persistent_gemm.hip; K % 8 == 0, N % 8 == 0)
 template <typename T, bool GLU>
 static int dispatch_cfg(GemmArgs a, int cfg, hipStream_t s) {
   switch (cfg) {
@@ -1695,13 +859,11 @@ static int dispatch_cfg(GemmArgs a, int cfg, hipStream_t s) {
     case 2: return launch_tiled<T, 32, 256, 1, 4, GLU>(a, s);
     case 5: return launch_tiled<T, 32, 128, 1, 2, GLU>(a, s);
     case 4: return a.K % 32 == 0 ? launch_dma<T, 128, 128, 2, 2, GLU>(a, s) : MI_MOE_EUNSUPPORTED;
-    case 7: return persistent_ok(a) ? launch_persistent<T, 256, 256, 4, 2, GLU>(a, s) : MI_MOE_EUNSUPPORTED;
+    case 7: return mi_gemm_persistent(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, s);
     case 8:  // the persistent kernel with the tile order fixed: XCDs own contiguous ranges ...
-      a.remap |= PERSIST_REMAP_FIXED;
-      return persistent_ok(a) ? launch_persistent<T, 256, 256, 4, 2, GLU>(a, s) : MI_MOE_EUNSUPPORTED;
     case 9:  // ... or take consecutive blocks of one chip-wide round
-      a.remap |= PERSIST_REMAP_FIXED | PERSIST_REMAP_INTERLEAVE;
-      return persistent_ok(a) ? launch_persistent<T, 256, 256, 4, 2, GLU>(a, s) : MI_MOE_EUNSUPPORTED;
+      a.remap |= PERSIST_REMAP_FIXED | (cfg == 9 ? PERSIST_REMAP_INTERLEAVE : 0);
+      return mi_gemm_persistent(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, s);
     default: return MI_MOE_EUNSUPPORTED;
   }
 }
@@ -1732,7 +894,7 @@ static bool tiled_aligned(const GemmArgs& a, int elt_bytes) {
 
 static int pick_cfg(const GemmArgs& a) {
   const long avg = a.E > 0 ? (long)a.L / a.E : a.L;  // rows per expert if the load were uniform
-  if (avg >= 192 && persistent_ok(a)) return 7;
+  if (avg >= 192 && mi_gemm_persistent_ok(a)) return 7;
   if (avg >= 512) return 0;
   if (avg >= 48) return a.K % 32 == 0 ? 4 : 1;
   // A few rows per expert: every weight byte is used once and the kernel is a weight stream, which wants many
@@ -1841,11 +1003,10 @@ extern "C" int mi_moe_scattered_gemm_wt_ws(const void* in, const void* w_kn, voi
   a.L = L; a.K = K; a.N = N; a.E = E; a.kdiv = k; a.n_tiles = 0;
   a.gather = !grouped_in; a.scatter = !grouped_out; a.remap = 1; a.ws = ws; a.pre = nullptr;
   a.out_nt = persistent_out_nt(a, false, 2);
-  if (!tiled_shape_ok(a, L, false, 2) || !persistent_ok(a)) return MI_MOE_EUNSUPPORTED;
+  if (!tiled_shape_ok(a, L, false, 2) || !mi_gemm_persistent_ok(a)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == MI_MOE_BF16) return launch_persistent<bf16_t, 256, 256, 4, 2, false, true>(a, s);
-  return launch_persistent<f16_t, 256, 256, 4, 2, false, true>(a, s);
+  return mi_gemm_persistent(a, dtype, PG_WEIGHT_KN, s);
 }
 
 extern "C" int mi_moe_scattered_gemm_wt(const void* in, const void* w_kn, void* out, const int32_t* sorted_scattered,
@@ -1892,13 +1053,12 @@ extern "C" int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_
   a.gather = 1; a.scatter = 0; a.remap = 1; a.ws = nullptr; a.pre = pre_out;
   // only the persistent kernel writes the pre-activation: shapes it does not take, and loads for which another
   // kernel would be picked, are the caller's two-call path
-  if (!persistent_ok(a) || pick_cfg(a) != 7) return MI_MOE_EUNSUPPORTED;
+  if (!mi_gemm_persistent_ok(a) || pick_cfg(a) != 7) return MI_MOE_EUNSUPPORTED;
   if (!tiled_shape_ok(a, L, true, 2)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
   a.out_nt = 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == MI_MOE_BF16) return launch_persistent<bf16_t, 256, 256, 4, 2, true, false, true>(a, s);
-  return launch_persistent<f16_t, 256, 256, 4, 2, true, false, true>(a, s);
+  return mi_gemm_persistent(a, dtype, PG_SWIGLU_KEEP, s);
 }
 
 extern "C" int mi_moe_up_swiglu_cfg(const void* x, const void* w_fc, void* act_out, const int32_t* sorted_scattered,

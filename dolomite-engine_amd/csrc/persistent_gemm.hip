@@ -1,0 +1,831 @@
+// Persistent grouped GEMM for large expert loads: one workgroup per CU walks a list of 256 x 256 tiles.
+//
+//   out[orow(i), :] = in[irow(i), :] @ W[e_i]^T     for every row i of the expert-sorted order
+//
+// (the scattered_experts op called at lm_engine/hf_models/modeling_utils/mlp_blocks/moe.py:91-101), with the SwiGLU of
+// activations/glu.py:42-43 in the epilogue (GLU), with the pre-activation written next to it for training (KEEP), or
+// with the weights stored (E, K, N) as both data gradients of the backward need them (WT).
+//
+// What bounds it and why it looks like this
+//   * Four waves, ONE per SIMD, each owning a 128 x 128 piece of the tile: 256 accumulators per lane, the whole AGPR
+//     half of the register file.  A K slice of 64 then costs a wave 32 fragment reads for its 128 matrix instructions
+//     (eight waves of 64 x 128 need 48 per 128), the LDS is busy for three quarters of the matrix time and not all of
+//     it, and the chip -- which runs these kernels against its power limit -- spends the difference on clock.
+//   * Operands come to LDS by DMA in whole 128-byte lines (64 values of a row): the same bytes in 64-byte halves
+//     doubled the L2 requests and lost 6 % of the rate.  The DMA is spread evenly over the slice, one instruction per
+//     eight matrix instructions; in two bursts per slice it costs 5 %, in one burst 12 %: an instruction whose
+//     queue is full holds the wave, and with one wave per SIMD that idles the matrix pipe.
+//   * The LDS ring has five units of 32 KB -- the rows of one operand for one slice -- which is all of the LDS: while
+//     slice k is multiplied, slice k + 1 is complete or landing, the activations of slice k + 2 arrive in the fifth
+//     unit, and its weights replace slice k once everybody has read it.  One barrier per slice.
+//   * Fragments are read one half slice ahead into a second register set; every LDS read, DMA instruction and scalar
+//     step sits alone between two matrix instructions (a matrix instruction leaves three free issue slots).
+//   * The accumulators are addressed by number in inline assembly.  As C++ values they are 64 four-register tuples
+//     that fill the AGPR file to the last register, and the compiler moved and spilled them at every tile boundary.
+//     Every phase names all of them as clobbered, so nothing of the compiler's can live there.
+//   * A tile boundary has no barrier: a wave stages its results through the eight 1 KB pieces of the free ring unit
+//     that its own DMA fills next.  The stores stay in flight under the next tile's first slice (they are counted,
+//     vmcnt retires in issue order).  The tile list of a workgroup is decoded once, a lane per tile.
+// Measured (8192 x 8192 x 8192, one expert): the loop runs at 0.94 of the matrix pipe's cycles without DMA; the form it
+// replaces -- eight waves in two groups that alternated between a memory and a matrix phase, 64-byte rows -- reached
+// 0.80 with DMA.
+#include "gemm_common.h"
+
+#include <type_traits>
+
+
+#define PG_BK 64        // K slice: one 128-byte line of a 16-bit row
+#define PG_U 32768      // bytes of a ring unit: 256 rows of one operand (WT weights: 64 rows of 256 columns)
+#define PG_LDS (5 * PG_U)
+#define PG_OOB 0xffffff00u  // byte offset past every buffer: such a lane of the DMA writes zeros
+
+// Splitting the last round along K.  A workgroup's tiles all take the same time, so when the tiles of an XCD do not
+// fill its last round, the workgroups without a tile wait for one tile time.  With a workspace, the `rem` tiles of
+// that round are cut into `parts` = min(slots / rem, PERSIST_SPLIT_MAX) ranges of K slices, one per workgroup; a
+// part writes its fp32 accumulators to the workspace instead of running the epilogue, and a second, small launch
+// (grouped_gemm_split_finish_kernel) adds the parts of every split tile in part order and runs the epilogue, so
+// the result does not depend on timing.  A round is only split if that shortens it by at least
+// PERSIST_SPLIT_MIN_SAVED slices: the partial tiles' trip through memory and the second launch cost 40-80 us
+// (measured), about 50 slices' worth.
+#define PERSIST_SPLIT_MAX 4
+#define PERSIST_SPLIT_MIN_SAVED 60
+#define PERSIST_SPLIT_MIN_SLICES 16
+
+// whether a contraction of length K can be shortened by PERSIST_SPLIT_MIN_SAVED slices at all (launch_persistent
+// applies the same rule, plus one on the grid)
+static bool persistent_may_split(int K) {
+  const int nk = K / PG_BK;
+  return nk - nk / PERSIST_SPLIT_MAX >= PERSIST_SPLIT_MIN_SAVED;
+}
+
+// Which tiles a workgroup runs.  Workgroup b sits on XCD b % 8 (the hardware deals workgroup ids round-robin to the
+// XCDs) in slot b / 8.  Two ways of dealing the band-ordered tile list to them:
+//   * contiguous (the default): XCD x owns the x-th eighth of the list and deals it to its slots in turn, so the
+//     CUs of an XCD work on neighbouring tiles out of one L2 and an XCD stays with its experts;
+//   * interleaved (PERSIST_REMAP_INTERLEAVE): round r of the whole chip is the tiles [r * grid, (r + 1) * grid), XCD
+//     x taking the x-th run of grid / 8 of them.  All XCDs then work on neighbouring tiles at the same time.  When
+//     an expert has more column tiles than a band is wide (intermediate size 14336: 112 column tiles, bands of 8),
+//     consecutive bands read the same activation rows, and the XCDs share them through the memory-side cache
+//     instead of each fetching them from HBM in its own time: Mixtral-shape layer 5.02 -> 4.73 ms.  With few
+//     column tiles (the band is the whole row) it changes little either way (-1.3 % on the Granite-1B shape,
+//     +1.1 % on the Granite-3B shape), so the host asks for it only from 8 column tiles on.
+// Either way the tiles that do not fill the last round can be cut along K (see PERSIST_SPLIT_MAX).
+
+struct SplitPlan {
+  int base, stride;  // tile of this workgroup in round i < full_rounds: base + i * stride
+  int full_rounds;   // rounds in which every slot has a tile
+  int rem;           // tiles of the last round, the first of them being rem_base
+  int rem_base;
+  int parts;         // K ranges each of them is cut into (1: not split)
+  int lslot;         // this workgroup's slot in the last round: part lslot / rem of tile rem_base + lslot % rem
+  int ws_base;       // first partial-tile slot of the last round's tiles in the workspace
+};
+
+// xcd / slot of the workgroup (slot < nslot); for the finishing kernel, slot is the tile of the last round it adds up
+__device__ __forceinline__ SplitPlan persist_split_plan(int total, int xcd, int slot, int nslot, int nk, bool have_ws,
+                                                        bool interleave) {
+  SplitPlan sp;
+  int cap;  // slots that share one last round
+  if (interleave) {
+    cap = nslot * 8;
+    sp.lslot = xcd * nslot + slot;
+    sp.base = sp.lslot;
+    sp.stride = cap;
+    sp.full_rounds = total / cap;
+    sp.rem = total - sp.full_rounds * cap;
+    sp.rem_base = sp.full_rounds * cap;
+    sp.ws_base = 0;
+  } else {
+    cap = nslot;
+    const int per = (total + 7) >> 3;
+    int n_x = total - xcd * per;
+    n_x = n_x < 0 ? 0 : (n_x < per ? n_x : per);
+    sp.lslot = slot;
+    sp.base = xcd * per + slot;
+    sp.stride = nslot;
+    sp.full_rounds = n_x / nslot;
+    sp.rem = n_x - sp.full_rounds * nslot;
+    sp.rem_base = xcd * per + sp.full_rounds * nslot;
+    sp.ws_base = xcd * nslot;
+  }
+  sp.parts = 1;
+  if (have_ws && sp.rem > 0) {
+    int p = cap / sp.rem;
+    if (p > PERSIST_SPLIT_MAX) p = PERSIST_SPLIT_MAX;
+    if (p >= 2 && nk / p >= PERSIST_SPLIT_MIN_SLICES && nk - nk / p >= PERSIST_SPLIT_MIN_SAVED) sp.parts = p;
+  }
+  return sp;
+}
+
+
+#define ALL_AGPRS \
+    "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
+    "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", \
+    "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", \
+    "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", \
+    "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", \
+    "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", \
+    "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", \
+    "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", \
+    "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", \
+    "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", \
+    "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", \
+    "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191", \
+    "a192", "a193", "a194", "a195", "a196", "a197", "a198", "a199", "a200", "a201", "a202", "a203", "a204", "a205", "a206", "a207", \
+    "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", "a222", "a223", \
+    "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", \
+    "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
+
+// ---- the accumulators: a0 .. a255, addressed by number (see the head of the file) -------------------------------
+// Block (nb, mb) of a wave -- 16 weight rows x 16 activation rows -- lives in a[4 (8 mb + nb) ..]: register i of a
+// lane is output column 16 nb + 4 (lane / 16) + i of activation row 16 mb + lane % 16.
+template <typename T> __device__ __forceinline__ void pg_mfma(int acc, u32x4 w, u32x4 x) {
+  if constexpr (std::is_same<T, bf16_t>::value)
+    asm volatile("v_mfma_f32_16x16x32_bf16 a[%0:%1], %2, %3, a[%0:%1]" : : "i"(acc), "i"(acc + 3), "v"(w), "v"(x));
+  else
+    asm volatile("v_mfma_f32_16x16x32_f16 a[%0:%1], %2, %3, a[%0:%1]" : : "i"(acc), "i"(acc + 3), "v"(w), "v"(x));
+}
+// first half slice of a tile: onto zero, so that the accumulators need not be cleared
+template <typename T> __device__ __forceinline__ void pg_mfma_first(int acc, u32x4 w, u32x4 x) {
+  if constexpr (std::is_same<T, bf16_t>::value)
+    asm volatile("v_mfma_f32_16x16x32_bf16 a[%0:%1], %2, %3, 0" : : "i"(acc), "i"(acc + 3), "v"(w), "v"(x));
+  else
+    asm volatile("v_mfma_f32_16x16x32_f16 a[%0:%1], %2, %3, 0" : : "i"(acc), "i"(acc + 3), "v"(w), "v"(x));
+}
+__device__ __forceinline__ float pg_acc(int acc) {
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "i"(acc));
+  return v;
+}
+// (a wait inside the statement: the matrix instructions that wrote a register take up to 19 issue slots to do so)
+__device__ __forceinline__ void pg_acc_settle() { asm volatile("s_nop 15\n\ts_nop 7" : : : "memory", ALL_AGPRS); }
+__device__ __forceinline__ void pg_own_agprs() { asm volatile("" : : : "memory", ALL_AGPRS); }
+
+// ---- DMA: M0 = LDS byte address of the wave's 1 KB piece, then 16 bytes per lane from buffer + lane offset + scalar
+// offset; a lane whose offset lies past the buffer writes zeros.  Inline assembly, because the compiler makes every
+// later LDS read wait for a DMA it knows of; the waits are written by hand here.
+__device__ __forceinline__ void pg_dma_dst(uint32_t lds, int j) {
+  asm volatile("s_add_u32 m0, %0, %1" : : "s"(lds), "i"(j * 4096) : "scc");
+}
+__device__ __forceinline__ void pg_dma(uint32_t off, u32x4 srd, uint32_t soff) {
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(off), "s"(srd), "s"(soff) : "memory");
+}
+__device__ __forceinline__ u32x4 pg_srd(const void* base, uint64_t bytes) {
+  const uint64_t b = (uint64_t)base;
+  const uint32_t n = bytes < (uint64_t)PG_OOB ? (uint32_t)bytes : PG_OOB;
+  return (u32x4){(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, n, 0x00020000u};
+}
+__device__ __forceinline__ constexpr int pg_wait(int vm, int lgkm) {
+  // gfx9 encoding: vmcnt = {imm[15:14], imm[3:0]}, expcnt = imm[6:4] (7 = no wait), lgkmcnt = imm[11:8]
+  return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8);
+}
+#define PG_SCHED() __builtin_amdgcn_sched_barrier(0)
+
+struct PgTile {
+  int expert, nt, row_begin, row_end;
+};
+
+// The tile list of one workgroup, a lane per tile (64 tiles at a time).  A lane of the four table registers holds an
+// expert: row tiles of experts 0..e and the end of its rows.  An expert's tiles are numbered band by band: a band is
+// up to 8 column tiles wide and runs over all of the expert's row tiles, row tile slowest.  The 32 workgroups of an
+// XCD, which take 32 consecutive tiles at a time, then cover about 4 row tiles x 8 column tiles: 12 operand slabs for
+// 32 tiles, and each weight slab is fetched once per band instead of once per row tile.  Up to 8 column tiles the
+// band is the whole row, so that complete output rows are written at about the same time.
+struct PgTable {
+  int incl[4], end[4];
+  int total;  // row tiles of all experts
+};
+template <int BM> __device__ __forceinline__ void pg_table(const int32_t* __restrict__ off, int E, PgTable& tb) {
+  const int lane = threadIdx.x & 63;
+  int carry = 0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    tb.incl[c] = 0;
+    tb.end[c] = 0;
+    if (c * 64 >= E) continue;
+    const int e = c * 64 + lane;
+    const int end = e < E ? off[e] : 0;
+    const int prev = (e < E && e > 0) ? off[e - 1] : 0;
+    int incl = e < E ? (end - prev + BM - 1) / BM : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    tb.incl[c] = incl + carry;
+    tb.end[c] = end;
+    carry += __builtin_amdgcn_readlane(incl, 63);
+  }
+  tb.total = carry;
+}
+template <int BM> __device__ __forceinline__ PgTile pg_locate(const PgTable& tb, int E, int n_tiles, int tile) {
+  const int q = tile / n_tiles;  // experts own contiguous tile ranges: (row tiles before) * n_tiles
+  int ex = 0, first = 0, prev = 0, incl = 0x7fffffff, rend = 0x7fffffff;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int n = E - c * 64 < 64 ? E - c * 64 : 64;
+    for (int l = 0; l < n; ++l) {
+      const int s = __builtin_amdgcn_readlane(tb.incl[c], l), en = __builtin_amdgcn_readlane(tb.end[c], l);
+      const bool past = q >= s;
+      ex += past ? 1 : 0;
+      first = past ? s : first;
+      prev = past ? en : prev;
+      incl = past ? incl : (s < incl ? s : incl);
+      rend = past ? rend : (en < rend ? en : rend);
+    }
+  }
+  const int tile_band = n_tiles < 8 ? n_tiles : 8;
+  const int local = tile - first * n_tiles, per_band = (incl - first) * tile_band;
+  const int band = local / per_band;
+  const int rem = local - band * per_band;
+  const int left = n_tiles - band * tile_band;
+  const int width = left < tile_band ? left : tile_band;
+  const int mt = rem / width;
+  PgTile t;
+  t.expert = ex;
+  t.nt = band * tile_band + rem - mt * width;
+  t.row_begin = prev + mt * BM;
+  t.row_end = rend;
+  return t;
+}
+
+template <typename T, bool GLU, bool WT, bool KEEP>
+__global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArgs a) {
+  static_assert(!KEEP || GLU, "the pre-activation belongs to the SwiGLU form");
+  static_assert(!WT || !GLU, "transposed-weight form");
+  constexpr int BM = 256;
+  constexpr int BN = GLU ? 128 : 256;               // output columns per tile
+  constexpr int NSTORE = KEEP ? 48 : (GLU ? 16 : 32);  // stores of a wave in the epilogue of an interior tile
+  typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
+  typedef short tr_s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) tr_s16x4* tr_ptr_t;
+
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const uint32_t lds0 = (uint32_t)(size_t)(lds_ptr_t)smem_raw;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1;          // 128 activation rows, 128 weight rows (SwiGLU: 64 up, 64 gate)
+  const int frow = lane & 15, fq = lane >> 4;       // fragment: row frow, k = 8 fq + [0, 8) of the half slice
+
+  // ---- which tiles -----------------------------------------------------------------------------------------------
+  PgTable tb;
+  pg_table<BM>(a.expert_offsets, a.E, tb);
+  const int total = tb.total * a.n_tiles;
+  const int nfull = a.K / PG_BK;                    // whole slices; a partial one is padded with zeros
+  int nk = (a.K + PG_BK - 1) / PG_BK;
+  if (nk < 2) nk = 2;                               // (the ring wants two: a second slice of zeros)
+  const SplitPlan sp = persist_split_plan(total, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, nk, a.ws != nullptr,
+                                          (a.remap & PERSIST_REMAP_INTERLEAVE) != 0);
+  const int my_part = sp.parts > 1 ? sp.lslot / sp.rem : 0, my_rem_tile = sp.rem > 0 ? sp.lslot % sp.rem : 0;
+  const int n_items = sp.full_rounds + (sp.lslot < sp.rem * sp.parts ? 1 : 0);
+  if (n_items == 0) return;
+  // K slices [k0, k1) of item i
+  auto item_k = [&](int i, int& k0, int& k1) {
+    const bool part = i == sp.full_rounds && sp.parts > 1;
+    k0 = part ? my_part * nk / sp.parts : 0;
+    k1 = part ? (my_part + 1) * nk / sp.parts : nk;
+  };
+  PgTile list;                                      // lane l: item (64-item block) + l
+  auto fetch = [&](int i) -> PgTile {               // called with i = 0, 1, 2, ...; past the last item: the last item
+    if (i >= n_items) i = n_items - 1;
+    else if ((i & 63) == 0) {
+      const int it = i + lane;
+      const int tile = it < sp.full_rounds ? sp.base + it * sp.stride : sp.rem_base + my_rem_tile;
+      list = pg_locate<BM>(tb, a.E, a.n_tiles, it < n_items ? tile : 0);
+    }
+    const int l = i & 63;
+    PgTile t;
+    t.expert = __builtin_amdgcn_readlane(list.expert, l);
+    t.nt = __builtin_amdgcn_readlane(list.nt, l);
+    t.row_begin = __builtin_amdgcn_readlane(list.row_begin, l);
+    t.row_end = __builtin_amdgcn_readlane(list.row_end, l);
+    return t;
+  };
+
+  // ---- DMA sources ---------------------------------------------------------------------------------------------------
+  // Unit image: row r of 128 bytes keeps its 16-byte chunks at slots chunk ^ ((r >> 1) & 7), which serves the 16 rows x
+  // 4 chunks of a fragment without bank conflicts.  Instruction j of a wave fills rows 8 (4 j + wave) .. + 8 in lane
+  // order, so the swizzle is applied on the global side: lane l fetches chunk (l % 8) ^ ((r >> 1) & 7).
+  const int drow = wave * 8 + (lane >> 3);          // row of instruction 0 (instruction j: + 32 j)
+  const int lchunk = (lane & 7) ^ ((wave & 1) * 4 + (lane >> 4));
+  const uint32_t row_bytes = (uint32_t)a.K * 2u;
+  const u32x4 xsrd = pg_srd(a.in, (uint64_t)(a.gather ? a.L / a.kdiv : a.L) * row_bytes);
+  const uint64_t w_bytes = (uint64_t)a.E * (GLU ? 2 : 1) * a.N * row_bytes;
+  auto make_wsrd = [&](const PgTile& t) -> u32x4 {
+    const uint64_t o = ((uint64_t)t.expert * (GLU ? 2 : 1) * a.N * a.K + (uint64_t)t.nt * BN * (WT ? 1 : a.K)) * 2u;
+    return pg_srd(static_cast<const unsigned char*>(a.w) + o, w_bytes - o);
+  };
+  // sorted-order row index of the activation rows a lane fetches (clamped into the tile's expert: rows past its end
+  // are never stored), and the byte offsets they give
+  auto load_rows = [&](const PgTile& t, int (&raw)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = t.row_begin + drow + 32 * j;
+      raw[j] = r < t.row_end ? r : t.row_end - 1;
+    }
+    if (a.gather) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) raw[j] = a.sorted_scattered[raw[j]];
+    }
+  };
+  auto make_xoff = [&](const int (&raw)[8], uint32_t (&off)[8]) {
+    // (top-k is a power of two in most configurations: a shift instead of a division)
+    const int sh = !a.gather ? 0 : a.kshift;
+    if (sh >= 0) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) off[j] = (uint32_t)(raw[j] >> sh) * row_bytes + lchunk * 16u;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) off[j] = (uint32_t)(raw[j] / a.kdiv) * row_bytes + lchunk * 16u;
+    }
+  };
+  // Weight rows are at fixed distances (rows past N are another matrix's, or past the buffer: never stored).
+  // WT: instruction j fills rows 8 j + 2 wave + lane / 32 of the slice; 16-byte piece l % 32 of row r holds the logical
+  // piece whose 32-byte group is (piece / 2) ^ (r % 4 | (r / 8 % 4) << 2): the swizzle the transposing reads expect.
+  uint32_t woff[8];
+  auto make_woff = [&]() {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (WT) {
+        const int r = 8 * j + 2 * wave + (lane >> 5), f = (r & 3) | ((j & 3) << 2);
+        woff[j] = ((uint32_t)r * a.N + ((((lane & 31) >> 1) ^ f) << 4) + (lane & 1) * 8) * 2u;
+      } else {
+        const int r = GLU ? 32 * (j & 3) + (j >= 4 ? a.N : 0) : 32 * j;
+        woff[j] = (uint32_t)(r + drow) * row_bytes + lchunk * 16u;
+      }
+    }
+  };
+  const uint32_t w_step = WT ? (uint32_t)a.N * (2u * PG_BK) : 2u * PG_BK;  // bytes from slice to slice
+  // a slice with fewer than 64 values: the lanes past them fetch zeros
+  auto mask_x = [&](uint32_t (&off)[8], int k) {
+    const bool gone = lchunk * 8 >= a.K - k * PG_BK;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) off[j] = gone ? PG_OOB : off[j];
+  };
+  auto mask_w = [&](int k) {
+    if constexpr (WT) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) woff[j] = 8 * j + 2 * wave + (lane >> 5) >= a.K - k * PG_BK ? PG_OOB : woff[j];
+    } else {
+      mask_x(woff, k);
+    }
+  };
+
+  // ---- fragment reads ------------------------------------------------------------------------------------------------
+  const uint32_t fswz = (frow >> 1) & 7;
+  const uint32_t fx = (wm * 128 + frow) * 128, fw = (wn * (GLU ? 64 : 128) + frow) * 128;
+  const uint32_t fc0 = lds0 + ((fq ^ fswz) * 16), fc1 = lds0 + (((fq + 4) ^ fswz) * 16);
+  // WT: ds_read_b64_tr_b16 transposes 4 rows x 16 columns across 16 lanes: lane i of the group supplies the address of
+  // (row i / 4, columns 4 (i % 4) ..) and receives column i of the four rows.  Lane group q reads rows 8q .. 8q + 3 and,
+  // 2 KiB further, 8q + 4 .. 8q + 7: together the 8 contraction values the matrix instruction wants.
+  const uint32_t trb = (8 * fq + (frow >> 2)) * 512 + ((((frow >> 2) | (fq << 2))) << 5) + (frow & 3) * 8;
+  u32x4 wf[2][8], xf[2][8];
+  auto read_w = [&](uint32_t base, int ks, int nb) -> u32x4 {
+    if constexpr (WT) {
+      const uint32_t ad = base + (trb ^ ((uint32_t)(wn * 8 + nb) << 5));
+      const tr_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(size_t)(ad + ks * 16384));
+      const tr_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(size_t)(ad + ks * 16384 + 2048));
+      return __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    } else {
+      typedef __attribute__((address_space(3))) const u32x4* p;
+      return *(p)(size_t)(base + (GLU && nb >= 4 ? 16384 + (nb - 4) * 2048 : nb * 2048));
+    }
+  };
+  auto read_x = [&](uint32_t base, int mb) -> u32x4 {
+    typedef __attribute__((address_space(3))) const u32x4* p;
+    return *(p)(size_t)(base + mb * 2048);
+  };
+
+  // ---- ring and source state ------------------------------------------------------------------------------------------
+  // Slots of X_k, W_k, X_k+1, W_k+1 and the free one (X_k+2; then W_k+2 goes to the slot of X_k); X = activations.
+  uint32_t p0 = 0, p1 = PG_U, p2 = 2 * PG_U, p3 = 3 * PG_U, p4 = 4 * PG_U;
+  uint32_t xoff[8], xoff_n[8];
+  u32x4 wsrd, wsrd_n;
+  int kx, kx_end, kx_ev, kw, kw_end, kw_ev;         // next slice of the source tile, its end, the next one with an event
+  int k0_n, k1_n;                                   // slices of the next item
+  auto event_of = [&](int end) { return nfull < end ? nfull : end; };
+  auto x_event = [&]() {
+    if (kx == kx_end) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) xoff[j] = xoff_n[j];
+      kx = k0_n;
+      kx_end = k1_n;
+    }
+    if (kx >= nfull) mask_x(xoff, kx);
+    kx_ev = event_of(kx_end);
+  };
+  auto w_event = [&]() {
+    if (kw == kw_end) {
+      wsrd = wsrd_n;
+      if (nfull != nk) make_woff();
+      kw = k0_n;
+      kw_end = k1_n;
+    }
+    if (kw >= nfull) mask_w(kw);
+    kw_ev = event_of(kw_end);
+  };
+
+  // One half slice: 64 matrix instructions.  B = 0: values [0, 32) of slice k out of the registers read before, while
+  // values [32, 64) are read and X_k+2 is fetched; B = 1: those, while slice k + 1 is read and W_k+2 is fetched.
+  // `hook(m)` runs after matrix instruction m.
+  const uint32_t dma0 = lds0 + wave * 1024;
+  uint32_t rw, rx;                                  // addresses of the next half's fragments
+  auto half = [&](auto btag, auto ftag, uint32_t dst, auto hook) {
+    constexpr int B = decltype(btag)::value;
+    constexpr bool FIRST = decltype(ftag)::value;
+    const uint32_t soff = B ? (uint32_t)kw * w_step : (uint32_t)kx * (2u * PG_BK);
+    pg_own_agprs();
+#pragma unroll
+    for (int m = 0; m < 64; ++m) {
+      const int nb = m & 7, mb = m >> 3;
+      if constexpr (FIRST) pg_mfma_first<T>((mb * 8 + nb) * 4, wf[B][nb], xf[B][mb]);
+      else pg_mfma<T>((mb * 8 + nb) * 4, wf[B][nb], xf[B][mb]);
+      if (m % 2 == 0 && m < 32) {
+        const int q = m / 2;
+        PG_SCHED();
+        if (q < 8) wf[B ^ 1][q] = read_w(rw, B ^ 1, q);
+        else xf[B ^ 1][q - 8] = read_x(rx, q - 8);
+        PG_SCHED();
+      }
+      if (m % 8 == 1) {
+        PG_SCHED();
+        pg_dma_dst(dst, m / 8);
+        PG_SCHED();
+      }
+      if (m % 8 == 3) {
+        PG_SCHED();
+        pg_dma(B ? woff[m / 8] : xoff[m / 8], B ? wsrd : xsrd, soff);
+        PG_SCHED();
+      }
+      hook(m);
+    }
+  };
+  auto read_bases = [&](int ks, uint32_t ps_w, uint32_t ps_x) {
+    rw = WT ? lds0 + ps_w : (ks ? fc1 : fc0) + fw + ps_w;
+    rx = (ks ? fc1 : fc0) + fx + ps_x;
+    asm volatile("" : "+v"(rx));
+    if constexpr (!WT) asm volatile("" : "+v"(rw));
+  };
+  // stores_after_dma: the epilogue of an interior tile lies between the DMA this slice waits for and now
+  auto step = [&](auto ftag, bool stores_after_dma) {
+    if (kx >= kx_ev) x_event();
+    half(std::integral_constant<int, 0>{}, ftag, dma0 + p4, [&](int m) {
+      if (m == 62) {
+        PG_SCHED();
+        ++kx;
+        read_bases(0, p3, p2);
+        PG_SCHED();
+      }
+    });
+    // slice k + 1 has landed (X_k+2 stays in flight); slice k is in everybody's registers
+    if (decltype(ftag)::value && stores_after_dma) __builtin_amdgcn_s_waitcnt(pg_wait(8 + NSTORE, 0));
+    else __builtin_amdgcn_s_waitcnt(pg_wait(8, 0));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    PG_SCHED();
+    if (kw >= kw_ev) w_event();
+    half(std::integral_constant<int, 1>{}, std::false_type{}, dma0 + p0, [&](int m) {
+      if (m == 62) ++kw;
+      if (m == 60) {
+        PG_SCHED();
+        const uint32_t t0 = p0, t1 = p1;
+        p0 = p2;
+        p1 = p3;
+        p2 = p4;
+        p3 = t0;
+        p4 = t1;
+        asm volatile("" : "+s"(p0), "+s"(p1), "+s"(p2), "+s"(p3), "+s"(p4));
+        PG_SCHED();
+      }
+      if (m == 62) {
+        PG_SCHED();
+        read_bases(1, p1, p0);
+        PG_SCHED();
+      }
+    });
+  };
+
+  // ---- epilogue: accumulators -> (SwiGLU) -> the wave's pieces of the free ring unit -> 16-byte stores ------------------
+  // Plain: four passes of 32 rows x 128 columns (256-byte rows, 4 to a piece); SwiGLU: two of 64 rows x 64 columns.
+  // Chunk c of scratch row r lies at slot c ^ (r % 16) (SwiGLU: c ^ (r / 2 % 8)): writes and reads free of conflicts,
+  // and the read-back is linear in the lane.
+  T* __restrict__ out = static_cast<T*>(a.out);
+  constexpr int SB = GLU ? 128 : 256;               // bytes of a scratch row
+  constexpr int RPP = 1024 / SB;                    // scratch rows per piece and per store instruction
+  constexpr int PASS_ROWS = 8 * RPP, NPASS = 128 / PASS_ROWS, MBP = PASS_ROWS / 16, NBO = GLU ? 4 : 8;
+  const uint32_t scr_swz = GLU ? (frow >> 1) & 7 : frow;
+  const uint32_t scr_w = (frow / RPP) * 4096 + (frow % RPP) * SB + (((fq >> 1) ^ scr_swz) * 16) + (fq & 1) * 8;
+  const int srow = lane / (SB / 16), sslot = lane % (SB / 16);
+  const int scc0 = GLU ? sslot ^ ((srow >> 1) & 7) : sslot ^ (srow & 15);  // chunk of store 0; store it: ^ 4 (it % ..)
+  int orow_lo, orow_hi;                             // output rows of the wave's rows lane and 64 + lane
+  auto load_out_rows = [&](const PgTile& t, int& lo, int& hi) {
+    const int r0 = t.row_begin + wm * 128 + lane;
+    lo = r0;
+    hi = r0 + 64;
+    if (a.scatter) {
+      lo = a.sorted_scattered[lo < t.row_end ? lo : t.row_end - 1];
+      hi = a.sorted_scattered[hi < t.row_end ? hi : t.row_end - 1];
+    }
+  };
+  // WHAT: 0 the kernel's result (SwiGLU: up * silu(gate)); 1 / 2 (KEEP): the up / the gate half of h, into a.pre.  KEEP
+  // forms the result from the ROUNDED halves, as the separate activation kernel forms it from the stored h.
+  auto epilogue_as = [&](auto what_tag, auto interior_tag, auto nt_tag, const PgTile& t) {
+    constexpr int WHAT = decltype(what_tag)::value;
+    constexpr bool INTERIOR = decltype(interior_tag)::value, NT = decltype(nt_tag)::value;
+    typedef __attribute__((address_space(3))) u32x2* wp_t;
+    typedef __attribute__((address_space(3))) const u32x4* rp_t;
+    unsigned char* dst = reinterpret_cast<unsigned char*>(WHAT == 0 ? out : static_cast<T*>(a.pre));
+    const uint32_t ld = (WHAT == 0 ? a.N : 2 * a.N) * 2u;
+    const uint32_t s0 = dma0 + p4;
+    const int col0 = t.nt * BN + wn * (GLU ? 64 : 128);
+#pragma unroll
+    for (int p = 0; p < NPASS; ++p) {
+#pragma unroll
+      for (int mbp = 0; mbp < MBP; ++mbp)
+#pragma unroll
+        for (int nb = 0; nb < NBO; ++nb) {
+          const int blk = (p * MBP + mbp) * 8 + nb;
+          float v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (WHAT == 1) {
+              v[i] = pg_acc(blk * 4 + i);
+            } else if (WHAT == 2) {
+              v[i] = pg_acc((blk + 4) * 4 + i);
+            } else if (GLU) {
+              float up = pg_acc(blk * 4 + i), gt = pg_acc((blk + 4) * 4 + i);
+              if (KEEP) {
+                up = Elt<T>::round(up);
+                gt = Elt<T>::round(gt);
+              }
+              v[i] = up * gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
+            } else {
+              v[i] = pg_acc(blk * 4 + i);
+            }
+          }
+          *(wp_t)(size_t)(s0 + (scr_w ^ (nb * 32)) + mbp * (16 / RPP) * 4096) =
+              (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+        }
+      asm volatile("" ::: "memory");
+      // (four at a time: one LDS latency for all of them)
+#pragma unroll
+      for (int it0 = 0; it0 < 8; it0 += 4) {
+        u32x4 val[4];
+        int orow[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int r = p * PASS_ROWS + (it0 + j) * RPP;  // + srow: row of the wave's 128
+          val[j] = *(rp_t)(size_t)(s0 + (it0 + j) * 4096 + lane * 16);
+          orow[j] = __builtin_amdgcn_ds_bpermute(((r & 63) + srow) * 4, r < 64 ? orow_lo : orow_hi);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int it = it0 + j;
+          const int row = t.row_begin + wm * 128 + p * PASS_ROWS + it * RPP + srow;
+          const int col = col0 + (scc0 ^ (GLU ? 4 * (it & 1) : 4 * (it & 3))) * 8;
+          if (INTERIOR || (row < t.row_end && col < a.N)) {
+            u32x4* q = reinterpret_cast<u32x4*>(dst + (uint64_t)(uint32_t)orow[j] * ld + (uint32_t)((WHAT == 2 ? a.N : 0) + col) * 2u);
+            if constexpr (NT) __builtin_nontemporal_store(val[j], q);
+            else *q = val[j];
+          }
+        }
+      }
+      asm volatile("" ::: "memory");
+    }
+  };
+  typedef std::integral_constant<int, 0> what_result;
+  typedef std::integral_constant<int, 1> what_up;
+  typedef std::integral_constant<int, 2> what_gate;
+  auto epilogue = [&](const PgTile& t, bool interior) {
+    if constexpr (KEEP) {
+      // the activation and both halves of the pre-activation (plain stores: the backward reads them again)
+      if (interior) {
+        epilogue_as(what_result{}, std::true_type{}, std::false_type{}, t);
+        epilogue_as(what_up{}, std::true_type{}, std::false_type{}, t);
+        epilogue_as(what_gate{}, std::true_type{}, std::false_type{}, t);
+      } else {
+        epilogue_as(what_result{}, std::false_type{}, std::false_type{}, t);
+        epilogue_as(what_up{}, std::false_type{}, std::false_type{}, t);
+        epilogue_as(what_gate{}, std::false_type{}, std::false_type{}, t);
+      }
+    } else if (interior) {
+      if (a.out_nt) epilogue_as(what_result{}, std::true_type{}, std::true_type{}, t);
+      else epilogue_as(what_result{}, std::true_type{}, std::false_type{}, t);
+    } else {
+      if (a.out_nt) epilogue_as(what_result{}, std::false_type{}, std::true_type{}, t);
+      else epilogue_as(what_result{}, std::false_type{}, std::false_type{}, t);
+    }
+  };
+  // a part of a split tile: accumulators -> workspace, block b of thread t at [b][t]
+  auto store_part = [&]() {
+    f32x4* base = static_cast<f32x4*>(a.ws) +
+                  ((size_t)sp.ws_base + (size_t)my_rem_tile * sp.parts + my_part) * (64 * 256) + threadIdx.x;
+#pragma unroll
+    for (int b = 0; b < 64; ++b) {
+      const f32x4 v = {pg_acc(4 * b), pg_acc(4 * b + 1), pg_acc(4 * b + 2), pg_acc(4 * b + 3)};
+      base[b * 256] = v;
+    }
+  };
+
+  // ---- prologue -----------------------------------------------------------------------------------------------------------
+  PgTile cur = fetch(0), nxt = fetch(1);
+  int k0, k1;
+  item_k(0, k0, k1);
+  {
+    int raw[8], raw_n[8];
+    load_rows(cur, raw);
+    load_rows(nxt, raw_n);
+    load_out_rows(cur, orow_lo, orow_hi);
+    make_xoff(raw, xoff);
+    make_xoff(raw_n, xoff_n);
+  }
+  make_woff();
+  wsrd = make_wsrd(cur);
+  wsrd_n = make_wsrd(nxt);
+  item_k(n_items > 1 ? 1 : 0, k0_n, k1_n);
+  asm volatile("" : "+v"(orow_lo), "+v"(orow_hi));
+  __builtin_amdgcn_s_waitcnt(pg_wait(0, 0));
+  kx = kw = k0;
+  kx_end = kw_end = k1;
+  kx_ev = kw_ev = event_of(k1);
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    if (kx >= nfull) mask_x(xoff, kx);
+    if (kw >= nfull) mask_w(kw);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      pg_dma_dst(dma0 + (s ? p2 : p0), j);
+      asm volatile("s_nop 0");
+      pg_dma(xoff[j], xsrd, (uint32_t)kx * (2u * PG_BK));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      pg_dma_dst(dma0 + (s ? p3 : p1), j);
+      asm volatile("s_nop 0");
+      pg_dma(woff[j], wsrd, (uint32_t)kw * w_step);
+    }
+    ++kx;
+    ++kw;
+  }
+  __builtin_amdgcn_s_waitcnt(pg_wait(16, 0));
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read_bases(0, p1, p0);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) wf[0][i] = read_w(rw, 0, i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) xf[0][i] = read_x(rx, i);
+  read_bases(1, p1, p0);
+
+  // ---- tile loop ------------------------------------------------------------------------------------------------------------
+  bool stores_pending = false;
+  for (int i = 0;; ++i) {
+    step(std::true_type{}, stores_pending);
+    for (int k = k0 + 1; k < k1; ++k) step(std::false_type{}, false);
+    pg_acc_settle();
+    if (k1 - k0 != nk) {
+      // a part of a split tile, always a workgroup's last item: the finishing launch adds the parts up
+      store_part();
+      break;
+    }
+    // rows of the tile after next, and where the next tile's results go: requested here, taken after the epilogue
+    const PgTile after = fetch(i + 2);
+    int raw[8], lo_n, hi_n;
+    load_rows(after, raw);
+    load_out_rows(nxt, lo_n, hi_n);
+    const bool interior = cur.row_begin + BM <= cur.row_end && (cur.nt + 1) * BN <= a.N;
+    epilogue(cur, interior);
+    if (i + 1 >= n_items) break;
+    stores_pending = interior;
+    make_xoff(raw, xoff_n);
+    wsrd_n = make_wsrd(after);
+    orow_lo = lo_n;
+    orow_hi = hi_n;
+    k0 = k0_n;
+    k1 = k1_n;
+    if (i + 2 < n_items) item_k(i + 2, k0_n, k1_n);  // (else: surplus DMA re-reads the last item's first slices)
+    cur = nxt;
+    nxt = after;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(xoff_n[j]));  // (the waits for the loads above belong here)
+    asm volatile("" : "+v"(orow_lo), "+v"(orow_hi));
+  }
+  __builtin_amdgcn_s_waitcnt(pg_wait(0, 0));  // surplus DMA must not outlive the workgroup's LDS
+}
+
+// The tiles the persistent kernel cut along K (see PERSIST_SPLIT_MAX): one workgroup per (XCD, tile of its last round)
+// and quarter of the accumulator blocks recomputes the same plan, adds the tile's partial accumulators in part order
+// and writes them the way the persistent kernel's epilogue does (same arithmetic, same rounding; thread t holds what
+// thread t of a part held).  Workgroups whose tile does not exist or was not split return at once.
+template <typename T, bool GLU>
+__global__ __launch_bounds__(256) void grouped_gemm_split_finish_kernel(GemmArgs a, int nslot) {
+  constexpr int BM = 256, BN = GLU ? 128 : 256;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
+  PgTable tb;
+  pg_table<BM>(a.expert_offsets, a.E, tb);
+  // contiguous: workgroup b adds up tile b / 8 of XCD b % 8's last round; interleaved: tile b of the chip's last round
+  const bool interleave = (a.remap & PERSIST_REMAP_INTERLEAVE) != 0;
+  const int xcd = interleave ? 0 : (int)(blockIdx.x & 7), j = interleave ? (int)blockIdx.x : (int)(blockIdx.x >> 3);
+  const SplitPlan sp = persist_split_plan(tb.total * a.n_tiles, xcd, 0, nslot, (a.K + PG_BK - 1) / PG_BK, true, interleave);
+  if (sp.parts == 1 || j >= sp.rem) return;
+  const PgTile t = pg_locate<BM>(tb, a.E, a.n_tiles, sp.rem_base + j);
+
+  constexpr int MBS = 2;  // row blocks of this workgroup: 2 q, 2 q + 1
+  const int q = blockIdx.y;
+  const f32x4* part = static_cast<const f32x4*>(a.ws) + ((size_t)sp.ws_base + (size_t)j * sp.parts) * (64 * 256) +
+                      q * (MBS * 8 * 256) + tid;
+  f32x4 sum[MBS * 8];
+#pragma unroll
+  for (int b = 0; b < MBS * 8; ++b) sum[b] = __builtin_nontemporal_load(part + b * 256);
+  for (int p = 1; p < sp.parts; ++p) {
+    part += 64 * 256;
+#pragma unroll
+    for (int b = 0; b < MBS * 8; ++b) {
+      const f32x4 v = __builtin_nontemporal_load(part + b * 256);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) sum[b][c] += v[c];
+    }
+  }
+  const int frow = lane & 15, fq = lane >> 4;
+  T* __restrict__ out = static_cast<T*>(a.out);
+#pragma unroll
+  for (int mb = 0; mb < MBS; ++mb) {
+    const int row = t.row_begin + wm * 128 + (q * MBS + mb) * 16 + frow;
+    if (row >= t.row_end) continue;
+    const int orow = a.scatter ? a.sorted_scattered[row] : row;
+#pragma unroll
+    for (int nb = 0; nb < (GLU ? 4 : 8); ++nb) {
+      const int col = t.nt * BN + wn * (GLU ? 64 : 128) + nb * 16 + fq * 4;
+      if (col >= a.N) continue;
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float up = sum[mb * 8 + nb][i];
+        if (GLU) {
+          const float gt = sum[mb * 8 + nb + 4][i];
+          v[i] = up * gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
+        } else {
+          v[i] = up;
+        }
+      }
+      const u32x2 p2 = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+      *reinterpret_cast<u32x2*>(out + (size_t)orow * a.N + col) = p2;
+    }
+  }
+}
+
+// ---- host side ----------------------------------------------------------------------------------------------------------------
+template <typename T, bool GLU, bool WT, bool KEEP>
+static int launch_persistent(GemmArgs a, hipStream_t s) {
+  constexpr int BM = 256, BN = GLU ? 128 : 256;
+  auto kern = grouped_gemm_persistent_kernel<T, GLU, WT, KEEP>;
+  static std::atomic<uint64_t> lds_ok{0};
+  int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), PG_LDS, lds_ok);
+  if (rc != MI_MOE_OK) return rc;
+  a.n_tiles = mi_ceil_div(a.N, BN);
+  a.kshift = -1;
+  if (a.kdiv > 0 && (a.kdiv & (a.kdiv - 1)) == 0)
+    for (a.kshift = 0; (1 << a.kshift) < a.kdiv;) ++a.kshift;
+  if (!(a.remap & PERSIST_REMAP_FIXED) && a.n_tiles >= 8) a.remap |= PERSIST_REMAP_INTERLEAVE;  // (see there)
+  int cus = 0;
+  if ((rc = mi_cu_count(&cus)) != MI_MOE_OK) return rc;
+  const long max_tiles = ((long)a.L / BM + (a.E < a.L ? a.E : a.L)) * a.n_tiles;
+  long grid = cus < max_tiles ? cus : max_tiles;
+  grid = (grid + 7) / 8 * 8;
+  // no contraction length that a split could shorten by PERSIST_SPLIT_MIN_SAVED slices, or one slot per XCD
+  if (!mi_gemm_persistent_splits(a.K) || grid < 16 || a.pre != nullptr) a.ws = nullptr;  // (the finishing launch writes the result only)
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), PG_LDS, s, a);
+  if ((rc = mi_launch_status()) != MI_MOE_OK || a.ws == nullptr) return rc;
+  // the tiles that were cut: at most half of the slots of a round that was split hold tiles (rounded up: an odd
+  // number of slots per XCD)
+  const int nslot = (int)(grid / 8);
+  hipLaunchKernelGGL((grouped_gemm_split_finish_kernel<T, GLU>), dim3(8u * (unsigned)((nslot + 1) / 2), 4), dim3(256), 0, s, a,
+                     nslot);
+  return mi_launch_status();
+}
+
+bool mi_gemm_persistent_splits(int K) { return persistent_may_split(K); }
+
+bool mi_gemm_persistent_ok(const GemmArgs& a) {
+  return a.K % 8 == 0 && a.N % 8 == 0 && a.E <= PERSIST_MAX_E && mi_aligned(a.out, 16);
+}
+
+int mi_gemm_persistent(const GemmArgs& a, int dtype, int form, hipStream_t s) {
+  if (!mi_gemm_persistent_ok(a)) return MI_MOE_EUNSUPPORTED;
+  if (dtype == MI_MOE_BF16) {
+    switch (form) {
+      case PG_PLAIN: return launch_persistent<bf16_t, false, false, false>(a, s);
+      case PG_SWIGLU: return launch_persistent<bf16_t, true, false, false>(a, s);
+      case PG_SWIGLU_KEEP: return launch_persistent<bf16_t, true, false, true>(a, s);
+      case PG_WEIGHT_KN: return launch_persistent<bf16_t, false, true, false>(a, s);
+    }
+  } else if (dtype == MI_MOE_F16) {
+    switch (form) {
+      case PG_PLAIN: return launch_persistent<f16_t, false, false, false>(a, s);
+      case PG_SWIGLU: return launch_persistent<f16_t, true, false, false>(a, s);
+      case PG_SWIGLU_KEEP: return launch_persistent<f16_t, true, false, true>(a, s);
+      case PG_WEIGHT_KN: return launch_persistent<f16_t, false, true, false>(a, s);
+    }
+  }
+  return MI_MOE_EDTYPE;
+}

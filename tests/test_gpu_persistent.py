@@ -1,0 +1,54 @@
+"""The persistent grouped GEMM at the sizes where its tiles, slices and tile list can go wrong: contractions shorter than
+a slice, of exactly one or two slices and with every kind of partial last slice, expert sizes around the 256-row tile,
+output columns around the 256- and 128-column tiles, experts without rows, more tiles than one block of a workgroup's
+tile list holds.  Against an fp32 product of the same rounded operands: fp32 accumulation leaves the one rounding of the
+result, half a unit in the last place (2^-9 of the value in bf16, 2^-12 in fp16), plus the reordering error of the fp32
+sum, far below the absolute term for these magnitudes."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.bfloat16: dict(rtol=2.0 ** -8, atol=2e-3), torch.float16: dict(rtol=2.0 ** -11, atol=5e-4)}
+
+
+def _reference(x, w, counts):
+    return torch.cat([p.float() @ w[e].float().t() for e, p in enumerate(x.split(counts))])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,K,N", [
+    ([300, 20], 8, 264), ([257, 255], 64, 256), ([256, 1], 72, 8), ([511], 120, 136), ([513, 0, 3], 128, 248),
+    ([260], 136, 512), ([700, 33], 920, 520), ([1] * 256, 200, 64), ([129, 128, 127], 1000, 1544),
+    ([40000], 64, 1024),  # 628 tiles of one expert; with 8 CUs per XCD's worth of slots still several per workgroup
+])
+def test_persistent_edges(device, dtype, counts, K, N):
+    from dolomite_engine_amd import ops
+
+    g = torch.Generator().manual_seed(K * 7 + N + len(counts))
+    E, L = len(counts), sum(counts)
+    print(f"persistent E={E} L={L} K={K} N={N} {dtype}", flush=True)
+    off = torch.tensor(counts).cumsum(0).int().to(device)
+    ss = torch.randperm(L, generator=g).int().to(device)
+    x = torch.randn(L, K, generator=g).to(dtype).to(device)
+    w = (torch.randn(E, N, K, generator=g) * 0.05).to(dtype).to(device)
+    ref = _reference(x, w, counts)
+    grouped = ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=7)
+    torch.testing.assert_close(grouped.float(), ref, **TOL[dtype])
+    scattered = ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=7)
+    assert torch.equal(scattered[ss.long()], grouped)
+    by_slot = torch.empty_like(x)
+    by_slot[ss.long()] = x
+    assert torch.equal(ops.scattered_gemm(by_slot, w, 1, ss, off, False, True, cfg=7), grouped)
+    w_kn = w.transpose(1, 2).contiguous()
+    assert torch.equal(ops.scattered_gemm(x, w_kn, 1, ss, off, True, True, weight_kn=True), grouped)
+    if N % 16 == 0:
+        half = N // 2
+        act = ops.up_swiglu(by_slot, w, 1, ss, off, cfg=7)
+        want = ref[:, :half] * torch.nn.functional.silu(ref[:, half:])
+        torch.testing.assert_close(act.float(), want, **TOL[dtype])
+        if L >= 192 * E:
+            act_k, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off)
+            assert torch.equal(h, grouped)
+            torch.testing.assert_close(act_k.float(), want, rtol=TOL[dtype]["rtol"] * 4, atol=TOL[dtype]["atol"] * 4)
