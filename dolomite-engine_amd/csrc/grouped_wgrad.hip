@@ -24,30 +24,20 @@
 //     An item of an expert with several groups writes an fp32 partial tile and a second kernel sums the partials
 //     of the expert in group order and rounds once (deterministic); an expert with one group is written directly,
 //     one without rows gets zeros from the second kernel.
-//   * HBM -> LDS by DMA (no registers), a ring of four 32-row slices with three in flight, and the forward
-//     kernel's ping-pong schedule: the two waves of a SIMD alternate between a memory phase and a matrix phase.
-//     A row's address is a scalar (index loads go through the scalar cache), the lanes add constant offsets.
-#include "common.h"
-
-#include <type_traits>
+//   * One wave per SIMD with 128 x 128 accumulators in the AGPR half of the register file, 64-row slices, and the
+//     five-unit DMA ring of persistent_gemm.hip (see there for why): one barrier per slice, one LDS read or DMA
+//     instruction between any two matrix instructions.  A lane loads the indices of its eight rows of a gathered
+//     operand two slices ahead and forms one offset per DMA instruction between matrix instructions (as scalar
+//     arithmetic -- eleven instructions per DMA instruction, in one gap -- the gather cost 12 % of the loop).
+//     Measured against the form it replaces (eight waves in two groups, 32-row slices, two barriers each), 40 experts,
+//     262144 rows: 1024 x 1536 with b gathered 724 -> 646 us (1277 TFLOP/s), 1536 x 512 with a gathered 381 -> 349 us;
+//     4072 rows in 32 experts, 1024 x 1024: 38.7 -> 34.0 us.
+#include "mfma_core.h"
 
 #define WGRAD_MAX_E 256
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
 #define MI_LDS __attribute__((address_space(3)))
-
-template <typename T> struct WgradMfma;
-template <> struct WgradMfma<bf16_t> {
-  static __device__ __forceinline__ f32x4 run(s16x8 a, s16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct WgradMfma<f16_t> {
-  static __device__ __forceinline__ f32x4 run(s16x8 a, s16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
 
 struct WgradArgs {
   const void* a;                  // (rows_a, M)
@@ -55,131 +45,116 @@ struct WgradArgs {
   const int32_t* a_idx;           // (L,) row of `a` for sorted row r, or null: r itself
   const int32_t* b_idx;           // same for `b`
   const int32_t* expert_offsets;  // (E,) inclusive ends of the experts' row ranges
-  float* partial;                 // [group][M][N]
+  float* partial;                 // [group][tile][accumulator block][thread] (see store_part)
   void* dw;                       // (E, M, N): written directly for an expert with a single group
   int* next_item;                 // plan: [0..8) per-XCD work counters, zero on entry; [8..17) first slot of each XCD
                                   // in the list; [32..) the groups in the order the XCDs work through them
   int L, M, N, E, chunk, m_tiles, n_tiles;
+  int a_rows, b_rows;
 };
 
-__device__ __forceinline__ constexpr int wgrad_waitcnt(int vm, int lgkm) {
-  // gfx9 encoding: vmcnt = {imm[15:14], imm[3:0]}, expcnt = imm[6:4] (7 = no wait), lgkmcnt = imm[11:8]
-  return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8);
-}
-
-// etab[2e] = groups of experts 0..e, etab[2e+1] = offsets[e]; returns nothing, all threads must call
-__device__ __forceinline__ void wgrad_build_table(const int32_t* __restrict__ offsets, int E, int chunk, int* etab, int lane,
-                                                  int wave) {
-  if (wave == 0) {
-    int carry = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + lane;
-      const int end = e < E ? offsets[e] : 0;
-      const int prev = (e < E && e > 0) ? offsets[e - 1] : 0;
-      int incl = e < E ? (end - prev + chunk - 1) / chunk : 0;
+// lane l of register c: expert 64 c + l -- groups of experts 0..e, and the end of its rows
+struct WgradTable {
+  int groups[4], end[4];
+};
+__device__ __forceinline__ void wgrad_table(const int32_t* __restrict__ off, int E, int chunk, WgradTable& tb) {
+  const int lane = threadIdx.x & 63;
+  int carry = 0;
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        int v = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += v;
-      }
-      incl += carry;
-      if (e < E) {
-        etab[2 * e] = incl;
-        etab[2 * e + 1] = end;
-      }
-      carry = __shfl(incl, 63, 64);
+  for (int c = 0; c < 4; ++c) {
+    tb.groups[c] = 0x7fffffff;
+    tb.end[c] = 0;
+    if (c * 64 >= E) continue;
+    const int e = c * 64 + lane;
+    const int end = e < E ? off[e] : 0;
+    const int prev = (e < E && e > 0) ? off[e - 1] : 0;
+    int incl = e < E ? (end - prev + chunk - 1) / chunk : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
     }
+    incl += carry;
+    carry = __builtin_amdgcn_readlane(incl, 63);
+    tb.groups[c] = e < E ? incl : 0x7fffffff;
+    tb.end[c] = end;
   }
-  __syncthreads();
 }
 
-// Two rows of a tile (512 bytes each) into 1 KiB of LDS starting at `lds_addr`: lanes 0-31 fetch 16 bytes each
-// from base + row_lo + off, lanes 32-63 from base + row_hi + off (32-bit byte offsets); lane l lands at
-// lds_addr + 16 l.  The row offsets are scalars (a gathered operand has an unrelated address per row) and the
-// lane offsets never change; their per-lane sum lives in a register that only this statement names.  Written as
-// assembly for the same reason as in the forward kernel: the compiler would order every later LDS read behind the
-// builtin form of this instruction with vmcnt(0).
-__device__ __forceinline__ void wgrad_dma_row_pair(const void* base, uint32_t row_lo, uint32_t row_hi, uint32_t off,
-                                                   uint64_t upper_half, uint32_t lds_addr) {
-  uint32_t tmp;
-  uint64_t saved;
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_mov_b64 %1, exec\n\t"
-      "v_add_u32 %0, %4, %3\n\t"
-      "s_mov_b64 exec, %7\n\t"
-      "v_add_u32 %0, %5, %3\n\t"
-      "s_mov_b64 exec, %1\n\t"
-      "global_load_lds_dwordx4 %0, %6"
-      : "=&v"(tmp), "=&s"(saved)
-      : "s"(lds_addr), "v"(off), "s"(row_lo), "s"(row_hi), "s"(base), "s"(upper_half)
-      : "memory", "m0");
-}
+// An expert with n rows has ceil(n / chunk) groups of equal size (a multiple of 32 rows, the last one shorter).
+__device__ __forceinline__ int wgrad_group_rows(int n, int groups) { return ((n + groups - 1) / groups + 31) & ~31; }
 
-template <typename T>
-__global__ __launch_bounds__(512) void grouped_wgrad_kernel(WgradArgs a) {
-  constexpr int BK = 32, TILE = 256;
-  constexpr int OP_BYTES = BK * TILE * 2;  // one operand's 32 rows x 256 columns
-  constexpr int STAGE_BYTES = 2 * OP_BYTES;
-  constexpr int NSTAGE = 4, AHEAD = 3;
-  constexpr int NLD = 4;                   // DMA instructions per wave and slice (4 row pairs)
-  typedef const __attribute__((address_space(4))) int32_t* const_idx_t;
-  typedef int32_t i32x8_a4 __attribute__((ext_vector_type(8), aligned(4)));
-  typedef const __attribute__((address_space(4))) i32x8_a4* const_idx8_t;
+#define WG_BK 64        // rows of a slice
+#define WG_U 32768      // bytes of a ring unit: one operand's 64 rows x 256 columns
+#define WG_LDS (5 * WG_U)
+
+// GA / GB: operand a / b is gathered through its index array
+template <typename T, bool GA, bool GB>
+__global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
+  constexpr int TILE = 256;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  int* etab = reinterpret_cast<int*>(smem_raw + NSTAGE * STAGE_BYTES);
-  int* item_slot = etab + 2 * a.E;
+  int* item_slot = reinterpret_cast<int*>(smem_raw);  // (between items, when the ring is drained)
+  const uint32_t lds0 = (uint32_t)(size_t)(MI_LDS void*)smem_raw;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1;          // 128 rows (m) x 128 columns (n) of the tile
+  const int fi = lane & 15, fq = lane >> 4;
+  const int upper = lane >> 5;
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 3, wn = wave >> 2;
-
-  wgrad_build_table(a.expert_offsets, a.E, a.chunk, etab, lane, wave);
+  WgradTable tb;
+  wgrad_table(a.expert_offsets, a.E, a.chunk, tb);
   const int tiles = a.m_tiles * a.n_tiles;
   const int xcd = blockIdx.x & 7;
-
-  // An expert with n rows has ceil(n / chunk) groups of equal size (a multiple of 32 rows, the last one shorter).
-  auto group_rows = [&](int n, int groups) { return ((n + groups - 1) / groups + 31) & ~31; };
   // this XCD's groups: slots [xfirst, xfirst + xgroups) of the planned list
   const int xfirst = a.next_item[8 + xcd];
   const int xgroups = a.next_item[8 + xcd + 1] - xfirst;
   const int* __restrict__ xlist = a.next_item + 32 + xfirst;
   const int items_x = xgroups * tiles;
 
-  // ---- loader role: waves 0-3 stage operand A, waves 4-7 operand B; each wave rows 8 wq .. 8 wq + 7 of a slice --
-  const bool load_b = wave >= 4;
-  const int wq = wave & 3;
-  const unsigned char* src = static_cast<const unsigned char*>(load_b ? a.b : a.a);
-  const const_idx_t idx = reinterpret_cast<const_idx_t>(reinterpret_cast<uintptr_t>(load_b ? a.b_idx : a.a_idx));
-  const int ld = load_b ? a.N : a.M;  // columns of the operand
-  const uint32_t ldbytes32 = (uint32_t)ld * (uint32_t)sizeof(T);  // operands stay below 4 GiB (checked on the host)
-  // LDS position lane % 32 of row `krow` holds the logical 16-byte piece whose 32-byte group is
-  // (position / 2) ^ f(krow), f(krow) = (krow & 3) | (((krow >> 3) & 3) << 2); row pair p of the wave is
-  // krow = 8 wq + 2 p + lane / 32, so f only depends on the parity of p
-  int lcol[2];  // first column (element) of the lane's piece, for even / odd row pairs
+  // ---- DMA: wave w fetches rows 16 w .. 16 w + 15 of a slice, instruction j the rows j (lanes 0-31) and 8 + j: a lane
+  // then needs the indices of eight consecutive rows of a gathered operand, two loads of 16 bytes per slice.  (The two
+  // rows of an instruction are neighbours in LDS; the contraction may take the rows in any order that both operands
+  // share.)
+  // Position lane % 32 of LDS row r holds the logical 16-byte piece whose 32-byte group is (position / 2) ^ f(r),
+  // f(r) = r % 4 | (r / 8 % 4) << 2, the swizzle the transposing reads expect: four lane offsets in all.
+  uint32_t piece[4];
 #pragma unroll
-  for (int par = 0; par < 2; ++par) {
-    const int f = ((2 * par + (lane >> 5)) & 3) | (wq << 2);
-    lcol[par] = (((((lane & 31) >> 1) ^ f) & 15) << 4) + (lane & 1) * 8;
+  for (int v = 0; v < 4; ++v) {
+    const int f = ((2 * (v & 1) + upper) & 3) | (((2 * wave + (v >> 1)) & 3) << 2);
+    piece[v] = (uint32_t)((((((lane & 31) >> 1) ^ f) & 15) << 4) + (lane & 1) * 8) * 2u;
   }
-  const uint32_t lds0 = (uint32_t)(size_t)(MI_LDS void*)smem_raw;
-  const uint32_t wave_lds = lds0 + (load_b ? OP_BYTES : 0) + 8 * wq * (TILE * 2);
+  auto piece_of = [&](int j) { return piece[(j & 1) + 2 * (j >> 2)]; };
+  const uint32_t a_ld = (uint32_t)a.M * 2u, b_ld = (uint32_t)a.N * 2u;  // bytes of a row
+  // (columns past an operand's width read the next row's: their products only reach results that are never stored)
+  const uint64_t a_bytes = (uint64_t)a.a_rows * a_ld, b_bytes = (uint64_t)a.b_rows * b_ld;
+  const uint32_t dma0 = lds0 + wave * 8192;
 
-  // ---- fragment read addresses (per lane): row 8q + 4h + i/4, column group F ^ f(row), piece i % 4 ----------
-  const int fi = lane & 15, fq = lane >> 4;
-  const int fl = (fi >> 2) | (fq << 2);
-  const uint32_t frag_base = (8 * fq + (fi >> 2)) * (TILE * 2) + (fl << 5) + (fi & 3) * 8;
+  // ---- fragment reads: ds_read_b64_tr_b16, row 8 q + 4 h + i / 4, 32-byte column group F ^ f(row), piece i % 4 --------
+  const uint32_t trb = (8 * fq + (fi >> 2)) * (TILE * 2) + ((((fi >> 2) | (fq << 2))) << 5) + (fi & 3) * 8;
+  auto read_frag = [&](uint32_t base, int ks, int F) -> u32x4 {
+    const uint32_t addr = base + (trb ^ ((uint32_t)F << 5));
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((MI_LDS s16x4*)(size_t)(addr + ks * 16384));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((MI_LDS s16x4*)(size_t)(addr + ks * 16384 + 2048));
+    return __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
 
   // Items of an XCD are handed out in order through a counter: the workgroups of the XCD stay on neighbouring
   // items (same group of rows, shared through the L2) and none of them idles while another still has a queue.
-  // (instantiated twice: for an operand gathered through an index array and for one read in place)
-  auto run_items = [&](auto gather_tag) {
-  constexpr bool GATHER = decltype(gather_tag)::value;
+  // The next item is drawn when the current one has three slices left: early enough that the draw's trip to memory is
+  // over when it ends, late enough that a workgroup does not hold an item another one could start.
+  constexpr int DRAW_AHEAD = 3;
+  int drawn = 0;
+  if (threadIdx.x == 0) drawn = atomicAdd(a.next_item + xcd, 1);
   for (;;) {
-    if (tid == 0) *item_slot = atomicAdd(a.next_item + xcd, 1);
-    __syncthreads();
+    // (bare barriers: a fence would also wait for the last item's stores)
+    if (threadIdx.x == 0) *item_slot = drawn;
+    __builtin_amdgcn_s_waitcnt(pg_wait(63, 0));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     const int item = __builtin_amdgcn_readfirstlane(*item_slot);
-    __syncthreads();
+    __builtin_amdgcn_s_waitcnt(pg_wait(63, 0));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     if (item >= items_x) break;
     const int grp = __builtin_amdgcn_readfirstlane(xlist[item / tiles]);
     // A group's tiles are numbered in bands of 8 row tiles, column tile slowest inside a band: the 32 workgroups
@@ -196,189 +171,256 @@ __global__ __launch_bounds__(512) void grouped_wgrad_kernel(WgradArgs a) {
 
     // group -> expert and its row range (wave-uniform)
     int r0 = 0, r1 = 1, expert = 0, expert_groups = 1;
-    for (int e0 = 0; e0 < a.E; e0 += 64) {
-      const int e = e0 + lane;
-      const int incl = e < a.E ? etab[2 * e] : 0x7fffffff;
-      const uint64_t hit = __ballot(incl > grp);
-      if (hit) {
-        const int ex = e0 + __ffsll((long long)hit) - 1;
-        const int first = ex > 0 ? etab[2 * (ex - 1)] : 0;
-        const int prev = ex > 0 ? etab[2 * (ex - 1) + 1] : 0;
-        expert = ex;
-        expert_groups = etab[2 * ex] - first;
-        const int rows = group_rows(etab[2 * ex + 1] - prev, etab[2 * ex] - first);
-        r0 = prev + (grp - first) * rows;
-        r1 = etab[2 * ex + 1];
-        if (r1 > r0 + rows) r1 = r0 + rows;
-        break;
-      }
-    }
-    r0 = __builtin_amdgcn_readfirstlane(r0);
-    r1 = __builtin_amdgcn_readfirstlane(r1);
-    expert = __builtin_amdgcn_readfirstlane(expert);
-    expert_groups = __builtin_amdgcn_readfirstlane(expert_groups);
-    const int nk = (r1 - r0 + BK - 1) / BK;
-
-    // lane offsets of this tile; columns past the operand's width re-read the tile's first piece (their
-    // products only reach output rows / columns that are never stored)
-    const int col0 = (load_b ? nt : mt) * TILE;
-    uint32_t loff[2];
+    {
+      int first = 0, prev = 0;
+      bool found = false;
 #pragma unroll
-    for (int par = 0; par < 2; ++par) loff[par] = (uint32_t)((col0 + lcol[par] < ld ? lcol[par] : 0) * sizeof(T));
-    const unsigned char* tile_src = src + (size_t)col0 * sizeof(T);
-
-    // rows of slice `slice` this wave fetches: sorted rows r0 + 32 slice + 8 wq + [0, 8), clamped into the group
-    // (rows past its end are fetched again from its last row and masked out of the last slice's fragments)
-    auto load_idx = [&](int slice, int (&rw)[8]) {
-      const int first = r0 + slice * BK + 8 * wq;
-      if (GATHER && first + 7 < r1) {
-        // the usual case: eight consecutive indices in one scalar load
-        const i32x8_a4 v = *reinterpret_cast<const_idx8_t>(idx + first);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) rw[i] = v[i];
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          int r = first + i;
-          if (r > r1 - 1) r = r1 - 1;
-          rw[i] = GATHER ? idx[r] : r;
+      for (int c = 0; c < 4; ++c) {
+        if (found || c * 64 >= a.E) continue;
+        const uint64_t hit = __ballot(tb.groups[c] > grp);
+        const int l = hit ? __ffsll((long long)hit) - 1 : 64;
+        if (l > 0) {
+          first = __builtin_amdgcn_readlane(tb.groups[c], l - 1);
+          prev = __builtin_amdgcn_readlane(tb.end[c], l - 1);
+        }
+        if (l < 64) {
+          expert = c * 64 + l;
+          expert_groups = __builtin_amdgcn_readlane(tb.groups[c], l) - first;
+          const int end = __builtin_amdgcn_readlane(tb.end[c], l);
+          const int rows = wgrad_group_rows(end - prev, expert_groups);
+          r0 = prev + (grp - first) * rows;
+          r1 = r0 + rows < end ? r0 + rows : end;
+          found = true;
         }
       }
-    };
-    auto dma_slice = [&](const int (&rw)[8], int stage) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p)
-        wgrad_dma_row_pair(tile_src, (uint32_t)rw[2 * p] * ldbytes32, (uint32_t)rw[2 * p + 1] * ldbytes32, loff[p & 1],
-                           0xffffffff00000000ull, wave_lds + stage * STAGE_BYTES + 2 * p * (TILE * 2));
-    };
-
-    f32x4 acc[4][8];
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < 8; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    s16x8 af[4], bf[8];
-    auto read_frag = [&](int stage, int opoff, int F) -> s16x8 {
-      const uint32_t addr = lds0 + stage * STAGE_BYTES + opoff + (frag_base ^ ((uint32_t)F << 5));
-      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((MI_LDS s16x4*)(size_t)addr);
-      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((MI_LDS s16x4*)(size_t)(addr + 4 * TILE * 2));
-      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    };
-    auto read_frags = [&](int stage) {
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) af[mb] = read_frag(stage, 0, 4 * wm + mb);
-#pragma unroll
-      for (int nb = 0; nb < 8; ++nb) bf[nb] = read_frag(stage, OP_BYTES, 8 * wn + nb);
-    };
-    auto multiply = [&]() {
-#pragma unroll
-      for (int nb = 0; nb < 8; ++nb)
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb) acc[mb][nb] = WgradMfma<T>::run(af[mb], bf[nb], acc[mb][nb]);
-    };
-    // the last slice of a group may be short: element j of a fragment is row 8 (lane / 16) + j of the slice
-    const int last_rows = r1 - r0 - (nk - 1) * BK;
-    auto mask_frags = [&]() {
-      uint32_t m[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int k = 8 * fq + 2 * t;
-        m[t] = (k < last_rows ? 0x0000ffffu : 0u) | (k + 1 < last_rows ? 0xffff0000u : 0u);
-      }
-      auto apply = [&](s16x8& v) {
-        u32x4 w = __builtin_bit_cast(u32x4, v);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) w[t] &= m[t];
-        v = __builtin_bit_cast(s16x8, w);
-      };
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) apply(af[mb]);
-#pragma unroll
-      for (int nb = 0; nb < 8; ++nb) apply(bf[nb]);
-    };
-
-    // ---- K loop: the forward kernel's ping-pong schedule.  The waves wn == 0 and wn == 1 (one of each per SIMD)
-    // run the same code one phase apart: while one group issues its 32 matrix instructions out of registers, the
-    // other reads its fragments of the slice and issues its share of the DMA for the slice three ahead.
-    int rw[8];
-    load_idx(0, rw);
-    dma_slice(rw, 0);
-    load_idx(1, rw);
-    dma_slice(rw, 1);
-    load_idx(2, rw);
-    dma_slice(rw, 2);
-    load_idx(3, rw);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(wgrad_waitcnt((AHEAD - 1) * NLD, 0));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (wn == 1) __builtin_amdgcn_s_barrier();
-    for (int g = 0; g < nk; ++g) {
-      const int cur = g & (NSTAGE - 1), fill = (g + AHEAD) & (NSTAGE - 1);
-      // slices past the group's end are fetched like the others (clamped rows) and never multiplied.  The DMA goes
-      // first: its row indices came in long ago, and a wait for them behind the fragment reads would also wait
-      // for those (scalar loads and LDS reads share a counter)
-      dma_slice(rw, fill);
-      read_frags(cur);
-      if (g == nk - 1 && last_rows < BK) mask_frags();
-      asm volatile("" ::: "memory");
-      // own DMA of slice g + 1 has landed (g + 2 and g + 3 stay in flight); fragments are in registers
-      __builtin_amdgcn_s_waitcnt(wgrad_waitcnt((NSTAGE - 2) * NLD, 0));
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      // the row indices of the next DMA come in through the scalar cache while the matrix pipe works
-      load_idx(g + 4, rw);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply();
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
     }
-    if (wn == 0) __builtin_amdgcn_s_barrier();
-    // surplus DMA (slices nk .. nk + 2) must land before the next item reuses the ring
-    __builtin_amdgcn_s_waitcnt(wgrad_waitcnt(0, 0));
+    const int nrows = r1 - r0, nk = (nrows + WG_BK - 1) / WG_BK, nfull = nrows / WG_BK;
+
+    const u32x4 asrd = pg_srd(static_cast<const unsigned char*>(a.a) + (size_t)mt * (TILE * 2), a_bytes - (uint64_t)mt * (TILE * 2));
+    const u32x4 bsrd = pg_srd(static_cast<const unsigned char*>(a.b) + (size_t)nt * (TILE * 2), b_bytes - (uint64_t)nt * (TILE * 2));
+    // lane offsets of the eight instructions: of an operand read in place relative to the slice's first row, of a
+    // gathered one recomputed every slice from the row indices; rows past the group's end give zeros
+    const int lrow = 16 * wave + 8 * upper;         // + j: row of the slice
+    uint32_t aoff[8], boff[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      aoff[j] = (uint32_t)(lrow + j) * a_ld + piece_of(j);
+      boff[j] = (uint32_t)(lrow + j) * b_ld + piece_of(j);
+    }
+    auto mask_rows = [&](uint32_t (&off)[8], int sl) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) off[j] = lrow + j >= nrows - sl * WG_BK ? PG_OOB : off[j];
+    };
+    // Row indices of slice sl for this lane.  Requested in assembly (the compiler would wait for everything in flight
+    // before their first use); they are older than the DMA that the slice's barrier leaves in flight, so they have
+    // arrived behind it.  Indices past the end of the array read as 0 and are masked with their rows.
+    const u32x4 isrd = pg_srd(GA ? a.a_idx : a.b_idx, (uint64_t)a.L * 4u), isrd_b = pg_srd(a.b_idx, (uint64_t)a.L * 4u);
+    const uint32_t ioff = (uint32_t)lrow * 4u;
+    auto load_idx = [&](u32x4 srd, int sl, u32x4 (&ix)[2]) {
+      const uint32_t so = (uint32_t)(r0 + sl * WG_BK) * 4u;
+      asm volatile("buffer_load_dwordx4 %0, %2, %3, %4 offen\n\tbuffer_load_dwordx4 %1, %2, %3, %4 offen offset:16"
+                   : "=&v"(ix[0]), "=&v"(ix[1]) : "v"(ioff), "s"(srd), "s"(so) : "memory");
+    };
+    auto gathered_off = [&](const u32x4 (&ix)[2], int j, uint32_t ld) -> uint32_t { return ix[j >> 2][j & 3] * ld + piece_of(j); };
+
+    // ---- ring (see persistent_gemm.hip): slots of A_k, B_k, A_k+1, B_k+1 and the free one ---------------------------------
+    uint32_t p0 = 0, p1 = WG_U, p2 = 2 * WG_U, p3 = 3 * WG_U, p4 = 4 * WG_U;
+    u32x4 ai[2], bi[2];                             // row indices of A_k+3 / B_k+2 where gathered
+    u32x4 wf[2][8], xf[2][8];                       // fragments of b (columns n) and a (rows m)
+    uint32_t rw, rx;
+    int ks_a, ks_b;                                 // next slice of either operand to fetch
+    auto half = [&](auto btag, auto ftag, uint32_t dst, auto hook) {
+      constexpr int B = decltype(btag)::value;
+      constexpr bool FIRST = decltype(ftag)::value;
+      constexpr bool G = B ? GB : GA;
+      const uint32_t soff = G ? 0u : (uint32_t)(r0 + (B ? ks_b : ks_a) * WG_BK) * (B ? b_ld : a_ld);
+      pg_own_agprs();
+#pragma unroll
+      for (int m = 0; m < 64; ++m) {
+        const int nb = m & 7, mb = m >> 3;
+        if constexpr (FIRST) pg_mfma_first<T>((mb * 8 + nb) * 4, wf[B][nb], xf[B][mb]);
+        else pg_mfma<T>((mb * 8 + nb) * 4, wf[B][nb], xf[B][mb]);
+        if (m % 2 == 0 && m < 32) {
+          const int q = m / 2;
+          PG_SCHED();
+          if (q < 8) wf[B ^ 1][q] = read_frag(rw, B ^ 1, 8 * wn + q);
+          else xf[B ^ 1][q - 8] = read_frag(rx, B ^ 1, 8 * wm + q - 8);
+          PG_SCHED();
+        }
+        if (m % 8 == 1) {
+          PG_SCHED();
+          pg_dma_dst(dst, m / 8 * 1024);
+          PG_SCHED();
+        }
+        if (m % 8 == 3) {
+          PG_SCHED();
+          pg_dma(B ? boff[m / 8] : aoff[m / 8], B ? bsrd : asrd, soff);
+          PG_SCHED();
+        }
+        hook(m);
+      }
+    };
+    auto read_bases = [&](uint32_t ps_b, uint32_t ps_a) {
+      rw = lds0 + ps_b;
+      rx = lds0 + ps_a;
+    };
+    auto step = [&](auto ftag) {
+      // the indices of A_k+3 and B_k+2 go out ahead of this half's DMA and have arrived at its end
+      if (GA) load_idx(isrd, ks_a + 1, ai);
+      if (GB) load_idx(isrd_b, ks_b, bi);
+      if (ks_a >= nfull) mask_rows(aoff, ks_a);
+      half(std::integral_constant<int, 0>{}, ftag, dma0 + p4, [&](int m) {
+        if (m == 62) {
+          PG_SCHED();
+          ++ks_a;
+          read_bases(p3, p2);
+          PG_SCHED();
+        }
+      });
+      // slice k + 1 has landed (A_k+2 stays in flight); slice k is in everybody's registers
+      __builtin_amdgcn_s_waitcnt(pg_wait(8, 0));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      PG_SCHED();
+      const bool b_short = ks_b >= nfull;
+      if (!GB && b_short) mask_rows(boff, ks_b);
+      if (GB && b_short) {
+        // (the last slice or two of a group)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) boff[j] = gathered_off(bi, j, b_ld);
+        mask_rows(boff, ks_b);
+      }
+      // SHORT: the offsets of this half's gathered rows are already there, masked (the last slice or two of a group)
+      auto second = [&](auto short_tag) {
+        half(std::integral_constant<int, 1>{}, std::false_type{}, dma0 + p0, [&](int m) {
+          if (GB && !decltype(short_tag)::value && m % 8 == 2) {
+            PG_SCHED();
+            boff[m / 8] = gathered_off(bi, m / 8, b_ld);
+            PG_SCHED();
+          }
+          if (GA && m % 8 == 5) {
+            PG_SCHED();
+            aoff[m / 8] = gathered_off(ai, m / 8, a_ld);
+            PG_SCHED();
+          }
+          if (m == 60) {
+            PG_SCHED();
+            ++ks_b;
+            const uint32_t t0 = p0, t1 = p1;
+            p0 = p2;
+            p1 = p3;
+            p2 = p4;
+            p3 = t0;
+            p4 = t1;
+            asm volatile("" : "+s"(p0), "+s"(p1), "+s"(p2), "+s"(p3), "+s"(p4));
+            read_bases(p1, p0);
+            PG_SCHED();
+          }
+        });
+      };
+      if (GB && b_short) second(std::true_type{});
+      else second(std::false_type{});
+    };
+
+    // ---- first two slices -------------------------------------------------------------------------------------------
+    u32x4 ix[3][2];
+    if (GA || GB) {
+      if (GA && GB) load_idx(isrd_b, 0, bi);
+#pragma unroll
+      for (int sl = 0; sl < 3; ++sl) load_idx(isrd, sl, ix[sl]);
+      asm volatile("s_waitcnt vmcnt(0)" : "+v"(ix[0][0]), "+v"(ix[0][1]), "+v"(ix[1][0]), "+v"(ix[1][1]), "+v"(ix[2][0]),
+                   "+v"(ix[2][1]), "+v"(bi[0]), "+v"(bi[1]) : : "memory");
+    }
+#pragma unroll
+    for (int sl = 0; sl < 2; ++sl) {
+      if (GA && GB && sl == 1) {
+        load_idx(isrd_b, 1, bi);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(bi[0]), "+v"(bi[1]) : : "memory");
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (GA) aoff[j] = gathered_off(ix[sl], j, a_ld);
+        if (GB) boff[j] = gathered_off(GA ? bi : ix[sl], j, b_ld);
+      }
+      if (sl >= nfull) {
+        mask_rows(aoff, sl);
+        mask_rows(boff, sl);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        pg_dma_dst(dma0 + (sl ? p2 : p0), j * 1024);
+        asm volatile("s_nop 0");
+        pg_dma(aoff[j], asrd, GA ? 0u : (uint32_t)(r0 + sl * WG_BK) * a_ld);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        pg_dma_dst(dma0 + (sl ? p3 : p1), j * 1024);
+        asm volatile("s_nop 0");
+        pg_dma(boff[j], bsrd, GB ? 0u : (uint32_t)(r0 + sl * WG_BK) * b_ld);
+      }
+    }
+    if (GA) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) aoff[j] = gathered_off(ix[2], j, a_ld);
+    }
+    ks_a = ks_b = 2;
+    __builtin_amdgcn_s_waitcnt(pg_wait(16, 0));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read_bases(p1, p0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wf[0][i] = read_frag(rw, 0, 8 * wn + i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) xf[0][i] = read_frag(rx, 0, 8 * wm + i);
+
+    // ---- slices -------------------------------------------------------------------------------------------------------
+    step(std::true_type{});
+    int k = 1;
+    for (; k < nk - DRAW_AHEAD; ++k) step(std::false_type{});
+    if (threadIdx.x == 0) drawn = atomicAdd(a.next_item + xcd, 1);
+    for (; k < nk; ++k) step(std::false_type{});
+    pg_acc_settle();
+    // surplus DMA (two slices of zeros) has to land before the ring is used again
+    __builtin_amdgcn_s_waitcnt(pg_wait(0, 0));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 
-    // ---- output tile: register i of block (mb, nb) is row 16 mb + 4 (lane / 16) + i, column 16 nb + lane % 16.
-    // An expert with one group is final: rounded and written straight into dw (whole 32-byte sectors per 16
-    // lanes).  Otherwise an fp32 partial tile for the reduction kernel.
+    // ---- output tile: register i of block (mb, nb) is row 16 mb + lane % 16, column 16 nb + 4 (lane / 16) + i -------------
+    // An expert with one group is final: rounded, staged through 8 KB of LDS per wave (32 rows x 128 columns at a time,
+    // 16-byte chunk c of row r at slot c ^ (r % 16)) and stored as whole 256-byte rows.  Otherwise the fp32
+    // accumulators go to the group's partial slab as they are: block b of thread t at [b][t].
     if (expert_groups == 1) {
       T* __restrict__ out = static_cast<T*>(a.dw) + (size_t)expert * a.M * a.N;
+      unsigned char* scratch = smem_raw + 1024 + wave * 8192;  // (past the item slot)
+      const bool interior = (mt + 1) * TILE <= a.M && (nt + 1) * TILE <= a.N;
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
+      for (int p = 0; p < 4; ++p) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = mt * TILE + wm * 64 + mb * 16 + 4 * fq + i;
-          if (m < a.M) {
+        for (int mbp = 0; mbp < 2; ++mbp)
 #pragma unroll
-            for (int nb = 0; nb < 8; ++nb) {
-              const int n = nt * TILE + wn * 128 + nb * 16 + fi;
-              if (n < a.N) Elt<T>::store(out + (size_t)m * a.N + n, acc[mb][nb][i]);
-            }
+          for (int nb = 0; nb < 8; ++nb) {
+            const int blk = ((2 * p + mbp) * 8 + nb) * 4;
+            const float v0 = pg_acc(blk), v1 = pg_acc(blk + 1), v2 = pg_acc(blk + 2), v3 = pg_acc(blk + 3);
+            *reinterpret_cast<u32x2*>(scratch + (mbp * 16 + fi) * 256 + (((2 * nb + (fq >> 1)) ^ fi) * 16) + (fq & 1) * 8) =
+                (u32x2){pack2<T>(v0, v1), pack2<T>(v2, v3)};
           }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+          const int r = 4 * it + (lane >> 4);
+          const u32x4 v = *reinterpret_cast<const u32x4*>(scratch + r * 256 + (lane & 15) * 16);
+          const int m = mt * TILE + wm * 128 + p * 32 + r, n = nt * TILE + wn * 128 + ((lane & 15) ^ (r & 15)) * 8;
+          if (interior || (m < a.M && n < a.N)) *reinterpret_cast<u32x4*>(out + (size_t)m * a.N + n) = v;
         }
+        asm volatile("" ::: "memory");
+      }
     } else {
-      float* __restrict__ out = a.partial + (size_t)grp * a.M * a.N;
+      f32x4* base = reinterpret_cast<f32x4*>(a.partial) + ((size_t)grp * tiles + (size_t)mt * a.n_tiles + nt) * (64 * 256) + threadIdx.x;
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = mt * TILE + wm * 64 + mb * 16 + 4 * fq + i;
-          if (m < a.M) {
-#pragma unroll
-            for (int nb = 0; nb < 8; ++nb) {
-              const int n = nt * TILE + wn * 128 + nb * 16 + fi;
-              if (n < a.N) out[(size_t)m * a.N + n] = acc[mb][nb][i];
-            }
-          }
-        }
+      for (int b = 0; b < 64; ++b)
+        base[b * 256] = (f32x4){pg_acc(4 * b), pg_acc(4 * b + 1), pg_acc(4 * b + 2), pg_acc(4 * b + 3)};
     }
   }
-  };
-  if (idx != nullptr) run_items(std::true_type{});
-  else run_items(std::false_type{});
 }
 
 // Plan of one launch (one workgroup, in front of the main kernel): zero the eight work counters, rank the
@@ -466,12 +508,12 @@ __global__ __launch_bounds__(1024) void wgrad_plan_kernel(const int32_t* __restr
 
 // dW[e] = sum of expert e's partial slabs in group order, rounded once (experts with several groups); zeros for an
 // expert without rows.  blockIdx.y walks the plan's list of such experts (without a plan -- a call with no rows at
-// all -- every expert gets zeros); the blocks of an entry stride over the expert's 8-value chunks, four slabs'
-// loads in flight per chunk.
+// all -- every expert gets zeros); the blocks of an entry stride over the expert's (tile, accumulator block, thread)
+// pieces of four values, four slabs' loads in flight per piece.
 template <typename T>
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ partial,
                                                            const int* __restrict__ plan, int red_at,
-                                                           T* __restrict__ dw, long mn) {
+                                                           T* __restrict__ dw, int M, int N, int n_tiles, int tiles) {
   int e = blockIdx.y, first = 0, count = 0;
   if (plan != nullptr) {
     if ((int)blockIdx.y >= plan[17]) return;
@@ -480,36 +522,27 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restri
     first = entry[1];
     count = entry[2];
   }
-  const long n8 = mn / 8;
-  const float* base = partial + (size_t)first * mn;
-  T* out = dw + (size_t)e * mn;
-  for (long id = (long)blockIdx.x * 256 + threadIdx.x; id < n8; id += (long)gridDim.x * 256) {
-    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-    const float* p = base + id * 8;
+  const size_t slab = (size_t)tiles * (64 * 256);  // f32x4 per group
+  const f32x4* base = reinterpret_cast<const f32x4*>(partial) + (size_t)first * slab;
+  T* out = dw + (size_t)e * M * N;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // piece (tile, b, thread): row 128 (wave % 2) + 16 (b / 8) + lane % 16, column 128 (wave / 2) + 16 (b % 8) + 4 (lane / 16)
+  const int dm = (wave & 1) * 128 + (lane & 15), dn = (wave >> 1) * 128 + (lane >> 4) * 4;
+  for (long id = blockIdx.x; id < (long)tiles * 64; id += gridDim.x) {
+    const int tile = (int)(id >> 6), b = (int)(id & 63);
+    const int m = (tile / n_tiles) * 256 + dm + (b >> 3) * 16, n = (tile % n_tiles) * 256 + dn + (b & 7) * 16;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    const f32x4* p = base + id * 256 + tid;
     int g = 0;
     for (; g + 4 <= count; g += 4) {
-      f32x4 v[8];
+      f32x4 v[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[2 * j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + (size_t)(g + j) * mn));
-        v[2 * j + 1] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + (size_t)(g + j) * mn + 4));
-      }
+      for (int j = 0; j < 4; ++j) v[j] = __builtin_nontemporal_load(p + (size_t)(g + j) * slab);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        s0 += v[2 * j];
-        s1 += v[2 * j + 1];
-      }
+      for (int j = 0; j < 4; ++j) s += v[j];
     }
-    for (; g < count; ++g) {
-      s0 += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + (size_t)g * mn));
-      s1 += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + (size_t)g * mn + 4));
-    }
-    u32x4 o;
-    o[0] = pack2<T>(s0[0], s0[1]);
-    o[1] = pack2<T>(s0[2], s0[3]);
-    o[2] = pack2<T>(s1[0], s1[1]);
-    o[3] = pack2<T>(s1[2], s1[3]);
-    *reinterpret_cast<u32x4*>(out + id * 8) = o;
+    for (; g < count; ++g) s += __builtin_nontemporal_load(p + (size_t)g * slab);
+    if (m < M && n < N) *reinterpret_cast<u32x2*>(out + (size_t)m * N + n) = (u32x2){pack2<T>(s[0], s[1]), pack2<T>(s[2], s[3])};
   }
 }
 
@@ -535,12 +568,39 @@ static int wgrad_chunk(int L, int E, int M, int N) {
 static long wgrad_max_groups(int L, int E, int chunk) { return (long)L / chunk + (E < L ? E : L); }
 static size_t wgrad_plan_bytes(long groups, int E) { return ((size_t)(32 + groups + 3 * (long)E) * sizeof(int) + 255) / 256 * 256; }
 
+// partial slabs: whole 256 x 256 tiles
+static size_t wgrad_slab_bytes(long groups, int M, int N) {
+  return (size_t)groups * (size_t)mi_ceil_div(M, 256) * (size_t)mi_ceil_div(N, 256) * (256 * 256 * sizeof(float));
+}
+
 extern "C" size_t mi_moe_grouped_wgrad_workspace_bytes(int L, int E, int M, int N) {
   if (L < 1 || E < 1 || M < 1 || N < 1) return 0;
   // [partial slabs][plan: 32 ints (work counters, first slots) + one int per group + three per expert, padded to
   // 256 bytes]
   const long groups = wgrad_max_groups(L, E, wgrad_chunk(L, E, M, N));
-  return (size_t)groups * (size_t)M * (size_t)N * sizeof(float) + wgrad_plan_bytes(groups, E);
+  return wgrad_slab_bytes(groups, M, N) + wgrad_plan_bytes(groups, E);
+}
+
+template <typename T, bool GA, bool GB> static int launch_wgrad_as(const WgradArgs& g, int grid, hipStream_t s) {
+  auto kern = grouped_wgrad_kernel<T, GA, GB>;
+  static std::atomic<uint64_t> lds_ok{0};
+  const int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), WG_LDS, lds_ok);
+  if (rc != MI_MOE_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), WG_LDS, s, g);
+  return mi_launch_status();
+}
+
+template <typename T> static int launch_wgrad(const WgradArgs& g, int grid, int red_at, hipStream_t s) {
+  if (g.L > 0) {
+    const int rc = g.a_idx != nullptr ? (g.b_idx != nullptr ? launch_wgrad_as<T, true, true>(g, grid, s) : launch_wgrad_as<T, true, false>(g, grid, s))
+                                      : (g.b_idx != nullptr ? launch_wgrad_as<T, false, true>(g, grid, s) : launch_wgrad_as<T, false, false>(g, grid, s));
+    if (rc != MI_MOE_OK) return rc;
+  }
+  const int tiles = g.m_tiles * g.n_tiles;
+  const int rblocks = tiles * 64 < 256 ? tiles * 64 : 256;
+  hipLaunchKernelGGL((wgrad_reduce_kernel<T>), dim3((unsigned)rblocks, (unsigned)g.E), dim3(256), 0, s, g.partial, g.next_item,
+                     red_at, static_cast<T*>(g.dw), g.M, g.N, g.n_tiles, tiles);
+  return mi_launch_status();
 }
 
 extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx,
@@ -556,7 +616,6 @@ extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const v
   if (L > 0 && (!a || !b)) return MI_MOE_ENULL;
   if (!mi_aligned(a, 16) || !mi_aligned(b, 16) || !mi_aligned(dw, 16) || !mi_aligned(workspace, 16)) return MI_MOE_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const long mn = (long)M * N;
   if (L > 0 && (!workspace || workspace_bytes < mi_moe_grouped_wgrad_workspace_bytes(L, E, M, N))) return MI_MOE_EWORKSPACE;
 
   WgradArgs g;
@@ -565,41 +624,23 @@ extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const v
   g.dw = dw;
   g.next_item = nullptr;
   g.L = L; g.M = M; g.N = N; g.E = E;
+  g.a_rows = a_rows; g.b_rows = b_rows;
   g.chunk = wgrad_chunk(L, E, M, N);
   const long max_groups = wgrad_max_groups(L, E, g.chunk);
   const int red_at = (int)(32 + max_groups);
   if (L > 0) {
-    g.next_item = reinterpret_cast<int*>(static_cast<unsigned char*>(workspace) +
-                                         (size_t)max_groups * (size_t)M * (size_t)N * sizeof(float));
+    g.next_item = reinterpret_cast<int*>(static_cast<unsigned char*>(workspace) + wgrad_slab_bytes(max_groups, M, N));
     hipLaunchKernelGGL(wgrad_plan_kernel, dim3(1), dim3(1024), 0, s, expert_offsets, E, g.chunk, g.next_item, red_at);
   }
   g.m_tiles = mi_ceil_div(M, 256);
   g.n_tiles = mi_ceil_div(N, 256);
-  const size_t lds = 4 * 2 * 32 * 256 * 2 + (size_t)E * 8 + 16;
   int cus = 0;
   int rc = mi_cu_count(&cus);
   if (rc != MI_MOE_OK) return rc;
   const long max_items = max_groups * g.m_tiles * g.n_tiles;
   long grid = cus < max_items ? cus : max_items;
   grid = (grid + 7) / 8 * 8;
-  long rblocks = (mn / 8 + 255) / 256;
-  if (rblocks > 256) rblocks = 256;
-  if (dtype == MI_MOE_BF16) {
-    auto kern = grouped_wgrad_kernel<bf16_t>;
-    static std::atomic<uint64_t> lds_ok{0};
-    if ((rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), MI_LDS_MAX_BYTES, lds_ok)) != MI_MOE_OK) return rc;
-    if (L > 0) hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, g);
-    hipLaunchKernelGGL((wgrad_reduce_kernel<bf16_t>), dim3((unsigned)rblocks, (unsigned)E), dim3(256), 0, s, g.partial,
-                       g.next_item, red_at, static_cast<bf16_t*>(dw), mn);
-  } else {
-    auto kern = grouped_wgrad_kernel<f16_t>;
-    static std::atomic<uint64_t> lds_ok{0};
-    if ((rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), MI_LDS_MAX_BYTES, lds_ok)) != MI_MOE_OK) return rc;
-    if (L > 0) hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, g);
-    hipLaunchKernelGGL((wgrad_reduce_kernel<f16_t>), dim3((unsigned)rblocks, (unsigned)E), dim3(256), 0, s, g.partial,
-                       g.next_item, red_at, static_cast<f16_t*>(dw), mn);
-  }
-  return mi_launch_status();
+  return dtype == MI_MOE_BF16 ? launch_wgrad<bf16_t>(g, (int)grid, red_at, s) : launch_wgrad<f16_t>(g, (int)grid, red_at, s);
 }
 
 // ---- fp32 weight gradient on the matrix cores ----------------------------------------------------------------
