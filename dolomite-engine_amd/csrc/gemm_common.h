@@ -9,7 +9,7 @@ struct GemmArgs {
   const void* w;
   void* out;
   const int32_t* sorted_scattered;
-  const int32_t* expert_offsets;
+  const int32_t* expert_offsets;  // null: one expert that owns all L rows
   int L;        // rows of the sorted order
   int K;        // contraction length
   int N;        // output columns (SwiGLU: I, with 2N weight rows per expert)
@@ -41,3 +41,15 @@ bool mi_gemm_persistent_ok(const GemmArgs& a);
 // whether a contraction of length K can be cut along K (the only calls that use a workspace)
 bool mi_gemm_persistent_splits(int K);
 int mi_gemm_persistent(const GemmArgs& a, int dtype, int form, hipStream_t s);
+
+// ---- stream_gemm.hip: K a multiple of one 16-byte chunk, N % 4 == 0 ------------------------------------------------------
+// whether the stream is the faster form for this problem (elt: bytes of an element)
+bool mi_gemm_stream_pick(const GemmArgs& a, int elt);
+// rb: row blocks of 16 per unit (1, 2, 4); nw: waves that split the contraction (1, 2, 4; rb 4: 1, 2); 0, 0: by the rule
+int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipStream_t s);
+
+// ---- grouped_gemm.hip: one expert that owns every row, rows in place (no index arrays): out = in @ W^T, or with SwiGLU ------
+int mi_gemm_one_expert(const void* in, const void* w, void* out, int L, int K, int N, bool glu, int dtype, mi_moe_stream_t stream);
+
+// end of expert e's rows
+__device__ __forceinline__ int mi_expert_end(const int32_t* __restrict__ off, int L, int e) { return off ? off[e] : L; }

@@ -97,14 +97,14 @@ struct TileCoord {
 };
 
 template <int BM>
-__device__ __forceinline__ bool decode_tile(const int32_t* __restrict__ off, int E, int n_tiles, int remap,
+__device__ __forceinline__ bool decode_tile(const int32_t* __restrict__ off, int L, int E, int n_tiles, int remap,
                                             TileCoord& tc) {
   const int lane = threadIdx.x & 63;
   // pass 1: total number of row tiles
   int total_m = 0;
   for (int e0 = 0; e0 < E; e0 += 64) {
     const int e = e0 + lane;
-    const int end = e < E ? off[e] : 0;
+    const int end = e < E ? mi_expert_end(off, L, e) : 0;
     const int prev = (e < E && e > 0) ? off[e - 1] : 0;
     int t = e < E ? (end - prev + BM - 1) / BM : 0;
 #pragma unroll
@@ -128,7 +128,7 @@ __device__ __forceinline__ bool decode_tile(const int32_t* __restrict__ off, int
   int carry = 0;
   for (int e0 = 0; e0 < E; e0 += 64) {
     const int e = e0 + lane;
-    const int end = e < E ? off[e] : 0;
+    const int end = e < E ? mi_expert_end(off, L, e) : 0;
     const int prev = (e < E && e > 0) ? off[e - 1] : 0;
     const int t = e < E ? (end - prev + BM - 1) / BM : 0;
     int incl = t;
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_kernel(GemmArgs a) {
   const int wm = wave % WM, wn = wave / WM;
 
   TileCoord tc;
-  if (!decode_tile<BM>(a.expert_offsets, a.E, a.n_tiles, a.remap, tc)) return;
+  if (!decode_tile<BM>(a.expert_offsets, a.L, a.E, a.n_tiles, a.remap, tc)) return;
   const int expert = tc.expert, row_begin = tc.row_begin, row_end = tc.row_end, nt = tc.nt;
 
   // ---- per-thread global sources ---------------------------------------------------------------
@@ -550,7 +550,7 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GemmArgs 
   const int wm = wave % WM, wn = wave / WM;
 
   TileCoord tc;
-  if (!decode_tile<BM>(a.expert_offsets, a.E, a.n_tiles, a.remap, tc)) return;
+  if (!decode_tile<BM>(a.expert_offsets, a.L, a.E, a.n_tiles, a.remap, tc)) return;
   const int expert = tc.expert, row_begin = tc.row_begin, row_end = tc.row_end, nt = tc.nt;
 
   // ---- DMA sources: instruction j of this wave fills stage rows [(j*NW + wave)*16, +16) -----------
@@ -718,7 +718,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_naive_kernel(GemmArgs a) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= a.L || col >= a.N) return;
   int expert = 0;
-  while (expert < a.E - 1 && a.expert_offsets[expert] <= row) ++expert;
+  while (expert < a.E - 1 && a.expert_offsets[expert] <= row) ++expert;  // (one expert: no offsets)
   const int src = a.gather ? a.sorted_scattered[row] / a.kdiv : row;
   const int orow = a.scatter ? a.sorted_scattered[row] : row;
   const T* x = static_cast<const T*>(a.in) + (size_t)src * a.K;
@@ -850,6 +850,7 @@ static int launch_naive(GemmArgs a, hipStream_t s) {
 //   0 / 1 / 2  register-staged 256x256 / 128x128 / 32x256 (any K % 8 == 0)
 //   3          one thread per output element (any shape, any dtype)
 //   4          DMA-staged 128x128, one tile per workgroup (K % 32 == 0)
+//   100 + 10 rb + nw  weight stream (stream_gemm.hip): row blocks of 16 per unit, waves that split the contraction
 //   7 / 8 / 9  persistent 256x256 tiles (persistent_gemm.hip; K % 8 == 0, N % 8 == 0)
 template <typename T, bool GLU>
 static int dispatch_cfg(GemmArgs a, int cfg, hipStream_t s) {
@@ -896,14 +897,7 @@ static int pick_cfg(const GemmArgs& a) {
   const long avg = a.E > 0 ? (long)a.L / a.E : a.L;  // rows per expert if the load were uniform
   if (avg >= 192 && mi_gemm_persistent_ok(a)) return 7;
   if (avg >= 512) return 0;
-  if (avg >= 48) return a.K % 32 == 0 ? 4 : 1;
-  // A few rows per expert: every weight byte is used once and the kernel is a weight stream, which wants many
-  // workgroups.  Measured at 8 - 256 tokens (kernel times, up / down projection): hidden 1536, 40 experts -- 32 x 256
-  // tiles 29 - 31 / 13.5 - 17 us, 32 x 128 tiles 23 - 27 / 12 - 17 us, DMA-staged 128 x 128 tiles 28 - 30 / 13 - 16 us;
-  // hidden 1024, 32 experts -- 20 - 22 / 12 - 15, 16 - 21 / 9 - 13, 15 - 16 / 9 - 11 us.  A very long contraction
-  // (the down-projection of an intermediate size of 14336: 226 against 188 us at 64 tokens) wants the deeper ring of
-  // the DMA-staged kernel too.
-  return (a.K % 32 == 0 && (a.K <= 1024 || a.K >= 8192)) ? 4 : 5;
+  return a.K % 32 == 0 ? 4 : 1;
 }
 
 // cfg < 0 picks a matrix-core kernel from the shape.  Nothing drops to the one-thread-per-output kernel on its own:
@@ -935,6 +929,8 @@ static int run_gemm(GemmArgs a, int dtype, bool glu, int cfg, int in_rows_bound,
   const int elt = dtype == MI_MOE_F32 ? 4 : 2;
   if (!tiled_shape_ok(a, in_rows_bound, glu, elt)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, elt)) return MI_MOE_EALIGN;
+  if (cfg >= 100) return mi_gemm_stream(a, dtype, glu, (cfg - 100) / 10, cfg % 10, s);
+  if (cfg < 0 && mi_gemm_stream_pick(a, elt)) return mi_gemm_stream(a, dtype, glu, 0, 0, s);
   if (dtype == MI_MOE_F32) {
     if (cfg < 0) {
       // fp32 matrix instructions are slow enough that what matters is how many CUs have a tile.  Measured (up /
@@ -961,6 +957,15 @@ static int check_common(const void* in, const void* w, void* out, const int32_t*
   if (!in || !w || !out || !off) return MI_MOE_ENULL;
   if (need_ss && !ss) return MI_MOE_ENULL;
   return MI_MOE_OK;
+}
+
+int mi_gemm_one_expert(const void* in, const void* w, void* out, int L, int K, int N, bool glu, int dtype, mi_moe_stream_t stream) {
+  GemmArgs a;
+  a.in = in; a.w = w; a.out = out;
+  a.sorted_scattered = nullptr; a.expert_offsets = nullptr;
+  a.L = L; a.K = K; a.N = N; a.E = 1; a.kdiv = 1; a.n_tiles = 0;
+  a.gather = 0; a.scatter = 0; a.remap = 1; a.ws = nullptr; a.pre = nullptr;
+  return run_gemm(a, dtype, glu, -1, L, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mi_moe_scattered_gemm_ws(const void* in, const void* w, void* out, const int32_t* sorted_scattered,

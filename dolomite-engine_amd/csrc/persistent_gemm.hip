@@ -129,7 +129,7 @@ struct PgTable {
   int incl[4], end[4];
   int total;  // row tiles of all experts
 };
-template <int BM> __device__ __forceinline__ void pg_table(const int32_t* __restrict__ off, int E, PgTable& tb) {
+template <int BM> __device__ __forceinline__ void pg_table(const int32_t* __restrict__ off, int L, int E, PgTable& tb) {
   const int lane = threadIdx.x & 63;
   int carry = 0;
 #pragma unroll
@@ -138,7 +138,7 @@ template <int BM> __device__ __forceinline__ void pg_table(const int32_t* __rest
     tb.end[c] = 0;
     if (c * 64 >= E) continue;
     const int e = c * 64 + lane;
-    const int end = e < E ? off[e] : 0;
+    const int end = e < E ? mi_expert_end(off, L, e) : 0;
     const int prev = (e < E && e > 0) ? off[e - 1] : 0;
     int incl = e < E ? (end - prev + BM - 1) / BM : 0;
 #pragma unroll
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
 
   // ---- which tiles -----------------------------------------------------------------------------------------------
   PgTable tb;
-  pg_table<BM>(a.expert_offsets, a.E, tb);
+  pg_table<BM>(a.expert_offsets, a.L, a.E, tb);
   const int total = tb.total * a.n_tiles;
   const int nfull = a.K / PG_BK;                    // whole slices; a partial one is padded with zeros
   int nk = (a.K + PG_BK - 1) / PG_BK;
@@ -656,7 +656,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_split_finish_kernel(GemmArgs
   constexpr int BM = 256, BN = GLU ? 128 : 256;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
   PgTable tb;
-  pg_table<BM>(a.expert_offsets, a.E, tb);
+  pg_table<BM>(a.expert_offsets, a.L, a.E, tb);
   // contiguous: workgroup b adds up tile b / 8 of XCD b % 8's last round; interleaved: tile b of the chip's last round
   const bool interleave = (a.remap & PERSIST_REMAP_INTERLEAVE) != 0;
   const int xcd = interleave ? 0 : (int)(blockIdx.x & 7), j = interleave ? (int)blockIdx.x : (int)(blockIdx.x >> 3);

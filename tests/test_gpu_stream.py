@@ -1,0 +1,39 @@
+"""The weight-stream form of the grouped GEMM at the sizes where its units can go wrong: one row, rows around a block of
+16 and around a chunk, experts without rows, contractions of one slice, shorter than the ring, with a partial last slice
+and of fewer slices than waves, and output columns that end inside a unit.  Against an fp32 product of the same rounded
+operands (float64 for fp32): 16-bit results carry one rounding, half a unit in the last place; fp32 results differ by the
+order of at most 1000 sums of magnitude below 1 (relative 1e-5 of the largest)."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.bfloat16: dict(rtol=2.0 ** -8, atol=2e-3), torch.float16: dict(rtol=2.0 ** -11, atol=5e-4),
+       torch.float32: dict(rtol=1e-5, atol=2e-5)}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("counts,K,N", [([1], 64, 32), ([0, 1, 0, 17, 16, 15], 136, 72), ([33, 32, 31, 0, 64, 65], 1000, 260),
+                                        ([2] * 70, 8, 16), ([5, 0, 3], 512, 1536), ([40, 1], 264, 28)])
+@pytest.mark.parametrize("cfg", [-1, 111, 112, 114, 121, 122, 124, 141, 142])
+def test_stream_edges(device, dtype, counts, K, N, cfg):
+    from dolomite_engine_amd import ops
+
+    g = torch.Generator().manual_seed(K + N + len(counts))
+    E, L, k = len(counts), sum(counts), 1
+    print(f"stream E={E} L={L} K={K} N={N} cfg={cfg} {dtype}", flush=True)
+    off = torch.tensor(counts).cumsum(0).int().to(device)
+    ss = torch.randperm(L, generator=g).int().to(device)
+    x = torch.randn(L, K, generator=g).to(dtype).to(device)
+    w = (torch.randn(E, 2 * N, K, generator=g) * 0.05).to(dtype).to(device)
+    wide = torch.float64 if dtype == torch.float32 else torch.float32
+    ref = torch.cat([p.to(wide) @ w[e].to(wide).t() for e, p in enumerate(x.split(counts))])
+    plain = ops.scattered_gemm(x, w, k, ss, off, True, False, cfg=cfg)
+    torch.testing.assert_close(plain[ss.long()].to(wide), ref, **TOL[dtype])
+    by_slot = torch.empty_like(x)
+    by_slot[ss.long()] = x
+    assert torch.equal(ops.scattered_gemm(by_slot, w, k, ss, off, False, False, cfg=cfg), plain)
+    act = ops.up_swiglu(by_slot, w, k, ss, off, cfg=cfg)
+    want = ref[:, :N] * torch.nn.functional.silu(ref[:, N:])
+    torch.testing.assert_close(act.to(wide), want, **TOL[dtype])
