@@ -238,6 +238,21 @@ class MoE(nn.Module):
         if residual is not None:
             residual = residual.reshape(-1, self.hidden_size)
 
+        if (
+            not self.training
+            and self._fused_swiglu
+            and is_kernel_allowed(Kernel.scattermoe)
+            and hidden_states.is_cuda
+            and ops._TIMER is None
+            and not self._needs_grad(hidden_states)
+            and isinstance(self.dropout, nn.Identity)
+        ):
+            # inference: all stages behind one library call (None: something the stage-by-stage code below has to look at)
+            y = self._forward_native(hidden_states, residual, residual_scale, pre_norm)
+            if y is not None:
+                add_aux_loss(0)
+                return y if self.use_padding_free_transformer else y.reshape(batch_size, sequence_length, self.hidden_size)
+
         routed = None
         presorted = None
         if pre_norm is None and self._use_fused_router(hidden_states) and ops.router_fused_sort_supported(
@@ -309,6 +324,49 @@ class MoE(nn.Module):
 
         return hidden_states
 
+    def _forward_native(self, hidden_states: torch.Tensor, residual: torch.Tensor | None,
+                        residual_scale: float | None, pre_norm: tuple | None) -> torch.Tensor | None:
+        """The whole eval-mode forward through ops.layer_forward; None where it does not take the call."""
+        fc, proj = self.c_fc, self.c_proj
+        if fc.bias is not None or proj.bias is not None:
+            return None
+        shared_fc = shared_proj = None
+        if self.shared_intermediate_size is not None:
+            if self.c_fc_shared.bias is not None or self.c_proj_shared.bias is not None:
+                return None
+            shared_fc, shared_proj = self.c_fc_shared.weight, self.c_proj_shared.weight
+        weight_q = fc.weight_q
+        if weight_q is not None:
+            weights = (weight_q, proj.weight_q, fc.weight_scale, proj.weight_scale)
+            if weights[1] is None:
+                return None
+        else:
+            weights = (fc.weight, proj.weight, None, None)
+            if weights[1] is None:
+                return None
+        gate_weight = self.gate.weight
+        logits = None
+        if pre_norm is None and not ops.router_fused_supported(hidden_states, self.num_experts, self.top_k):
+            logits = self._unfused_logits(hidden_states)
+        return ops.layer_forward(hidden_states, gate_weight, self.router_logit_bias, self.top_k, *weights,
+                                 shared_fc, shared_proj, residual, residual_scale, pre_norm, logits)
+
+    def _unfused_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
+        """Router logits of shapes the router kernel does not take (more than 256 experts, a hidden size that is not a
+        multiple of 16): they come from torch, the selection still follows the kernel's tie rule (value descending,
+        expert index ascending) in training and in inference alike."""
+        ops._warn_once(("router_unfused", self.num_experts, self.hidden_size, hidden_states.dtype),
+                       f"MoE router with {self.num_experts} experts, hidden size {self.hidden_size}, "
+                       f"{hidden_states.dtype}: not a shape of the fused router kernel; the logits are computed "
+                       "by torch's linear layer")
+        return self._biased_logits(hidden_states)
+
+    def _biased_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
+        router_logits = self.gate(hidden_states)
+        if self.router_logit_bias is not None:
+            router_logits = (router_logits.float() + self.router_logit_bias.float()).to(router_logits.dtype)
+        return router_logits
+
     def _needs_grad(self, hidden_states: torch.Tensor) -> bool:
         return torch.is_grad_enabled() and (
             hidden_states.requires_grad or any(p.requires_grad for p in self.parameters())
@@ -343,18 +401,8 @@ class MoE(nn.Module):
             return (*ops.router_fused(hidden_states, self.gate.weight, self.top_k, bias=self.router_logit_bias,
                                       return_logits=self.training), None)
 
-        router_logits = self.gate(hidden_states)
-        if self.router_logit_bias is not None:
-            router_logits = (router_logits.float() + self.router_logit_bias.float()).to(router_logits.dtype)
-
         if is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda:
-            # shapes the router kernel does not take (more than 256 experts, a hidden size that is not a multiple
-            # of 16): the logits come from torch, the selection still follows the kernel's tie rule (value
-            # descending, expert index ascending) in training and in inference alike
-            ops._warn_once(("router_unfused", self.num_experts, self.hidden_size, hidden_states.dtype),
-                           f"MoE router with {self.num_experts} experts, hidden size {self.hidden_size}, "
-                           f"{hidden_states.dtype}: not a shape of the fused router kernel; the logits are computed "
-                           "by torch's linear layer")
+            router_logits = self._unfused_logits(hidden_states)
             with torch.no_grad():
                 router_weights, selected_experts = ops.router_topk_softmax(router_logits.detach(), self.top_k)
             if torch.is_grad_enabled() and router_logits.requires_grad:
@@ -363,6 +411,7 @@ class MoE(nn.Module):
                 picked = router_logits.gather(-1, selected_experts.long())
                 router_weights = F.softmax(picked.float(), dim=-1).type_as(hidden_states)
         else:
+            router_logits = self._biased_logits(hidden_states)
             router_weights, selected_experts = self._get_topk(router_logits)
             router_weights = F.softmax(router_weights.float(), dim=-1)
             router_weights = router_weights.type_as(hidden_states)

@@ -13,6 +13,8 @@ compositions are in ``autograd.py``).
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -907,3 +909,81 @@ def down_fp8(act: torch.Tensor, w_proj_q: torch.Tensor, w_proj_scale: torch.Tens
         check(lib.mi_moe_down_fp8_cfg(_ptr(act), _ptr(w_proj_q), _ptr(scale), _ptr(o), _ptr(ss), _ptr(off), L, I, H,
                                      E, _code(act.dtype), int(tiled), int(cfg), _stream()))
     return o
+
+
+# ------------------------------------------------------------------------------------------------
+# the whole inference forward
+# ------------------------------------------------------------------------------------------------
+
+
+@functools.lru_cache(maxsize=256)
+def _layer_sizes(T: int, H: int, E: int, k: int, I: int, S: int, code: int, has_norm: int) -> tuple[int, int]:
+    """(workspace bytes, contraction length that may use the split-K workspace or 0): functions of the sizes alone."""
+    lib = _lib.load()
+    splits = 0
+    if code != F32:
+        splits = next((K for K in (H, I) if lib.mi_moe_grouped_gemm_splits(K, code)), 0)
+    return lib.mi_moe_layer_workspace_bytes(T, H, E, k, I, S, code, has_norm), splits
+
+
+def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor | None, k: int, w_fc: torch.Tensor,
+                  w_proj: torch.Tensor, fc_scale: torch.Tensor | None, proj_scale: torch.Tensor | None,
+                  shared_fc: torch.Tensor | None, shared_proj: torch.Tensor | None, residual: torch.Tensor | None,
+                  residual_scale: float | None, pre_norm: tuple | None, logits: torch.Tensor | None = None):
+    """The eval-mode forward of a SwiGLU layer without biases in one library call: the launches of the single stages, in
+    their order, with every intermediate in one workspace.  Returns y (T, H), or None for anything the stages' own
+    wrappers have to look at (another device or dtype, strided operands, shapes outside the kernels' granularity, fp8
+    weights that are widened for the call); nothing has run then."""
+    dev, dtype = x.get_device(), x.dtype
+    code = _DTYPE_CODE.get(dtype)
+    if code is None or dev < 0 or dev != _current_device() or x.dim() != 2 or not x.is_contiguous():
+        return None
+    T, H = x.shape
+    E = gate_weight.shape[0]
+    fp8 = fc_scale is not None
+    I = (fc_scale if fp8 else w_fc).shape[1] // 2
+    S = 0 if shared_fc is None else shared_fc.shape[0] // 2
+    unit = 4 if code == F32 else (16 if fp8 else 8)
+    if T < 1 or H % unit or I % unit or S % (4 if code == F32 else 8) or gate_weight.shape[1] != H:
+        return None
+    norm_w, eps = (None, 0.0) if pre_norm is None else pre_norm
+    same = [gate_weight]
+    if fp8:
+        if T * k >= FP8_DENSE_ROWS_PER_EXPERT * E or w_fc.dtype != torch.float8_e4m3fn or w_proj.dtype != torch.float8_e4m3fn:
+            return None
+        for t in (w_fc, w_proj, fc_scale, proj_scale):
+            if t.get_device() != dev or not t.is_contiguous():
+                return None
+        if fc_scale.dtype != torch.float32 or proj_scale.dtype != torch.float32:
+            return None
+    else:
+        same += (w_fc, w_proj)
+    for t in (shared_fc, shared_proj, residual, norm_w, logits):
+        if t is not None:
+            same.append(t)
+    for t in same:
+        if t.dtype != dtype or t.get_device() != dev or not t.is_contiguous():
+            return None
+    if residual is not None and residual.shape != x.shape:
+        return None
+    if bias is not None and (bias.dtype != torch.float32 or bias.get_device() != dev or not bias.is_contiguous()):
+        return None
+    if pre_norm is not None:
+        if not rmsnorm_router_fused_supported(x, E, k) or (norm_w is not None and norm_w.shape != (H,)):
+            return None
+    elif logits is None and not router_fused_supported(x, E, k):
+        return None
+    ws_bytes, splits = _layer_sizes(T, H, E, k, I, S, code, pre_norm is not None)
+    y = torch.empty_like(x)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+    gemm_ws, gemm_bytes = _gemm_workspace(x.device, splits, dtype) if splits else (None, 0)
+    rc = _lib.load().mi_moe_layer_forward(
+        x.data_ptr(), _ptr(norm_w), eps, pre_norm is not None, gate_weight.data_ptr(), _ptr(bias), _ptr(logits),
+        w_fc.data_ptr(), _ptr(fc_scale), w_proj.data_ptr(), _ptr(proj_scale),
+        (int(w_fc.dim() == 1) | int(w_proj.dim() == 1) << 1) if fp8 else 0, _ptr(shared_fc), _ptr(shared_proj), _ptr(residual),
+        1.0 if residual_scale is None else residual_scale, residual_scale is not None, y.data_ptr(), T, H, E, k, I, S, code,
+        ws.data_ptr(), ws_bytes, _ptr(gemm_ws), gemm_bytes, _RAW_STREAM(dev) if _RAW_STREAM is not None else _stream())
+    if rc in (_lib.MI_MOE_EUNSUPPORTED, _lib.MI_MOE_EALIGN):
+        return None
+    check(rc)
+    return y

@@ -410,6 +410,25 @@ int mi_moe_down_fp8_cfg(const void* act, const void* w_proj_q, const float* w_pr
 int mi_moe_fp8_dequant(const void* w_q, const float* w_scale, void* w_out, int E, int out, int in, int glu,
                        int w_tiled, int dtype, mi_moe_stream_t stream);
 
+/* ---- the whole inference forward -------------------------------------------------------------------------------------
+ * MoE.forward in eval mode (moe.py:212-290) with a SwiGLU activation, as one call: the launches of the entry points above in
+ * the order the layer runs them, every intermediate in one workspace.
+ *   x (T, H); has_norm: x is first RMS-normalised with weight norm_w (H, or NULL) and norm_eps (mi_moe_rmsnorm_router_fused);
+ *   gate_w (E, H) with gate_bias (E floats, or NULL), or logits (T, E) already formed by the caller (then gate_w is not read);
+ *   w_fc (E, 2I, H), w_proj (E, H, I) of `dtype`, or e4m3fn bytes when fc_scale / proj_scale (fp32, E x rows) are given, bit 0 /
+ *   bit 1 of w_tiled saying that w_fc / w_proj is in the streamed-tile order;
+ *   S > 0: shared experts shared_fc (2S, H), shared_proj (H, S); residual (T, H) or NULL, residual_scale if has_scale, as in
+ *   mi_moe_combine_block_tail; y (T, H).
+ * ws: mi_moe_layer_workspace_bytes() bytes, 256-byte aligned; gemm_ws: as in the _ws calls (or NULL).  Shapes that one of the
+ * stages does not take return that stage's code; launches before it have then run, y has not been written. */
+size_t mi_moe_layer_workspace_bytes(int T, int H, int E, int k, int I, int S, int dtype, int has_norm);
+int mi_moe_layer_forward(const void* x, const void* norm_w, float norm_eps, int has_norm, const void* gate_w,
+                         const float* gate_bias, const void* logits, const void* w_fc, const float* fc_scale,
+                         const void* w_proj, const float* proj_scale, int w_tiled, const void* shared_fc,
+                         const void* shared_proj, const void* residual, float residual_scale, int has_scale, void* y,
+                         int T, int H, int E, int k, int I, int S, int dtype, void* ws, size_t ws_bytes, void* gemm_ws,
+                         size_t gemm_ws_bytes, mi_moe_stream_t stream);
+
 /*
  * Diagnostics (no counterpart in the reference; nothing in the layer calls them): the pieces of the persistent
  * grouped GEMM's inner loop in isolation, for a benchmark that wants a measured ceiling beside the GEMM's own

@@ -1,0 +1,58 @@
+"""The eval-mode forward behind one library call against the stage-by-stage calls it stands for: the same kernels on the
+same inputs in the same order, so the results are equal bit for bit.  (An installed stage timer makes the module run its
+stages one by one.)"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+class _Timer:
+    def __init__(self):
+        self.stages = []
+
+    def begin(self, name):
+        self.stages.append(name)
+
+    def end(self, name):
+        pass
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,E,k,I,shared,fp8,norm,tail", [
+    (1, 1536, 40, 8, 512, None, False, True, True), (64, 1024, 32, 8, 512, None, False, False, False),
+    (1, 64, 4, 1, 32, 16, False, False, True), (333, 920, 17, 4, 520, 344, False, False, False),
+    (700, 256, 8, 2, 512, 64, False, True, False), (40, 512, 64, 6, 256, None, True, False, True),
+    (900, 512, 8, 2, 384, None, True, False, False), (50, 256, 130, 4, 64, None, False, False, False),
+    (2000, 256, 8, 2, 128, None, True, False, False),  # so many rows per expert that the fp8 weights are widened
+])
+def test_native_forward_equals_stages(device, dtype, T, H, E, k, I, shared, fp8, norm, tail):
+    from dolomite_engine_amd import Kernel, MoE, enable_kernels, ops
+
+    if fp8 and dtype == torch.float32:
+        pytest.skip("fp8 weights go with 16-bit activations")
+    torch.manual_seed(T + H)
+    m = MoE(hidden_size=H, intermediate_size=I, shared_intermediate_size=shared, num_experts=E, num_experts_per_tok=k,
+            activation_function="swiglu", add_bias=False, dropout=0.0, init_method="normal", initializer_range=0.05,
+            m_width=None, num_layers=1, use_padding_free_transformer=True).to(dtype).to(device).eval()
+    if fp8:
+        m.quantize_expert_weights_fp8()
+    x = torch.randn(T, H, device=device, dtype=dtype)
+    kwargs = {}
+    if norm:
+        kwargs["pre_norm"] = (1 + 0.1 * torch.randn(H, device=device, dtype=dtype), 1e-5)
+    if tail:
+        kwargs.update(residual=torch.randn(T, H, device=device, dtype=dtype), residual_scale=0.22)
+    timer = _Timer()
+    with torch.no_grad(), enable_kernels([Kernel.scattermoe]):
+        native = m(x, **kwargs)
+        ops.set_stage_timer(timer)
+        try:
+            stages = m(x, **kwargs)
+        finally:
+            ops.set_stage_timer(None)
+        again = m(x, **kwargs)
+    assert timer.stages, "the second forward was meant to run stage by stage"
+    assert torch.equal(native, stages)
+    assert torch.equal(native, again)
