@@ -42,6 +42,14 @@ bool mi_gemm_persistent_ok(const GemmArgs& a);
 bool mi_gemm_persistent_splits(int K);
 int mi_gemm_persistent(const GemmArgs& a, int dtype, int form, hipStream_t s);
 
+// ---- persistent_fp8.hip: fp8 weights (wscale, w_tiled); K % 16 == 0, K > 256, N % 8 == 0, at most PERSIST_MAX_E experts,
+// 16-byte aligned output ----------------------------------------------------------------------------------------------
+enum { FP8_BY_SHAPE = 1, FP8_PERSISTENT = 3, FP8_STAGED = 4 };  // forms of mi_gemm_fp8_tiled
+bool mi_gemm_fp8_persistent_ok(const GemmArgs& a);
+// whether they are the faster form than the register-staged tiles
+bool mi_gemm_fp8_persistent_pick(int L, int K, int N, int E, bool glu);
+int mi_gemm_fp8_persistent(const GemmArgs& a, int dtype, bool glu, hipStream_t s);
+
 // ---- stream_gemm.hip: K a multiple of one 16-byte chunk, N % 4 == 0 ------------------------------------------------------
 // whether the stream is the faster form for this problem (elt: bytes of an element)
 bool mi_gemm_stream_pick(const GemmArgs& a, int elt);

@@ -786,8 +786,21 @@ static int launch_dma(GemmArgs a, hipStream_t s) {
   return mi_launch_status();
 }
 
-// fp8 expert weights on the register-staged tiles: out[orow(i)] = scale[e_i] * (in[irow(i)] @ Wq[e_i]^T), with SwiGLU
-// over the [up ; gate] halves when glu.  Called by decode_fp8.hip for batches beyond a few rows per expert (the
+// Cache policy of the persistent kernel's output stores.  The plain form's output -- the (slots, hidden) rows the
+// combine streams once -- is stored non-temporal, so that it does not push the operands out of the caches:
+// down-projection of the 16384-token, 32-expert shape 0.169 -> 0.146 ms (its combine 0.048 -> 0.053 ms), little
+// either way on the other shapes.  The SwiGLU form's output is the next GEMM's operand: up to about the size the
+// memory-side cache can hold next to the weights it stays cached (134 MB on that shape: non-temporal stores would
+// make the GEMM that reads it back 8 % slower); beyond that it would not survive until it is read and only evicts
+// the operands on its way (268 MB on the 32768-token, 40-expert shape: both GEMMs 1 % faster non-temporal).
+static int persistent_out_nt(const GemmArgs& a, bool glu, int elt) {
+  if (!glu) return 1;
+  return (double)a.L * a.N * elt > 192.0 * 1024 * 1024;
+}
+
+// fp8 expert weights on tiles: out[orow(i)] = scale[e_i] * (in[irow(i)] @ Wq[e_i]^T), with SwiGLU over the [up ; gate]
+// halves when glu -- the persistent kernel of persistent_fp8.hip, or the register-staged tiles for what it does not take
+// and for small problems.  Called by decode_fp8.hip for batches beyond a few rows per expert (the
 // streaming kernels there read an expert's weights once per 16 of its rows).  Shapes: K % 16 == 0, N % 4 == 0,
 // w_tiled only with K % 128 == 0; MI_MOE_EUNSUPPORTED otherwise.
 template <typename T, bool GLU>
@@ -800,7 +813,7 @@ static int dispatch_w8(const GemmArgs& a, hipStream_t s) {
 
 int mi_gemm_fp8_tiled(const void* in, const void* wq, const float* scale, void* out, const int32_t* sorted_scattered,
                       const int32_t* expert_offsets, int L, int K, int N, int E, int kdiv, int gather, int scatter,
-                      int glu, int w_tiled, int dtype, hipStream_t s) {
+                      int glu, int w_tiled, int dtype, int form, hipStream_t s) {
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16) return MI_MOE_EDTYPE;
   if (L == 0) return MI_MOE_OK;
   if (K % 16 != 0 || N % 4 != 0 || (w_tiled && K % 128 != 0)) return MI_MOE_EUNSUPPORTED;
@@ -816,6 +829,9 @@ int mi_gemm_fp8_tiled(const void* in, const void* wq, const float* scale, void* 
   a.L = L; a.K = K; a.N = N; a.E = E; a.kdiv = kdiv > 0 ? kdiv : 1; a.kshift = -1; a.n_tiles = 0;
   a.gather = gather; a.scatter = scatter; a.remap = 1; a.ws = nullptr; a.pre = nullptr; a.out_nt = 0;
   a.wscale = scale; a.w_tiled = w_tiled;
+  a.out_nt = persistent_out_nt(a, glu != 0, 2);
+  if (form == FP8_PERSISTENT || (form == FP8_BY_SHAPE && mi_gemm_fp8_persistent_ok(a) && mi_gemm_fp8_persistent_pick(L, K, N, E, glu != 0)))
+    return mi_gemm_fp8_persistent(a, dtype, glu != 0, s);
   if (dtype == MI_MOE_BF16) return glu ? dispatch_w8<bf16_t, true>(a, s) : dispatch_w8<bf16_t, false>(a, s);
   return glu ? dispatch_w8<f16_t, true>(a, s) : dispatch_w8<f16_t, false>(a, s);
 }
@@ -903,18 +919,6 @@ static int pick_cfg(const GemmArgs& a) {
 // cfg < 0 picks a matrix-core kernel from the shape.  Nothing drops to the one-thread-per-output kernel on its own:
 // a problem the matrix-core kernels cannot take is refused (MI_MOE_EALIGN for a misaligned pointer,
 // MI_MOE_EUNSUPPORTED for the shape) and the caller asks for cfg 3 explicitly if it wants the slow kernel.
-// Cache policy of the persistent kernel's output stores.  The plain form's output -- the (slots, hidden) rows the
-// combine streams once -- is stored non-temporal, so that it does not push the operands out of the caches:
-// down-projection of the 16384-token, 32-expert shape 0.169 -> 0.146 ms (its combine 0.048 -> 0.053 ms), little
-// either way on the other shapes.  The SwiGLU form's output is the next GEMM's operand: up to about the size the
-// memory-side cache can hold next to the weights it stays cached (134 MB on that shape: non-temporal stores would
-// make the GEMM that reads it back 8 % slower); beyond that it would not survive until it is read and only evicts
-// the operands on its way (268 MB on the 32768-token, 40-expert shape: both GEMMs 1 % faster non-temporal).
-static int persistent_out_nt(const GemmArgs& a, bool glu, int elt) {
-  if (!glu) return 1;
-  return (double)a.L * a.N * elt > 192.0 * 1024 * 1024;
-}
-
 static int run_gemm(GemmArgs a, int dtype, bool glu, int cfg, int in_rows_bound, hipStream_t s) {
   a.out_nt = persistent_out_nt(a, glu, dtype == MI_MOE_F32 ? 4 : 2);
   if (a.L == 0) return MI_MOE_OK;

@@ -29,6 +29,7 @@
 // 0.80 with DMA.
 #include "gemm_common.h"
 #include "mfma_core.h"
+#include "persistent_tiles.h"
 
 
 #define PG_BK 64        // K slice: one 128-byte line of a 16-bit row
@@ -41,12 +42,8 @@
 // part writes its fp32 accumulators to the workspace instead of running the epilogue, and a second, small launch
 // (grouped_gemm_split_finish_kernel) adds the parts of every split tile in part order and runs the epilogue, so
 // the result does not depend on timing.  A round is only split if that shortens it by at least
-// PERSIST_SPLIT_MIN_SAVED slices: the partial tiles' trip through memory and the second launch cost 40-80 us
+// PERSIST_SPLIT_MIN_SAVED (persistent_tiles.h) slices: the partial tiles' trip through memory and the second launch cost 40-80 us
 // (measured), about 50 slices' worth.
-#define PERSIST_SPLIT_MAX 4
-#define PERSIST_SPLIT_MIN_SAVED 60
-#define PERSIST_SPLIT_MIN_SLICES 16
-
 // whether a contraction of length K can be shortened by PERSIST_SPLIT_MIN_SAVED slices at all (launch_persistent
 // applies the same rule, plus one on the grid)
 static bool persistent_may_split(int K) {
@@ -54,134 +51,6 @@ static bool persistent_may_split(int K) {
   return nk - nk / PERSIST_SPLIT_MAX >= PERSIST_SPLIT_MIN_SAVED;
 }
 
-// Which tiles a workgroup runs.  Workgroup b sits on XCD b % 8 (the hardware deals workgroup ids round-robin to the
-// XCDs) in slot b / 8.  Two ways of dealing the band-ordered tile list to them:
-//   * contiguous (the default): XCD x owns the x-th eighth of the list and deals it to its slots in turn, so the
-//     CUs of an XCD work on neighbouring tiles out of one L2 and an XCD stays with its experts;
-//   * interleaved (PERSIST_REMAP_INTERLEAVE): round r of the whole chip is the tiles [r * grid, (r + 1) * grid), XCD
-//     x taking the x-th run of grid / 8 of them.  All XCDs then work on neighbouring tiles at the same time.  When
-//     an expert has more column tiles than a band is wide (intermediate size 14336: 112 column tiles, bands of 8),
-//     consecutive bands read the same activation rows, and the XCDs share them through the memory-side cache
-//     instead of each fetching them from HBM in its own time: Mixtral-shape layer 5.02 -> 4.73 ms.  With few
-//     column tiles (the band is the whole row) it changes little either way (-1.3 % on the Granite-1B shape,
-//     +1.1 % on the Granite-3B shape), so the host asks for it only from 8 column tiles on.
-// Either way the tiles that do not fill the last round can be cut along K (see PERSIST_SPLIT_MAX).
-
-struct SplitPlan {
-  int base, stride;  // tile of this workgroup in round i < full_rounds: base + i * stride
-  int full_rounds;   // rounds in which every slot has a tile
-  int rem;           // tiles of the last round, the first of them being rem_base
-  int rem_base;
-  int parts;         // K ranges each of them is cut into (1: not split)
-  int lslot;         // this workgroup's slot in the last round: part lslot / rem of tile rem_base + lslot % rem
-  int ws_base;       // first partial-tile slot of the last round's tiles in the workspace
-};
-
-// xcd / slot of the workgroup (slot < nslot); for the finishing kernel, slot is the tile of the last round it adds up
-__device__ __forceinline__ SplitPlan persist_split_plan(int total, int xcd, int slot, int nslot, int nk, bool have_ws,
-                                                        bool interleave) {
-  SplitPlan sp;
-  int cap;  // slots that share one last round
-  if (interleave) {
-    cap = nslot * 8;
-    sp.lslot = xcd * nslot + slot;
-    sp.base = sp.lslot;
-    sp.stride = cap;
-    sp.full_rounds = total / cap;
-    sp.rem = total - sp.full_rounds * cap;
-    sp.rem_base = sp.full_rounds * cap;
-    sp.ws_base = 0;
-  } else {
-    cap = nslot;
-    const int per = (total + 7) >> 3;
-    int n_x = total - xcd * per;
-    n_x = n_x < 0 ? 0 : (n_x < per ? n_x : per);
-    sp.lslot = slot;
-    sp.base = xcd * per + slot;
-    sp.stride = nslot;
-    sp.full_rounds = n_x / nslot;
-    sp.rem = n_x - sp.full_rounds * nslot;
-    sp.rem_base = xcd * per + sp.full_rounds * nslot;
-    sp.ws_base = xcd * nslot;
-  }
-  sp.parts = 1;
-  if (have_ws && sp.rem > 0) {
-    int p = cap / sp.rem;
-    if (p > PERSIST_SPLIT_MAX) p = PERSIST_SPLIT_MAX;
-    if (p >= 2 && nk / p >= PERSIST_SPLIT_MIN_SLICES && nk - nk / p >= PERSIST_SPLIT_MIN_SAVED) sp.parts = p;
-  }
-  return sp;
-}
-
-
-
-struct PgTile {
-  int expert, nt, row_begin, row_end;
-};
-
-// The tile list of one workgroup, a lane per tile (64 tiles at a time).  A lane of the four table registers holds an
-// expert: row tiles of experts 0..e and the end of its rows.  An expert's tiles are numbered band by band: a band is
-// up to 8 column tiles wide and runs over all of the expert's row tiles, row tile slowest.  The 32 workgroups of an
-// XCD, which take 32 consecutive tiles at a time, then cover about 4 row tiles x 8 column tiles: 12 operand slabs for
-// 32 tiles, and each weight slab is fetched once per band instead of once per row tile.  Up to 8 column tiles the
-// band is the whole row, so that complete output rows are written at about the same time.
-struct PgTable {
-  int incl[4], end[4];
-  int total;  // row tiles of all experts
-};
-template <int BM> __device__ __forceinline__ void pg_table(const int32_t* __restrict__ off, int L, int E, PgTable& tb) {
-  const int lane = threadIdx.x & 63;
-  int carry = 0;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    tb.incl[c] = 0;
-    tb.end[c] = 0;
-    if (c * 64 >= E) continue;
-    const int e = c * 64 + lane;
-    const int end = e < E ? mi_expert_end(off, L, e) : 0;
-    const int prev = (e < E && e > 0) ? off[e - 1] : 0;
-    int incl = e < E ? (end - prev + BM - 1) / BM : 0;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    tb.incl[c] = incl + carry;
-    tb.end[c] = end;
-    carry += __builtin_amdgcn_readlane(incl, 63);
-  }
-  tb.total = carry;
-}
-template <int BM> __device__ __forceinline__ PgTile pg_locate(const PgTable& tb, int E, int n_tiles, int tile) {
-  const int q = tile / n_tiles;  // experts own contiguous tile ranges: (row tiles before) * n_tiles
-  int ex = 0, first = 0, prev = 0, incl = 0x7fffffff, rend = 0x7fffffff;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int n = E - c * 64 < 64 ? E - c * 64 : 64;
-    for (int l = 0; l < n; ++l) {
-      const int s = __builtin_amdgcn_readlane(tb.incl[c], l), en = __builtin_amdgcn_readlane(tb.end[c], l);
-      const bool past = q >= s;
-      ex += past ? 1 : 0;
-      first = past ? s : first;
-      prev = past ? en : prev;
-      incl = past ? incl : (s < incl ? s : incl);
-      rend = past ? rend : (en < rend ? en : rend);
-    }
-  }
-  const int tile_band = n_tiles < 8 ? n_tiles : 8;
-  const int local = tile - first * n_tiles, per_band = (incl - first) * tile_band;
-  const int band = local / per_band;
-  const int rem = local - band * per_band;
-  const int left = n_tiles - band * tile_band;
-  const int width = left < tile_band ? left : tile_band;
-  const int mt = rem / width;
-  PgTile t;
-  t.expert = ex;
-  t.nt = band * tile_band + rem - mt * width;
-  t.row_begin = prev + mt * BM;
-  t.row_end = rend;
-  return t;
-}
 
 template <typename T, bool GLU, bool WT, bool KEEP>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArgs a) {

@@ -803,11 +803,18 @@ def fp8_untile(tiled: torch.Tensor, E: int, out_rows: int, K: int, glu: bool) ->
 
 
 # Average rows per expert from which the fp8 calls widen the weights for the call and run the persistent 16-bit
-# kernels instead of the library's own fp8 kernels (streaming for a few rows per expert, tiles that widen the bytes
-# on their way into LDS beyond): the widening is one pass over all weights whatever the batch, and the persistent
-# kernel is the faster GEMM.  Measured on the decode workload's shape (both projections): 384 rows per expert 1.34 ms
-# on the fp8 tiles / 1.58 ms widened, 768 rows 2.27 / 2.23 ms, 1536 rows 4.16 / 3.55 ms.
+# kernels instead of the library's own fp8 kernels: the widening is one pass over all weights whatever the batch, and
+# the 16-bit kernel is the faster GEMM.  Against the library's persistent fp8 tiles it pays from about 3000 rows per
+# expert on (64 experts of 2816 x 4096 and 4096 x 1408 weights, both projections, us, fp8 tiles / widened: 768 rows
+# 1536 / 2040, 1536 rows 2924 / 3173, 2304 rows 4215 / 4295, 3072 rows 5614 / 5473); shapes those tiles do not take run
+# on the register-staged ones, where it pays from 768 (384 rows 1.34 ms / 1.58, 768 rows 2.27 / 2.23).
 FP8_DENSE_ROWS_PER_EXPERT = 768
+FP8_DENSE_ROWS_PERSISTENT = 2816
+
+
+def _fp8_widens(L: int, K: int, N: int, E: int) -> bool:
+    persistent = K > 256 and N % 8 == 0 and E <= 256
+    return L >= (FP8_DENSE_ROWS_PERSISTENT if persistent else FP8_DENSE_ROWS_PER_EXPERT) * E
 
 
 def fp8_dequant(w_q: torch.Tensor, scale: torch.Tensor, in_features: int, glu: bool, dtype: torch.dtype) -> torch.Tensor:
@@ -842,10 +849,11 @@ def up_swiglu_fp8(x: torch.Tensor, w_fc_q: torch.Tensor, w_fc_scale: torch.Tenso
                   widen: bool | None = None, cfg: int = -1) -> torch.Tensor:
     """As up_swiglu with e4m3fn weights and fp32 per-output-channel scales (E, 2I).  The weights are either
     row-major (E, 2I, H) or, as a flat tensor, in the layout of :func:`fp8_tile` (``glu=True``).  From
-    FP8_DENSE_ROWS_PER_EXPERT rows per expert on average the weights are widened for the call and
+    a few thousand rows per expert on average (_fp8_widens) the weights are widened for the call and
     :func:`up_swiglu` runs on the copy (``widen``: True / False force either way).  Below that the library picks
-    between its streaming kernels (decode: a few rows per expert) and the tile kernels that widen the fp8 bytes on
-    their way into LDS (``cfg``: 0 / 1 force either, -1 picks by the batch)."""
+    between its streaming kernels (decode: a few rows per expert) and the tile kernels, which are the persistent fp8
+    tiles or the register-staged ones (``cfg``: 0 / 1 force streaming or tiles, 3 / 4 persistent or staged tiles, -1
+    picks by the batch)."""
     _dev(x, w_fc_q, w_fc_scale, sorted_scattered_idxs, expert_offsets)
     _no_grad(x)
     if w_fc_q.dtype != torch.float8_e4m3fn:
@@ -867,7 +875,7 @@ def up_swiglu_fp8(x: torch.Tensor, w_fc_q: torch.Tensor, w_fc_scale: torch.Tenso
         raise ValueError("shape mismatch")
     if x.shape[0] * k != L:
         raise ValueError("shape mismatch")
-    if (L >= FP8_DENSE_ROWS_PER_EXPERT * E if widen is None else widen) and H % 16 == 0 and L > 0:
+    if (_fp8_widens(L, H, I2 // 2, E) if widen is None else widen) and H % 16 == 0 and L > 0:
         return up_swiglu(x, fp8_dequant(w_fc_q, scale, H, True, x.dtype), k, ss, off)
     act = torch.empty((L, I2 // 2), dtype=x.dtype, device=x.device)
     with _stage("up_swiglu_fp8"):
@@ -880,8 +888,7 @@ def down_fp8(act: torch.Tensor, w_proj_q: torch.Tensor, w_proj_scale: torch.Tens
              sorted_scattered_idxs: torch.Tensor, expert_offsets: torch.Tensor,
              widen: bool | None = None, cfg: int = -1) -> torch.Tensor:
     """Down-projection with e4m3fn weights, row-major (E, H, I) or tiled (:func:`fp8_tile`, ``glu=False``):
-    act (L, I) grouped -> (L, H) in flat-slot order (widened weights from FP8_DENSE_ROWS_PER_EXPERT rows per expert
-    on, ``cfg`` below that, as in :func:`up_swiglu_fp8`)."""
+    act (L, I) grouped -> (L, H) in flat-slot order (``widen`` and ``cfg`` as in :func:`up_swiglu_fp8`)."""
     _dev(act, w_proj_q, w_proj_scale, sorted_scattered_idxs, expert_offsets)
     _no_grad(act)
     if w_proj_q.dtype != torch.float8_e4m3fn:
@@ -902,7 +909,7 @@ def down_fp8(act: torch.Tensor, w_proj_q: torch.Tensor, w_proj_scale: torch.Tens
         raise ValueError("shape mismatch")
     if ss.numel() != L:
         raise ValueError("shape mismatch")
-    if (L >= FP8_DENSE_ROWS_PER_EXPERT * E if widen is None else widen) and I % 16 == 0 and L > 0:
+    if (_fp8_widens(L, I, H, E) if widen is None else widen) and I % 16 == 0 and L > 0:
         return scattered_gemm(act, fp8_dequant(w_proj_q, scale, I, False, act.dtype), 1, ss, off, True, False)
     o = torch.empty((L, H), dtype=act.dtype, device=act.device)
     with _stage("down_fp8"):
@@ -949,7 +956,7 @@ def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor
     norm_w, eps = (None, 0.0) if pre_norm is None else pre_norm
     same = [gate_weight]
     if fp8:
-        if T * k >= FP8_DENSE_ROWS_PER_EXPERT * E or w_fc.dtype != torch.float8_e4m3fn or w_proj.dtype != torch.float8_e4m3fn:
+        if _fp8_widens(T * k, H, I, E) or _fp8_widens(T * k, I, H, E) or w_fc.dtype != torch.float8_e4m3fn or w_proj.dtype != torch.float8_e4m3fn:
             return None
         for t in (w_fc, w_proj, fc_scale, proj_scale):
             if t.get_device() != dev or not t.is_contiguous():

@@ -394,9 +394,10 @@ int mi_moe_down_fp8(const void* act, const void* w_proj_q, const float* w_proj_s
                     const int32_t* sorted_scattered, const int32_t* expert_offsets, int L, int I, int H,
                     int E, int dtype, int w_tiled, mi_moe_stream_t stream);
 /* The same two calls with the kernel family chosen by the caller: cfg -1 picks by the batch (what the calls above
- * do), 0 the streaming kernels (an expert's weights are read once per 16 of its rows: decode), 1 the tile kernels of
- * the grouped GEMM with the fp8 bytes widened on their way into LDS (an expert's weights are read once per row tile:
- * from a few dozen rows per expert on). */
+ * do), 0 the streaming kernels (an expert's weights are read once per 16 of its rows: decode), 1 the tile kernels
+ * (an expert's weights are read once per row tile: from about 14 rows per expert on) as picked by the shape, 3 the persistent
+ * tiles that keep fp8 in LDS (in > 256, out % 8 == 0, E <= 256, 16-byte aligned output; MI_MOE_EUNSUPPORTED otherwise), 4 the
+ * register-staged tiles that widen the bytes on their way into LDS. */
 int mi_moe_up_swiglu_fp8_cfg(const void* x, const void* w_fc_q, const float* w_fc_scale, void* act_out,
                              const int32_t* sorted_scattered, const int32_t* expert_offsets, int L, int H, int I,
                              int E, int k, int dtype, int w_tiled, int cfg, mi_moe_stream_t stream);
