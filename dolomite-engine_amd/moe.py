@@ -330,6 +330,8 @@ class MoE(nn.Module):
         fc, proj = self.c_fc, self.c_proj
         if fc.bias is not None or proj.bias is not None:
             return None
+        if type(proj) is not ParameterizedExperts or proj._forward_hooks or proj._forward_pre_hooks:
+            return None  # (the stage-by-stage code calls the down-projection as a module)
         shared_fc = shared_proj = None
         if self.shared_intermediate_size is not None:
             if self.c_fc_shared.bias is not None or self.c_proj_shared.bias is not None:

@@ -933,14 +933,19 @@ def _layer_sizes(T: int, H: int, E: int, k: int, I: int, S: int, code: int, has_
     return lib.mi_moe_layer_workspace_bytes(T, H, E, k, I, S, code, has_norm), splits
 
 
+@functools.lru_cache(maxsize=256)
+def _fp8_tiled_bytes(E: int, N: int, K: int, glu: int) -> int:
+    return _lib.load().mi_moe_fp8_tiled_bytes(E, N, K, glu)
+
+
 def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor | None, k: int, w_fc: torch.Tensor,
                   w_proj: torch.Tensor, fc_scale: torch.Tensor | None, proj_scale: torch.Tensor | None,
                   shared_fc: torch.Tensor | None, shared_proj: torch.Tensor | None, residual: torch.Tensor | None,
                   residual_scale: float | None, pre_norm: tuple | None, logits: torch.Tensor | None = None):
     """The eval-mode forward of a SwiGLU layer without biases in one library call: the launches of the single stages, in
     their order, with every intermediate in one workspace.  Returns y (T, H), or None for anything the stages' own
-    wrappers have to look at (another device or dtype, strided operands, shapes outside the kernels' granularity, fp8
-    weights that are widened for the call); nothing has run then."""
+    wrappers have to look at (another device or dtype, strided operands, shapes that do not fit together or are
+    outside the kernels' granularity, fp8 weights that are widened for the call); nothing has been kept then."""
     dev, dtype = x.get_device(), x.dtype
     code = _DTYPE_CODE.get(dtype)
     if code is None or dev < 0 or dev != _current_device() or x.dim() != 2 or not x.is_contiguous():
@@ -948,8 +953,24 @@ def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor
     T, H = x.shape
     E = gate_weight.shape[0]
     fp8 = fc_scale is not None
-    I = (fc_scale if fp8 else w_fc).shape[1] // 2
+    I2 = (fc_scale if fp8 else w_fc).shape[1]
+    I = I2 // 2
     S = 0 if shared_fc is None else shared_fc.shape[0] // 2
+    # the library sees pointers only: every operand's shape is the one the sizes above imply
+    if I2 % 2 or (shared_fc is not None and (shared_fc.shape != (2 * S, H) or shared_proj.shape != (H, S))):
+        return None
+    if fp8:
+        if fc_scale.shape != (E, I2) or proj_scale.shape != (E, H):
+            return None
+        for w, rows, K, N, glu in ((w_fc, I2, H, I, 1), (w_proj, H, I, H, 0)):
+            if w.dim() != 1 and w.shape != (E, rows, K):
+                return None
+            if w.dim() == 1 and not 0 < w.numel() == _fp8_tiled_bytes(E, N, K, glu):
+                return None
+    elif w_fc.shape != (E, I2, H) or w_proj.shape != (E, H, I):
+        return None
+    if (logits is not None and logits.shape != (T, E)) or (bias is not None and bias.shape != (E,)):
+        return None
     unit = 4 if code == F32 else (16 if fp8 else 8)
     if T < 1 or H % unit or I % unit or S % (4 if code == F32 else 8) or gate_weight.shape[1] != H:
         return None
@@ -988,7 +1009,7 @@ def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor
         x.data_ptr(), _ptr(norm_w), eps, pre_norm is not None, gate_weight.data_ptr(), _ptr(bias), _ptr(logits),
         w_fc.data_ptr(), _ptr(fc_scale), w_proj.data_ptr(), _ptr(proj_scale),
         (int(w_fc.dim() == 1) | int(w_proj.dim() == 1) << 1) if fp8 else 0, _ptr(shared_fc), _ptr(shared_proj), _ptr(residual),
-        1.0 if residual_scale is None else residual_scale, residual_scale is not None, y.data_ptr(), T, H, E, k, I, S, code,
+        1.0 if residual_scale is None else float(residual_scale), residual_scale is not None, y.data_ptr(), T, H, E, k, I, S, code,
         ws.data_ptr(), ws_bytes, _ptr(gemm_ws), gemm_bytes, _RAW_STREAM(dev) if _RAW_STREAM is not None else _stream())
     if rc in (_lib.MI_MOE_EUNSUPPORTED, _lib.MI_MOE_EALIGN):
         return None

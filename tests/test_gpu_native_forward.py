@@ -56,3 +56,28 @@ def test_native_forward_equals_stages(device, dtype, T, H, E, k, I, shared, fp8,
     assert timer.stages, "the second forward was meant to run stage by stage"
     assert torch.equal(native, stages)
     assert torch.equal(native, again)
+
+
+def test_native_forward_refuses_what_does_not_fit(device):
+    """The one-call forward takes pointers: operands whose shapes do not fit together go to the stage-by-stage code, which
+    raises, and a forward hook on the down-projection still runs."""
+    from dolomite_engine_amd import Kernel, MoE, enable_kernels
+
+    def layer():
+        return MoE(hidden_size=128, intermediate_size=64, shared_intermediate_size=32, num_experts=4, num_experts_per_tok=2,
+                   activation_function="swiglu", add_bias=False, dropout=0.0, init_method="normal", initializer_range=0.05,
+                   m_width=None, num_layers=1, use_padding_free_transformer=True).bfloat16().to(device).eval()
+
+    x = torch.randn(9, 128, device=device, dtype=torch.bfloat16)
+    with torch.no_grad(), enable_kernels([Kernel.scattermoe]):
+        for name, width in (("c_fc", 64), ("c_proj", 32), ("c_proj_shared", 16)):
+            m = layer()
+            sub = getattr(m, name)
+            sub.weight = torch.nn.Parameter(sub.weight.detach()[..., :width].contiguous())
+            with pytest.raises(ValueError):
+                m(x)
+        m = layer()
+        seen = []
+        want = m(x)
+        m.c_proj.register_forward_hook(lambda *a: seen.append(1))
+        assert torch.equal(m(x), want) and seen
