@@ -249,13 +249,14 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(const int32_
 }
 
 // Whole problem in one block: histogram, expert scan and scatter without touching a workspace.
-__global__ __launch_bounds__(SORT_THREADS) void sort_single_block_kernel(const int32_t* __restrict__ ids, int L,
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void sort_single_block_kernel(const int32_t* __restrict__ ids, int L,
                                                                          int E, int nbits,
                                                                          int32_t* __restrict__ sorted_expert,
                                                                          int32_t* __restrict__ sorted_scattered,
                                                                          int32_t* __restrict__ expert_offsets) {
-  extern __shared__ int smem[];  // SORT_WAVES * E counters, then E totals
-  sort_single_block(ids, L, E, nbits, sorted_expert, sorted_scattered, expert_offsets, smem);
+  extern __shared__ int smem[];  // WAVES * E counters, then E totals
+  sort_single_block<WAVES>(ids, L, E, nbits, sorted_expert, sorted_scattered, expert_offsets, smem);
 }
 
 
@@ -277,9 +278,21 @@ extern "C" int mi_moe_sort_bin(const int32_t* topk_idx, int T, int k, int E, int
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   if (L <= SORT_SINGLE_BLOCK_MAX) {
-    size_t lds = (size_t)(SORT_WAVES + 1) * E * sizeof(int);
-    hipLaunchKernelGGL(sort_single_block_kernel, dim3(1), dim3(SORT_THREADS), lds, s, topk_idx, L, E, nbits,
-                       sorted_expert, sorted_scattered, expert_offsets);
+    if (L <= SORT_FEW_IDS) {
+      const size_t lds = (size_t)(SORT_WAVES + 1) * E * sizeof(int);
+      hipLaunchKernelGGL(sort_single_block_kernel<SORT_WAVES>, dim3(1), dim3(SORT_THREADS), lds, s, topk_idx, L, E, nbits,
+                         sorted_expert, sorted_scattered, expert_offsets);
+    } else {
+      const size_t lds = (size_t)(SORT_MANY_WAVES + 1) * E * sizeof(int);
+      if (lds > 64 * 1024) {  // (more than 963 experts)
+        static std::atomic<uint64_t> lds_ok{0};
+        const int rc = mi_allow_lds_once(reinterpret_cast<const void*>(sort_single_block_kernel<SORT_MANY_WAVES>),
+                                         (SORT_MANY_WAVES + 1) * SORT_MAX_E * (int)sizeof(int), lds_ok);
+        if (rc != MI_MOE_OK) return rc;
+      }
+      hipLaunchKernelGGL(sort_single_block_kernel<SORT_MANY_WAVES>, dim3(1), dim3(SORT_MANY_WAVES * 64), lds, s, topk_idx, L,
+                         E, nbits, sorted_expert, sorted_scattered, expert_offsets);
+    }
     return mi_launch_status();
   }
   const int nblk = mi_ceil_div(L, SORT_CHUNK);

@@ -18,6 +18,30 @@ __device__ __forceinline__ int wave_incl_scan_i32(int v, int lane) {
   return v;
 }
 
+// One step of the stable scatter: a wave's 64 slots from `slot - lane` on, lane l holding slot's expert e (ok: a valid one).
+// mybase[e]: output position of the wave's next slot of expert e.
+__device__ __forceinline__ void sort_scatter_step(int slot, int e, bool ok, int nbits, int* mybase,
+                                                  int32_t* __restrict__ sorted_expert,
+                                                  int32_t* __restrict__ sorted_scattered) {
+  const int lane = threadIdx.x & 63;
+  if (!ok) e = 0;
+  uint64_t peers = __ballot(ok);
+  for (int b = 0; b < nbits; ++b) {
+    uint64_t bal = __ballot((e >> b) & 1);
+    peers &= ((e >> b) & 1) ? bal : ~bal;
+  }
+  if (ok) {
+    const uint64_t below = peers & ((1ull << lane) - 1ull);
+    const int rank = __popcll(below);
+    const int pos = mybase[e] + rank;
+    sorted_expert[pos] = e;
+    sorted_scattered[pos] = slot;
+    // every lane of the group has read mybase[e] (one LDS instruction, wave-wide) before the
+    // group's first lane bumps it for the next step
+    if (below == 0ull) mybase[e] += __popcll(peers);
+  }
+}
+
 // Stable scatter of one chunk [chunk_begin, chunk_end).  wbase[w * E + e] must hold, on entry, the
 // output position of the first slot of expert e seen by wave w.
 __device__ __forceinline__ void sort_scatter_chunk(const int32_t* __restrict__ ids, int chunk_begin, int chunk_end,
@@ -32,24 +56,8 @@ __device__ __forceinline__ void sort_scatter_chunk(const int32_t* __restrict__ i
   for (int s0 = begin; s0 < end; s0 += 64) {
     const int slot = s0 + lane;
     const bool valid = slot < end;
-    int e = valid ? ids[slot] : 0;
-    const bool ok = valid && (unsigned)e < (unsigned)E;
-    if (!ok) e = 0;
-    uint64_t peers = __ballot(ok);
-    for (int b = 0; b < nbits; ++b) {
-      uint64_t bal = __ballot((e >> b) & 1);
-      peers &= ((e >> b) & 1) ? bal : ~bal;
-    }
-    if (ok) {
-      const uint64_t below = peers & ((1ull << lane) - 1ull);
-      const int rank = __popcll(below);
-      const int pos = mybase[e] + rank;
-      sorted_expert[pos] = e;
-      sorted_scattered[pos] = slot;
-      // every lane of the group has read mybase[e] (one LDS instruction, wave-wide) before the
-      // group's first lane bumps it for the next step
-      if (below == 0ull) mybase[e] += __popcll(peers);
-    }
+    const int e = valid ? ids[slot] : 0;
+    sort_scatter_step(slot, e, valid && (unsigned)e < (unsigned)E, nbits, mybase, sorted_expert, sorted_scattered);
   }
 }
 
@@ -66,24 +74,37 @@ __device__ __forceinline__ void sort_wave_hist(const int32_t* __restrict__ ids, 
   }
 }
 
-// Whole problem in one block of SORT_THREADS threads: histogram, expert scan and scatter without touching a
-// workspace.  `smem`: (SORT_WAVES + 1) * E ints of LDS.
+// Whole problem in one block of WAVES waves, at most 512 ids a wave: histogram, expert scan and scatter without touching a
+// workspace.  `smem`: (WAVES + 1) * E ints of LDS.  It is a chain of latencies, so a wave's ids are loaded at once and
+// kept for both passes, and sixteen waves share them from SORT_FEW_IDS ids on (four waves that loaded the ids step by
+// step, twice: 12.5 us for 2840 ids of 40 experts, now 5.6).
+#define SORT_ID_STEPS 8
+template <int WAVES>
 __device__ __forceinline__ void sort_single_block(const int32_t* __restrict__ ids, int L, int E, int nbits,
                                                   int32_t* __restrict__ sorted_expert,
                                                   int32_t* __restrict__ sorted_scattered,
                                                   int32_t* __restrict__ expert_offsets, int* smem) {
+  constexpr int THREADS = WAVES * 64;
   int* wcnt = smem;
-  int* totals = smem + SORT_WAVES * E;
+  int* totals = smem + WAVES * E;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < SORT_WAVES * E; i += SORT_THREADS) wcnt[i] = 0;
+  const int per_wave = mi_ceil_div_dev(mi_ceil_div_dev(L, WAVES), 64) * 64;
+  int id[SORT_ID_STEPS];
+#pragma unroll
+  for (int j = 0; j < SORT_ID_STEPS; ++j) {
+    const int slot = wave * per_wave + j * 64 + lane;
+    id[j] = j * 64 < per_wave && slot < L ? ids[slot] : -1;
+  }
+  for (int i = threadIdx.x; i < WAVES * E; i += THREADS) wcnt[i] = 0;
   __syncthreads();
-  const int per_wave = mi_ceil_div_dev(mi_ceil_div_dev(L, SORT_WAVES), 64) * 64;
-  sort_wave_hist(ids, 0, L, per_wave, E, wcnt);
+#pragma unroll
+  for (int j = 0; j < SORT_ID_STEPS; ++j)
+    if ((unsigned)id[j] < (unsigned)E) atomicAdd(&wcnt[wave * E + id[j]], 1);
   __syncthreads();
-  for (int e = threadIdx.x; e < E; e += SORT_THREADS) {
+  for (int e = threadIdx.x; e < E; e += THREADS) {
     int t = 0;
 #pragma unroll
-    for (int w = 0; w < SORT_WAVES; ++w) t += wcnt[w * E + e];
+    for (int w = 0; w < WAVES; ++w) t += wcnt[w * E + e];
     totals[e] = t;
   }
   __syncthreads();
@@ -101,17 +122,23 @@ __device__ __forceinline__ void sort_single_block(const int32_t* __restrict__ id
     }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < E; e += SORT_THREADS) {
+  for (int e = threadIdx.x; e < E; e += THREADS) {
     int run = totals[e];
 #pragma unroll
-    for (int w = 0; w < SORT_WAVES; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       int c = wcnt[w * E + e];
       wcnt[w * E + e] = run;
       run += c;
     }
   }
   __syncthreads();
-  sort_scatter_chunk(ids, 0, L, per_wave, E, nbits, wcnt, sorted_expert, sorted_scattered);
+#pragma unroll
+  for (int j = 0; j < SORT_ID_STEPS; ++j)
+    if (j * 64 < per_wave)
+      sort_scatter_step(wave * per_wave + j * 64 + lane, id[j], (unsigned)id[j] < (unsigned)E, nbits, wcnt + wave * E,
+                        sorted_expert, sorted_scattered);
 }
 
-#define SORT_SINGLE_BLOCK_MAX 8192
+#define SORT_MANY_WAVES 16
+#define SORT_FEW_IDS 512            // up to here four waves sort
+#define SORT_SINGLE_BLOCK_MAX 8192  // SORT_MANY_WAVES * 64 * SORT_ID_STEPS
