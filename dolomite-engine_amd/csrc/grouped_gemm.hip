@@ -909,10 +909,30 @@ static bool tiled_aligned(const GemmArgs& a, int elt_bytes) {
   return mi_aligned(a.in, 16) && mi_aligned(a.w, 16) && mi_aligned(a.out, 4 * elt_bytes);
 }
 
-static int pick_cfg(const GemmArgs& a) {
+// So few 256 x 256 tiles that most CUs would have none: smaller tiles give four times as many workgroups.  Measured, us,
+// 256 x 256 tiles against 128 x 128: one expert (shared experts, the router's gradient) of 2048 rows, 1024 -> 1024 (SwiGLU,
+// 64 tiles) 24.5 / 15.7, of 1429 rows (24 tiles) 23.3 / 12.9, of 3001 rows, 920 -> 344 fp16 (36 tiles) 23.3 / 17.0; 4096
+// rows 1536 -> 512 (64 tiles) 31.6 / 20.8; but 512 -> 1536 (96 tiles) 15.6 / 16.7, 17 experts of 235 rows, 920 -> 520 (85
+// tiles) 26.0 / 26.2.
+static bool few_large_tiles(const GemmArgs& a, bool glu) {
+  return (double)a.E * mi_ceil_div((a.L + a.E - 1) / a.E, 256) * mi_ceil_div(a.N, glu ? 128 : 256) <= 72;
+}
+
+#define PERSIST_MIN_ROWS 120  // rows per expert on average
+
+static int pick_cfg(const GemmArgs& a, bool glu) {
   const long avg = a.E > 0 ? (long)a.L / a.E : a.L;  // rows per expert if the load were uniform
-  if (avg >= 192 && mi_gemm_persistent_ok(a)) return 7;
-  if (avg >= 512) return 0;
+  // (128 x 128 tiles need a second row tile, and a second pass over the weights, for the experts with more than 128 rows.
+  // Persistent / 128 x 128 tiles, us, up and down projection: hidden 1536, 40 experts, 80 rows per expert 35.8 / 31.6 and
+  // 23.7 / 17.8, 120 rows 38.2 / 38.8 and 22.0 / 29.7, 160 rows 37.2 / 46.1 and 20.6 / 32.0; hidden 4096, 8 experts, I 14336,
+  // 100 rows 450 / 407 and 284 / 212, 130 rows 435 / 694 and 308 / 372; hidden 1024, 32 experts, 150 rows 27.0 / 26.8 and
+  // 18.0 / 19.1)
+  if (avg >= PERSIST_MIN_ROWS && mi_gemm_persistent_ok(a) && !few_large_tiles(a, glu)) return 7;
+  if (avg >= 512 && !few_large_tiles(a, glu)) return 0;
+  // A few rows per expert, just beyond the weight stream's range: many small tiles, except where the contraction is so
+  // short or so long that the deeper ring of the DMA tiles wins (31 rows per expert, hidden 1536, 40 experts: layer 74 us
+  // with the 32 x 128 tiles, 82 with the DMA tiles).
+  if (avg < 48 && !(a.K % 32 == 0 && (a.K <= 1024 || a.K >= 8192))) return 5;
   return a.K % 32 == 0 ? 4 : 1;
 }
 
@@ -948,7 +968,7 @@ static int run_gemm(GemmArgs a, int dtype, bool glu, int cfg, int in_rows_bound,
     }
     return glu ? dispatch_cfg_f32<true>(a, cfg, s) : dispatch_cfg_f32<false>(a, cfg, s);
   }
-  if (cfg < 0) cfg = pick_cfg(a);
+  if (cfg < 0) cfg = pick_cfg(a, glu);
   if (dtype == MI_MOE_BF16) return glu ? dispatch_cfg<bf16_t, true>(a, cfg, s) : dispatch_cfg<bf16_t, false>(a, cfg, s);
   return glu ? dispatch_cfg<f16_t, true>(a, cfg, s) : dispatch_cfg<f16_t, false>(a, cfg, s);
 }
@@ -1062,7 +1082,7 @@ extern "C" int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_
   a.gather = 1; a.scatter = 0; a.remap = 1; a.ws = nullptr; a.pre = pre_out;
   // only the persistent kernel writes the pre-activation: shapes it does not take, and loads for which another
   // kernel would be picked, are the caller's two-call path
-  if (!mi_gemm_persistent_ok(a) || pick_cfg(a) != 7) return MI_MOE_EUNSUPPORTED;
+  if (!mi_gemm_persistent_ok(a) || (long)L / E < PERSIST_MIN_ROWS) return MI_MOE_EUNSUPPORTED;
   if (!tiled_shape_ok(a, L, true, 2)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
   a.out_nt = 0;
