@@ -232,6 +232,8 @@ class FusedRouter(torch.autograd.Function):
         else:
             logits, gates, experts = ops.router_fused(x, gate_w, k, bias=bias, return_logits=True)
             ctx.mark_non_differentiable(experts)
+        # (the integer outputs have no gradient: without this a zero tensor is filled for each of them in every backward)
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(x, gate_w, logits, experts)
         return logits, gates, experts, se, ss, off
 
@@ -245,8 +247,12 @@ class FusedRouter(torch.autograd.Function):
         rows, off = one_expert_rows(T, x.device)
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            # (T, E) @ (E, H): the gate weight transposed to (H, E) is the "(out, in)" weight of one expert
-            dx = ops.scattered_gemm(dl, gate_w.t().contiguous().unsqueeze(0), 1, rows, off, True, True)
+            # (T, E) @ (E, H): the gate weight as it lies is the "(in, out)" weight of one expert; the transposed-weight
+            # kernel takes it in 16 bits and multiples of 8, else a transposed copy is the "(out, in)" weight
+            if dl.dtype != torch.float32 and gate_w.shape[0] % 8 == 0 and H % 8 == 0:
+                dx = ops.scattered_gemm(dl, gate_w.unsqueeze(0), 1, rows, off, True, True, weight_kn=True)
+            else:
+                dx = ops.scattered_gemm(dl, gate_w.t().contiguous().unsqueeze(0), 1, rows, off, True, True)
         if ctx.needs_input_grad[1]:
             dw = ops.grouped_wgrad(dl, x, off)[0]
         return dx, dw, None, None
