@@ -7,6 +7,7 @@
 #define SORT_THREADS 256
 #define SORT_WAVES (SORT_THREADS / 64)
 #define SORT_CHUNK 2048
+#define SORT_SMALL_CHUNK 512
 #define SORT_MAX_E 1024
 
 __device__ __forceinline__ int wave_incl_scan_i32(int v, int lane) {
