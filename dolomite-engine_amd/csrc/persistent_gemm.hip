@@ -118,8 +118,8 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
     const uint64_t o = ((uint64_t)t.expert * (GLU ? 2 : 1) * a.N * a.K + (uint64_t)t.nt * BN * (WT ? 1 : a.K)) * 2u;
     return pg_srd(static_cast<const unsigned char*>(a.w) + o, w_bytes - o);
   };
-  // sorted-order row index of the activation rows a lane fetches (clamped into the tile's expert: rows past its end
-  // are never stored), and the byte offsets they give
+  // sorted-order row index of the activation rows a lane fetches (clamped into the tile's expert), and the byte offsets
+  // they give; rows past the expert's end lie past the buffer: zeros, no traffic, and multipliers at rest
   auto load_rows = [&](const PgTile& t, int (&raw)[8]) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
       for (int j = 0; j < 8; ++j) raw[j] = a.sorted_scattered[raw[j]];
     }
   };
-  auto make_xoff = [&](const int (&raw)[8], uint32_t (&off)[8]) {
+  auto make_xoff = [&](const PgTile& t, const int (&raw)[8], uint32_t (&off)[8]) {
     // (top-k is a power of two in most configurations: a shift instead of a division)
     const int sh = !a.gather ? 0 : a.kshift;
     if (sh >= 0) {
@@ -141,6 +141,8 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
 #pragma unroll
       for (int j = 0; j < 8; ++j) off[j] = (uint32_t)(raw[j] / a.kdiv) * row_bytes + lchunk * 16u;
     }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) off[j] = t.row_begin + drow + 32 * j < t.row_end ? off[j] : PG_OOB;
   };
   // Weight rows are at fixed distances (rows past N are another matrix's, or past the buffer: never stored).
   // WT: instruction j fills rows 8 j + 2 wave + lane / 32 of the slice; 16-byte piece l % 32 of row r holds the logical
@@ -439,8 +441,8 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
     load_rows(cur, raw);
     load_rows(nxt, raw_n);
     load_out_rows(cur, orow_lo, orow_hi);
-    make_xoff(raw, xoff);
-    make_xoff(raw_n, xoff_n);
+    make_xoff(cur, raw, xoff);
+    make_xoff(nxt, raw_n, xoff_n);
   }
   make_woff();
   wsrd = make_wsrd(cur);
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
     epilogue(cur, interior);
     if (i + 1 >= n_items) break;
     stores_pending = interior;
-    make_xoff(raw, xoff_n);
+    make_xoff(after, raw, xoff_n);
     wsrd_n = make_wsrd(after);
     orow_lo = lo_n;
     orow_hi = hi_n;
