@@ -261,17 +261,19 @@ __global__ __launch_bounds__(WAVES * 64) void sort_single_block_kernel(const int
 }
 
 
-// Slots per block: small chunks as long as the table of chunk histograms stays small (128 KB).  A block walks its chunk 64
-// slots a wave and step, and with 2048 slots a chunk most CUs have no block: 12004 slots of 17 experts 16.5 -> 10.3
-// us for the three passes.
-static int sort_chunk(int L, int E) {
-  return (long)E * mi_ceil_div(L, SORT_SMALL_CHUNK) <= 32768 ? SORT_SMALL_CHUNK : SORT_CHUNK;
+// Slots per block: small chunks as long as the table of chunk histograms stays small (64 KB) and fits the caller's
+// workspace, which has to hold the table of SORT_CHUNK chunks only (one sized for a larger batch stays enough for every
+// smaller one).  A block walks its chunk 64 slots a wave and step, and with 2048 slots a chunk most CUs have no block:
+// 12004 slots of 17 experts 16.5 -> 10.3 us for the three passes, 131072 slots of 32 experts 19.6 -> 16.3.
+static size_t sort_table_bytes(int L, int E, int chunk) { return ((size_t)E * mi_ceil_div(L, chunk) + (size_t)E) * sizeof(int32_t); }
+static int sort_chunk(int L, int E, size_t ws_bytes) {
+  return (long)E * mi_ceil_div(L, SORT_SMALL_CHUNK) <= 16384 && ws_bytes >= sort_table_bytes(L, E, SORT_SMALL_CHUNK) ? SORT_SMALL_CHUNK
+                                                                                                                    : SORT_CHUNK;
 }
 
 extern "C" size_t mi_moe_sort_bin_workspace_bytes(int L, int E) {
   if (L <= SORT_SINGLE_BLOCK_MAX || E < 1) return 0;
-  size_t nblk = (size_t)mi_ceil_div(L, sort_chunk(L, E));
-  return ((size_t)E * nblk + (size_t)E) * sizeof(int32_t);
+  return sort_table_bytes(L, E, sort_chunk(L, E, ~(size_t)0));
 }
 
 extern "C" int mi_moe_sort_bin(const int32_t* topk_idx, int T, int k, int E, int32_t* sorted_expert,
@@ -303,8 +305,8 @@ extern "C" int mi_moe_sort_bin(const int32_t* topk_idx, int T, int k, int E, int
     }
     return mi_launch_status();
   }
-  const int chunk = sort_chunk(L, E), nblk = mi_ceil_div(L, chunk);
-  if (ws_bytes < mi_moe_sort_bin_workspace_bytes(L, E) || !ws) return MI_MOE_EWORKSPACE;
+  const int chunk = sort_chunk(L, E, ws_bytes), nblk = mi_ceil_div(L, chunk);
+  if (ws_bytes < sort_table_bytes(L, E, chunk) || !ws) return MI_MOE_EWORKSPACE;
   if (!mi_aligned(ws, 16)) return MI_MOE_EALIGN;
   int32_t* w = static_cast<int32_t*>(ws);
   hipLaunchKernelGGL(chunk == SORT_CHUNK ? sort_hist_kernel<SORT_CHUNK> : sort_hist_kernel<SORT_SMALL_CHUNK>, dim3(nblk),
