@@ -52,7 +52,7 @@ int mi_gemm_fp8_persistent(const GemmArgs& a, int dtype, bool glu, hipStream_t s
 
 // ---- stream_gemm.hip: K a multiple of one 16-byte chunk, N % 4 == 0 ------------------------------------------------------
 // whether the stream is the faster form for this problem (elt: bytes of an element)
-bool mi_gemm_stream_pick(const GemmArgs& a, int elt);
+bool mi_gemm_stream_pick(const GemmArgs& a, bool glu, int elt);
 // rb: row blocks of 16 per unit (1, 2, 4); nw: waves that split the contraction (1, 2, 4; rb 4: 1, 2); 0, 0: by the rule
 int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipStream_t s);
 

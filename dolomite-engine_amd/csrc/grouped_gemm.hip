@@ -954,7 +954,7 @@ static int run_gemm(GemmArgs a, int dtype, bool glu, int cfg, int in_rows_bound,
   if (!tiled_shape_ok(a, in_rows_bound, glu, elt)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, elt)) return MI_MOE_EALIGN;
   if (cfg >= 100) return mi_gemm_stream(a, dtype, glu, (cfg - 100) / 10, cfg % 10, s);
-  if (cfg < 0 && mi_gemm_stream_pick(a, elt)) return mi_gemm_stream(a, dtype, glu, 0, 0, s);
+  if (cfg < 0 && mi_gemm_stream_pick(a, glu, elt)) return mi_gemm_stream(a, dtype, glu, 0, 0, s);
   if (dtype == MI_MOE_F32) {
     if (cfg < 0) {
       // fp32 matrix instructions are slow enough that what matters is how many CUs have a tile.  Measured (up /

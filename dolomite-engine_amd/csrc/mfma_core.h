@@ -10,7 +10,9 @@
 
 #include <type_traits>
 
-#define PG_OOB 0xfffff000u  // byte offset past every buffer: such a lane of the DMA writes zeros
+// Byte offset past every buffer: such a lane of the DMA writes zeros.  (A 16-bit operand of the accepted sizes, under
+// 2^31 elements in whole 16-byte chunks, ends here at the latest; the range check does not wrap with the scalar offset.)
+#define PG_OOB 0xfffffff0u
 #define PG_SCHED() __builtin_amdgcn_sched_barrier(0)
 
 #define ALL_AGPRS \

@@ -274,7 +274,14 @@ template <typename T> static int launch_stream_t(const GemmArgs& a, bool glu, in
 // So: up to 16 rows per expert always; up to 28 with a contraction long enough to keep the rings full, up to 56 where it
 // is very long or where the tile kernels would pad a ragged one; fp32 as long as there are too few results to give
 // every CU a tile.
-bool mi_gemm_stream_pick(const GemmArgs& a, int elt) {
+// Never where an operand passes the 32-bit byte offsets of the DMA (fp32 only: the general rule counts elements).
+static bool stream_offsets_ok(const GemmArgs& a, bool glu, int elt) {
+  const double row = (double)a.K * elt;
+  return (a.gather ? a.L / a.kdiv : a.L) * row <= (double)PG_OOB && (glu ? 2.0 : 1.0) * a.N * row <= (double)PG_OOB;
+}
+
+bool mi_gemm_stream_pick(const GemmArgs& a, bool glu, int elt) {
+  if (!stream_offsets_ok(a, glu, elt)) return false;
   const long rows = a.L, e = a.E;
   if (elt == 4) return rows <= 64 * e || rows * a.N <= (1L << 20);
   if (rows <= 16 * e) return true;
@@ -284,6 +291,7 @@ bool mi_gemm_stream_pick(const GemmArgs& a, int elt) {
 
 int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipStream_t s) {
   const int elt = dtype == MI_MOE_F32 ? 4 : 2;
+  if (!stream_offsets_ok(a, glu, elt)) return MI_MOE_EUNSUPPORTED;
   const double avg = (double)a.L / a.E;
   if (rb == 0) {
     // row blocks: most experts in one chunk; beyond that (fp32) long contractions re-read less with large chunks
