@@ -924,8 +924,9 @@ def down_fp8(act: torch.Tensor, w_proj_q: torch.Tensor, w_proj_scale: torch.Tens
 
 
 @functools.lru_cache(maxsize=256)
-def _layer_sizes(T: int, H: int, E: int, k: int, I: int, S: int, code: int, has_norm: int) -> tuple[int, int]:
-    """(workspace bytes, contraction length that may use the split-K workspace or 0): functions of the sizes alone."""
+def _layer_sizes(dev: int, T: int, H: int, E: int, k: int, I: int, S: int, code: int, has_norm: int) -> tuple[int, int]:
+    """(workspace bytes, contraction length that may use the split-K workspace or 0): functions of the sizes and of the
+    current device's compute units alone."""
     lib = _lib.load()
     splits = 0
     if code != F32:
@@ -1001,7 +1002,7 @@ def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor
             return None
     elif logits is None and not router_fused_supported(x, E, k):
         return None
-    ws_bytes, splits = _layer_sizes(T, H, E, k, I, S, code, pre_norm is not None)
+    ws_bytes, splits = _layer_sizes(dev, T, H, E, k, I, S, code, pre_norm is not None)
     y = torch.empty_like(x)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
     gemm_ws, gemm_bytes = _gemm_workspace(x.device, splits, dtype) if splits else (None, 0)
