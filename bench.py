@@ -258,11 +258,10 @@ def measure_ceilings(w, inputs, device, iters=20):
 
 
 def measure_inner_loop_probes(device, slices=6144):
-    """The pieces of the persistent grouped GEMM's inner loop in isolation (mi_moe_probe_kloop: one workgroup per
-    CU, the GEMM's own 256 x 256 tile, slice, ring and schedule, on 2 MiB of L2-resident random bf16 data): the
-    matrix instructions alone, with the LDS fragment reads, the L2 -> LDS DMA alone, and all of it together.  What
-    "all of it" reaches is the ceiling of the GEMM's K loop on this GPU -- before gather, expert tails, tile
-    boundaries and epilogues."""
+    """The pieces of an eight-wave GEMM inner loop in isolation (mi_moe_probe_kloop: one workgroup per CU, a 256 x 256
+    tile of 64 x 128 wave tiles, on 2 MiB of L2-resident random bf16 data): the matrix instructions alone, with the LDS
+    fragment reads, the L2 -> LDS DMA alone, and all of it together.  "mfma_only" is what the matrix cores sustain at
+    the clock the chip settles at; the grouped GEMM's own loop (four waves of 128 x 128) is not bound by the others."""
     import torch
 
     from dolomite_engine_amd import _lib

@@ -1,16 +1,17 @@
-// Diagnostic kernels: the pieces of the persistent grouped GEMM's inner loop (grouped_gemm.hip) run in isolation,
-// so that a benchmark can put a measured ceiling next to the GEMM's own figure on the same GPU in the same process.
+// Diagnostic kernels: the pieces of an eight-wave GEMM inner loop run in isolation, so that a benchmark can put measured
+// rates of the matrix cores, the LDS and the DMA next to the grouped GEMM's figure on the same GPU in the same process.
+// (The persistent grouped GEMM, persistent_gemm.hip, runs four waves of 128 x 128 and is not bound by modes 1 and 3.)
 // Nothing in the layer calls these; they compute nothing useful.
 //
-// One workgroup of eight waves per compute unit works through `slices` K slices of a 256 x 256 bf16 tile exactly
-// as the GEMM does (32-wide slices, wave tile 64 x 128, twelve 16-byte fragment reads and 32 v_mfma_f32_16x16x32 per
+// One workgroup of eight waves per compute unit works through `slices` K slices of a 256 x 256 bf16 tile
+// (32-wide slices, wave tile 64 x 128, twelve 16-byte fragment reads and 32 v_mfma_f32_16x16x32 per
 // wave and slice, four 1 KiB DMA instructions per wave and slice into a ring of four 32 KiB stages), with parts
 // switched off:
 //   mode 0   matrix instructions only (operands read once): what the matrix cores sustain on this data at the
 //            clock the chip settles at
 //   mode 1   + the LDS fragment reads of every slice (no DMA: the ring keeps its first contents)
 //   mode 2   DMA only: L2 -> LDS fill rate of one workgroup per CU (addresses walk an L2-resident span)
-//   mode 3   everything, in the GEMM's two-group ping-pong schedule
+//   mode 3   everything, in two wave groups that alternate between memory and matrix phases
 // `data` supplies the bytes (the caller chooses them: random bf16 values draw more power than zeros and lower the
 // clock).  flops per slice and workgroup: 2 * 256 * 256 * 32; DMA bytes per slice and workgroup: 32 KiB.
 #include "common.h"

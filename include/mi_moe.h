@@ -155,7 +155,8 @@ int mi_moe_count(const int32_t* ids, int L, int E, uint32_t* counts_out, mi_moe_
  *   sorted_expert     (T*k,) int32  non-decreasing expert ids
  *   sorted_scattered  (T*k,) int32  flat slot id (t*k + j) of each sorted row; stable
  *   expert_offsets    (E,)   int32  INCLUSIVE prefix sum of the per-expert counts
- *   ws / ws_bytes     scratch of at least mi_moe_sort_bin_workspace_bytes(T*k, E) bytes, 16-byte aligned
+ *   ws / ws_bytes     scratch of at least mi_moe_sort_bin_workspace_bytes(T*k, E) bytes, 16-byte aligned; one sized for
+ *                     more slots of as many experts serves fewer
  */
 size_t mi_moe_sort_bin_workspace_bytes(int L, int E);
 int mi_moe_sort_bin(const int32_t* topk_idx, int T, int k, int E, int32_t* sorted_expert,
@@ -431,13 +432,13 @@ int mi_moe_layer_forward(const void* x, const void* norm_w, float norm_eps, int 
                          size_t gemm_ws_bytes, mi_moe_stream_t stream);
 
 /*
- * Diagnostics (no counterpart in the reference; nothing in the layer calls them): the pieces of the persistent
- * grouped GEMM's inner loop in isolation, for a benchmark that wants a measured ceiling beside the GEMM's own
- * figure.  One workgroup of eight waves per compute unit runs `slices` K slices of a 256 x 256 bf16 tile the way
- * the GEMM does (32 matrix instructions 16x16x32, twelve 16-byte LDS fragment reads and four 1 KiB DMA
+ * Diagnostics (no counterpart in the reference; nothing in the layer calls them): the pieces of an eight-wave
+ * GEMM inner loop in isolation, for a benchmark that wants measured rates beside the grouped GEMM's own
+ * figure (which runs four waves of 128 x 128 and is not bound by modes 1 and 3).  One workgroup of eight waves per compute unit runs `slices` K slices of a 256 x 256 bf16 tile
+ * (32 matrix instructions 16x16x32, twelve 16-byte LDS fragment reads and four 1 KiB DMA
  * instructions per wave and slice, ring of four 32 KiB stages) with parts switched off:
  *   mode 0  matrix instructions only        mode 1  + the LDS fragment reads
- *   mode 2  DMA only (L2 -> LDS fill)       mode 3  everything, in the GEMM's two-group ping-pong schedule
+ *   mode 2  DMA only (L2 -> LDS fill)       mode 3  everything, in two alternating wave groups
  * Per workgroup and slice: 2 * 256 * 256 * 32 flops, 32 KiB of DMA.  data: at least 2 MiB + 4 KiB of bytes of the
  * caller's choice (random bf16 values draw more power than zeros), 16-byte aligned, read only; sink:
  * mi_moe_probe_sink_bytes() bytes that the kernels write (one float per thread, so that nothing is optimised away).
