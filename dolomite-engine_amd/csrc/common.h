@@ -76,6 +76,9 @@ template <> __device__ __forceinline__ float unpack_hi<f16_t>(uint32_t v) {
 }
 
 __device__ __forceinline__ float silu_f32(float g) { return g / (1.0f + __expf(-g)); }
+// the same with the reciprocal instruction (1 ulp) in place of the division, for the tile kernels' epilogues.  A SwiGLU is
+// up * silu(gate) in this order: up * gate first overflows for finite results (up = 1e20, gate = -1e20 gives -0, not NaN).
+__device__ __forceinline__ float silu_rcp_f32(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
 
 // ---- host helpers ---------------------------------------------------------------------------
 

@@ -316,8 +316,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
           for (int i = 0; i < 4; ++i) {
             v[i] = pg_acc(blk * 4 + i) * sc[i];
             if (GLU) {
-              const float gt = pg_acc((blk + 4) * 4 + i) * sg[i];
-              v[i] = v[i] * gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
+              v[i] = v[i] * silu_rcp_f32(pg_acc((blk + 4) * 4 + i) * sg[i]);
             }
           }
           *(wp_t)(size_t)(s0 + (scr_w ^ (nb * 32)) + mbp * (16 / RPP) * 2048) =

@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
                 up = Elt<T>::round(up);
                 gt = Elt<T>::round(gt);
               }
-              v[i] = up * gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
+              v[i] = up * silu_rcp_f32(gt);
             } else {
               v[i] = pg_acc(blk * 4 + i);
             }
@@ -568,7 +568,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_split_finish_kernel(GemmArgs
         const float up = sum[mb * 8 + nb][i];
         if (GLU) {
           const float gt = sum[mb * 8 + nb + 4][i];
-          v[i] = up * gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
+          v[i] = up * silu_rcp_f32(gt);
         } else {
           v[i] = up;
         }
