@@ -2,14 +2,18 @@
 //
 //   out[orow(i), :] = in[irow(i), :] @ W[e_i]^T     (+ SwiGLU), as in persistent_gemm.hip
 //
-// Every weight byte is used once per row chunk, so what counts is how many bytes a CU has in flight, and at the smallest
+// Weights are read once per row chunk, so what counts is how many bytes a CU has in flight, and at the smallest
 // sizes (one token: 8 of 40 experts, 38 MB of weights) how many CUs have any.
 //   * A unit is 32 weight rows (SwiGLU: 16 up, 16 gate) of one expert for a chunk of up to 16 RB of its rows.  The NW
 //     waves of a workgroup split the contraction: each streams its range of K through a ring of its own -- no barrier
 //     until the partial sums meet in LDS, where they are added in wave order.  Slices are whole 128-byte lines.
 //   * Operands come by DMA; rows past the expert's end and values past K are lanes past the buffer: zeros, and no
 //     traffic.  (The 128-row tile kernels fetch 112 copies of an expert's last row for 16 real ones.)
-//   * Weights nobody reads again are fetched non-temporally (see decode_fp8.hip).
+//   * An expert with one chunk has its weights fetched non-temporally (see decode_fp8.hip).  With several, the chunks of a
+//     unit run side by side on one XCD and share the fetch through its L2: loads are uneven even when the router is not
+//     (16 rows per expert on average are 10 to 22), and an expert of 200 MB read once per chunk, all its units at a time, came
+//     from HBM each time.  8 experts, 4096 -> 14336, both projections, us, units innermost -> now: 64 tokens 630 -> 463 (tile
+//     kernels 516), 48 tokens that all want the same two experts 332 -> 203 (240).
 #include "gemm_common.h"
 #include "mfma_core.h"
 
@@ -43,7 +47,7 @@ template <bool NT> __device__ __forceinline__ void stream_dma(uint32_t lds, uint
 
 #define STREAM_STAGES 4
 
-template <typename T, bool GLU, int RB, int NW, bool NT>
+template <typename T, bool GLU, int RB, int NW>
 __global__ __launch_bounds__(NW * 64) void grouped_gemm_stream_kernel(GemmArgs a) {
   constexpr int CE = 16 / sizeof(T);                // elements of a 16-byte chunk
   constexpr int BK = 8 * CE;                        // K slice: 128 bytes of a row
@@ -59,8 +63,9 @@ __global__ __launch_bounds__(NW * 64) void grouped_gemm_stream_kernel(GemmArgs a
 
   // ---- unit -> (expert, row chunk, weight rows) -----------------------------------------------------------------------
   int expert = 0, row_begin = 0, row_end = 0, nt = 0;
+  bool once = true;                                 // one chunk: nobody else reads this unit's weights
   {
-    // (one pass over the offsets: a lane per expert, row chunks in expert order, units innermost)
+    // (one pass over the offsets: a lane per expert, its blocks side by side)
     const int mt = blockIdx.x / a.n_tiles;
     nt = blockIdx.x - mt * a.n_tiles;
     int carry = 0;
@@ -82,7 +87,18 @@ __global__ __launch_bounds__(NW * 64) void grouped_gemm_stream_kernel(GemmArgs a
         const int l = __ffsll((long long)hit) - 1;
         expert = e0 + l;
         row_end = __builtin_amdgcn_readlane(end, l);
-        row_begin = __builtin_amdgcn_readlane(prev, l) + (mt - __builtin_amdgcn_readlane(incl - mine, l)) * BM;
+        row_begin = __builtin_amdgcn_readlane(prev, l);
+        const int chunks = __builtin_amdgcn_readlane(mine, l);
+        if (chunks > 1) {
+          once = false;
+          // eight units, all their chunks, the next eight: blocks eight apart are on one XCD
+          const int local = blockIdx.x - __builtin_amdgcn_readlane(incl - mine, l) * a.n_tiles;
+          const int g = local / (8 * chunks), rem = local - g * 8 * chunks;
+          const int width = a.n_tiles - 8 * g < 8 ? a.n_tiles - 8 * g : 8;
+          const int chunk = rem / width;
+          nt = 8 * g + rem - chunk * width;
+          row_begin += chunk * BM;
+        }
         found = true;
       }
       carry = __builtin_amdgcn_readlane(incl, 63);
@@ -121,7 +137,7 @@ __global__ __launch_bounds__(NW * 64) void grouped_gemm_stream_kernel(GemmArgs a
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const bool gone = ((lane & 7) ^ (4 * (j & 1) + odd)) * CE >= a.K - k * BK;
-        stream_dma<NT>(st + j * 1024, gone ? PG_OOB : woff[j], wsrd, soff);
+        stream_dma<false>(st + j * 1024, gone ? PG_OOB : woff[j], wsrd, soff);
       }
 #pragma unroll
       for (int j = 0; j < NX; ++j) {
@@ -129,8 +145,13 @@ __global__ __launch_bounds__(NW * 64) void grouped_gemm_stream_kernel(GemmArgs a
         stream_dma<false>(st + (4 + j) * 1024, gone ? PG_OOB : xoff[j], xsrd, soff);
       }
     } else {
+      if (once) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) stream_dma<NT>(st + j * 1024, woff[j], wsrd, soff);
+        for (int j = 0; j < 4; ++j) stream_dma<true>(st + j * 1024, woff[j], wsrd, soff);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) stream_dma<false>(st + j * 1024, woff[j], wsrd, soff);
+      }
 #pragma unroll
       for (int j = 0; j < NX; ++j) stream_dma<false>(st + (4 + j) * 1024, xoff[j], xsrd, soff);
     }
@@ -224,9 +245,9 @@ __global__ __launch_bounds__(NW * 64) void grouped_gemm_stream_kernel(GemmArgs a
 }
 
 // ---- host side ------------------------------------------------------------------------------------------------------------
-template <typename T, bool GLU, int RB, int NW, bool NT> static int launch_stream(GemmArgs a, hipStream_t s) {
+template <typename T, bool GLU, int RB, int NW> static int launch_stream(GemmArgs a, hipStream_t s) {
   constexpr int lds = NW * STREAM_STAGES * (4 + 2 * RB) * 1024;
-  auto kern = grouped_gemm_stream_kernel<T, GLU, RB, NW, NT>;
+  auto kern = grouped_gemm_stream_kernel<T, GLU, RB, NW>;
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> lds_ok{0};
     const int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), lds, lds_ok);
@@ -240,40 +261,44 @@ template <typename T, bool GLU, int RB, int NW, bool NT> static int launch_strea
   return mi_launch_status();
 }
 
-template <typename T, bool GLU, int RB> static int launch_stream_nw(const GemmArgs& a, int nw, bool nt, hipStream_t s) {
+template <typename T, bool GLU, int RB> static int launch_stream_nw(const GemmArgs& a, int nw, hipStream_t s) {
   switch (nw) {
-    case 1: return nt ? launch_stream<T, GLU, RB, 1, true>(a, s) : launch_stream<T, GLU, RB, 1, false>(a, s);
-    case 2: return nt ? launch_stream<T, GLU, RB, 2, true>(a, s) : launch_stream<T, GLU, RB, 2, false>(a, s);
+    case 1: return launch_stream<T, GLU, RB, 1>(a, s);
+    case 2: return launch_stream<T, GLU, RB, 2>(a, s);
     case 4:
-      if constexpr (RB <= 2) return nt ? launch_stream<T, GLU, RB, 4, true>(a, s) : launch_stream<T, GLU, RB, 4, false>(a, s);
+      if constexpr (RB <= 2) return launch_stream<T, GLU, RB, 4>(a, s);
       break;  // (RB 4: four rings of 48 KB do not fit)
   }
   return MI_MOE_EUNSUPPORTED;
 }
 
-template <typename T> static int launch_stream_t(const GemmArgs& a, bool glu, int rb, int nw, bool nt, hipStream_t s) {
+template <typename T> static int launch_stream_t(const GemmArgs& a, bool glu, int rb, int nw, hipStream_t s) {
   switch (rb) {
-    case 1: return glu ? launch_stream_nw<T, true, 1>(a, nw, nt, s) : launch_stream_nw<T, false, 1>(a, nw, nt, s);
-    case 2: return glu ? launch_stream_nw<T, true, 2>(a, nw, nt, s) : launch_stream_nw<T, false, 2>(a, nw, nt, s);
-    case 4: return glu ? launch_stream_nw<T, true, 4>(a, nw, nt, s) : launch_stream_nw<T, false, 4>(a, nw, nt, s);
+    case 1: return glu ? launch_stream_nw<T, true, 1>(a, nw, s) : launch_stream_nw<T, false, 1>(a, nw, s);
+    case 2: return glu ? launch_stream_nw<T, true, 2>(a, nw, s) : launch_stream_nw<T, false, 2>(a, nw, s);
+    case 4: return glu ? launch_stream_nw<T, true, 4>(a, nw, s) : launch_stream_nw<T, false, 4>(a, nw, s);
     default: return MI_MOE_EUNSUPPORTED;
   }
 }
 
-// Where the stream is the faster form.  Measured with cold weights, us, up / down projection, stream against the tile
-// kernels (bf16 unless stated):
-//   hidden 1536, 40 experts, I 512     1 token 7.0 / 4.7 (19.6 / 8.3), 16: 22.5 / 12.7 (33.0 / 13.5), 64: 24.7 / 13.6
-//                                      (33.5 / 13.9), 128 (26 rows per expert): 30.0 / 16.4 (33.4 / 15.0), 256: 41.6 / 21.3
-//                                      (43.3 / 16.2)
-//   hidden 1024, 32 experts, I 512     64 tokens (16 rows) 13.3 / 8.8 (14.9 / 9.6), 128: 18.1 / 12.1 (16.0 / 10.3)
-//   hidden 4096, 8 experts, I 14336    1 token 76 / 36 (96 / 129), 64 (16 rows) 309 / 150 (344 / 187), 128: 394 / 186 (470 / 206)
-//   hidden 920, 17 experts, I 520 fp16 64 tokens 10.3 / 6.7 (17.3 / 11.6), 200 (47 rows) 14.8 / 9.0 (21.8 / 13.9)
-//   fp32, hidden 256, 8 experts, I 512 128 tokens (32 rows) 8.3 / 6.2 (13.8 / 21.0), 512: 14.9 / 9.0 (15.1 / 24.2), 2048: 40.6 /
-//                                      22.6 (36.6 / 24.9)
-//   fp32, hidden 1000, 17 experts      128 tokens 27.8 / 15.4 (44.8 / 26.1), 1024: 144 / 69 (123 / 71)
-// So: up to 16 rows per expert always; up to 28 with a contraction long enough to keep the rings full, up to 56 where it
-// is very long or where the tile kernels would pad a ragged one; fp32 as long as there are too few results to give
-// every CU a tile.
+// Where the stream is the faster form.  Measured with cold weights, us, up / down projection, experts chosen by random logits,
+// stream against the tile kernels (bf16 unless stated):
+//   hidden 1536, 40 experts, I 512     1 token 7.7 / 5.8 (25.6 / 8.3), 16: 23.7 / 14.4 (33.7 / 17.4), 64: 24.4 / 15.9 (33.3 /
+//                                      18.2), 96 (19 rows per expert): 28.4 (33.6), 128: 31.2 (33.6), and with Zipf(1.1) loads
+//                                      34.5 (33.4)
+//   hidden 1024, 32 experts, I 512     64 tokens (16 rows) 16.2 / 9.3 (17.6 / 11.2)
+//   hidden 2048, 16 experts, I 1024    64 tokens (16 rows) 26.0 / 15.4 (40.0 / 17.3), 80: 27.5 (39.9)
+//   hidden 4096, 8 experts, I 14336    1 token 79 / 36 (85 / 97), 64 (16 rows) 313 / 150 (333 / 184), 128: 399 / 188 (491 / 190);
+//                                      192 (48 rows) 439 / 211 (375 / 194)
+//   hidden 920, 17 experts, I 520 fp16 64 tokens 12.9 / 8.6 (22.1 / 14.3), 128 (30 rows) 21.8 / 12.1 (22.3 / 14.4), 200 (47 rows) 24.4 /
+//                                      13.5 (24.3 / 14.8), all of them on four experts 20.4 / 13.1 (16.4 / 10.8)
+//   fp32, hidden 256, 8 experts, I 512 128 tokens (32 rows) 9.3 / 6.9 (13.4 / 21.2), 512: 15.5 / 8.6 (15.3 / 23.9), 2048: 35.9 /
+//                                      23.4 (36.9 / 24.5)
+//   fp32, hidden 1000, 17 experts      128 tokens 43.7 / 26.3 (51.2 / 29.5), 512: 86 / 48 on the tiles, 84 / 48 on the stream
+// So: up to 16 rows per expert always; up to 24 with a contraction long enough to keep the rings full, below 48 where it
+// is very long, up to 40 where the tile kernels would pad a ragged one; fp32 as long as there are too few results to give
+// every CU a tile.  (Weights that the memory-side cache still holds from the last call -- one layer in a loop -- favour the
+// tiles: 40 experts, 80 tokens, 26.6 / 14.1 against 23.6 / 14.5.)
 // Never where an operand passes the 32-bit byte offsets of the DMA (fp32 only: the general rule counts elements).
 static bool stream_offsets_ok(const GemmArgs& a, bool glu, int elt) {
   const double row = (double)a.K * elt;
@@ -285,8 +310,8 @@ bool mi_gemm_stream_pick(const GemmArgs& a, bool glu, int elt) {
   const long rows = a.L, e = a.E;
   if (elt == 4) return rows <= 64 * e || rows * a.N <= (1L << 20);
   if (rows <= 16 * e) return true;
-  if (a.K % 32 != 0 || a.K >= 4096) return rows <= 56 * e;
-  return a.K >= 1280 && rows <= 28 * e;
+  if (a.K >= 4096) return rows < 48 * e;
+  return a.K % 32 != 0 ? rows <= 40 * e : a.K >= 1280 && rows <= 24 * e;
 }
 
 int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipStream_t s) {
@@ -294,21 +319,22 @@ int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipSt
   if (!stream_offsets_ok(a, glu, elt)) return MI_MOE_EUNSUPPORTED;
   const double avg = (double)a.L / a.E;
   if (rb == 0) {
-    // row blocks: most experts in one chunk; beyond that (fp32) long contractions re-read less with large chunks
-    rb = avg <= 16 ? 1 : (avg <= (elt == 4 ? 48 : 28) ? 2 : (elt == 4 && a.K <= 768 ? 1 : 4));
+    // row blocks: most experts in one chunk, and nearly all where a second one means long reads (13 of 16 rows on average);
+    // beyond that (fp32) long contractions re-read less with large chunks
+    rb = avg <= (elt == 2 && a.K >= 1280 ? 13 : 16) ? 1 : (avg <= (elt == 4 ? 48 : 28) ? 2 : (elt == 4 && a.K <= 768 ? 1 : 4));
     // waves per unit: enough of them for the chip when there are few units (1 token: 256 units, 7.0 us with four waves
-    // each, 9 with one), and always four on a long contraction
+    // each, 9 with one), always four on a long contraction, two with chunks of 32 rows on a fairly long one (hidden 1536, 96
+    // tokens: 33.8 -> 28.4 us)
     const int bm = 16 * rb, nk = mi_ceil_div(a.K, 128 / elt);
     const long touched = a.E < a.L ? a.E : a.L;
     const long units = touched * (long)(avg <= bm ? 1 : (avg + bm - 1) / bm) * mi_ceil_div(a.N, glu ? 16 : 32);
     nw = (units <= 320 || (nk >= 64 && units <= 2048)) && nk >= 4 ? 4 : (units <= 640 && nk >= 4 ? 2 : 1);
+    if (nw == 1 && rb == 2 && elt == 2 && nk >= 24) nw = 2;
     if (rb == 4 && nw == 4) nw = 2;
   }
-  // weights that one chunk per expert reads once are not worth a place in the caches (16 tokens: 25.8 -> 22.5 us)
-  const bool nt = avg <= 0.85 * 16 * rb;
   switch (dtype) {
-    case MI_MOE_F32: return launch_stream_t<float>(a, glu, rb, nw, nt, s);
-    case MI_MOE_F16: return launch_stream_t<f16_t>(a, glu, rb, nw, nt, s);
-    default: return launch_stream_t<bf16_t>(a, glu, rb, nw, nt, s);
+    case MI_MOE_F32: return launch_stream_t<float>(a, glu, rb, nw, s);
+    case MI_MOE_F16: return launch_stream_t<f16_t>(a, glu, rb, nw, s);
+    default: return launch_stream_t<bf16_t>(a, glu, rb, nw, s);
   }
 }

@@ -37,3 +37,32 @@ def test_stream_edges(device, dtype, counts, K, N, cfg):
     act = ops.up_swiglu(by_slot, w, k, ss, off, cfg=cfg)
     want = ref[:, :N] * torch.nn.functional.silu(ref[:, N:])
     torch.testing.assert_close(act.to(wide), want, **TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("counts,K,N", [([300, 7, 0, 33], 136, 296), ([16, 17, 129], 1096, 28), ([0, 513], 72, 520)])
+@pytest.mark.parametrize("cfg", [-1, 111, 124, 142])
+def test_stream_many_chunks(device, dtype, counts, K, N, cfg):
+    """Experts of many row chunks beside experts of one: the chunks of a unit are eight blocks apart, in groups of eight units
+    of which the last is smaller (10, 1 and 17 units plain; 19, 2 and 33 of SwiGLU).  A row's result does not depend on which
+    rows share its chunk: equal to the call in which every expert's rows are in another order, bit for bit."""
+    from dolomite_engine_amd import ops
+
+    g = torch.Generator().manual_seed(K + N)
+    E, L = len(counts), sum(counts)
+    print(f"stream chunks {counts} K={K} N={N} cfg={cfg} {dtype}", flush=True)
+    off = torch.tensor(counts).cumsum(0).int().to(device)
+    ss = torch.randperm(L, generator=g).int().to(device)
+    x = torch.randn(L, K, generator=g).to(dtype).to(device)
+    w = (torch.randn(E, 2 * N, K, generator=g) * 0.05).to(dtype).to(device)
+    wide = torch.float64 if dtype == torch.float32 else torch.float32
+    ref = torch.cat([p.to(wide) @ w[e].to(wide).t() for e, p in enumerate(x.split(counts))])
+    plain = ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=cfg)
+    torch.testing.assert_close(plain.to(wide), ref, **TOL[dtype])
+    other = torch.cat([p.flip(0) for p in torch.arange(L).split(counts)]).to(device)
+    assert torch.equal(ops.scattered_gemm(x[other].contiguous(), w, 1, ss, off, True, True, cfg=cfg), plain[other])
+    by_slot = torch.empty_like(x)
+    by_slot[ss.long()] = x
+    act = ops.up_swiglu(by_slot, w, 1, ss, off, cfg=cfg)
+    want = ref[:, :N] * torch.nn.functional.silu(ref[:, N:])
+    torch.testing.assert_close(act.to(wide), want, **TOL[dtype])
