@@ -290,13 +290,13 @@ template <typename T> static int launch_stream_t(const GemmArgs& a, bool glu, in
 //   hidden 2048, 16 experts, I 1024    64 tokens (16 rows) 26.0 / 15.4 (40.0 / 17.3), 80: 27.5 (39.9)
 //   hidden 4096, 8 experts, I 14336    1 token 79 / 36 (85 / 97), 64 (16 rows) 313 / 150 (333 / 184), 128: 399 / 188 (491 / 190);
 //                                      192 (48 rows) 439 / 211 (375 / 194)
-//   hidden 920, 17 experts, I 520 fp16 64 tokens 12.9 / 8.6 (22.1 / 14.3), 128 (30 rows) 21.8 / 12.1 (22.3 / 14.4), 200 (47 rows) 24.4 /
-//                                      13.5 (24.3 / 14.8), all of them on four experts 20.4 / 13.1 (16.4 / 10.8)
-//   fp32, hidden 256, 8 experts, I 512 128 tokens (32 rows) 9.3 / 6.9 (13.4 / 21.2), 512: 15.5 / 8.6 (15.3 / 23.9), 2048: 35.9 /
-//                                      23.4 (36.9 / 24.5)
+//   hidden 920, 17 experts, I 520 fp16 64 tokens 12.9 / 8.6 (22.1 / 14.3), 128 (30 rows) 16.5 / 9.4 (22.3 / 14.4), 200 (47 rows) 19.1 /
+//                                      10.4 (24.3 / 14.8), all of them on four experts 17.7 / 11.1 (16.4 / 10.8)
+//   fp32, hidden 256, 8 experts, I 512 128 tokens (32 rows) 9.3 / 6.9 (13.4 / 21.2), 512: 15.5 / 8.6 (15.3 / 23.9), 2048: 36.0 /
+//                                      23.4 (37.0 / 24.5)
 //   fp32, hidden 1000, 17 experts      128 tokens 43.7 / 26.3 (51.2 / 29.5), 512: 86 / 48 on the tiles, 84 / 48 on the stream
 // So: up to 16 rows per expert always; up to 24 with a contraction long enough to keep the rings full, below 48 where it
-// is very long, up to 40 where the tile kernels would pad a ragged one; fp32 as long as there are too few results to give
+// is very long, up to 56 where the tile kernels would pad a ragged one; fp32 as long as there are too few results to give
 // every CU a tile.  (Weights that the memory-side cache still holds from the last call -- one layer in a loop -- favour the
 // tiles: 40 experts, 80 tokens, 26.6 / 14.1 against 23.6 / 14.5.)
 // Never where an operand passes the 32-bit byte offsets of the DMA (fp32 only: the general rule counts elements).
@@ -311,7 +311,7 @@ bool mi_gemm_stream_pick(const GemmArgs& a, bool glu, int elt) {
   if (elt == 4) return rows <= 64 * e || rows * a.N <= (1L << 20);
   if (rows <= 16 * e) return true;
   if (a.K >= 4096) return rows < 48 * e;
-  return a.K % 32 != 0 ? rows <= 40 * e : a.K >= 1280 && rows <= 24 * e;
+  return a.K % 32 != 0 ? rows <= 56 * e : a.K >= 1280 && rows <= 24 * e;
 }
 
 int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipStream_t s) {
@@ -320,8 +320,9 @@ int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipSt
   const double avg = (double)a.L / a.E;
   if (rb == 0) {
     // row blocks: most experts in one chunk, and nearly all where a second one means long reads (13 of 16 rows on average);
-    // beyond that (fp32) long contractions re-read less with large chunks
-    rb = avg <= (elt == 2 && a.K >= 1280 ? 13 : 16) ? 1 : (avg <= (elt == 4 ? 48 : 28) ? 2 : (elt == 4 && a.K <= 768 ? 1 : 4));
+    // fp32 beyond that: small chunks, whatever the load (17 experts, hidden 1000, 256 tokens, up-projection, us, 16 / 64 rows a
+    // chunk: even load 54 / 45, Zipf(1.1) 53 / 67, tiles 65)
+    rb = avg <= (elt == 2 && a.K >= 1280 ? 13 : 16) ? 1 : (avg <= (elt == 4 ? 48 : 28) ? 2 : (elt == 4 ? 1 : 4));
     // waves per unit: enough of them for the chip when there are few units (1 token: 256 units, 7.0 us with four waves
     // each, 9 with one), always four on a long contraction, two with chunks of 32 rows on a fairly long one (hidden 1536, 96
     // tokens: 33.8 -> 28.4 us)
@@ -330,7 +331,9 @@ int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipSt
     const long units = touched * (long)(avg <= bm ? 1 : (avg + bm - 1) / bm) * mi_ceil_div(a.N, glu ? 16 : 32);
     nw = (units <= 320 || (nk >= 64 && units <= 2048)) && nk >= 4 ? 4 : (units <= 640 && nk >= 4 ? 2 : 1);
     if (nw == 1 && rb == 2 && elt == 2 && nk >= 24) nw = 2;
-    if (rb == 4 && nw == 4) nw = 2;
+    // (chunks of 64 rows: two rings of 48 KB cost more than they bring, 17 experts, hidden 920, 128 tokens 21.8 / 12.1 us with two
+    // waves, 16.5 / 9.4 with one -- except on the very long contractions: K 14336, 128 tokens 188 / 252)
+    if (rb == 4) nw = nw > 1 && nk >= 64 ? 2 : 1;
   }
   switch (dtype) {
     case MI_MOE_F32: return launch_stream_t<float>(a, glu, rb, nw, s);
