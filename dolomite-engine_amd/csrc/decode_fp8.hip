@@ -466,8 +466,11 @@ int mi_gemm_fp8_tiled(const void* in, const void* wq, const float* scale, void* 
 // Rows per expert (on average) from which the tile kernels take over: the streaming kernels read an expert's
 // weights once per 16 of its rows, a tile kernel once per row tile.  Measured on 64 experts of 2 x 1408 x 4096 and
 // 4096 x 1408 weights, top-6, both projections, streaming / tiles: 12 rows per expert 220 us / 252, 13.5 rows 246 / 247,
-// 15 rows 279 / 235, 24 rows 426 / 255.  (The register-staged tiles, where they are picked: 12 rows 266, 18 rows 273.)
+// 15 rows 279 / 235, 24 rows 426 / 255.  (The register-staged tiles, where they are picked: 12 rows 266, 18 rows 273.)  With fewer
+// tiles than would fill the chip twice over the streaming kernels hold out longer (14 rows per expert: 8 experts, K 14336,
+// N 4096, 128 tiles, 118 / 150; 40 experts, K 1536, I 512, 160 tiles, 22 / 29).
 #define FP8_PERSISTENT_MIN_ROWS 14
+#define FP8_PERSISTENT_MIN_TILES 400
 #define FP8_TILED_MIN_ROWS 16
 
 static int run_decode(DecodeArgs a, int dtype, bool glu, hipStream_t s, int cfg) {
@@ -478,7 +481,8 @@ static int run_decode(DecodeArgs a, int dtype, bool glu, hipStream_t s, int cfg)
   if ((a.gather || a.scatter) && !a.sorted_scattered) return MI_MOE_ENULL;
   if (a.K % 16 != 0 || a.N % 4 != 0) return MI_MOE_EUNSUPPORTED;
   // cfg: -1 by the batch, 0 the streaming kernels, else a form of mi_gemm_fp8_tiled
-  const long min_rows = mi_gemm_fp8_persistent_pick(a.L, a.K, a.N, a.E, glu) ? FP8_PERSISTENT_MIN_ROWS : FP8_TILED_MIN_ROWS;
+  const bool many = (long)a.E * mi_ceil_div(a.N, glu ? 128 : 256) >= FP8_PERSISTENT_MIN_TILES;
+  const long min_rows = many && mi_gemm_fp8_persistent_pick(a.L, a.K, a.N, a.E, glu) ? FP8_PERSISTENT_MIN_ROWS : FP8_TILED_MIN_ROWS;
   if (cfg > 0 || (cfg < 0 && (long)a.L >= min_rows * a.E))
     return mi_gemm_fp8_tiled(a.in, a.wq, a.scale, a.out, a.sorted_scattered, a.expert_offsets, a.L, a.K, a.N, a.E,
                              a.kdiv, a.gather, a.scatter, glu ? 1 : 0, a.tiled ? 1 : 0, dtype, cfg < 0 ? FP8_BY_SHAPE : cfg, s);
