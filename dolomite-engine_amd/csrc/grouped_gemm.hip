@@ -912,10 +912,19 @@ static bool tiled_aligned(const GemmArgs& a, int elt_bytes) {
 // So few 256 x 256 tiles that most CUs would have none: smaller tiles give four times as many workgroups.  Measured, us,
 // 256 x 256 tiles against 128 x 128: one expert (shared experts, the router's gradient) of 2048 rows, 1024 -> 1024 (SwiGLU,
 // 64 tiles) 24.5 / 15.7, of 1429 rows (24 tiles) 23.3 / 12.9, of 3001 rows, 920 -> 344 fp16 (36 tiles) 23.3 / 17.0; 4096
-// rows 1536 -> 512 (64 tiles) 31.6 / 20.8; but 512 -> 1536 (96 tiles) 15.6 / 16.7, 17 experts of 235 rows, 920 -> 520 (85
-// tiles) 26.0 / 26.2.
+// rows 1536 -> 512 (64 tiles) 31.6 / 20.8; but 512 -> 1536 (96 tiles) 15.6 / 16.7.
+// Beyond that the 128 x 128 tiles win while they are at most one to a CU (experts chosen by random logits, cold weights, up
+// projection: 24 experts of 120 rows, 1024 -> 512 (240 of them) 28.9 / 20.9; 12 experts, 2048 -> 1024 (240) 47.2 / 36.4; 6 experts,
+// 4096 -> 1792 (210) 81.8 / 63.6; but 32 experts, 1024 -> 512 (320) 29.3 / 32.8 and 24 of 150 rows (384) 29.2 / 27.0, with their
+// down-projections 48.2 / 46.3), and where K is ragged, which costs the 256 x 256 tiles' DMA half lines, while they are
+// all resident, two to a CU (920 -> 520: 24 experts of 240 rows (432) 35.2 / 32.8, 17 of 300 (459) 32.2 / 29.3, 20 of 300 (540) 33.0 /
+// 46.7, 24 of 300 (648) 34.6 / 49.1).
 static bool few_large_tiles(const GemmArgs& a, bool glu) {
-  return (double)a.E * mi_ceil_div((a.L + a.E - 1) / a.E, 256) * mi_ceil_div(a.N, glu ? 128 : 256) <= 72;
+  const int avg = (a.L + a.E - 1) / a.E;
+  if ((double)a.E * mi_ceil_div(avg, 256) * mi_ceil_div(a.N, glu ? 128 : 256) <= 72) return true;
+  // (a quarter of the experts has a row tile more than the average one)
+  const double small = (double)a.E * mi_ceil_div(avg, 128) * mi_ceil_div(a.N, glu ? 64 : 128);
+  return a.K % 32 == 0 ? 1.25 * small <= 256 : small <= 512;
 }
 
 #define PERSIST_MIN_ROWS 120  // rows per expert on average
