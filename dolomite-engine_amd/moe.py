@@ -245,7 +245,7 @@ class MoE(nn.Module):
             and hidden_states.is_cuda
             and ops._TIMER is None
             and not self._needs_grad(hidden_states)
-            and isinstance(self.dropout, nn.Identity)
+            and self._stages_as_written()
         ):
             # inference: all stages behind one library call (None: something the stage-by-stage code below has to look at)
             y = self._forward_native(hidden_states, residual, residual_scale, pre_norm)
@@ -324,14 +324,22 @@ class MoE(nn.Module):
 
         return hidden_states
 
+    def _stages_as_written(self) -> bool:
+        """Whether the stage-by-stage code would run what the one-call forward stands for: no stage replaced (by a subclass,
+        on the class or on the instance), no hook on, and no other forward in, a module that it calls."""
+        cls, own = type(self), self.__dict__
+        for name, function in _STAGES.items():
+            if getattr(cls, name) is not function or name in own:
+                return False
+        return (_called_as_written(self.c_proj, ParameterizedExperts, _EXPERTS_FORWARD)
+                and _called_as_written(self.dropout, nn.Identity, _IDENTITY_FORWARD) and not _any_global_hook())
+
     def _forward_native(self, hidden_states: torch.Tensor, residual: torch.Tensor | None,
                         residual_scale: float | None, pre_norm: tuple | None) -> torch.Tensor | None:
         """The whole eval-mode forward through ops.layer_forward; None where it does not take the call."""
         fc, proj = self.c_fc, self.c_proj
         if fc.bias is not None or proj.bias is not None:
             return None
-        if type(proj) is not ParameterizedExperts or proj._forward_hooks or proj._forward_pre_hooks:
-            return None  # (the stage-by-stage code calls the down-projection as a module)
         shared_fc = shared_proj = None
         if self.shared_intermediate_size is not None:
             if self.c_fc_shared.bias is not None or self.c_proj_shared.bias is not None:
@@ -340,12 +348,10 @@ class MoE(nn.Module):
         weight_q = fc.weight_q
         if weight_q is not None:
             weights = (weight_q, proj.weight_q, fc.weight_scale, proj.weight_scale)
-            if weights[1] is None:
-                return None
         else:
             weights = (fc.weight, proj.weight, None, None)
-            if weights[1] is None:
-                return None
+        if weights[1] is None:
+            return None
         gate_weight = self.gate.weight
         logits = None
         if pre_norm is None and not ops.router_fused_supported(hidden_states, self.num_experts, self.top_k):
@@ -592,3 +598,20 @@ class MoE(nn.Module):
             raise RuntimeError("fp8 expert weights do not support biases")
         self.c_fc.quantize_fp8(tiled=tiled, glu=self._fused_swiglu)
         self.c_proj.quantize_fp8(tiled=tiled, glu=False)
+
+
+# What the one-call forward stands for, as it is written above (see MoE._stages_as_written).
+_STAGES = {name: getattr(MoE, name) for name in ("_route", "_use_fused_router", "_compute_experts",
+                                                 "_compute_shared_experts")}
+_EXPERTS_FORWARD = ParameterizedExperts.forward
+_IDENTITY_FORWARD = nn.Identity.forward
+
+
+def _called_as_written(module: nn.Module, cls: type, forward) -> bool:
+    return (type(module) is cls and cls.forward is forward and not module._forward_hooks
+            and not module._forward_pre_hooks and "forward" not in module.__dict__)
+
+
+def _any_global_hook() -> bool:
+    hooks = torch.nn.modules.module
+    return bool(hooks._global_forward_hooks or hooks._global_forward_pre_hooks)

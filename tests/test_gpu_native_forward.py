@@ -81,3 +81,70 @@ def test_native_forward_refuses_what_does_not_fit(device):
         want = m(x)
         m.c_proj.register_forward_hook(lambda *a: seen.append(1))
         assert torch.equal(m(x), want) and seen
+
+
+def _layer(device, **kwargs):
+    from dolomite_engine_amd import MoE
+
+    sizes = dict(hidden_size=128, intermediate_size=64, shared_intermediate_size=32, num_experts=4, num_experts_per_tok=2)
+    return MoE(**{**sizes, **kwargs}, activation_function="swiglu", add_bias=False, dropout=0.0, init_method="normal",
+                        initializer_range=0.05, m_width=None, num_layers=1,
+                        use_padding_free_transformer=True).bfloat16().to(device).eval()
+
+
+@pytest.mark.parametrize("stage", ["_compute_experts", "_compute_shared_experts", "_route", "c_proj.forward",
+                                   "dropout.forward"])
+@pytest.mark.parametrize("where", ["subclass", "class", "instance"])
+def test_native_forward_leaves_replaced_stages_alone(device, monkeypatch, stage, where):
+    """A stage that a subclass or a caller replaced is called in eval() as it is in train()."""
+    from dolomite_engine_amd import Kernel, MoE, enable_kernels
+
+    torch.manual_seed(5)
+    x = torch.randn(300, 128, device=device, dtype=torch.bfloat16)
+    m = _layer(device, num_experts=72)  # (up to 64, the router and the sort are one call and _route is not called)
+    owner = m
+    *path, name = stage.split(".")
+    for part in path:
+        owner = getattr(owner, part)
+    original = getattr(type(owner), name)
+    seen = []
+
+    def replacement(self, *args, **kwargs):
+        seen.append(1)
+        return original(self, *args, **kwargs)
+
+    with torch.no_grad(), enable_kernels([Kernel.scattermoe]):
+        want = m(x)
+        if where == "subclass":
+            owner.__class__ = type("Replaced", (type(owner),), {name: replacement})
+        elif where == "class":
+            monkeypatch.setattr(type(owner), name, replacement)
+        else:
+            owner.__dict__[name] = replacement.__get__(owner)
+        assert torch.equal(m(x), want)
+    assert seen
+
+
+@pytest.mark.parametrize("module", ["c_proj", "dropout", None])
+@pytest.mark.parametrize("pre", [False, True])
+def test_native_forward_leaves_hooks_alone(device, module, pre):
+    """Hooks on the modules that the stages call, and hooks on every module, run in eval() too."""
+    from dolomite_engine_amd import Kernel, enable_kernels
+
+    torch.manual_seed(6)
+    x = torch.randn(9, 128, device=device, dtype=torch.bfloat16)
+    m = _layer(device)
+    seen = []
+    with torch.no_grad(), enable_kernels([Kernel.scattermoe]):
+        want = m(x)
+        if module is not None:
+            register = getattr(getattr(m, module), "register_forward_pre_hook" if pre else "register_forward_hook")
+        else:
+            hooks = torch.nn.modules.module
+            register = hooks.register_module_forward_pre_hook if pre else hooks.register_module_forward_hook
+        handle = register(lambda mod, *a: seen.append(type(mod).__name__))
+        try:
+            assert torch.equal(m(x), want)
+        finally:
+            handle.remove()
+    assert seen and (module is not None or "ParameterizedExperts" in seen)
