@@ -238,6 +238,7 @@ class MoE(nn.Module):
         if residual is not None:
             residual = residual.reshape(-1, self.hidden_size)
 
+        logits = None
         if (
             not self.training
             and self._fused_swiglu
@@ -248,7 +249,7 @@ class MoE(nn.Module):
             and self._stages_as_written()
         ):
             # inference: all stages behind one library call (None: something the stage-by-stage code below has to look at)
-            y = self._forward_native(hidden_states, residual, residual_scale, pre_norm)
+            y, logits = self._forward_native(hidden_states, residual, residual_scale, pre_norm)
             if y is not None:
                 add_aux_loss(0)
                 return y if self.use_padding_free_transformer else y.reshape(batch_size, sequence_length, self.hidden_size)
@@ -277,7 +278,7 @@ class MoE(nn.Module):
 
         if routed is None:
             # (with a gradient the router function may hand back the expert sort as well)
-            *routed, presorted = self._route(hidden_states)
+            *routed, presorted = self._route(hidden_states) if logits is None else self._route(hidden_states, logits)
         router_logits, router_weights, selected_experts = routed
 
         # the tail can only be folded in where nothing sits between the expert sum and it
@@ -334,16 +335,17 @@ class MoE(nn.Module):
         return (_called_as_written(self.c_proj, ParameterizedExperts, _EXPERTS_FORWARD)
                 and _called_as_written(self.dropout, nn.Identity, _IDENTITY_FORWARD) and not _any_global_hook())
 
-    def _forward_native(self, hidden_states: torch.Tensor, residual: torch.Tensor | None,
-                        residual_scale: float | None, pre_norm: tuple | None) -> torch.Tensor | None:
-        """The whole eval-mode forward through ops.layer_forward; None where it does not take the call."""
+    def _forward_native(self, hidden_states: torch.Tensor, residual: torch.Tensor | None, residual_scale: float | None,
+                        pre_norm: tuple | None) -> tuple[torch.Tensor | None, torch.Tensor | None]:
+        """The whole eval-mode forward through ops.layer_forward, None where it does not take the call; and the router's
+        logits if they had to be formed by torch before that was known, for the stage-by-stage code to go on from."""
         fc, proj = self.c_fc, self.c_proj
         if fc.bias is not None or proj.bias is not None:
-            return None
+            return None, None
         shared_fc = shared_proj = None
         if self.shared_intermediate_size is not None:
             if self.c_fc_shared.bias is not None or self.c_proj_shared.bias is not None:
-                return None
+                return None, None
             shared_fc, shared_proj = self.c_fc_shared.weight, self.c_proj_shared.weight
         weight_q = fc.weight_q
         if weight_q is not None:
@@ -351,13 +353,13 @@ class MoE(nn.Module):
         else:
             weights = (fc.weight, proj.weight, None, None)
         if weights[1] is None:
-            return None
+            return None, None
         gate_weight = self.gate.weight
         logits = None
         if pre_norm is None and not ops.router_fused_supported(hidden_states, self.num_experts, self.top_k):
             logits = self._unfused_logits(hidden_states)
         return ops.layer_forward(hidden_states, gate_weight, self.router_logit_bias, self.top_k, *weights,
-                                 shared_fc, shared_proj, residual, residual_scale, pre_norm, logits)
+                                 shared_fc, shared_proj, residual, residual_scale, pre_norm, logits), logits
 
     def _unfused_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         """Router logits of shapes the router kernel does not take (more than 256 experts, a hidden size that is not a
@@ -394,12 +396,12 @@ class MoE(nn.Module):
         """moe.py:246-257: (router_logits, router_weights, selected_experts)."""
         return self._route(hidden_states)[:3]
 
-    def _route(self, hidden_states: torch.Tensor):
+    def _route(self, hidden_states: torch.Tensor, logits: torch.Tensor | None = None):
         """moe.py:246-257, plus the expert sort where the router produced it: (router_logits, router_weights,
         selected_experts, presorted or None).  On the kernel path the gate GEMM, top-k and softmax are one kernel in
         every dtype; in eval mode the (T, E) logits are never written (only the training aux loss and the backward
         read them); with a gradient the same kernel runs inside autograd.FusedRouter, whose backward is kernels
-        too."""
+        too.  ``logits``: the result of _unfused_logits, where the caller has it already."""
         if (is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda
                 and ops.router_fused_supported(hidden_states, self.num_experts, self.top_k)):
             if self._needs_grad(hidden_states):
@@ -410,7 +412,7 @@ class MoE(nn.Module):
                                       return_logits=self.training), None)
 
         if is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda:
-            router_logits = self._unfused_logits(hidden_states)
+            router_logits = self._unfused_logits(hidden_states) if logits is None else logits
             with torch.no_grad():
                 router_weights, selected_experts = ops.router_topk_softmax(router_logits.detach(), self.top_k)
             if torch.is_grad_enabled() and router_logits.requires_grad:

@@ -148,3 +148,22 @@ def test_native_forward_leaves_hooks_alone(device, module, pre):
         finally:
             handle.remove()
     assert seen and (module is not None or "ParameterizedExperts" in seen)
+
+
+@pytest.mark.parametrize("hidden,intermediate,fp8,tokens", [(132, 64, False, 9), (136, 64, False, 9), (136, 64, True, 9),
+                                                            (136, 60, False, 9)])
+def test_gate_runs_once_per_forward(device, hidden, intermediate, fp8, tokens):
+    """Hidden sizes that no router kernel takes: torch forms the logits, once, also where the one-call forward then refuses
+    the layer (hidden or intermediate size no multiple of 8, fp8 weights with a hidden size that is no multiple of 16)."""
+    from dolomite_engine_amd import Kernel, enable_kernels
+
+    torch.manual_seed(7)
+    m = _layer(device, hidden_size=hidden, intermediate_size=intermediate)
+    if fp8:
+        m.quantize_expert_weights_fp8()
+    seen = []
+    m.gate.register_forward_hook(lambda *a: seen.append(1))
+    x = torch.randn(tokens, hidden, device=device, dtype=torch.bfloat16)
+    with torch.no_grad(), enable_kernels([Kernel.scattermoe]):
+        m(x)
+    assert len(seen) == 1
