@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
             *reinterpret_cast<u32x2*>(scratch + (mbp * 16 + fi) * 256 + (((2 * nb + (fq >> 1)) ^ fi) * 16) + (fq & 1) * 8) =
                 (u32x2){pack2<T>(v0, v1), pack2<T>(v2, v3)};
           }
-        asm volatile("" ::: "memory");
+        pg_own_agprs();
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
           const int r = 4 * it + (lane >> 4);
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
           const int m = mt * TILE + wm * 128 + p * 32 + r, n = nt * TILE + wn * 128 + ((lane & 15) ^ (r & 15)) * 8;
           if (interior || (m < a.M && n < a.N)) *reinterpret_cast<u32x4*>(out + (size_t)m * a.N + n) = v;
         }
-        asm volatile("" ::: "memory");
+        pg_own_agprs();
       }
     } else {
       // (blocks wholly past M or N do not exist: a router's gradient, 40 x 1536, is a sixth of its tiles)
@@ -420,6 +420,7 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
       f32x4* base = reinterpret_cast<f32x4*>(a.partial) + (((size_t)grp * m_blocks + mb0) * n_blocks + nb0) * 64 + lane;
 #pragma unroll
       for (int mb = 0; mb < 8; ++mb) {
+        pg_own_agprs();
         if (mb0 + mb >= m_blocks) continue;
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb) {

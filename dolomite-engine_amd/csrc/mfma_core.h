@@ -2,8 +2,11 @@
 // register file (persistent_gemm.hip, grouped_wgrad.hip), and DMA from memory to LDS.
 //
 // The accumulators are addressed by number.  As C++ values they would be 64 four-register tuples that fill the AGPR file
-// to the last register, and the compiler moved and spilled them at every tile boundary.  Every phase of the kernels
-// names all of them as clobbered (pg_own_agprs, pg_acc_settle), so nothing of the compiler's can live there.
+// to the last register, and the compiler moved and spilled them at every tile boundary.  To the compiler all of them are
+// lost at every pg_own_agprs and pg_acc_settle: nothing of its own can live there from one of these to behind the next.
+// They stand at the start of each half slice, at the end of a tile, and between the groups of accumulators that an
+// epilogue reads.  Between two of them it could still place a value that lives no longer than that; what the built
+// kernels do with a0 .. a255 is checked on the built code (tests/test_accumulator_registers.py).
 #pragma once
 
 #include "common.h"

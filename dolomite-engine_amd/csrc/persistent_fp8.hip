@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
               (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
         }
       }
-      asm volatile("" ::: "memory");
+      pg_own_agprs();
 #pragma unroll
       for (int it0 = 0; it0 < 8; it0 += 4) {
         u32x4 val[4];
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
           }
         }
       }
-      asm volatile("" ::: "memory");
+      pg_own_agprs();
     }
   };
   auto epilogue = [&](const PgTile& t, bool interior) {

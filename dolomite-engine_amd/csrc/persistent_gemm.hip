@@ -371,7 +371,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
           *(wp_t)(size_t)(s0 + (scr_w ^ (nb * 32)) + mbp * (16 / RPP) * 4096) =
               (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
         }
-      asm volatile("" ::: "memory");
+      pg_own_agprs();
       // (four at a time: one LDS latency for all of them)
 #pragma unroll
       for (int it0 = 0; it0 < 8; it0 += 4) {
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
           }
         }
       }
-      asm volatile("" ::: "memory");
+      pg_own_agprs();
     }
   };
   typedef std::integral_constant<int, 0> what_result;
@@ -427,6 +427,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
                   ((size_t)sp.ws_base + (size_t)my_rem_tile * sp.parts + my_part) * (64 * 256) + threadIdx.x;
 #pragma unroll
     for (int b = 0; b < 64; ++b) {
+      if (b % 8 == 0) pg_own_agprs();
       const f32x4 v = {pg_acc(4 * b), pg_acc(4 * b + 1), pg_acc(4 * b + 2), pg_acc(4 * b + 3)};
       base[b * 256] = v;
     }
