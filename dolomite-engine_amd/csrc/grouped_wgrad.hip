@@ -281,6 +281,9 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
       __builtin_amdgcn_s_waitcnt(pg_wait(8, 0));
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
+      // (the indices are there from here on: the compiler took them as ready where they were requested)
+      if (GA) asm volatile("" : "+v"(ai[0]), "+v"(ai[1]));
+      if (GB) asm volatile("" : "+v"(bi[0]), "+v"(bi[1]));
       PG_SCHED();
       const bool b_short = ks_b >= nfull;
       if (!GB && b_short) mask_rows(boff, ks_b);

@@ -6,7 +6,7 @@
 // lost at every pg_own_agprs and pg_acc_settle: nothing of its own can live there from one of these to behind the next.
 // They stand at the start of each half slice, at the end of a tile, and between the groups of accumulators that an
 // epilogue reads.  Between two of them it could still place a value that lives no longer than that; what the built
-// kernels do with a0 .. a255 is checked on the built code (tests/test_accumulator_registers.py).
+// kernels do with a0 .. a255 is checked on the built code (tests/test_built_kernels.py).
 #pragma once
 
 #include "common.h"
