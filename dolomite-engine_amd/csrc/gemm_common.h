@@ -53,8 +53,10 @@ int mi_gemm_fp8_persistent(const GemmArgs& a, int dtype, bool glu, hipStream_t s
 // ---- stream_gemm.hip: K a multiple of one 16-byte chunk, N % 4 == 0 ------------------------------------------------------
 // whether the stream is the faster form for this problem (elt: bytes of an element)
 bool mi_gemm_stream_pick(const GemmArgs& a, bool glu, int elt);
-// rb: row blocks of 16 per unit (1, 2, 4); nw: waves that split the contraction (1, 2, 4; rb 4: 1, 2); 0, 0: by the rule
-int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipStream_t s);
+// form: 10 x row blocks of 16 per unit (1, 2, 4) + waves that split the contraction (1, 2, 4; row blocks 4: 1, 2); below 10: by
+// the rule, which is
+int mi_gemm_stream_form(const GemmArgs& a, bool glu, int elt);
+int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int form, hipStream_t s);
 
 // ---- grouped_gemm.hip: one expert that owns every row, rows in place (no index arrays): out = in @ W^T, or with SwiGLU ------
 int mi_gemm_one_expert(const void* in, const void* w, void* out, int L, int K, int N, bool glu, int dtype, mi_moe_stream_t stream);

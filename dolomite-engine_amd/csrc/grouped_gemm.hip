@@ -929,8 +929,19 @@ static bool few_large_tiles(const GemmArgs& a, bool glu) {
 
 #define PERSIST_MIN_ROWS 120  // rows per expert on average
 
-static int pick_cfg(const GemmArgs& a, bool glu) {
+// The configuration for cfg -1: one of the numbers of mi_moe_scattered_gemm_cfg (100 + row blocks and waves: the weight stream).
+static int pick_cfg(const GemmArgs& a, bool glu, int elt) {
+  if (mi_gemm_stream_pick(a, glu, elt)) return 100 + mi_gemm_stream_form(a, glu, elt);
   const long avg = a.E > 0 ? (long)a.L / a.E : a.L;  // rows per expert if the load were uniform
+  if (elt == 4) {
+    // fp32 matrix instructions are slow enough that what matters is how many CUs have a tile.  Measured (up /
+    // down projection, us): 128 x 128 tiles beat 256 x 256 at every size tried (262144 rows, 40 experts, hidden
+    // 1536: 3240 / 1678 against 3359 / 1690; 65536 rows, 32 experts: 1136 / 585 against 1338 / 686), and below
+    // about two 128 x 128 tiles per CU the 32 x 256 tiles win (the reference's correctness configuration, 1024
+    // rows in 8 experts: 15 / 24 against 23 / 37; 4096 rows: 38 / 25 against 43 / 38 and, for 256 x 256, 73 / 127).
+    const long tiles128 = ((long)a.L / 128 + a.E / 2 + 1) * mi_ceil_div((glu ? 2 : 1) * a.N, 128);
+    return avg < 48 ? 5 : ((avg >= 512 && tiles128 >= 512) ? 1 : 2);
+  }
   // (128 x 128 tiles need a second row tile, and a second pass over the weights, for the experts with more than 128 rows.
   // Persistent / 128 x 128 tiles, us, up and down projection: hidden 1536, 40 experts, 80 rows per expert 35.8 / 31.6 and
   // 23.7 / 17.8, 120 rows 38.2 / 38.8 and 22.0 / 29.7, 160 rows 37.2 / 46.1 and 20.6 / 32.0; hidden 4096, 8 experts, I 14336,
@@ -962,22 +973,9 @@ static int run_gemm(GemmArgs a, int dtype, bool glu, int cfg, int in_rows_bound,
   const int elt = dtype == MI_MOE_F32 ? 4 : 2;
   if (!tiled_shape_ok(a, in_rows_bound, glu, elt)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, elt)) return MI_MOE_EALIGN;
-  if (cfg >= 100) return mi_gemm_stream(a, dtype, glu, (cfg - 100) / 10, cfg % 10, s);
-  if (cfg < 0 && mi_gemm_stream_pick(a, glu, elt)) return mi_gemm_stream(a, dtype, glu, 0, 0, s);
-  if (dtype == MI_MOE_F32) {
-    if (cfg < 0) {
-      // fp32 matrix instructions are slow enough that what matters is how many CUs have a tile.  Measured (up /
-      // down projection, us): 128 x 128 tiles beat 256 x 256 at every size tried (262144 rows, 40 experts, hidden
-      // 1536: 3240 / 1678 against 3359 / 1690; 65536 rows, 32 experts: 1136 / 585 against 1338 / 686), and below
-      // about two 128 x 128 tiles per CU the 32 x 256 tiles win (the reference's correctness configuration, 1024
-      // rows in 8 experts: 15 / 24 against 23 / 37; 4096 rows: 38 / 25 against 43 / 38 and, for 256 x 256, 73 / 127).
-      const long avg = a.E > 0 ? (long)a.L / a.E : a.L;
-      const long tiles128 = ((long)a.L / 128 + a.E / 2 + 1) * mi_ceil_div((glu ? 2 : 1) * a.N, 128);
-      cfg = avg < 48 ? 5 : ((avg >= 512 && tiles128 >= 512) ? 1 : 2);
-    }
-    return glu ? dispatch_cfg_f32<true>(a, cfg, s) : dispatch_cfg_f32<false>(a, cfg, s);
-  }
-  if (cfg < 0) cfg = pick_cfg(a, glu);
+  if (cfg < 0) cfg = pick_cfg(a, glu, elt);
+  if (cfg >= 100) return mi_gemm_stream(a, dtype, glu, cfg - 100, s);
+  if (dtype == MI_MOE_F32) return glu ? dispatch_cfg_f32<true>(a, cfg, s) : dispatch_cfg_f32<false>(a, cfg, s);
   if (dtype == MI_MOE_BF16) return glu ? dispatch_cfg<bf16_t, true>(a, cfg, s) : dispatch_cfg<bf16_t, false>(a, cfg, s);
   return glu ? dispatch_cfg<f16_t, true>(a, cfg, s) : dispatch_cfg<f16_t, false>(a, cfg, s);
 }
@@ -990,6 +988,15 @@ static int check_common(const void* in, const void* w, void* out, const int32_t*
   if (!in || !w || !out || !off) return MI_MOE_ENULL;
   if (need_ss && !ss) return MI_MOE_ENULL;
   return MI_MOE_OK;
+}
+
+extern "C" int mi_moe_grouped_gemm_choice(int L, int K, int N, int E, int glu, int dtype) {
+  if (L < 1 || K < 1 || N < 1 || E < 1 || E > 65536) return MI_MOE_ESHAPE;
+  if (dtype != MI_MOE_F32 && dtype != MI_MOE_F16 && dtype != MI_MOE_BF16) return MI_MOE_EDTYPE;
+  const int elt = dtype == MI_MOE_F32 ? 4 : 2;
+  GemmArgs a = {};  // (null pointers count as aligned)
+  a.L = L; a.K = K; a.N = N; a.E = E; a.kdiv = 1;
+  return tiled_shape_ok(a, L, glu != 0, elt) ? pick_cfg(a, glu != 0, elt) : MI_MOE_EUNSUPPORTED;
 }
 
 int mi_gemm_one_expert(const void* in, const void* w, void* out, int L, int K, int N, bool glu, int dtype, mi_moe_stream_t stream) {

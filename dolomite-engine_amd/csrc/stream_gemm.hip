@@ -314,27 +314,31 @@ bool mi_gemm_stream_pick(const GemmArgs& a, bool glu, int elt) {
   return a.K % 32 != 0 ? rows <= 56 * e : a.K >= 1280 && rows <= 24 * e;
 }
 
-int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int rb, int nw, hipStream_t s) {
+int mi_gemm_stream_form(const GemmArgs& a, bool glu, int elt) {
+  const double avg = (double)a.L / a.E;
+  // row blocks: most experts in one chunk, and nearly all where a second one means long reads (13 of 16 rows on average);
+  // fp32 beyond that: small chunks, whatever the load (17 experts, hidden 1000, 256 tokens, up-projection, us, 16 / 64 rows a
+  // chunk: even load 54 / 45, Zipf(1.1) 53 / 67, tiles 65)
+  const int rb = avg <= (elt == 2 && a.K >= 1280 ? 13 : 16) ? 1 : (avg <= (elt == 4 ? 48 : 28) ? 2 : (elt == 4 ? 1 : 4));
+  // waves per unit: enough of them for the chip when there are few units (1 token: 256 units, 7.0 us with four waves
+  // each, 9 with one), always four on a long contraction, two with chunks of 32 rows on a fairly long one (hidden 1536, 96
+  // tokens: 33.8 -> 28.4 us)
+  const int bm = 16 * rb, nk = mi_ceil_div(a.K, 128 / elt);
+  const long touched = a.E < a.L ? a.E : a.L;
+  const long units = touched * (long)(avg <= bm ? 1 : (avg + bm - 1) / bm) * mi_ceil_div(a.N, glu ? 16 : 32);
+  int nw = (units <= 320 || (nk >= 64 && units <= 2048)) && nk >= 4 ? 4 : (units <= 640 && nk >= 4 ? 2 : 1);
+  if (nw == 1 && rb == 2 && elt == 2 && nk >= 24) nw = 2;
+  // (chunks of 64 rows: two rings of 48 KB cost more than they bring, 17 experts, hidden 920, 128 tokens 21.8 / 12.1 us with two
+  // waves, 16.5 / 9.4 with one -- except on the very long contractions: K 14336, 128 tokens 188 / 252)
+  if (rb == 4) nw = nw > 1 && nk >= 64 ? 2 : 1;
+  return 10 * rb + nw;
+}
+
+int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int form, hipStream_t s) {
   const int elt = dtype == MI_MOE_F32 ? 4 : 2;
   if (!stream_offsets_ok(a, glu, elt)) return MI_MOE_EUNSUPPORTED;
-  const double avg = (double)a.L / a.E;
-  if (rb == 0) {
-    // row blocks: most experts in one chunk, and nearly all where a second one means long reads (13 of 16 rows on average);
-    // fp32 beyond that: small chunks, whatever the load (17 experts, hidden 1000, 256 tokens, up-projection, us, 16 / 64 rows a
-    // chunk: even load 54 / 45, Zipf(1.1) 53 / 67, tiles 65)
-    rb = avg <= (elt == 2 && a.K >= 1280 ? 13 : 16) ? 1 : (avg <= (elt == 4 ? 48 : 28) ? 2 : (elt == 4 ? 1 : 4));
-    // waves per unit: enough of them for the chip when there are few units (1 token: 256 units, 7.0 us with four waves
-    // each, 9 with one), always four on a long contraction, two with chunks of 32 rows on a fairly long one (hidden 1536, 96
-    // tokens: 33.8 -> 28.4 us)
-    const int bm = 16 * rb, nk = mi_ceil_div(a.K, 128 / elt);
-    const long touched = a.E < a.L ? a.E : a.L;
-    const long units = touched * (long)(avg <= bm ? 1 : (avg + bm - 1) / bm) * mi_ceil_div(a.N, glu ? 16 : 32);
-    nw = (units <= 320 || (nk >= 64 && units <= 2048)) && nk >= 4 ? 4 : (units <= 640 && nk >= 4 ? 2 : 1);
-    if (nw == 1 && rb == 2 && elt == 2 && nk >= 24) nw = 2;
-    // (chunks of 64 rows: two rings of 48 KB cost more than they bring, 17 experts, hidden 920, 128 tokens 21.8 / 12.1 us with two
-    // waves, 16.5 / 9.4 with one -- except on the very long contractions: K 14336, 128 tokens 188 / 252)
-    if (rb == 4) nw = nw > 1 && nk >= 64 ? 2 : 1;
-  }
+  if (form < 10) form = mi_gemm_stream_form(a, glu, elt);
+  const int rb = form / 10, nw = form % 10;
   switch (dtype) {
     case MI_MOE_F32: return launch_stream_t<float>(a, glu, rb, nw, s);
     case MI_MOE_F16: return launch_stream_t<f16_t>(a, glu, rb, nw, s);

@@ -201,22 +201,26 @@ int mi_moe_scattered_gemm(const void* in, const void* w, void* out, const int32_
  * The same product with the expert weights stored (E, K, N), i.e. out[orow(i), :] = in[irow(i), :] @ w_kn[e_i]:
  * the form of both data gradients of the backward of scattered_experts (moe.py:91-101), d_act = dy @ w_proj[e] and
  * dx = d_h @ w_fc[e], with the weights as the module keeps them (no transposed copy).  F16 / BF16, and only the
- * shapes the persistent tile kernel takes (K % 32 == 0, K >= 128, N % 8 == 0, E <= 256, 16-byte aligned
- * pointers); MI_MOE_EUNSUPPORTED otherwise (the caller can transpose and use mi_moe_scattered_gemm).
+ * shapes the persistent tile kernel takes (K % 8 == 0, N % 8 == 0, E <= 256, 16-byte aligned pointers);
+ * MI_MOE_EUNSUPPORTED otherwise (the caller can transpose and use mi_moe_scattered_gemm).
  */
 int mi_moe_scattered_gemm_wt(const void* in, const void* w_kn, void* out, const int32_t* sorted_scattered,
                              const int32_t* expert_offsets, int L, int K, int N, int E, int k, int grouped_in,
                              int grouped_out, int dtype, mi_moe_stream_t stream);
 
 /* Same call with an explicit kernel configuration (tuning / benchmarking / tests): cfg = -1 picks one
- * from the shape; 0 / 1 / 2 = register-staged 256x256 / 128x128 / 32x256 tiles (all three element types);
+ * from the shape; 0 / 1 / 2 / 5 = register-staged 256x256 / 128x128 / 32x256 / 32x128 tiles (all three element types);
  * 3 = one thread per output element (any shape); 4 = DMA-staged 128x128 (K % 32 == 0); 7 = persistent
- * DMA-staged 256x256 tiles with 32-wide K slices and the two wave groups of a SIMD alternating between
- * LDS/DMA work and matrix instructions (K % 32 == 0, K >= 128, N % 8 == 0, E <= 256; what -1 picks for
- * large expert loads); 8 / 9 = 7 with the order in which the XCDs take the tiles fixed to "each XCD a contiguous
- * eighth of the tile list" / "consecutive 32-tile blocks of one chip-wide round" (7 picks the second from 8 column
- * tiles on; same results either way); 4 and 7 .. 9 are F16 / BF16 only.  A configuration that does not take the
- * shape or type returns MI_MOE_EUNSUPPORTED. */
+ * DMA-staged 256x256 tiles, four waves of 128x128 and K slices of 64 (K % 8 == 0, N % 8 == 0, E <= 256, `out` 16-byte
+ * aligned; what -1 picks for large expert loads); 8 / 9 = 7 with the order in which the XCDs take the tiles fixed to
+ * "each XCD a contiguous eighth of the tile list" / "consecutive 32-tile blocks of one chip-wide round" (7 picks the second
+ * from 8 column tiles on; same results either way); 4 and 7 .. 9 are F16 / BF16 only.  100 + 10 r + w = the weight
+ * stream for a few rows per expert (all three element types) with chunks of 16 r rows (r = 1, 2, 4) and w waves that
+ * split the contraction (w = 1, 2, 4; r = 4: 1, 2); 100 = the stream in the form its own rule picks.  A configuration that
+ * does not take the shape or type returns MI_MOE_EUNSUPPORTED.
+ * mi_moe_grouped_gemm_choice tells which of these numbers cfg -1 is for a problem with 16-byte aligned operands (glu: the
+ * up-projection with SwiGLU, N = I), or returns the error code of a problem that none of them takes. */
+int mi_moe_grouped_gemm_choice(int L, int K, int N, int E, int glu, int dtype);
 int mi_moe_scattered_gemm_cfg(const void* in, const void* w, void* out, const int32_t* sorted_scattered,
                               const int32_t* expert_offsets, int L, int K, int N, int E, int k,
                               int grouped_in, int grouped_out, int dtype, int cfg, mi_moe_stream_t stream);
@@ -270,9 +274,9 @@ int mi_moe_up_swiglu_ws(const void* x, const void* w_fc, void* act_out, const in
  * less than mi_moe_scattered_gemm followed by mi_moe_swiglu_forward.  h is rounded to `dtype` and act_out is formed
  * from the ROUNDED halves, as mi_moe_swiglu_forward forms it from the stored h (what GLUActivation does to the
  * output of the grouped GEMM, glu.py:42-43), with this kernel's reciprocal in place of that kernel's division.
- * F16 / BF16 and the shapes and loads for which cfg -1 picks the persistent tile kernel (H % 32 == 0, H >= 128,
- * I % 8 == 0, E <= 256, on average >= 192 rows per expert); MI_MOE_EUNSUPPORTED otherwise, and the caller makes
- * the two calls.  h_out 16-byte aligned.
+ * F16 / BF16, H % 8 == 0, I % 8 == 0, E <= 256, on average >= 120 rows per expert; MI_MOE_EUNSUPPORTED otherwise, and
+ * the caller makes the two calls.  (Where the problem has so few 256 x 256 tiles that smaller ones are faster, this call
+ * makes the two launches itself; act_out is then formed with the division.)  act_out and h_out 16-byte aligned.
  */
 int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_out, void* h_out, const int32_t* sorted_scattered,
                           const int32_t* expert_offsets, int L, int H, int I, int E, int k, int dtype,
