@@ -258,10 +258,10 @@ def measure_ceilings(w, inputs, device, iters=20):
 
 
 def measure_inner_loop_probes(device, slices=6144):
-    """The pieces of an eight-wave GEMM inner loop in isolation (mi_moe_probe_kloop: one workgroup per CU, a 256 x 256
-    tile of 64 x 128 wave tiles, on 2 MiB of L2-resident random bf16 data): the matrix instructions alone, with the LDS
-    fragment reads, the L2 -> LDS DMA alone, and all of it together.  "mfma_only" is what the matrix cores sustain at
-    the clock the chip settles at; the grouped GEMM's own loop (four waves of 128 x 128) is not bound by the others."""
+    """The pieces of the persistent grouped GEMM's inner loop in isolation (mi_moe_probe_kloop: one workgroup per CU, a
+    256 x 256 tile of four 128 x 128 wave tiles, on 2 MiB of L2-resident random bf16 data): the matrix instructions alone,
+    with the LDS fragment reads, the L2 -> LDS DMA alone, and all of it together.  "mfma_only" is what the matrix cores
+    sustain at the clock the chip settles at."""
     import torch
 
     from dolomite_engine_amd import _lib
@@ -273,7 +273,7 @@ def measure_inner_loop_probes(device, slices=6144):
     cus = sink.numel() // (512 * 4)
     stream = torch.cuda.current_stream().cuda_stream
     out = {"workgroups": cus, "slices_per_workgroup": slices}
-    for mode, name in ((0, "mfma_only"), (1, "mfma_plus_lds_reads"), (2, "dma_only"), (3, "all_pingpong")):
+    for mode, name in ((0, "mfma_only"), (1, "mfma_plus_lds_reads"), (2, "dma_only"), (3, "all")):
         def launch():
             _lib.check(lib.mi_moe_probe_kloop(mode, data.data_ptr(), data.numel() * 2, slices, sink.data_ptr(),
                                               sink.numel(), stream))

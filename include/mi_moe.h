@@ -436,16 +436,16 @@ int mi_moe_layer_forward(const void* x, const void* norm_w, float norm_eps, int 
                          size_t gemm_ws_bytes, mi_moe_stream_t stream);
 
 /*
- * Diagnostics (no counterpart in the reference; nothing in the layer calls them): the pieces of an eight-wave
- * GEMM inner loop in isolation, for a benchmark that wants measured rates beside the grouped GEMM's own
- * figure (which runs four waves of 128 x 128 and is not bound by modes 1 and 3).  One workgroup of eight waves per compute unit runs `slices` K slices of a 256 x 256 bf16 tile
- * (32 matrix instructions 16x16x32, twelve 16-byte LDS fragment reads and four 1 KiB DMA
- * instructions per wave and slice, ring of four 32 KiB stages) with parts switched off:
+ * Diagnostics (no counterpart in the reference; nothing in the layer calls them): the pieces of the persistent grouped GEMM's
+ * inner loop in isolation, for a benchmark that wants measured rates beside the grouped GEMM's own figure.  One workgroup
+ * of four waves per compute unit runs `slices` K slices, 32 wide, of a 256 x 256 bf16 tile (per wave and slice 64 matrix
+ * instructions 16x16x32, sixteen 16-byte LDS fragment reads and eight 1 KiB DMA instructions, ring of five 32 KiB units) with
+ * parts switched off:
  *   mode 0  matrix instructions only        mode 1  + the LDS fragment reads
- *   mode 2  DMA only (L2 -> LDS fill)       mode 3  everything, in two alternating wave groups
+ *   mode 2  DMA only (L2 -> LDS fill)       mode 3  everything
  * Per workgroup and slice: 2 * 256 * 256 * 32 flops, 32 KiB of DMA.  data: at least 2 MiB + 4 KiB of bytes of the
  * caller's choice (random bf16 values draw more power than zeros), 16-byte aligned, read only; sink:
- * mi_moe_probe_sink_bytes() bytes that the kernels write (one float per thread, so that nothing is optimised away).
+ * mi_moe_probe_sink_bytes() bytes that the kernels write (two floats per thread, so that nothing is optimised away).
  */
 size_t mi_moe_probe_sink_bytes(void);
 int mi_moe_probe_kloop(int mode, const void* data, size_t data_bytes, int slices, void* sink, size_t sink_bytes,
