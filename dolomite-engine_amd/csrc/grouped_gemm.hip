@@ -787,12 +787,14 @@ static int launch_dma(GemmArgs a, hipStream_t s) {
 }
 
 // Cache policy of the persistent kernel's output stores.  The plain form's output -- the (slots, hidden) rows the
-// combine streams once -- is stored non-temporal, so that it does not push the operands out of the caches:
-// down-projection of the 16384-token, 32-expert shape 0.169 -> 0.146 ms (its combine 0.048 -> 0.053 ms), little
-// either way on the other shapes.  The SwiGLU form's output is the next GEMM's operand: up to about the size the
-// memory-side cache can hold next to the weights it stays cached (134 MB on that shape: non-temporal stores would
-// make the GEMM that reads it back 8 % slower); beyond that it would not survive until it is read and only evicts
-// the operands on its way (268 MB on the 32768-token, 40-expert shape: both GEMMs 1 % faster non-temporal).
+// combine streams once -- is stored non-temporal, so that it does not push the operands out of the caches.  Cached /
+// non-temporal, us, down-projection alone and up + down + combine: 32 experts, 512 -> 1024, 16384 tokens 156 / 151 and 431 / 423;
+// 40 experts, 512 -> 1536, 24576 tokens 314 / 308 and 889 / 881, 32768 tokens 404 / 395 and 1165 / 1148; 8 experts, 14336 -> 4096 the
+// same within 1 %.  The SwiGLU form's output is the next GEMM's operand: up to about the size the memory-side cache can hold
+// next to the weights it stays cached; beyond that it would not survive until it is read and only evicts the operands
+// on its way.  It matters little: up + down + combine 134 MB (32 experts, 16384 tokens) 426 / 431, 134 MB (40 experts) 603 / 605,
+// 235 MB (8 experts, I 14336) 2118 / 2135; 268 MB (16 experts, I 1024) 1358 / 1338, 268 MB (40 experts, 32768 tokens) 1154 / 1151,
+// 470 MB 4086 / 4073.
 static int persistent_out_nt(const GemmArgs& a, bool glu, int elt) {
   if (!glu) return 1;
   return (double)a.L * a.N * elt > 192.0 * 1024 * 1024;
@@ -863,7 +865,7 @@ static int launch_naive(GemmArgs a, hipStream_t s) {
 }
 
 // tile configurations
-//   0 / 1 / 2  register-staged 256x256 / 128x128 / 32x256 (any K % 8 == 0)
+//   0 / 1 / 2 / 5  register-staged 256x256 / 128x128 / 32x256 / 32x128 (any K % 8 == 0)
 //   3          one thread per output element (any shape, any dtype)
 //   4          DMA-staged 128x128, one tile per workgroup (K % 32 == 0)
 //   100 + 10 rb + nw  weight stream (stream_gemm.hip): row blocks of 16 per unit, waves that split the contraction

@@ -15,9 +15,12 @@
 //     x taking the x-th run of grid / 8 of them.  All XCDs then work on neighbouring tiles at the same time.  When
 //     an expert has more column tiles than a band is wide (intermediate size 14336: 112 column tiles, bands of 8),
 //     consecutive bands read the same activation rows, and the XCDs share them through the memory-side cache
-//     instead of each fetching them from HBM in its own time: Mixtral-shape layer 5.02 -> 4.73 ms.  With few
-//     column tiles (the band is the whole row) it changes little either way (-1.3 % on the Granite-1B shape,
-//     +1.1 % on the Granite-3B shape), so the host asks for it only from 8 column tiles on.
+//     instead of each fetching them from HBM in its own time.
+// The host asks for the second from 8 column tiles on.  Contiguous / interleaved, us: 8192 tokens, 8 experts, 14336 -> 4096 (16
+// column tiles) 1524 / 1429, 4096 -> 14336 (112) 2727 / 2691; 8192 tokens, 64 experts, 4096 -> 1408 (11) 928 / 911 and back (16)
+// 500 / 510; 16384 tokens, 16 experts, 2048 -> 1024 (8) 418 / 417 and back (8) 253 / 244; but below 8, where a band is the whole
+// row, 512 -> 1536 (6), 40 experts, 32768 tokens 395 / 420, 16384 tokens 213 / 224, 1024 -> 512 (4), 32 experts, 4096 tokens 80 / 84,
+// 1536 -> 512 (4) 335 / 340 (with an uneven load 604 / 597).
 // Either way the tiles that do not fill the last round can be cut along K (see PERSIST_SPLIT_MAX).
 
 struct SplitPlan {
