@@ -66,3 +66,24 @@ def test_stream_many_chunks(device, dtype, counts, K, N, cfg):
     act = ops.up_swiglu(by_slot, w, 1, ss, off, cfg=cfg)
     want = ref[:, :N] * torch.nn.functional.silu(ref[:, N:])
     torch.testing.assert_close(act.to(wide), want, **TOL[dtype])
+
+
+@pytest.mark.parametrize("rb,waves", [(1, 1), (1, 4), (2, 2), (4, 1)])
+def test_stream_fp32_beyond_one_chunk(device, rb, waves):
+    """fp32 beyond one chunk of rows per expert on average is another kernel (no non-temporal fetch for experts with one
+    chunk): a row more, past the line, changes no other row's result."""
+    from dolomite_engine_amd import ops
+
+    g = torch.Generator().manual_seed(rb)
+    K, N, rows, cfg = 520, 296, 32 * rb + 1, 100 + 10 * rb + waves
+    print(f"stream fp32 line cfg={cfg}", flush=True)
+    x = torch.randn(rows, K, generator=g).to(device)
+    w = (torch.randn(2, 2 * N, K, generator=g) * 0.05).to(device)
+    out = []
+    for first in (rows - 2, rows - 1):  # 16 rb rows per expert on average, and one row more in the first expert
+        xs = torch.cat((x[:first], x[-1:]))
+        off = torch.tensor([first, first + 1], dtype=torch.int32, device=device)
+        ss = torch.arange(first + 1, dtype=torch.int32, device=device)
+        out.append((ops.scattered_gemm(xs, w, 1, ss, off, True, True, cfg=cfg), ops.up_swiglu(xs, w, 1, ss, off, cfg=cfg)))
+    for at, past in zip(*out):
+        assert torch.equal(at[:rows - 2], past[:rows - 2]) and torch.equal(at[-1], past[-1])
