@@ -37,7 +37,7 @@ def _foreign(instructions):
     return out
 
 
-def test_checker_sees_foreign_writes():
+def test_foreign_writes_are_seen():
     own = ["v_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]", "v_accvgpr_read_b32 v1, a17", "v_mov_b32_e32 v1, v2"]
     planted = ["v_accvgpr_write_b32 a3, v1", "v_accvgpr_mov_b32 a1, a2", "scratch_load_dword a5, off, off",
                "ds_read_b128 a[4:7], v1 offset:16", "global_store_dwordx4 v[0:1], a[0:3], off"]
@@ -68,7 +68,7 @@ def _early_uses(instructions):
     return out
 
 
-def test_checker_sees_early_uses():
+def test_early_uses_are_seen():
     own = ["buffer_load_dwordx4 v[4:7], v1, s[0:3], s4 offen", "buffer_load_dwordx4 v8, s[0:3], s4 offen lds",
            "v_mov_b32_e32 v2, v3", "s_waitcnt vmcnt(8)", "v_mul_lo_u32 v9, v5, s3"]
     assert _early_uses(own) == []
