@@ -335,15 +335,22 @@ class MoE(nn.Module):
                 or "_route" in own or "_use_fused_router" in own or "_compute_experts" in own
                 or "_compute_shared_experts" in own or _HOOKS._global_forward_hooks or _HOOKS._global_forward_pre_hooks):
             return False
-        modules = own["_modules"]
-        return (_called_as_written(modules.get("c_proj"), ParameterizedExperts, _EXPERTS_FORWARD)
-                and _called_as_written(modules.get("dropout"), nn.Identity, _IDENTITY_FORWARD))
+        proj, dropout = self._modules_by_name("c_proj", "dropout")
+        return (_called_as_written(proj, ParameterizedExperts, _EXPERTS_FORWARD)
+                and _called_as_written(dropout, nn.Identity, _IDENTITY_FORWARD))
+
+    def _modules_by_name(self, *names: str) -> list[nn.Module | None]:
+        """The modules of these names (a subclass may have them as properties), past nn.Module's __getattr__."""
+        if type(self) is MoE:
+            modules = self.__dict__["_modules"]
+            return [modules.get(name) for name in names]
+        return [getattr(self, name) for name in names]
 
     def _forward_native(self, hidden_states: torch.Tensor, residual: torch.Tensor | None, residual_scale: float | None,
                         pre_norm: tuple | None) -> tuple[torch.Tensor | None, torch.Tensor | None]:
         """The whole eval-mode forward through ops.layer_forward, None where it does not take the call; and the router's
         logits if they had to be formed by torch before that was known, for the stage-by-stage code to go on from."""
-        fc, proj = self.c_fc, self.c_proj
+        fc, proj, gate = self._modules_by_name("c_fc", "c_proj", "gate")
         if fc.bias is not None or proj.bias is not None:
             return None, None
         shared_fc = shared_proj = None
@@ -358,7 +365,7 @@ class MoE(nn.Module):
             weights = (fc.weight, proj.weight, None, None)
         if weights[1] is None:
             return None, None
-        gate_weight = self.gate.weight
+        gate_weight = gate.weight
         logits = None
         if pre_norm is None and not ops.router_fused_supported(hidden_states, self.num_experts, self.top_k):
             logits = self._unfused_logits(hidden_states)
