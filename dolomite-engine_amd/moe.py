@@ -328,7 +328,7 @@ class MoE(nn.Module):
     def _stages_as_written(self) -> bool:
         """Whether the stage-by-stage code would run what the one-call forward stands for: no stage replaced (by a subclass,
         on the class or on the instance), no hook on, and no other forward in, a module that it calls.  (Written out, past
-        nn.Module's __getattr__: it runs on every forward, 2.6 -> 0.7 us.)"""
+        nn.Module's __getattr__: it runs on every forward, 2.6 -> 1.0 us.)"""
         cls, own = type(self), self.__dict__
         if (cls._route is not _ROUTE or cls._use_fused_router is not _USE_FUSED_ROUTER
                 or cls._compute_experts is not _COMPUTE_EXPERTS or cls._compute_shared_experts is not _COMPUTE_SHARED_EXPERTS
