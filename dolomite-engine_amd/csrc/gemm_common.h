@@ -23,6 +23,7 @@ struct GemmArgs {
   void* ws;     // persistent kernel: workspace for splitting the last round of tiles along K (or null)
   void* pre;    // persistent SwiGLU kernel: (L, 2N) pre-activation output next to the activation (or null)
   int out_nt;   // persistent kernel: store the output non-temporal (set in run_gemm)
+  uint32_t out_window;  // persistent kernel: rows of the output that 32-bit byte offsets reach (set by the launch)
   // fp8 weights (register-staged kernel, W8 form): w holds e4m3fn bytes, row-major (E, rows, K) or in the streamed-tile
   // layout of decode_fp8.hip; wscale (E, rows) fp32 is applied to the accumulators in the epilogue
   const float* wscale;

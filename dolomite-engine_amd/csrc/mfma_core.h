@@ -70,10 +70,10 @@ __device__ __forceinline__ void pg_dma_dst(uint32_t lds, int bytes) {
 __device__ __forceinline__ void pg_dma(uint32_t off, u32x4 srd, uint32_t soff) {
   asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(off), "s"(srd), "s"(soff) : "memory");
 }
+__device__ __forceinline__ uint32_t pg_srd_bytes(uint64_t bytes) { return bytes < (uint64_t)PG_OOB ? (uint32_t)bytes : PG_OOB; }
 __device__ __forceinline__ u32x4 pg_srd(const void* base, uint64_t bytes) {
   const uint64_t b = (uint64_t)base;
-  const uint32_t n = bytes < (uint64_t)PG_OOB ? (uint32_t)bytes : PG_OOB;
-  return (u32x4){(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, n, 0x00020000u};
+  return (u32x4){(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, pg_srd_bytes(bytes), 0x00020000u};
 }
 __device__ __forceinline__ constexpr int pg_wait(int vm, int lgkm) {
   // gfx9 encoding: vmcnt = {imm[15:14], imm[3:0]}, expcnt = imm[6:4] (7 = no wait), lgkmcnt = imm[11:8]

@@ -59,13 +59,14 @@ static bool persistent_may_split(int K) {
 }
 
 
-template <typename T, bool GLU, bool WT, bool KEEP>
-__global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArgs a) {
+// NT: results are stored non-temporal
+template <typename T, bool GLU, bool WT, bool KEEP, bool NT>
+__device__ __forceinline__ void persistent_body(const GemmArgs& a) {
   static_assert(!KEEP || GLU, "the pre-activation belongs to the SwiGLU form");
   static_assert(!WT || !GLU, "transposed-weight form");
   constexpr int BM = 256;
   constexpr int BN = GLU ? 128 : 256;               // output columns per tile
-  constexpr int NSTORE = KEEP ? 48 : (GLU ? 16 : 32);  // stores of a wave in the epilogue of an interior tile
+  constexpr int NSTORE = KEEP ? 48 : (GLU ? 16 : 32);  // stores of a wave in the epilogue
   typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
   typedef short tr_s16x4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) tr_s16x4* tr_ptr_t;
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
     asm volatile("" : "+v"(rx));
     if constexpr (!WT) asm volatile("" : "+v"(rw));
   };
-  // stores_after_dma: the epilogue of an interior tile lies between the DMA this slice waits for and now
+  // stores_after_dma: the epilogue of a tile lies between the DMA this slice waits for and now
   auto step = [&](auto ftag, bool stores_after_dma) {
     if (kw >= kw_ev) w_event();
     half(std::integral_constant<int, 0>{}, ftag, dma0 + p4, [&](int m) {
@@ -341,15 +342,35 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
   };
   // WHAT: 0 the kernel's result (SwiGLU: up * silu(gate)); 1 / 2 (KEEP): the up / the gate half of h, into a.pre.  KEEP
   // forms the result from the ROUNDED halves, as the separate activation kernel forms it from the stored h.
-  auto epilogue_as = [&](auto what_tag, auto interior_tag, auto nt_tag, const PgTile& t) {
+  // Every tile issues the same number of stores on one path; what does not exist is a lane past the buffer.  With a branch for
+  // edge tiles the compiler, which counts stores along the shortest way it can construct, waited for all of them wherever it
+  // needed the next tile's rows, and again in the next tile's first slice: 40 experts, 512 -> 1536, 32768 tokens 401 -> 390 us,
+  // 32 experts, 512 -> 1024, 16384 tokens 142 -> 139, 1536 -> 512 SwiGLU, 32768 tokens 613 -> 608.
+  // WHAT 0 writes the rows [row0, row0 + out_window) of the output: all of them, unless it has more than 4 GiB.
+  auto epilogue_as = [&](auto what_tag, const PgTile& t, uint32_t row0) __attribute__((always_inline)) {
     constexpr int WHAT = decltype(what_tag)::value;
-    constexpr bool INTERIOR = decltype(interior_tag)::value, NT = decltype(nt_tag)::value;
     typedef __attribute__((address_space(3))) u32x2* wp_t;
     typedef __attribute__((address_space(3))) const u32x4* rp_t;
-    unsigned char* dst = reinterpret_cast<unsigned char*>(WHAT == 0 ? out : static_cast<T*>(a.pre));
     const uint32_t ld = (WHAT == 0 ? a.N : 2 * a.N) * 2u;
+    // (rows of the pre-activation are the sorted order's: addressed from the tile's first, as the whole can exceed 4 GiB)
+    const int r0 = wm * 128 + lane, rows = t.row_end - t.row_begin;
+    const uint32_t window = WHAT == 0 ? a.out_window : (uint32_t)rows, left = WHAT == 0 ? a.L - row0 : (uint32_t)rows;
+    unsigned char* dst = WHAT == 0 ? reinterpret_cast<unsigned char*>(out) + (uint64_t)row0 * ld
+                                   : static_cast<unsigned char*>(a.pre) + (uint64_t)t.row_begin * ld;
+    const auto srd = __builtin_amdgcn_make_buffer_rsrc(dst, (short)0, (int)((left < window ? left : window) * ld), 0x00020000);
     const uint32_t s0 = dma0 + p4;
     const int col0 = t.nt * BN + wn * (GLU ? 64 : 128);
+    // byte offsets of the wave's rows lane and 64 + lane, and of the lane's columns in store it (% CP); saturating sums keep what
+    // does not exist past the buffer
+    constexpr int CP = GLU ? 2 : 4;
+    const uint32_t lo = WHAT == 0 ? (uint32_t)orow_lo - row0 : r0, hi = WHAT == 0 ? (uint32_t)orow_hi - row0 : r0 + 64;
+    const uint32_t rlo = r0 < rows && lo < window ? lo * ld : PG_OOB, rhi = r0 + 64 < rows && hi < window ? hi * ld : PG_OOB;
+    uint32_t coff[CP];
+#pragma unroll
+    for (int c = 0; c < CP; ++c) {
+      const int col = col0 + (scc0 ^ (4 * c)) * 8;
+      coff[c] = col < a.N ? (uint32_t)((WHAT == 2 ? a.N : 0) + col) * 2u : PG_OOB;
+    }
 #pragma unroll
     for (int p = 0; p < NPASS; ++p) {
 #pragma unroll
@@ -383,49 +404,30 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
 #pragma unroll
       for (int it0 = 0; it0 < 8; it0 += 4) {
         u32x4 val[4];
-        int orow[4];
+        uint32_t roff[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int r = p * PASS_ROWS + (it0 + j) * RPP;  // + srow: row of the wave's 128
           val[j] = *(rp_t)(size_t)(s0 + (it0 + j) * 4096 + lane * 16);
-          orow[j] = __builtin_amdgcn_ds_bpermute(((r & 63) + srow) * 4, r < 64 ? orow_lo : orow_hi);
+          roff[j] = (uint32_t)__builtin_amdgcn_ds_bpermute(((r & 63) + srow) * 4, (int)(r < 64 ? rlo : rhi));
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int it = it0 + j;
-          const int row = t.row_begin + wm * 128 + p * PASS_ROWS + it * RPP + srow;
-          const int col = col0 + (scc0 ^ (GLU ? 4 * (it & 1) : 4 * (it & 3))) * 8;
-          if (INTERIOR || (row < t.row_end && col < a.N)) {
-            u32x4* q = reinterpret_cast<u32x4*>(dst + (uint64_t)(uint32_t)orow[j] * ld + (uint32_t)((WHAT == 2 ? a.N : 0) + col) * 2u);
-            if constexpr (NT) __builtin_nontemporal_store(val[j], q);
-            else *q = val[j];
-          }
-        }
+        for (int j = 0; j < 4; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(val[j], srd, (int)__builtin_elementwise_add_sat(roff[j], coff[(it0 + j) % CP]), 0, NT ? 2 : 0);
       }
       pg_own_agprs();
     }
   };
-  typedef std::integral_constant<int, 0> what_result;
-  typedef std::integral_constant<int, 1> what_up;
-  typedef std::integral_constant<int, 2> what_gate;
-  auto epilogue = [&](const PgTile& t, bool interior) {
+  auto epilogue = [&](const PgTile& t) __attribute__((always_inline)) {
+    uint32_t row0 = 0;
+    do {
+      epilogue_as(std::integral_constant<int, 0>{}, t, row0);
+      row0 += a.out_window;
+    } while (row0 < (uint32_t)a.L);
     if constexpr (KEEP) {
-      // the activation and both halves of the pre-activation (plain stores: the backward reads them again)
-      if (interior) {
-        epilogue_as(what_result{}, std::true_type{}, std::false_type{}, t);
-        epilogue_as(what_up{}, std::true_type{}, std::false_type{}, t);
-        epilogue_as(what_gate{}, std::true_type{}, std::false_type{}, t);
-      } else {
-        epilogue_as(what_result{}, std::false_type{}, std::false_type{}, t);
-        epilogue_as(what_up{}, std::false_type{}, std::false_type{}, t);
-        epilogue_as(what_gate{}, std::false_type{}, std::false_type{}, t);
-      }
-    } else if (interior) {
-      if (a.out_nt) epilogue_as(what_result{}, std::true_type{}, std::true_type{}, t);
-      else epilogue_as(what_result{}, std::true_type{}, std::false_type{}, t);
-    } else {
-      if (a.out_nt) epilogue_as(what_result{}, std::false_type{}, std::true_type{}, t);
-      else epilogue_as(what_result{}, std::false_type{}, std::false_type{}, t);
+      // both halves of the pre-activation next to the activation
+      epilogue_as(std::integral_constant<int, 1>{}, t, 0);
+      epilogue_as(std::integral_constant<int, 2>{}, t, 0);
     }
   };
   // a part of a split tile: accumulators -> workspace, block b of thread t at [b][t]
@@ -434,7 +436,10 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
                   ((size_t)sp.ws_base + (size_t)my_rem_tile * sp.parts + my_part) * (64 * 256) + threadIdx.x;
 #pragma unroll
     for (int b = 0; b < 64; ++b) {
-      if (b % 8 == 0) pg_own_agprs();
+      if (b % 8 == 0) {
+        pg_own_agprs();
+        asm volatile("" : "+v"(base));              // (or the 64 addresses are kept in registers from the first tile on)
+      }
       const f32x4 v = {pg_acc(4 * b), pg_acc(4 * b + 1), pg_acc(4 * b + 2), pg_acc(4 * b + 3)};
       base[b * 256] = v;
     }
@@ -506,10 +511,13 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
     int raw[8], lo_n, hi_n;
     load_rows(after, raw);
     load_out_rows(nxt, lo_n, hi_n);
-    const bool interior = cur.row_begin + BM <= cur.row_end && (cur.nt + 1) * BN <= a.N;
-    epilogue(cur, interior);
+    epilogue(cur);
+    // (the waits for the loads above belong here: they count the epilogue's stores, which stay in flight)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(raw[j]));
+    asm volatile("" : "+v"(lo_n), "+v"(hi_n));
     if (i + 1 >= n_items) break;
-    stores_pending = interior;
+    stores_pending = true;
     make_xoff(after, raw, xoff_n);
     wsrd_n = make_wsrd(after);
     orow_lo = lo_n;
@@ -520,10 +528,22 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
     cur = nxt;
     nxt = after;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(xoff_n[j]));  // (the waits for the loads above belong here)
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(xoff_n[j]));
     asm volatile("" : "+v"(orow_lo), "+v"(orow_hi));
   }
   __builtin_amdgcn_s_waitcnt(pg_wait(0, 0));  // surplus DMA must not outlive the workgroup's LDS
+}
+
+template <typename T, bool GLU, bool WT, bool KEEP>
+__global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArgs a) {
+  if constexpr (!GLU) {
+    persistent_body<T, GLU, WT, KEEP, true>(a);
+  } else if constexpr (KEEP) {
+    persistent_body<T, GLU, WT, KEEP, false>(a);    // (the backward reads both again)
+  } else {
+    if (a.out_nt) persistent_body<T, GLU, WT, KEEP, true>(a);
+    else persistent_body<T, GLU, WT, KEEP, false>(a);
+  }
 }
 
 // The tiles the persistent kernel cut along K (see PERSIST_SPLIT_MAX): one workgroup per (XCD, tile of its last round)
@@ -596,6 +616,7 @@ static int launch_persistent(GemmArgs a, hipStream_t s) {
   int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), PG_LDS, lds_ok);
   if (rc != MI_MOE_OK) return rc;
   a.n_tiles = mi_ceil_div(a.N, BN);
+  a.out_window = PG_OOB / ((uint32_t)a.N * 2u);
   a.kshift = -1;
   if (a.kdiv > 0 && (a.kdiv & (a.kdiv - 1)) == 0)
     for (a.kshift = 0; (1 << a.kshift) < a.kdiv;) ++a.kshift;

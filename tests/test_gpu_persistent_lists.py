@@ -1,0 +1,63 @@
+"""Persistent grouped GEMM: the search for a tile's expert at the ends of its blocks of 64 experts, and outputs beyond what one
+32-bit byte offset reaches.  Bounds as in test_gpu_persistent.py: the one rounding of the result plus the order of the fp32 sum."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = dict(rtol=2.0 ** -8, atol=2e-3)
+
+
+@pytest.mark.parametrize("E", [1, 2, 63, 64, 65, 127, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("empty", ["none", "ends", "block", "most"])
+def test_expert_of_a_tile(device, E, empty):
+    from dolomite_engine_amd import ops
+
+    g = torch.Generator().manual_seed(E)
+    counts = torch.randint(1, 600, (E,), generator=g)
+    if empty == "ends":
+        counts[: E // 3] = 0
+        counts[E - E // 4:] = 0
+    elif empty == "block":
+        counts[63:65] = 0
+        counts[127:193] = 0
+    elif empty == "most":
+        counts[torch.rand(E, generator=g) < 0.9] = 0
+        counts[E // 2] = 257
+    L, K, N = int(counts.sum()), 64, 264
+    print(f"persistent experts E={E} {empty} L={L}", flush=True)
+    off = counts.cumsum(0).int().to(device)
+    ss = torch.randperm(L, generator=g).int().to(device)
+    x = torch.randn(L, K, generator=g).bfloat16().to(device)
+    w = (torch.randn(E, N, K, generator=g) * 0.05).bfloat16().to(device)
+    ref = torch.cat([p.float() @ w[e].float().t() for e, p in enumerate(x.split(counts.tolist()))])
+    torch.testing.assert_close(ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=7).float(), ref, **TOL)
+
+
+def test_output_beyond_4_gib(device):
+    from dolomite_engine_amd import ops
+
+    counts, K, N = [170001, 0, 100010], 64, 8192
+    L = sum(counts)  # 4.4 GB of results; as a pre-activation next to half of that
+    print(f"persistent output of {L} x {N}", flush=True)
+    g = torch.Generator(device).manual_seed(3)
+    off = torch.tensor(counts).cumsum(0).int().to(device)
+    ss = torch.randperm(L, generator=g, device=device).int()
+    x = torch.empty(L, K, device=device, dtype=torch.bfloat16).normal_(generator=g)
+    w = torch.empty(3, N, K, device=device, dtype=torch.bfloat16).normal_(0.0, 0.05, generator=g)
+    scattered = ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=7)
+    by_slot = torch.empty_like(x)
+    by_slot[ss.long()] = x
+    act, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off)
+    expert = torch.repeat_interleave(torch.arange(3, device=device), torch.tensor(counts, device=device))
+    for rows in torch.arange(L, device=device).split(10000):
+        ref = torch.empty(len(rows), N, device=device)
+        for e in range(3):
+            mine = expert[rows] == e
+            ref[mine] = x[rows][mine].float() @ w[e].float().t()
+        torch.testing.assert_close(scattered[ss[rows].long()].float(), ref, **TOL)
+        torch.testing.assert_close(h[rows].float(), ref, **TOL)
+        want = ref[:, :N // 2] * torch.nn.functional.silu(ref[:, N // 2:])
+        # (formed from the rounded halves)
+        torch.testing.assert_close(act[rows].float(), want, rtol=2.0 ** -6, atol=8e-3)
