@@ -43,6 +43,13 @@ bool mi_gemm_persistent_ok(const GemmArgs& a);
 bool mi_gemm_persistent_splits(int K);
 int mi_gemm_persistent(const GemmArgs& a, int dtype, int form, hipStream_t s);
 
+// ---- persistent_even.hip: the same with an expert's row tiles equally high, and other tiles (rows x columns) -----------------
+enum { EVEN_NONE = 0, EVEN_256x128 = 14, EVEN_160x256 = 15, EVEN_224x192 = 16, EVEN_256x256 = 18 };
+// the form that is faster than 256 x 256 tiles for this problem, or EVEN_NONE
+int mi_gemm_even_pick(const GemmArgs& a, int form);
+int mi_gemm_even(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s);
+int mi_gemm_even_train(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s);
+
 // ---- persistent_fp8.hip: fp8 weights (wscale, w_tiled); K % 16 == 0, K > 256, N % 8 == 0, at most PERSIST_MAX_E experts,
 // 16-byte aligned output ----------------------------------------------------------------------------------------------
 enum { FP8_BY_SHAPE = 1, FP8_PERSISTENT = 3, FP8_STAGED = 4 };  // forms of mi_gemm_fp8_tiled

@@ -883,6 +883,11 @@ static int dispatch_cfg(GemmArgs a, int cfg, hipStream_t s) {
     case 9:  // ... or take consecutive blocks of one chip-wide round
       a.remap |= PERSIST_REMAP_FIXED | (cfg == 9 ? PERSIST_REMAP_INTERLEAVE : 0);
       return mi_gemm_persistent(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, s);
+    case EVEN_256x128:  // the persistent kernel's even forms
+    case EVEN_160x256:
+    case EVEN_224x192:
+    case EVEN_256x256:
+      return mi_gemm_even(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, cfg, s);
     default: return MI_MOE_EUNSUPPORTED;
   }
 }

@@ -121,7 +121,8 @@ template <int BM> __device__ __forceinline__ void pg_table(const int32_t* __rest
 // The expert of a lane's row tile by binary search over the table's lanes: six exchanges, where the walk over the experts
 // that this replaces took 2.2 us of a launch with 40 of them (both projections of 40 experts, 1536 / 512, 2048 tokens 112 ->
 // 109 us; fp8 tiles, 64 experts, 4096 / 1408, 1024 tokens, layer 317 -> 312 us).
-template <int BM> __device__ __forceinline__ PgTile pg_locate(const PgTable& tb, int E, int n_tiles, int tile) {
+// EVEN: an expert's row tiles are equally high up to the last, in steps of 32 rows, and a tile ends with its own rows.
+template <int BM, bool EVEN = false> __device__ __forceinline__ PgTile pg_locate(const PgTable& tb, int E, int n_tiles, int tile) {
   asm volatile("" : "+s"(n_tiles));  // (or the divisions' reciprocals stay in registers from tile to tile)
   const int q = tile / n_tiles;  // experts own contiguous tile ranges: (row tiles before) * n_tiles
   // the 64 experts that hold it, and what lies before them
@@ -163,7 +164,15 @@ template <int BM> __device__ __forceinline__ PgTile pg_locate(const PgTable& tb,
   PgTile t;
   t.expert = chunk * 64 + l;
   t.nt = band * tile_band + rem - mt * width;
-  t.row_begin = prev + mt * BM;
-  t.row_end = rend;
+  if (EVEN) {
+    const int n = incl - first, h = (rend - prev + 32 * n - 1) / (32 * n) * 32;
+    t.row_begin = prev + mt * h;
+    t.row_end = t.row_begin + h < rend ? t.row_begin + h : rend;
+  } else {
+    t.row_begin = prev + mt * BM;
+    t.row_end = rend;
+  }
   return t;
 }
+// pairs of 16-row blocks of a tile
+__device__ __forceinline__ int pg_row_pairs(const PgTile& t) { return (t.row_end - t.row_begin + 31) >> 5; }

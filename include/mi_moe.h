@@ -214,13 +214,18 @@ int mi_moe_scattered_gemm_wt(const void* in, const void* w_kn, void* out, const 
  * DMA-staged 256x256 tiles, four waves of 128x128 and K slices of 64 (K % 8 == 0, N % 8 == 0, E <= 256, `out` 16-byte
  * aligned; what -1 picks for large expert loads); 8 / 9 = 7 with the order in which the XCDs take the tiles fixed to
  * "each XCD a contiguous eighth of the tile list" / "consecutive 32-tile blocks of one chip-wide round" (7 picks the second
- * from 8 column tiles on; same results either way); 4 and 7 .. 9 are F16 / BF16 only.  100 + 10 r + w = the weight
+ * from 8 column tiles on; same results either way); 14 / 15 / 16 / 18 = the same kernel with an expert's row tiles equally
+ * high and tiles of 256x128 / 160x256 / 224x192 / 256x256 (7 picks among these and its own by the rows per expert; the same
+ * results); 4, 7 .. 9 and 14 .. 18 are F16 / BF16 only.  100 + 10 r + w = the weight
  * stream for a few rows per expert (all three element types) with chunks of 16 r rows (r = 1, 2, 4) and w waves that
  * split the contraction (w = 1, 2, 4; r = 4: 1, 2); 100 = the stream in the form its own rule picks.  A configuration that
  * does not take the shape or type returns MI_MOE_EUNSUPPORTED.
  * mi_moe_grouped_gemm_choice tells which of these numbers cfg -1 is for a problem with 16-byte aligned operands (glu: the
  * up-projection with SwiGLU, N = I), or returns the error code of a problem that none of them takes. */
 int mi_moe_grouped_gemm_choice(int L, int K, int N, int E, int glu, int dtype);
+/* Which tiles configuration 7 takes on the current device for a problem without a workspace: 14, 15, 16 or 18 as above, 0 for
+ * its own 256x256.  form: 0 plain, 1 SwiGLU, 2 SwiGLU with the pre-activation, 3 transposed weights. */
+int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form);
 int mi_moe_scattered_gemm_cfg(const void* in, const void* w, void* out, const int32_t* sorted_scattered,
                               const int32_t* expert_offsets, int L, int K, int N, int E, int k,
                               int grouped_in, int grouped_out, int dtype, int cfg, mi_moe_stream_t stream);
