@@ -28,8 +28,8 @@
 static double tile_cost(const GemmArgs& a, int form, int nb, int bm, bool even, int cus) {
   const bool glu = form == PG_SWIGLU || form == PG_SWIGLU_KEEP;
   const double avg = (double)a.L / a.E, sd = a.E > 1 ? std::sqrt(avg) : 0.0;
-  double row_tiles = 0.0;
-  for (int i = -1; i <= 1; ++i) row_tiles += std::fmax(1.0, std::ceil((avg + i * sd) / bm)) / 3.0;
+  double row_tiles = sd > 0.0 ? 1.0 : std::ceil(avg / bm);  // (with as many experts beyond each multiple of bm as a normal load has)
+  for (int j = 1; sd > 0.0 && j * bm < avg + 4.0 * sd; ++j) row_tiles += 0.5 * std::erfc((j * bm - avg) / (sd * 1.41421356));
   const int cols = mi_ceil_div(a.N, (glu ? 16 : 32) * nb);
   const double all = a.E * row_tiles * cols / cus;
   double rounds = std::ceil(all);
