@@ -6,6 +6,12 @@
 // 60 - 68 us a pass whatever the kernels did.
 #include "gemm_common.h"
 
+// router_fused.hip
+bool mi_rmsnorm_router_sorts(int T, int H, int E);
+int mi_rmsnorm_router(const void* h, const void* ln_weight, float eps, const void* gate_w, const float* bias, int T, int H, int E,
+                      int k, int dtype, void* x_norm_out, void* logits_out, void* gates_out, int32_t* idx_out,
+                      int32_t* sorted_expert, int32_t* sorted_scattered, int32_t* expert_offsets, mi_moe_stream_t stream);
+
 namespace {
 
 struct LayerSpace {
@@ -76,8 +82,9 @@ extern "C" int mi_moe_layer_forward(const void* x, const void* norm_w, float nor
   if (has_norm) {
     if (logits) return MI_MOE_EUNSUPPORTED;
     void* xn = b + w.x_norm;
-    if ((rc = mi_moe_rmsnorm_router_fused(x, norm_w, norm_eps, gate_w, gate_bias, T, H, E, k, dtype, xn, nullptr, gates, experts,
-                                          stream)) != MI_MOE_OK)
+    sorted = mi_rmsnorm_router_sorts(T, H, E);
+    if ((rc = mi_rmsnorm_router(x, norm_w, norm_eps, gate_w, gate_bias, T, H, E, k, dtype, xn, nullptr, gates, experts,
+                                sorted ? se : nullptr, ss, off, stream)) != MI_MOE_OK)
       return rc;
     x = xn;
   } else if (logits) {

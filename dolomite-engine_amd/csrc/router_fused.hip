@@ -388,6 +388,155 @@ __global__ __launch_bounds__(ROUTER_LDS_WAVES * 64) void router_fused_lds_kernel
   }
 }
 
+// At most one group of 16 tokens per CU and a hidden size of up to 2048: a workgroup of eight waves has one group, wave p the K
+// steps p, p + 8, ..., and requests everything it will read -- its steps of the rows, of the gate weights (straight into the
+// matrix operands' registers: nobody else in the workgroup wants them) and of gamma -- at once.  One trip to memory, where the
+// kernel above makes three (rows, weights to LDS, with the norm the rows again); the parts are added in the same order, so the
+// results are the same bits.  SORT (one workgroup, at most 16 tokens): the one-block sort of the experts behind it.
+#define ROUTER_DIRECT_STEPS 4
+#define ROUTER_DIRECT_H (ROUTER_DIRECT_STEPS * ROUTER_LDS_WAVES * 64)
+#define ROUTER_SORT_TOKENS 16
+struct RouterSort {
+  int32_t *sorted_expert, *sorted_scattered, *expert_offsets;
+  int nbits;
+};
+template <typename T, bool NORM, bool SORT>
+__global__ __launch_bounds__(ROUTER_LDS_WAVES * 64) void router_fused_direct_kernel(
+    const T* __restrict__ x, const T* __restrict__ gw, const float* __restrict__ bias, int Trows, int H, int E, int k,
+    T* __restrict__ logits_out, T* __restrict__ gates, int32_t* __restrict__ idx, RouterNorm norm,
+    int32_t* __restrict__ chunk_hist, int nchunks, RouterSort sort) {
+  typedef typename RMfma<T>::vec frag_t;
+  constexpr int S = ROUTER_DIRECT_STEPS, W = ROUTER_LDS_WAVES;
+  __shared__ f32x4 red[(W - 1) * 4 * 64];
+  __shared__ float ssred[W * 16];
+  __shared__ int whist[64];
+  const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const int r = lane & 15, q = lane >> 4;
+  const int nsteps = (H + 63) >> 6, neb = (E + 15) >> 4;
+  const int t = blockIdx.x * 16 + r;
+  const T* xrow = x + (size_t)(t < Trows ? t : Trows - 1) * H;
+  if (threadIdx.x < 64) whist[threadIdx.x] = 0;
+
+  // the MFMA runs on all lanes: steps and k that do not exist contribute zeros
+  u32x4 xr[S][2], wr[S][4][2], gr[S][2];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int kpos = (s * W + part) * 64 + q * 16;
+    xr[s][0] = xr[s][1] = (u32x4){0u, 0u, 0u, 0u};
+    if (s * W + part < nsteps && kpos < H) {
+      xr[s][0] = *reinterpret_cast<const u32x4*>(xrow + kpos);
+      xr[s][1] = *reinterpret_cast<const u32x4*>(xrow + kpos + 8);
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int kpos = (s * W + part) * 64 + q * 16;
+    const bool valid = s * W + part < nsteps && kpos < H;
+#pragma unroll
+    for (int eb = 0; eb < 4; ++eb) {
+      wr[s][eb][0] = wr[s][eb][1] = (u32x4){0u, 0u, 0u, 0u};
+      if (eb < neb && valid) {
+        const int e = eb * 16 + r;
+        const T* wrow = gw + (size_t)(e < E ? e : E - 1) * H + kpos;
+        wr[s][eb][0] = *reinterpret_cast<const u32x4*>(wrow);
+        wr[s][eb][1] = *reinterpret_cast<const u32x4*>(wrow + 8);
+      }
+    }
+  }
+  float rstd = 1.0f;
+  if constexpr (NORM) {
+    const T* gamma = static_cast<const T*>(norm.gamma);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int kpos = (s * W + part) * 64 + q * 16;
+      const uint32_t one = pack2<T>(1.0f, 1.0f);
+      gr[s][0] = gr[s][1] = (u32x4){one, one, one, one};
+      if (gamma != nullptr && s * W + part < nsteps && kpos < H) {
+        if ((reinterpret_cast<uintptr_t>(gamma) & 15) == 0) {
+          gr[s][0] = *reinterpret_cast<const u32x4*>(gamma + kpos);
+          gr[s][1] = *reinterpret_cast<const u32x4*>(gamma + kpos + 8);
+          continue;
+        }
+        // (only its elements' alignment is asked of gamma)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          gr[s][0][i] = pack2<T>(Elt<T>::load(gamma + kpos + 2 * i), Elt<T>::load(gamma + kpos + 2 * i + 1));
+          gr[s][1][i] = pack2<T>(Elt<T>::load(gamma + kpos + 8 + 2 * i), Elt<T>::load(gamma + kpos + 9 + 2 * i));
+        }
+      }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a0 = unpack_lo<T>(xr[s][0][i]), a1 = unpack_hi<T>(xr[s][0][i]);
+        const float b0 = unpack_lo<T>(xr[s][1][i]), b1 = unpack_hi<T>(xr[s][1][i]);
+        ss = fmaf(a0, a0, ss); ss = fmaf(a1, a1, ss); ss = fmaf(b0, b0, ss); ss = fmaf(b1, b1, ss);
+      }
+    }
+    ss += __shfl_xor(ss, 16, MI_WAVE);
+    ss += __shfl_xor(ss, 32, MI_WAVE);
+    if (q == 0) ssred[part * 16 + r] = ss;
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int p = 0; p < W; ++p) ss += ssred[p * 16 + r];
+    rstd = 1.0f / sqrtf(ss / (float)H + norm.eps);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int kpos = (s * W + part) * 64 + q * 16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t x0 = xr[s][0][i], x1 = xr[s][1][i], g0 = gr[s][0][i], g1 = gr[s][1][i];
+        xr[s][0][i] = pack2<T>(unpack_lo<T>(x0) * rstd * unpack_lo<T>(g0), unpack_hi<T>(x0) * rstd * unpack_hi<T>(g0));
+        xr[s][1][i] = pack2<T>(unpack_lo<T>(x1) * rstd * unpack_lo<T>(g1), unpack_hi<T>(x1) * rstd * unpack_hi<T>(g1));
+      }
+      if (t < Trows && s * W + part < nsteps && kpos < H) {
+        T* xn = static_cast<T*>(norm.xnorm_out) + (size_t)t * H + kpos;
+        *reinterpret_cast<u32x4*>(xn) = xr[s][0];
+        *reinterpret_cast<u32x4*>(xn + 8) = xr[s][1];
+      } else if (s * W + part >= nsteps || kpos >= H) {  // (0 x inf of a row that is not finite)
+        xr[s][0] = xr[s][1] = (u32x4){0u, 0u, 0u, 0u};
+      }
+    }
+  }
+  f32x4 acc[4];
+#pragma unroll
+  for (int eb = 0; eb < 4; ++eb) acc[eb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s * W + part < nsteps) {
+#pragma unroll
+      for (int eb = 0; eb < 4; ++eb)
+        if (eb < neb) {
+          acc[eb] = RMfma<T>::run(__builtin_bit_cast(frag_t, wr[s][eb][0]), __builtin_bit_cast(frag_t, xr[s][0]), acc[eb]);
+          acc[eb] = RMfma<T>::run(__builtin_bit_cast(frag_t, wr[s][eb][1]), __builtin_bit_cast(frag_t, xr[s][1]), acc[eb]);
+        }
+    }
+  if (part != 0) {
+#pragma unroll
+    for (int eb = 0; eb < 4; ++eb) red[((part - 1) * 4 + eb) * 64 + lane] = acc[eb];
+  }
+  __syncthreads();
+  if (part == 0) {
+#pragma unroll
+    for (int p = 0; p < W - 1; ++p) {
+#pragma unroll
+      for (int eb = 0; eb < 4; ++eb) acc[eb] += red[(p * 4 + eb) * 64 + lane];
+    }
+    router_epilogue<T>(acc, t, t < Trows, q, bias, E, k, logits_out, gates, idx, chunk_hist != nullptr ? whist : nullptr);
+  }
+  if constexpr (SORT) {
+    __syncthreads();
+    sort_single_block<W>(idx, Trows * k, E, sort.nbits, sort.sorted_expert, sort.sorted_scattered, sort.expert_offsets,
+                         reinterpret_cast<int*>(red));
+  } else if (chunk_hist != nullptr) {
+    __syncthreads();
+    if (threadIdx.x < E && blockIdx.x < nchunks) chunk_hist[(size_t)threadIdx.x * nchunks + blockIdx.x] = whist[threadIdx.x];
+  }
+}
+
 // Many tokens, gate weights too large for LDS.  A workgroup of eight waves owns ROUTER_KS_TG groups of 16 tokens;
 // wave w takes the 64-wide K steps w, w + 8, ... of all of them (two steps' loads in flight at a time), so a wave
 // walks an eighth of the row, and a step's gate-weight fragments serve every group.  The partial logits meet in
@@ -762,6 +911,12 @@ static int launch_router_lds(const void* x, const void* gw, const float* bias, i
   int blocks = 0, waves = 0;
   int rc = router_lds_shape(T_, &blocks, &waves);
   if (rc != MI_MOE_OK) return rc;
+  if (waves == 1 && H <= ROUTER_DIRECT_H) {
+    hipLaunchKernelGGL((router_fused_direct_kernel<T, NORM, false>), dim3(blocks), dim3(ROUTER_LDS_WAVES * 64), 0, s,
+                       static_cast<const T*>(x), static_cast<const T*>(gw), bias, T_, H, E, k, static_cast<T*>(logits_out),
+                       static_cast<T*>(gates), idx, norm, chunk_hist, nchunks, RouterSort{});
+    return mi_launch_status();
+  }
   // few groups per workgroup (at most four waves would walk one): the idle waves take shares of the K steps
   // (router_fused_lds_kernel, KS); 3 groups leave two waves without a share
   const int ksplit = waves <= 4 ? (waves == 1 ? 8 : (waves == 2 ? 4 : 2)) : 1;
@@ -789,9 +944,26 @@ static int launch_router_lds(const void* x, const void* gw, const float* bias, i
   return mi_launch_status();
 }
 
+// at most 16 tokens: router (with the norm) and sort in one workgroup
+static bool router_one_group(int T_, int H, int E) { return T_ <= ROUTER_SORT_TOKENS && H <= ROUTER_DIRECT_H && router_lds_fits(H, E); }
+template <typename T, bool NORM>
+static int launch_router_one_group(const void* x, const void* gw, const float* bias, int T_, int H, int E, int k, void* logits_out,
+                                   void* gates, int32_t* idx, RouterNorm norm, int32_t* sorted_expert, int32_t* sorted_scattered,
+                                   int32_t* expert_offsets, hipStream_t s) {
+  RouterSort sort = {sorted_expert, sorted_scattered, expert_offsets, 0};
+  while ((1 << sort.nbits) < E) ++sort.nbits;
+  auto kern = sorted_expert != nullptr ? router_fused_direct_kernel<T, NORM, true> : router_fused_direct_kernel<T, NORM, false>;
+  hipLaunchKernelGGL(kern, dim3(1), dim3(ROUTER_LDS_WAVES * 64), 0, s, static_cast<const T*>(x), static_cast<const T*>(gw), bias,
+                     T_, H, E, k, static_cast<T*>(logits_out), static_cast<T*>(gates), idx, norm, static_cast<int32_t*>(nullptr), 0,
+                     sort);
+  return mi_launch_status();
+}
+
 template <typename T>
 static int launch_router(const void* x, const void* gw, const float* bias, int T_, int H, int E, int k,
                          void* logits_out, void* gates, int32_t* idx, hipStream_t s) {
+  if (router_one_group(T_, H, E))
+    return launch_router_one_group<T, false>(x, gw, bias, T_, H, E, k, logits_out, gates, idx, RouterNorm{}, nullptr, nullptr, nullptr, s);
   if (router_few_tokens(T_, H, E)) {  // split K across the waves of a workgroup instead
     hipLaunchKernelGGL((router_fused_small_kernel<T>), dim3(mi_ceil_div(T_, 16)), dim3(1024), 0, s,
                        static_cast<const T*>(x), static_cast<const T*>(gw), bias, T_, H, E, k,
@@ -822,6 +994,9 @@ template <typename T>
 static int launch_router_splitk_sort(const void* x, const void* gw, const float* bias, int T_, int H, int E, int k,
                                      void* logits_out, void* gates, int32_t* idx, int32_t* sorted_expert,
                                      int32_t* sorted_scattered, int32_t* expert_offsets, void* ws, hipStream_t s) {
+  if (router_one_group(T_, H, E))
+    return launch_router_one_group<T, false>(x, gw, bias, T_, H, E, k, logits_out, gates, idx, RouterNorm{}, sorted_expert,
+                                             sorted_scattered, expert_offsets, s);
   const int splits = router_splits(T_, H);
   const int steps_per_split = mi_ceil_div(mi_ceil_div(H, 64), splits);
   const int groups = mi_ceil_div(T_, 16);
@@ -966,7 +1141,7 @@ extern "C" int mi_moe_router_fused(const void* x, const void* gate_w, const floa
     return mi_router_general(x, gate_w, bias, T, H, E, k, dtype, logits_out, gates_out, idx_out, gws, s);
   }
   const size_t need = router_ws_bytes(T, H, E);
-  if (ws != nullptr && need > 0) {  // few tokens and a workspace: K split across workgroups
+  if (ws != nullptr && need > 0 && !router_one_group(T, H, E)) {  // few tokens and a workspace: K split across workgroups
     if (ws_bytes < need) return MI_MOE_EWORKSPACE;
     if (!mi_aligned(ws, 16)) return MI_MOE_EALIGN;
     if (dtype == MI_MOE_BF16)
@@ -987,10 +1162,12 @@ extern "C" int mi_moe_rmsnorm_router_fused_supported(int H, int E, int k, int dt
   return rmsnorm_router_lds_bytes(H, E, 2) <= 156u * 1024u;
 }
 
-extern "C" int mi_moe_rmsnorm_router_fused(const void* h, const void* ln_weight, float eps, const void* gate_w,
-                                           const float* bias, int T, int H, int E, int k, int dtype,
-                                           void* x_norm_out, void* logits_out, void* gates_out, int32_t* idx_out,
-                                           mi_moe_stream_t stream) {
+bool mi_rmsnorm_router_sorts(int T, int H, int E) { return T >= 1 && router_one_group(T, H, E); }
+
+// sorted_expert (mi_rmsnorm_router_sorts) or null: the sort in the same launch
+int mi_rmsnorm_router(const void* h, const void* ln_weight, float eps, const void* gate_w, const float* bias, int T, int H, int E,
+                      int k, int dtype, void* x_norm_out, void* logits_out, void* gates_out, int32_t* idx_out,
+                      int32_t* sorted_expert, int32_t* sorted_scattered, int32_t* expert_offsets, mi_moe_stream_t stream) {
   if (T < 0 || H < 1 || E < 1 || k < 1 || k > E) return MI_MOE_ESHAPE;
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16) return MI_MOE_EDTYPE;
   if (!mi_moe_rmsnorm_router_fused_supported(H, E, k, dtype)) return MI_MOE_EUNSUPPORTED;
@@ -999,8 +1176,23 @@ extern "C" int mi_moe_rmsnorm_router_fused(const void* h, const void* ln_weight,
   if (!mi_aligned(h, 16) || !mi_aligned(gate_w, 16) || !mi_aligned(x_norm_out, 16)) return MI_MOE_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RouterNorm norm = {ln_weight, x_norm_out, eps};
+  if (router_one_group(T, H, E)) {
+    if (dtype == MI_MOE_BF16)
+      return launch_router_one_group<bf16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, sorted_expert,
+                                                   sorted_scattered, expert_offsets, s);
+    return launch_router_one_group<f16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, sorted_expert,
+                                                sorted_scattered, expert_offsets, s);
+  }
   const size_t lds = rmsnorm_router_lds_bytes(H, E, 2);
   if (dtype == MI_MOE_BF16)
     return launch_router_lds<bf16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, lds, s);
   return launch_router_lds<f16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, lds, s);
+}
+
+extern "C" int mi_moe_rmsnorm_router_fused(const void* h, const void* ln_weight, float eps, const void* gate_w,
+                                           const float* bias, int T, int H, int E, int k, int dtype,
+                                           void* x_norm_out, void* logits_out, void* gates_out, int32_t* idx_out,
+                                           mi_moe_stream_t stream) {
+  return mi_rmsnorm_router(h, ln_weight, eps, gate_w, bias, T, H, E, k, dtype, x_norm_out, logits_out, gates_out, idx_out, nullptr,
+                           nullptr, nullptr, stream);
 }
