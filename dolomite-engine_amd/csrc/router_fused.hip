@@ -1141,12 +1141,14 @@ extern "C" int mi_moe_router_fused(const void* x, const void* gate_w, const floa
     return mi_router_general(x, gate_w, bias, T, H, E, k, dtype, logits_out, gates_out, idx_out, gws, s);
   }
   const size_t need = router_ws_bytes(T, H, E);
-  if (ws != nullptr && need > 0 && !router_one_group(T, H, E)) {  // few tokens and a workspace: K split across workgroups
+  if (ws != nullptr && need > 0) {  // few tokens and a workspace: K split across workgroups
     if (ws_bytes < need) return MI_MOE_EWORKSPACE;
     if (!mi_aligned(ws, 16)) return MI_MOE_EALIGN;
-    if (dtype == MI_MOE_BF16)
-      return launch_router_splitk<bf16_t>(x, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, ws, s);
-    return launch_router_splitk<f16_t>(x, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, ws, s);
+    if (!router_one_group(T, H, E)) {
+      if (dtype == MI_MOE_BF16)
+        return launch_router_splitk<bf16_t>(x, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, ws, s);
+      return launch_router_splitk<f16_t>(x, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, ws, s);
+    }
   }
   if (dtype == MI_MOE_BF16) return launch_router<bf16_t>(x, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, s);
   return launch_router<f16_t>(x, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, s);
