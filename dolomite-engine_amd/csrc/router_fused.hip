@@ -392,7 +392,8 @@ __global__ __launch_bounds__(ROUTER_LDS_WAVES * 64) void router_fused_lds_kernel
 // steps p, p + 8, ..., and requests everything it will read -- its steps of the rows, of the gate weights (straight into the
 // matrix operands' registers: nobody else in the workgroup wants them) and of gamma -- at once.  One trip to memory, where the
 // kernel above makes three (rows, weights to LDS, with the norm the rows again); the parts are added in the same order, so the
-// results are the same bits.  SORT (one workgroup, at most 16 tokens): the one-block sort of the experts behind it.
+// results are the same bits.  Hidden 1536, 40 experts, cold inputs, router + sort, us, before -> after: 1024 tokens 21.2 -> 20.6, 4096
+// 25.5 -> 24.6; with the norm, router alone 18.7 -> 16.2 and 22.9 -> 20.1.  SORT (one workgroup, at most 16 tokens): the one-block sort of the experts behind it.
 #define ROUTER_DIRECT_STEPS 4
 #define ROUTER_DIRECT_H (ROUTER_DIRECT_STEPS * ROUTER_LDS_WAVES * 64)
 #define ROUTER_SORT_TOKENS 16
@@ -944,8 +945,16 @@ static int launch_router_lds(const void* x, const void* gw, const float* bias, i
   return mi_launch_status();
 }
 
-// at most 16 tokens: router (with the norm) and sort in one workgroup
-static bool router_one_group(int T_, int H, int E) { return T_ <= ROUTER_SORT_TOKENS && H <= ROUTER_DIRECT_H && router_lds_fits(H, E); }
+// At most 16 tokens: router (with the norm) and sort in one workgroup.  Without the norm what it replaces has K split over workgroups
+// and one CU is slower at the bytes, so they are limited to 128 KB of rows and gate weights.  Layer, us, before -> after: 32 experts,
+// hidden 1024, 1 / 8 / 16 tokens 28.0 -> 24.9 / 33.3 -> 32.2 / 34.2 -> 33.3, with the norm 30.1 -> 26.4 / 36.1 -> 33.4 / 37.3 -> 35.0; 40
+// experts, hidden 1536 28.4 -> 26.0 / 46.9 -> 47.6 / 51.0 -> 52.0 (the last two stay), with the norm 30.6 -> 27.6 / 51.5 -> 48.8 / 56.7 -> 54.0.
+static bool router_norm_one_group(int T_, int H, int E) {
+  return T_ <= ROUTER_SORT_TOKENS && H <= ROUTER_DIRECT_H && router_lds_fits(H, E);
+}
+static bool router_one_group(int T_, int H, int E) {
+  return router_norm_one_group(T_, H, E) && (long)(T_ + E) * H <= 65536;
+}
 template <typename T, bool NORM>
 static int launch_router_one_group(const void* x, const void* gw, const float* bias, int T_, int H, int E, int k, void* logits_out,
                                    void* gates, int32_t* idx, RouterNorm norm, int32_t* sorted_expert, int32_t* sorted_scattered,
@@ -1164,7 +1173,7 @@ extern "C" int mi_moe_rmsnorm_router_fused_supported(int H, int E, int k, int dt
   return rmsnorm_router_lds_bytes(H, E, 2) <= 156u * 1024u;
 }
 
-bool mi_rmsnorm_router_sorts(int T, int H, int E) { return T >= 1 && router_one_group(T, H, E); }
+bool mi_rmsnorm_router_sorts(int T, int H, int E) { return T >= 1 && router_norm_one_group(T, H, E); }
 
 // sorted_expert (mi_rmsnorm_router_sorts) or null: the sort in the same launch
 int mi_rmsnorm_router(const void* h, const void* ln_weight, float eps, const void* gate_w, const float* bias, int T, int H, int E,
@@ -1178,7 +1187,7 @@ int mi_rmsnorm_router(const void* h, const void* ln_weight, float eps, const voi
   if (!mi_aligned(h, 16) || !mi_aligned(gate_w, 16) || !mi_aligned(x_norm_out, 16)) return MI_MOE_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RouterNorm norm = {ln_weight, x_norm_out, eps};
-  if (router_one_group(T, H, E)) {
+  if (router_norm_one_group(T, H, E)) {
     if (dtype == MI_MOE_BF16)
       return launch_router_one_group<bf16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, sorted_expert,
                                                    sorted_scattered, expert_offsets, s);
