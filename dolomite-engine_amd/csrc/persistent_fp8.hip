@@ -44,7 +44,7 @@ template <> __device__ __forceinline__ uint32_t pf_widen2<f16_t>(uint32_t v, boo
 template <typename T, bool GLU>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(GemmArgs a) {
   constexpr int BN = GLU ? 128 : 256;               // output columns per tile
-  constexpr int NSTORE = GLU ? 8 : 16;              // stores of a wave in the epilogue of an interior tile
+  constexpr int NSTORE = GLU ? 8 : 16;              // stores of a wave in the epilogue
   typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
   typedef __attribute__((address_space(3))) const u32x4* frag_ptr_t;
 
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
   typedef std::integral_constant<int, 3> half_d;
   // Between the halves of a slice: the next slice has landed -- behind it may be in flight what this wave requested
   // since: activations two slices less a half, weights one slice -- and this one is in everybody's registers.
-  // stores: the epilogue of an interior tile lies between those requests.
+  // stores: the epilogue of a tile lies between those requests.
   auto meet = [&](bool odd, bool stores) {
     if (isx) {
       if (stores) __builtin_amdgcn_s_waitcnt(pg_wait(12 + NSTORE, 0));
@@ -287,15 +287,32 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
   };
   int orow_l;
   float sc_lo, sc_hi;
-  auto epilogue_as = [&](auto interior_tag, auto nt_tag, const PgTile& t) {
-    constexpr bool INTERIOR = decltype(interior_tag)::value, NT = decltype(nt_tag)::value;
+  // Every tile issues the same number of stores on one path, what does not exist as lanes past the buffer, and none is waited for
+  // before the next tile's first slice (rows [row0, row0 + out_window): persistent_body.h).  Before, with a branch for edge tiles (all
+  // tiles of a middling load), and now: a layer of 64 experts, hidden 4096, 309.0 -> 305.0 us at 1024 tokens, 252.7 -> 250.4 at 180,
+  // 580 -> 575 at 2500.  Leaving out the matrix instructions of row blocks that a tile does not have gains 2 % at 180 tokens and loses
+  // 4 - 10 % from 600 on: with branches in a half slice the fragments are waited for at each, and four copies of the loop spill.
+  auto epilogue_as = [&](auto nt_tag, const PgTile& t, uint32_t row0) __attribute__((always_inline)) {
+    constexpr bool NT = decltype(nt_tag)::value;
     typedef __attribute__((address_space(3))) u32x2* wp_t;
-    unsigned char* dst = reinterpret_cast<unsigned char*>(out);
     const uint32_t ld = (uint32_t)a.N * 2u;
+    const uint32_t window = a.out_window, left = a.L - row0;
+    const auto osrd = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char*>(out) + (uint64_t)row0 * ld, (short)0,
+                                                        (int)((left < window ? left : window) * ld), 0x00020000);
     // activations: the slot behind the last one requested; weights: the second half of the one being requested
     const uint32_t s0 = !isx ? ring + 16384
                              : (ring + PF_XU >= lds_x + PF_NX * PF_XU ? ring + PF_XU - PF_NX * PF_XU : ring + PF_XU);
     const int col0 = t.nt * BN + wn * (GLU ? 64 : 128);
+    // byte offsets of the wave's row `lane`, and of the lane's columns in store it (% CP); the sums saturate
+    constexpr int CP = GLU ? 2 : 4;
+    const uint32_t orel = (uint32_t)orow_l - row0;
+    const uint32_t orow_off = wm * 64 + lane < t.row_end - t.row_begin && orel < window ? orel * ld : PG_OOB;
+    uint32_t coff[CP];
+#pragma unroll
+    for (int c = 0; c < CP; ++c) {
+      const int col = col0 + (scc0 ^ (4 * c)) * 8;
+      coff[c] = col < a.N ? (uint32_t)col * 2u : PG_OOB;
+    }
 #pragma unroll
     for (int p = 0; p < NPASS; ++p) {
       asm volatile("" : "+v"(sc_lo), "+v"(sc_hi));  // (or all the scales of both passes would be held at once)
@@ -327,35 +344,26 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
 #pragma unroll
       for (int it0 = 0; it0 < 8; it0 += 4) {
         u32x4 val[4];
-        int orow[4];
+        uint32_t roff[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           val[j] = *(frag_ptr_t)(size_t)(s0 + (it0 + j) * 2048 + lane * 16);
-          orow[j] = __builtin_amdgcn_ds_bpermute((p * PASS_ROWS + (it0 + j) * RPP + srow) * 4, orow_l);
+          roff[j] = (uint32_t)__builtin_amdgcn_ds_bpermute((p * PASS_ROWS + (it0 + j) * RPP + srow) * 4, (int)orow_off);
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int it = it0 + j;
-          const int row = t.row_begin + wm * 64 + p * PASS_ROWS + it * RPP + srow;
-          const int col = col0 + (scc0 ^ (GLU ? 4 * (it & 1) : 4 * (it & 3))) * 8;
-          if (INTERIOR || (row < t.row_end && col < a.N)) {
-            u32x4* q = reinterpret_cast<u32x4*>(dst + (uint64_t)(uint32_t)orow[j] * ld + (uint32_t)col * 2u);
-            if constexpr (NT) __builtin_nontemporal_store(val[j], q);
-            else *q = val[j];
-          }
-        }
+        for (int j = 0; j < 4; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(val[j], osrd, (int)__builtin_elementwise_add_sat(roff[j], coff[(it0 + j) % CP]), 0, NT ? 2 : 0);
       }
       pg_own_agprs();
     }
   };
-  auto epilogue = [&](const PgTile& t, bool interior) {
-    if (interior) {
-      if (a.out_nt) epilogue_as(std::true_type{}, std::true_type{}, t);
-      else epilogue_as(std::true_type{}, std::false_type{}, t);
-    } else {
-      if (a.out_nt) epilogue_as(std::false_type{}, std::true_type{}, t);
-      else epilogue_as(std::false_type{}, std::false_type{}, t);
-    }
+  auto epilogue = [&](const PgTile& t) __attribute__((always_inline)) {
+    uint32_t row0 = 0;
+    do {
+      if (a.out_nt) epilogue_as(std::true_type{}, t, row0);
+      else epilogue_as(std::false_type{}, t, row0);
+      row0 += a.out_window;
+    } while (row0 < (uint32_t)a.L);
   };
 
   // ---- prologue: activation slices 0-2; weight slices 0, 1 and the first four pieces of 2 ---------------------------------
@@ -431,10 +439,9 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
     float lo_n, hi_n;
     load_rows(after, rows);
     load_ends(nxt, orow_n, lo_n, hi_n);
-    const bool interior = cur.row_begin + PF_BM <= cur.row_end && (cur.nt + 1) * BN <= a.N;
-    epilogue(cur, interior);
+    epilogue(cur);
     if (i + 1 >= n_items) break;
-    stores_pending = interior;
+    stores_pending = true;
     make_xoff(after, rows, xoff_n);
     wsrd_n = make_wsrd(after);
     orow_l = orow_n;
@@ -456,6 +463,7 @@ template <typename T, bool GLU> static int launch_fp8_persistent(GemmArgs a, hip
   int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), PF_LDS, lds_ok);
   if (rc != MI_MOE_OK) return rc;
   a.n_tiles = mi_ceil_div(a.N, GLU ? 128 : 256);
+  a.out_window = PG_OOB / ((uint32_t)a.N * 2u);
   a.kshift = -1;
   if ((a.kdiv & (a.kdiv - 1)) == 0)
     for (a.kshift = 0; (1 << a.kshift) < a.kdiv;) ++a.kshift;
