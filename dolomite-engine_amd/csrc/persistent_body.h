@@ -205,7 +205,10 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a) {
 
   // One half slice: NB matrix instructions for each of the tile's 8 row blocks of a wave (EVEN: `pairs`).  B = 0: values [0, 32)
   // of slice k out of the registers read before, while values [32, 64) are read and W_k+2 is fetched; B = 1: those, while slice
-  // k + 1 is read and X_k+2 is fetched.  `hook()` runs behind the last read.
+  // k + 1 is read and X_k+2 is fetched.  `hook` has two parts, the ring's rotation and
+  // the next half's addresses: near the half's end, apart; EVEN, whose end a low tile leaves out: both behind the last read,
+  // which is more than the issue slots that one matrix instruction leaves (with the plain form's there too, a layer of 8 experts,
+  // 4096 / 14336, 8192 tokens: 4076 -> 4104 us).
   const uint32_t dma0 = lds0 + wave * 1024;
   uint32_t rw, rx;                                  // addresses of the next half's fragments
   auto half = [&](auto btag, auto ftag, int pairs, uint32_t dst, auto hook) __attribute__((always_inline)) {
@@ -242,7 +245,15 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a) {
           if (q < NB) wf[B ^ 1][q] = read_w(rw, B ^ 1, q);
           else xf[B ^ 1][q - NB] = read_x(rx, q - NB);
           PG_SCHED();
-          if (q == NR - 1) hook();
+          if (EVEN && q == NR - 1) {
+            hook(0);
+            hook(1);
+          }
+          PG_SCHED();
+        }
+        if (!EVEN && (m0 + i == NB * NX - 4 || m0 + i == NB * NX - 2)) {
+          PG_SCHED();
+          hook(m0 + i == NB * NX - 4 ? 0 : 1);
           PG_SCHED();
         }
 #pragma unroll
@@ -290,7 +301,8 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a) {
   // stores_after_dma: the epilogue of a tile lies between the DMA this slice waits for and now
   auto step = [&](auto ftag, int pairs, bool stores_after_dma) __attribute__((always_inline)) {
     if (kw >= kw_ev) w_event();
-    half(std::integral_constant<int, 0>{}, ftag, pairs, dma0 + p4, [&]() {
+    half(std::integral_constant<int, 0>{}, ftag, pairs, dma0 + p4, [&](int part) __attribute__((always_inline)) {
+      if (part == 0) return;
       ++kw;
       read_bases(0, p3, p2);
     });
@@ -302,16 +314,19 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a) {
     asm volatile("" ::: "memory");
     PG_SCHED();
     if (kx >= kx_ev) x_event();
-    half(std::integral_constant<int, 1>{}, std::false_type{}, pairs, dma0 + p0, [&]() {
-      const uint32_t t0 = p0, t1 = p1;
-      p0 = p2;
-      p1 = p3;
-      p2 = RING3 ? px2 : t0;
-      p3 = p4;
-      p4 = t1;
-      px2 = t0;
-      if (RING3) asm volatile("" : "+s"(px2));
-      asm volatile("" : "+s"(p0), "+s"(p1), "+s"(p2), "+s"(p3), "+s"(p4));
+    half(std::integral_constant<int, 1>{}, std::false_type{}, pairs, dma0 + p0, [&](int part) __attribute__((always_inline)) {
+      if (part == 0) {
+        const uint32_t t0 = p0, t1 = p1;
+        p0 = p2;
+        p1 = p3;
+        p2 = RING3 ? px2 : t0;
+        p3 = p4;
+        p4 = t1;
+        px2 = t0;
+        if (RING3) asm volatile("" : "+s"(px2));
+        asm volatile("" : "+s"(p0), "+s"(p1), "+s"(p2), "+s"(p3), "+s"(p4));
+        return;
+      }
       ++kx;
       read_bases(1, p1, p0);
     });
