@@ -369,8 +369,10 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a) {
     typedef __attribute__((address_space(3))) u32x2* wp_t;
     typedef __attribute__((address_space(3))) const u32x4* rp_t;
     const uint32_t ld = (WHAT == 0 ? a.N : 2 * a.N) * 2u;
-    // (rows of the pre-activation are the sorted order's: addressed from the tile's first, as the whole can exceed 4 GiB)
-    const int r0 = tile_row0, rows = t.row_end - t.row_begin;
+    // (rows of the pre-activation are the sorted order's: addressed from the tile's first, as the whole can exceed 4 GiB -- and so
+    // can what an expert has behind a tile that is not EVEN, whose end is the expert's)
+    const int behind = t.row_end - t.row_begin;
+    const int r0 = tile_row0, rows = behind < BM ? behind : BM;
     const uint32_t window = WHAT == 0 ? a.out_window : (uint32_t)rows, left = WHAT == 0 ? a.L - row0 : (uint32_t)rows;
     unsigned char* dst = WHAT == 0 ? reinterpret_cast<unsigned char*>(out) + (uint64_t)row0 * ld
                                    : static_cast<unsigned char*>(a.pre) + (uint64_t)t.row_begin * ld;

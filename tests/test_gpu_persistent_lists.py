@@ -61,3 +61,28 @@ def test_output_beyond_4_gib(device):
         want = ref[:, :N // 2] * torch.nn.functional.silu(ref[:, N // 2:])
         # (formed from the rounded halves)
         torch.testing.assert_close(act[rows].float(), want, rtol=2.0 ** -6, atol=8e-3)
+
+
+def test_pre_activation_of_an_expert_beyond_4_gib(device):
+    """The pre-activation's rows are addressed from their tile's first, whatever its expert still has behind them: with 262445 rows of
+    16 KB in one expert, a tile has just over 4 GiB of them behind its first row."""
+    from dolomite_engine_amd import _lib, ops
+
+    counts, K, N = [300, 262445], 64, 8192
+    L = sum(counts)
+    assert _lib.load().mi_moe_grouped_gemm_tile_choice(L, K, N // 2, 2, 2) == 0  # (256 x 256: the form whose tiles end with the expert)
+    print(f"persistent pre-activation of {L} x {N}", flush=True)
+    g = torch.Generator(device).manual_seed(4)
+    off = torch.tensor(counts).cumsum(0).int().to(device)
+    ss = torch.randperm(L, generator=g, device=device).int()
+    x = torch.empty(L, K, device=device, dtype=torch.bfloat16).normal_(generator=g)
+    w = torch.empty(2, N, K, device=device, dtype=torch.bfloat16).normal_(0.0, 0.05, generator=g)
+    stale = [torch.full((L, n), float("nan"), device=device, dtype=torch.bfloat16) for n in (N, N // 2)]
+    del stale  # (what is not written shows: the outputs are allocated where these were)
+    act, h = ops.up_swiglu_keep(x, w, 1, ss, off)
+    for e, begin, end in ((0, 0, counts[0]), (1, counts[0], L)):
+        for rows in torch.arange(begin, end, device=device).split(10000):
+            ref = x[ss[rows].long()].float() @ w[e].float().t()
+            torch.testing.assert_close(h[rows].float(), ref, **TOL)
+            want = ref[:, :N // 2] * torch.nn.functional.silu(ref[:, N // 2:])
+            torch.testing.assert_close(act[rows].float(), want, rtol=2.0 ** -6, atol=8e-3)  # (formed from the rounded halves)
