@@ -35,6 +35,7 @@ struct GemmArgs {
 #define PERSIST_REMAP_FIXED 4  // the caller chose the form (cfg 8 / 9): the host does not apply its own rule
 #define PERSIST_MAX_E 256
 #define PERSIST_WS_TILE_BYTES (256 * 256 * 4)
+#define PERSIST_PRE_MAX_I (1 << 22)  // 256 rows of a pre-activation this wide (2I elements of 16 bits) are 4 GiB
 
 enum { PG_PLAIN = 0, PG_SWIGLU = 1, PG_SWIGLU_KEEP = 2, PG_WEIGHT_KN = 3 };
 // K % 8 == 0 and N % 8 == 0, at most PERSIST_MAX_E experts, 16-byte aligned output

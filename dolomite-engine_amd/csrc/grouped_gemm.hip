@@ -1108,9 +1108,10 @@ extern "C" int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_
   if (!mi_gemm_persistent_ok(a) || (long)L / E < PERSIST_MIN_ROWS) return MI_MOE_EUNSUPPORTED;
   if (!tiled_shape_ok(a, L, true, 2)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
-  if (few_large_tiles(a, true)) {
+  if (few_large_tiles(a, true) || I >= PERSIST_PRE_MAX_I) {
     // too few tiles for one launch to pay: the product on its own rule, then the element-wise pass (one expert of 509 rows,
-    // 1024 -> 512, 28.2 -> 16.9 us; of 4096 rows, 1536 -> 512, 37.2 -> 26.9; 17 experts of 150 rows, 920 -> 520, 37.3 -> 31.2)
+    // 1024 -> 512, 28.2 -> 16.9 us; of 4096 rows, 1536 -> 512, 37.2 -> 26.9; 17 experts of 150 rows, 920 -> 520, 37.3 -> 31.2).
+    // Or rows so wide that a tile's part of the pre-activation exceeds 32-bit byte offsets
     a.out = pre_out;
     a.pre = nullptr;
     a.N = 2 * I;

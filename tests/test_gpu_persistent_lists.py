@@ -86,3 +86,25 @@ def test_pre_activation_of_an_expert_beyond_4_gib(device):
             torch.testing.assert_close(h[rows].float(), ref, **TOL)
             want = ref[:, :N // 2] * torch.nn.functional.silu(ref[:, N // 2:])
             torch.testing.assert_close(act[rows].float(), want, rtol=2.0 ** -6, atol=8e-3)  # (formed from the rounded halves)
+
+
+def test_pre_activation_rows_of_32_mib(device):
+    """Rows of the pre-activation so wide that those of a tile, of 256 or of 160, are beyond 4 GiB."""
+    from dolomite_engine_amd import ops
+
+    L, K, N = 300, 8, 2 * ((1 << 23) + 8)
+    print(f"pre-activation of {L} x {N}", flush=True)
+    g = torch.Generator(device).manual_seed(5)
+    off = torch.tensor([L], dtype=torch.int32, device=device)
+    ss = torch.randperm(L, generator=g, device=device).int()
+    x = torch.empty(L, K, device=device, dtype=torch.bfloat16).normal_(generator=g)
+    w = torch.empty(1, N, K, device=device, dtype=torch.bfloat16).normal_(0.0, 0.05, generator=g)
+    stale = [torch.full((L, n), float("nan"), device=device, dtype=torch.bfloat16) for n in (N, N // 2)]
+    del stale
+    act, h = ops.up_swiglu_keep(x, w, 1, ss, off)
+    rows = x[ss.long()].float()
+    for cols in torch.arange(N // 2, device=device).split(1 << 18):
+        up, gate = rows @ w[0, cols].float().t(), rows @ w[0, N // 2 + cols].float().t()
+        torch.testing.assert_close(h[:, cols].float(), up, **TOL)
+        torch.testing.assert_close(h[:, N // 2 + cols].float(), gate, **TOL)
+        torch.testing.assert_close(act[:, cols].float(), up * torch.nn.functional.silu(gate), rtol=2.0 ** -6, atol=8e-3)
