@@ -86,3 +86,20 @@ def test_even_training_forms(device, dtype, rows, E, K, N, tile, tile_kn):
     want = h.float()[:, :N] * torch.nn.functional.silu(h.float()[:, N:])  # (one rounding, and the rounded halves are exact)
     torch.testing.assert_close(act.float(), want, rtol=TOL[dtype]["rtol"], atol=TOL[dtype]["atol"])
     assert torch.equal(ops.scattered_gemm(x, w.transpose(1, 2).contiguous(), 1, ss, off, True, True, weight_kn=True), plain)
+
+
+def test_tile_choice_takes_no_time(device):
+    """The rule runs in front of every launch: its time does not grow with the load (1 ms is thirty times less than a sum over all
+    row tiles of an expert takes here, and a thousand times what is needed)."""
+    import time
+
+    from dolomite_engine_amd import _lib
+
+    choice = _lib.load().mi_moe_grouped_gemm_tile_choice
+    times = []
+    for _ in range(5):
+        start = time.perf_counter()
+        choice(1 << 30, 64, 64, 3, PLAIN)
+        times.append(time.perf_counter() - start)
+    print(f"tile choice of 2^30 rows: {min(times) * 1e6:.1f} us", flush=True)
+    assert min(times) < 1e-3
