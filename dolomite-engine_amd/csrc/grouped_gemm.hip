@@ -869,7 +869,24 @@ static int launch_naive(GemmArgs a, hipStream_t s) {
 //   3          one thread per output element (any shape, any dtype)
 //   4          DMA-staged 128x128, one tile per workgroup (K % 32 == 0)
 //   100 + 10 rb + nw  weight stream (stream_gemm.hip): row blocks of 16 per unit, waves that split the contraction
-//   7 / 8 / 9  persistent 256x256 tiles (persistent_gemm.hip; K % 8 == 0, N % 8 == 0)
+//   7          the persistent kernel (persistent_gemm.hip; K % 8 == 0, N % 8 == 0), tiles by its rule
+//   8 / 9      its 256x256 tiles with their order fixed
+//   14 / 15 / 16 / 18  its even tiles (persistent_even.hip)
+static int run_persistent(GemmArgs a, int dtype, int form, int cfg, hipStream_t s) {
+  switch (cfg) {
+    case 7: return mi_gemm_persistent(a, dtype, form, s);
+    case 8:  // 256 x 256 tiles with their order fixed: XCDs own contiguous ranges ...
+    case 9:  // ... or take consecutive blocks of one chip-wide round
+      a.remap |= PERSIST_REMAP_FIXED | (cfg == 9 ? PERSIST_REMAP_INTERLEAVE : 0);
+      return mi_gemm_persistent(a, dtype, form, s);
+    case EVEN_256x128:
+    case EVEN_160x256:
+    case EVEN_224x192:
+    case EVEN_256x256: return mi_gemm_even(a, dtype, form, cfg, s);
+    default: return MI_MOE_EUNSUPPORTED;
+  }
+}
+
 template <typename T, bool GLU>
 static int dispatch_cfg(GemmArgs a, int cfg, hipStream_t s) {
   switch (cfg) {
@@ -878,17 +895,7 @@ static int dispatch_cfg(GemmArgs a, int cfg, hipStream_t s) {
     case 2: return launch_tiled<T, 32, 256, 1, 4, GLU>(a, s);
     case 5: return launch_tiled<T, 32, 128, 1, 2, GLU>(a, s);
     case 4: return a.K % 32 == 0 ? launch_dma<T, 128, 128, 2, 2, GLU>(a, s) : MI_MOE_EUNSUPPORTED;
-    case 7: return mi_gemm_persistent(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, s);
-    case 8:  // the persistent kernel with the tile order fixed: XCDs own contiguous ranges ...
-    case 9:  // ... or take consecutive blocks of one chip-wide round
-      a.remap |= PERSIST_REMAP_FIXED | (cfg == 9 ? PERSIST_REMAP_INTERLEAVE : 0);
-      return mi_gemm_persistent(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, s);
-    case EVEN_256x128:  // the persistent kernel's even forms
-    case EVEN_160x256:
-    case EVEN_224x192:
-    case EVEN_256x256:
-      return mi_gemm_even(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, cfg, s);
-    default: return MI_MOE_EUNSUPPORTED;
+    default: return run_persistent(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, cfg, s);
   }
 }
 
@@ -1039,10 +1046,10 @@ extern "C" int mi_moe_scattered_gemm_cfg(const void* in, const void* w, void* ou
                                   grouped_out, dtype, cfg, nullptr, 0, stream);
 }
 
-extern "C" int mi_moe_scattered_gemm_wt_ws(const void* in, const void* w_kn, void* out,
-                                           const int32_t* sorted_scattered, const int32_t* expert_offsets, int L,
-                                           int K, int N, int E, int k, int grouped_in, int grouped_out, int dtype,
-                                           void* ws, size_t ws_bytes, mi_moe_stream_t stream) {
+extern "C" int mi_moe_scattered_gemm_wt_cfg(const void* in, const void* w_kn, void* out,
+                                            const int32_t* sorted_scattered, const int32_t* expert_offsets, int L,
+                                            int K, int N, int E, int k, int grouped_in, int grouped_out, int dtype, int cfg,
+                                            void* ws, size_t ws_bytes, mi_moe_stream_t stream) {
   int rc = check_common(in, w_kn, out, sorted_scattered, expert_offsets, L, K, N, E, k, dtype,
                         !grouped_in || !grouped_out);
   if (rc != MI_MOE_OK) return rc;
@@ -1057,8 +1064,15 @@ extern "C" int mi_moe_scattered_gemm_wt_ws(const void* in, const void* w_kn, voi
   a.out_nt = persistent_out_nt(a, false, 2);
   if (!tiled_shape_ok(a, L, false, 2) || !mi_gemm_persistent_ok(a)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return mi_gemm_persistent(a, dtype, PG_WEIGHT_KN, s);
+  return run_persistent(a, dtype, PG_WEIGHT_KN, cfg < 0 ? 7 : cfg, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mi_moe_scattered_gemm_wt_ws(const void* in, const void* w_kn, void* out,
+                                           const int32_t* sorted_scattered, const int32_t* expert_offsets, int L,
+                                           int K, int N, int E, int k, int grouped_in, int grouped_out, int dtype,
+                                           void* ws, size_t ws_bytes, mi_moe_stream_t stream) {
+  return mi_moe_scattered_gemm_wt_cfg(in, w_kn, out, sorted_scattered, expert_offsets, L, K, N, E, k, grouped_in, grouped_out,
+                                      dtype, -1, ws, ws_bytes, stream);
 }
 
 extern "C" int mi_moe_scattered_gemm_wt(const void* in, const void* w_kn, void* out, const int32_t* sorted_scattered,
@@ -1089,9 +1103,9 @@ extern "C" int mi_moe_up_swiglu_ws(const void* x, const void* w_fc, void* act_ou
   return run_gemm(a, dtype, true, cfg, L, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_out, void* pre_out,
-                                     const int32_t* sorted_scattered, const int32_t* expert_offsets, int L, int H, int I,
-                                     int E, int k, int dtype, mi_moe_stream_t stream) {
+extern "C" int mi_moe_up_swiglu_keep_cfg(const void* x, const void* w_fc, void* act_out, void* pre_out,
+                                         const int32_t* sorted_scattered, const int32_t* expert_offsets, int L, int H, int I,
+                                         int E, int k, int dtype, int cfg, mi_moe_stream_t stream) {
   int rc = check_common(x, w_fc, act_out, sorted_scattered, expert_offsets, L, H, I, E, k, dtype, true);
   if (rc != MI_MOE_OK) return rc;
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16) return MI_MOE_EDTYPE;
@@ -1105,10 +1119,11 @@ extern "C" int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_
   a.gather = 1; a.scatter = 0; a.remap = 1; a.ws = nullptr; a.pre = pre_out;
   // only the persistent kernel writes the pre-activation from its accumulators: shapes it does not take, and loads of a few
   // rows per expert, are the caller's two-call path
-  if (!mi_gemm_persistent_ok(a) || (long)L / E < PERSIST_MIN_ROWS) return MI_MOE_EUNSUPPORTED;
+  if (!mi_gemm_persistent_ok(a) || (cfg < 0 && (long)L / E < PERSIST_MIN_ROWS)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_shape_ok(a, L, true, 2)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
-  if (few_large_tiles(a, true) || I >= PERSIST_PRE_MAX_I) {
+  if (cfg >= 0 && I >= PERSIST_PRE_MAX_I) return MI_MOE_EUNSUPPORTED;
+  if (cfg < 0 && (few_large_tiles(a, true) || I >= PERSIST_PRE_MAX_I)) {
     // too few tiles for one launch to pay: the product on its own rule, then the element-wise pass (one expert of 509 rows,
     // 1024 -> 512, 28.2 -> 16.9 us; of 4096 rows, 1536 -> 512, 37.2 -> 26.9; 17 experts of 150 rows, 920 -> 520, 37.3 -> 31.2).
     // Or rows so wide that a tile's part of the pre-activation exceeds 32-bit byte offsets
@@ -1119,8 +1134,13 @@ extern "C" int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_
     return mi_moe_swiglu_forward(pre_out, act_out, L, I, dtype, stream);
   }
   a.out_nt = 0;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return mi_gemm_persistent(a, dtype, PG_SWIGLU_KEEP, s);
+  return run_persistent(a, dtype, PG_SWIGLU_KEEP, cfg < 0 ? 7 : cfg, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_out, void* pre_out,
+                                     const int32_t* sorted_scattered, const int32_t* expert_offsets, int L, int H, int I,
+                                     int E, int k, int dtype, mi_moe_stream_t stream) {
+  return mi_moe_up_swiglu_keep_cfg(x, w_fc, act_out, pre_out, sorted_scattered, expert_offsets, L, H, I, E, k, dtype, -1, stream);
 }
 
 extern "C" int mi_moe_up_swiglu_cfg(const void* x, const void* w_fc, void* act_out, const int32_t* sorted_scattered,

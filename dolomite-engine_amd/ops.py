@@ -362,6 +362,10 @@ def _gemm_workspace(device: torch.device, K: int, dtype: torch.dtype, enabled: b
     return ws, ws.numel()
 
 
+# forms of the persistent kernel (mi_moe_scattered_gemm_cfg)
+_PERSISTENT_CFGS = (7, 8, 9, 14, 15, 16, 18)
+
+
 def scattered_gemm(inputs: torch.Tensor, weight: torch.Tensor, k: int, sorted_scattered_idxs: torch.Tensor,
                    expert_offsets: torch.Tensor, grouped_in: bool, grouped_out: bool, cfg: int = -1,
                    weight_kn: bool = False, split_k: bool = True) -> torch.Tensor:
@@ -370,7 +374,8 @@ def scattered_gemm(inputs: torch.Tensor, weight: torch.Tensor, k: int, sorted_sc
     ``split_k``: hand the persistent kernel its workspace (see _gemm_workspace); False runs every tile whole.
 
     ``weight_kn``: the weight is (E, in, out) instead (``inputs @ weight[e]``, the form of the backward's data
-    gradients).  Shapes the transposed-weight kernel does not take are transposed once and run the normal way."""
+    gradients).  Shapes the transposed-weight kernel does not take are transposed once and run the normal way, and so are
+    configurations it does not have (of the persistent kernel's tiles only 14 and 16; any other ``cfg`` leaves it its rule)."""
     _dev(inputs, weight, sorted_scattered_idxs, expert_offsets)
     _no_grad(inputs, weight)
     inputs = inputs.contiguous()
@@ -393,9 +398,9 @@ def scattered_gemm(inputs: torch.Tensor, weight: torch.Tensor, k: int, sorted_sc
     ws, ws_bytes = _gemm_workspace(inputs.device, K, inputs.dtype, split_k)
     if weight_kn:
         with _stage("scattered_gemm"):
-            rc = lib.mi_moe_scattered_gemm_wt_ws(_ptr(inputs), _ptr(weight), _ptr(out), _ptr(ss), _ptr(off), L, K, N,
-                                                 E, k, int(grouped_in), int(grouped_out), _code(inputs.dtype),
-                                                 _ptr(ws), ws_bytes, _stream())
+            rc = lib.mi_moe_scattered_gemm_wt_cfg(_ptr(inputs), _ptr(weight), _ptr(out), _ptr(ss), _ptr(off), L, K, N,
+                                                  E, k, int(grouped_in), int(grouped_out), _code(inputs.dtype),
+                                                  cfg if cfg in _PERSISTENT_CFGS else -1, _ptr(ws), ws_bytes, _stream())
         if rc == 0:
             return out
         if rc not in (_lib.MI_MOE_EUNSUPPORTED, _lib.MI_MOE_EDTYPE, _lib.MI_MOE_EALIGN):
@@ -711,10 +716,11 @@ def up_swiglu(x: torch.Tensor, w_fc: torch.Tensor, k: int, sorted_scattered_idxs
 
 
 def up_swiglu_keep(x: torch.Tensor, w_fc: torch.Tensor, k: int, sorted_scattered_idxs: torch.Tensor,
-                   expert_offsets: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+                   expert_offsets: torch.Tensor, cfg: int = -1) -> tuple[torch.Tensor, torch.Tensor]:
     """Up-projection for training: (act (L, I), h (L, 2I)) -- the activation and the pre-activation the backward
     needs.  One launch (mi_moe_up_swiglu_keep) where the persistent tile kernel takes the problem, else the grouped
-    GEMM followed by the element-wise SwiGLU on the stored h; either way act is formed from the rounded h."""
+    GEMM followed by the element-wise SwiGLU on the stored h; either way act is formed from the rounded h.
+    ``cfg``: that launch with the tiles named (7, 8, 9, 14, 15, 16 or 18 as in scattered_gemm), whatever the load."""
     _dev(x, w_fc, sorted_scattered_idxs, expert_offsets)
     _no_grad(x, w_fc)
     x = x.contiguous()
@@ -732,11 +738,11 @@ def up_swiglu_keep(x: torch.Tensor, w_fc: torch.Tensor, k: int, sorted_scattered
         act = torch.empty((L, I2 // 2), dtype=x.dtype, device=x.device)
         h = torch.empty((L, I2), dtype=x.dtype, device=x.device)
         with _stage("up_swiglu"):
-            rc = lib.mi_moe_up_swiglu_keep(_ptr(x), _ptr(w_fc), _ptr(act), _ptr(h), _ptr(ss), _ptr(off), L, H, I2 // 2,
-                                           E, k, _code(x.dtype), _stream())
+            rc = lib.mi_moe_up_swiglu_keep_cfg(_ptr(x), _ptr(w_fc), _ptr(act), _ptr(h), _ptr(ss), _ptr(off), L, H, I2 // 2,
+                                               E, k, _code(x.dtype), cfg, _stream())
         if rc == 0:
             return act, h
-        if rc not in (_lib.MI_MOE_EUNSUPPORTED, _lib.MI_MOE_EALIGN):
+        if cfg >= 0 or rc not in (_lib.MI_MOE_EUNSUPPORTED, _lib.MI_MOE_EALIGN):
             check(rc)
     h = scattered_gemm(x, w_fc, k, ss, off, False, True)
     return swiglu_forward(h), h

@@ -210,13 +210,14 @@ int mi_moe_scattered_gemm_wt(const void* in, const void* w_kn, void* out, const 
 
 /* Same call with an explicit kernel configuration (tuning / benchmarking / tests): cfg = -1 picks one
  * from the shape; 0 / 1 / 2 / 5 = register-staged 256x256 / 128x128 / 32x256 / 32x128 tiles (all three element types);
- * 3 = one thread per output element (any shape); 4 = DMA-staged 128x128 (K % 32 == 0); 7 = persistent
- * DMA-staged 256x256 tiles, four waves of 128x128 and K slices of 64 (K % 8 == 0, N % 8 == 0, E <= 256, `out` 16-byte
- * aligned; what -1 picks for large expert loads); 8 / 9 = 7 with the order in which the XCDs take the tiles fixed to
- * "each XCD a contiguous eighth of the tile list" / "consecutive 32-tile blocks of one chip-wide round" (7 picks the second
- * from 8 column tiles on; same results either way); 14 / 15 / 16 / 18 = the same kernel with an expert's row tiles equally
- * high and tiles of 256x128 / 160x256 / 224x192 / 256x256 (7 picks among these and its own by the rows per expert; the same
- * results); 4, 7 .. 9 and 14 .. 18 are F16 / BF16 only.  100 + 10 r + w = the weight
+ * 3 = one thread per output element (any shape); 4 = DMA-staged 128x128 (K % 32 == 0); 7 = the persistent kernel, four
+ * waves and K slices of 64 (K % 8 == 0, N % 8 == 0, E <= 256, `out` 16-byte aligned; what -1 picks for large expert loads),
+ * with the tiles that its rule picks by the rows per expert; 8 / 9 = its 256x256 tiles with the order in which the XCDs
+ * take them fixed to "each XCD a contiguous eighth of the tile list" / "consecutive 32-tile blocks of one chip-wide round"
+ * (7 takes the second from 8 column tiles on); 14 / 15 / 16 / 18 = an expert's row tiles equally high and tiles of
+ * 256x128 / 160x256 / 224x192 / 256x256.  7 .. 18 give the same bits, except where a call with a workspace cuts tiles along K
+ * (mi_moe_scattered_gemm_ws; only 256x256 tiles of 7, 8 and 9): those add in another order.  4, 7 .. 9 and 14 .. 18 are
+ * F16 / BF16 only.  100 + 10 r + w = the weight
  * stream for a few rows per expert (all three element types) with chunks of 16 r rows (r = 1, 2, 4) and w waves that
  * split the contraction (w = 1, 2, 4; r = 4: 1, 2); 100 = the stream in the form its own rule picks.  A configuration that
  * does not take the shape or type returns MI_MOE_EUNSUPPORTED.
@@ -253,6 +254,10 @@ int mi_moe_scattered_gemm_ws(const void* in, const void* w, void* out, const int
 int mi_moe_scattered_gemm_wt_ws(const void* in, const void* w_kn, void* out, const int32_t* sorted_scattered,
                                 const int32_t* expert_offsets, int L, int K, int N, int E, int k, int grouped_in,
                                 int grouped_out, int dtype, void* ws, size_t ws_bytes, mi_moe_stream_t stream);
+/* ... with the tiles named: cfg 7 (-1: the same), 8, 9, 15 or 18 as above; MI_MOE_EUNSUPPORTED otherwise */
+int mi_moe_scattered_gemm_wt_cfg(const void* in, const void* w_kn, void* out, const int32_t* sorted_scattered,
+                                 const int32_t* expert_offsets, int L, int K, int N, int E, int k, int grouped_in,
+                                 int grouped_out, int dtype, int cfg, void* ws, size_t ws_bytes, mi_moe_stream_t stream);
 
 /*
  * Up-projection with SwiGLU fused into the epilogue:
@@ -286,6 +291,11 @@ int mi_moe_up_swiglu_ws(const void* x, const void* w_fc, void* act_out, const in
 int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_out, void* h_out, const int32_t* sorted_scattered,
                           const int32_t* expert_offsets, int L, int H, int I, int E, int k, int dtype,
                           mi_moe_stream_t stream);
+/* ... always the one launch, with the tiles named: cfg 7, 8, 9, 14, 15, 16 or 18 as above (-1: mi_moe_up_swiglu_keep), for any
+ * number of rows per expert and I < 2^22; MI_MOE_EUNSUPPORTED otherwise */
+int mi_moe_up_swiglu_keep_cfg(const void* x, const void* w_fc, void* act_out, void* h_out, const int32_t* sorted_scattered,
+                              const int32_t* expert_offsets, int L, int H, int I, int E, int k, int dtype, int cfg,
+                              mi_moe_stream_t stream);
 
 /*
  * Gate-weighted combine:  y[t, :] = sum_j gates[t, j] * o[t*k + j, :]   (fp32 accumulation).

@@ -140,6 +140,11 @@ def test_argument_validation_happens_before_any_launch():
     assert lib.mi_moe_up_swiglu_ws(p16, p16, p16, p16, p16, 16, 16, 8, 4, 2, _lib.BF16, -1, p16, 8, None) == E_WS
     assert lib.mi_moe_scattered_gemm_wt_ws(p16, p16, p16, p16, p16, 16, 16, 8, 4, 2, 0, 1, _lib.BF16, p16, 8, None) == E_WS
     assert lib.mi_moe_scattered_gemm_ws(p16, p16, p16, p16, p16, 16, 12, 8, 4, 2, 0, 1, _lib.BF16, -1, None, 0, None) == E_UNSUP
+    # the training forms with their tiles named: other configurations are refused
+    assert lib.mi_moe_scattered_gemm_wt_cfg(p16, p16, p16, p16, p16, 16, 16, 8, 4, 2, 0, 1, _lib.BF16, 14, None, 0, None) == E_UNSUP
+    assert lib.mi_moe_scattered_gemm_wt_cfg(p16, p16, p16, p16, p16, 16, 16, 8, 4, 2, 0, 1, _lib.BF16, 1, None, 0, None) == E_UNSUP
+    assert lib.mi_moe_up_swiglu_keep_cfg(p16, p16, p16, p16, p16, p16, 16, 16, 8, 4, 2, _lib.BF16, 1, None) == E_UNSUP
+    assert lib.mi_moe_up_swiglu_keep_cfg(p16, p16, p16, p16, p16, p16, 16, 8, 1 << 22, 4, 2, _lib.BF16, 8, None) == E_UNSUP
     assert lib.mi_moe_scattered_gemm(None, None, None, None, None, 16, 8, 8, 4, 2, 0, 1, 7, None) == E_DTYPE
     assert lib.mi_moe_scattered_gemm(None, None, None, None, None, 16, 8, 8, 4, 2, 0, 1, _lib.BF16, None) == E_NULL
     assert lib.mi_moe_scattered_gemm(None, None, None, None, None, 0, 8, 8, 4, 2, 0, 1, _lib.BF16, None) == 0

@@ -99,8 +99,10 @@ def test_scattered_gemm_weight_kn(device, dtype, T, E, k, K, N, mode):
                                           grouped_out=grouped_out)
     torch.testing.assert_close(out.cpu().float(), ref, **TOL[dtype])
     if dtype != torch.float32 and K % 32 == 0 and K >= 128 and N % 8 == 0:
-        same = ops.scattered_gemm(xd, wd.transpose(1, 2).contiguous(), k, ssd, offd, grouped_in, grouped_out, cfg=7)
-        assert torch.equal(out, same)
+        for cfg in (7, 8):
+            same = ops.scattered_gemm(xd, wd.transpose(1, 2).contiguous(), k, ssd, offd, grouped_in, grouped_out, cfg=cfg)
+            assert torch.equal(out, same)
+            assert torch.equal(out, ops.scattered_gemm(xd, wd, k, ssd, offd, grouped_in, grouped_out, cfg=cfg, weight_kn=True))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
@@ -218,14 +220,16 @@ def test_split_k_of_the_last_round(device, form, name, counts, K, N):
     rows_w = 2 * N if form == "swiglu" else N
     w = (torch.randn(E, rows_w, K, generator=g) * 0.05).to(torch.bfloat16).to(device)
     w_kn = w.transpose(1, 2).contiguous() if form == "weight_kn" else None
+    # the 256 x 256 tiles, the only ones that are cut, in the order that they have by themselves
+    cfg = 9 if -(-N // (128 if form == "swiglu" else 256)) >= 8 else 8
     print(f"split-K {form} {name}", flush=True)
 
     def run(split):
         if form == "swiglu":
-            return ops.up_swiglu(inp, w, 1, torch.arange(L, dtype=torch.int32, device=device), off, cfg=7, split_k=split)
+            return ops.up_swiglu(inp, w, 1, torch.arange(L, dtype=torch.int32, device=device), off, cfg=cfg, split_k=split)
         if form == "weight_kn":
-            return ops.scattered_gemm(inp, w_kn, 1, ss, off, True, False, weight_kn=True, split_k=split)
-        return ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=7, split_k=split)
+            return ops.scattered_gemm(inp, w_kn, 1, ss, off, True, False, cfg=cfg, weight_kn=True, split_k=split)
+        return ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=cfg, split_k=split)
 
     whole, split, again = run(False), run(True), run(True)
     assert torch.equal(split, again), "not reproducible"
@@ -267,17 +271,17 @@ def test_split_k_workspace_outlives_a_captured_graph(device):
     print("split-K workspace under graph capture", flush=True)
     assert ops._gemm_workspace(torch.device(device), 512, torch.bfloat16)[0] is None
     assert ops._gemm_workspace(torch.device(device), 8192, torch.float32)[0] is None
-    eager = ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=7)
+    eager = ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=8)
     torch.cuda.synchronize()
 
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
-        ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=7)   # creates the side stream's workspace
+        ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=8)   # creates the side stream's workspace
     torch.cuda.current_stream().wait_stream(side)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        out = ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=7)
+        out = ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=8)
     held = {k: v.data_ptr() for k, v in ops._GEMM_WS.items()}
     graph.replay()
     torch.cuda.synchronize()
@@ -289,7 +293,7 @@ def test_split_k_workspace_outlives_a_captured_graph(device):
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            ops.scattered_gemm(small_in, small_w, 1, ss, off, True, False, cfg=7)
+            ops.scattered_gemm(small_in, small_w, 1, ss, off, True, False, cfg=8)
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         torch.cuda.empty_cache()
@@ -344,12 +348,15 @@ def test_persistent_kernel_random_shapes(device, seed):
         inp = (torch.randn(L, K, generator=g) * 0.5).to(torch.bfloat16).to(device)
         w = (torch.randn(E, rows_w, K, generator=g) * (2.0 / K ** 0.5)).to(torch.bfloat16).to(device)
         print(f"persistent kernel seed {seed} case {case}: E={E} L={L} K={K} N={N} {form}", flush=True)
-        if form == "swiglu":
-            out = ops.up_swiglu(inp, w, 1, torch.arange(L, dtype=torch.int32, device=device), off, cfg=7)
-        elif form == "weight_kn":
-            out = ops.scattered_gemm(inp, w.transpose(1, 2).contiguous(), 1, ss, off, True, False, weight_kn=True)
-        else:
-            out = ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=7)
+        fixed_order = 9 if -(-N // (128 if form == "swiglu" else 256)) >= 8 else 8
+        outs = []
+        for cfg in (fixed_order, 7):  # 256 x 256 tiles in the order that they have by themselves, and the rule's tiles
+            if form == "swiglu":
+                outs.append(ops.up_swiglu(inp, w, 1, torch.arange(L, dtype=torch.int32, device=device), off, cfg=cfg))
+            elif form == "weight_kn":
+                outs.append(ops.scattered_gemm(inp, w.transpose(1, 2).contiguous(), 1, ss, off, True, False, cfg=cfg, weight_kn=True))
+            else:
+                outs.append(ops.scattered_gemm(inp, w, 1, ss, off, True, False, cfg=cfg))
         ref = torch.zeros((L, N), dtype=torch.float32, device=device)
         prev = 0
         for e, end in enumerate(off.tolist()):
@@ -361,8 +368,9 @@ def test_persistent_kernel_random_shapes(device, seed):
             scattered = torch.empty_like(ref)
             scattered[ss.long()] = ref
             ref = scattered
-        err = (out.float() - ref).abs().max().item()
-        assert err <= 1e-2 * ref.abs().max().item() + 1e-3, (case, E, L, K, N, form, err)
+        for out in outs:
+            err = (out.float() - ref).abs().max().item()
+            assert err <= 1e-2 * ref.abs().max().item() + 1e-3, (case, E, L, K, N, form, err)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])

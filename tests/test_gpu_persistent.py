@@ -36,27 +36,34 @@ def test_persistent_edges(device, dtype, counts, K, N):
     x = torch.randn(L, K, generator=g).to(dtype).to(device)
     w = (torch.randn(E, N, K, generator=g) * 0.05).to(dtype).to(device)
     ref = _reference(x, w, counts)
-    grouped = ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=7)
+    grouped = ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=8)
     torch.testing.assert_close(grouped.float(), ref, **TOL[dtype])
-    scattered = ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=7)
-    assert torch.equal(scattered[ss.long()], grouped)
     by_slot = torch.empty_like(x)
     by_slot[ss.long()] = x
-    assert torch.equal(ops.scattered_gemm(by_slot, w, 1, ss, off, False, True, cfg=7), grouped)
     w_kn = w.transpose(1, 2).contiguous()
-    assert torch.equal(ops.scattered_gemm(x, w_kn, 1, ss, off, True, True, weight_kn=True), grouped)
+    half, few = N // 2, True
     if N % 16 == 0:
-        half = N // 2
-        act = ops.up_swiglu(by_slot, w, 1, ss, off, cfg=7)
         want = ref[:, :half] * torch.nn.functional.silu(ref[:, half:])
-        torch.testing.assert_close(act.float(), want, **TOL[dtype])
-        if L >= 120 * E:
-            # (the persistent kernel, or with few tiles the product on smaller ones)
-            act_k, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off)
-            few = _lib.load().mi_moe_grouped_gemm_choice(L, K, half, E, 1, ops._code(dtype)) != 7
-            assert torch.equal(h, ops.scattered_gemm(by_slot, w, 1, ss, off, False, True, cfg=-1 if few else 7))
-            torch.testing.assert_close(h.float(), ref, **TOL[dtype])
-            torch.testing.assert_close(act_k.float(), want, rtol=TOL[dtype]["rtol"] * 4, atol=TOL[dtype]["atol"] * 4)
+        keep_tol = dict(rtol=TOL[dtype]["rtol"] * 4, atol=TOL[dtype]["atol"] * 4)
+        few = _lib.load().mi_moe_grouped_gemm_choice(L, K, half, E, 1, ops._code(dtype)) != 7
+    for cfg in (8, 9, 7):  # the 256 x 256 tiles in both orders, and the tiles that the rule picks
+        assert torch.equal(ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=cfg), grouped)
+        scattered = ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=cfg)
+        assert torch.equal(scattered[ss.long()], grouped)
+        assert torch.equal(ops.scattered_gemm(by_slot, w, 1, ss, off, False, True, cfg=cfg), grouped)
+        assert torch.equal(ops.scattered_gemm(x, w_kn, 1, ss, off, True, True, cfg=cfg, weight_kn=True), grouped)
+        if N % 16 == 0:
+            act = ops.up_swiglu(by_slot, w, 1, ss, off, cfg=cfg)
+            torch.testing.assert_close(act.float(), want, **TOL[dtype])
+            act_k, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off, cfg=cfg)
+            assert torch.equal(h, grouped)
+            torch.testing.assert_close(act_k.float(), want, **keep_tol)
+    if N % 16 == 0 and L >= 120 * E:
+        # (the persistent kernel, or with few tiles the product on smaller ones)
+        act_k, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off)
+        assert torch.equal(h, ops.scattered_gemm(by_slot, w, 1, ss, off, False, True, cfg=-1 if few else 7))
+        torch.testing.assert_close(h.float(), ref, **TOL[dtype])
+        torch.testing.assert_close(act_k.float(), want, **keep_tol)
 
 
 @pytest.mark.parametrize("items,K", [(64, 72), (65, 8), (66, 136), (130, 64)])
@@ -85,6 +92,10 @@ def test_persistent_tile_list(device, items, K, cfg):
     act = ops.up_swiglu(by_slot, w, 1, ss, off, cfg=cfg)
     want = ref[:, :N // 2] * torch.nn.functional.silu(ref[:, N // 2:])
     torch.testing.assert_close(act.float(), want, **TOL[torch.bfloat16])
-    if cfg == 9:
-        w_kn = w.transpose(1, 2).contiguous()
-        assert torch.equal(ops.scattered_gemm(x, w_kn, 1, ss, off, True, False, weight_kn=True), o)
+    w_kn = w.transpose(1, 2).contiguous()
+    for form in (cfg, -1):
+        assert torch.equal(ops.scattered_gemm(x, w_kn, 1, ss, off, True, False, cfg=form, weight_kn=True), o)
+    del w_kn
+    act_k, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off, cfg=cfg)
+    assert torch.equal(h, o[ss.long()])
+    torch.testing.assert_close(act_k.float(), want, rtol=4 * TOL[torch.bfloat16]["rtol"], atol=4 * TOL[torch.bfloat16]["atol"])

@@ -32,7 +32,8 @@ def test_expert_of_a_tile(device, E, empty):
     x = torch.randn(L, K, generator=g).bfloat16().to(device)
     w = (torch.randn(E, N, K, generator=g) * 0.05).bfloat16().to(device)
     ref = torch.cat([p.float() @ w[e].float().t() for e, p in enumerate(x.split(counts.tolist()))])
-    torch.testing.assert_close(ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=7).float(), ref, **TOL)
+    for cfg in (8, 14, 15, 16, 18, 7):  # (16: row tiles of 224, the others of 256 and 160)
+        torch.testing.assert_close(ops.scattered_gemm(x, w, 1, ss, off, True, True, cfg=cfg).float(), ref, **TOL)
 
 
 def test_output_beyond_4_gib(device):
@@ -46,10 +47,13 @@ def test_output_beyond_4_gib(device):
     ss = torch.randperm(L, generator=g, device=device).int()
     x = torch.empty(L, K, device=device, dtype=torch.bfloat16).normal_(generator=g)
     w = torch.empty(3, N, K, device=device, dtype=torch.bfloat16).normal_(0.0, 0.05, generator=g)
-    scattered = ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=7)
+    scattered = ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=8)
+    for cfg in (15, 18, 7):
+        assert torch.equal(ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=cfg), scattered)
+    assert torch.equal(ops.scattered_gemm(x, w.transpose(1, 2).contiguous(), 1, ss, off, True, False, cfg=8, weight_kn=True), scattered)
     by_slot = torch.empty_like(x)
     by_slot[ss.long()] = x
-    act, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off)
+    act, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off, cfg=8)
     expert = torch.repeat_interleave(torch.arange(3, device=device), torch.tensor(counts, device=device))
     for rows in torch.arange(L, device=device).split(10000):
         ref = torch.empty(len(rows), N, device=device)
@@ -65,12 +69,11 @@ def test_output_beyond_4_gib(device):
 
 def test_pre_activation_of_an_expert_beyond_4_gib(device):
     """The pre-activation's rows are addressed from their tile's first, whatever its expert still has behind them: with 262445 rows of
-    16 KB in one expert, a tile has just over 4 GiB of them behind its first row."""
-    from dolomite_engine_amd import _lib, ops
+    16 KB in one expert, a tile (of 256 x 256, whose end is the expert's) has just over 4 GiB of them behind its first row."""
+    from dolomite_engine_amd import ops
 
     counts, K, N = [300, 262445], 64, 8192
     L = sum(counts)
-    assert _lib.load().mi_moe_grouped_gemm_tile_choice(L, K, N // 2, 2, 2) == 0  # (256 x 256: the form whose tiles end with the expert)
     print(f"persistent pre-activation of {L} x {N}", flush=True)
     g = torch.Generator(device).manual_seed(4)
     off = torch.tensor(counts).cumsum(0).int().to(device)
@@ -79,7 +82,7 @@ def test_pre_activation_of_an_expert_beyond_4_gib(device):
     w = torch.empty(2, N, K, device=device, dtype=torch.bfloat16).normal_(0.0, 0.05, generator=g)
     stale = [torch.full((L, n), float("nan"), device=device, dtype=torch.bfloat16) for n in (N, N // 2)]
     del stale  # (what is not written shows: the outputs are allocated where these were)
-    act, h = ops.up_swiglu_keep(x, w, 1, ss, off)
+    act, h = ops.up_swiglu_keep(x, w, 1, ss, off, cfg=8)
     for e, begin, end in ((0, 0, counts[0]), (1, counts[0], L)):
         for rows in torch.arange(begin, end, device=device).split(10000):
             ref = x[ss[rows].long()].float() @ w[e].float().t()

@@ -71,13 +71,14 @@ def test_swiglu_keep_of_large_operands(device):
     w[0, N:, 1] = 1
     ss = torch.arange(L, dtype=torch.int32, device=device)
     off = torch.full((1,), L, dtype=torch.int32, device=device)
-    act, h = ops.up_swiglu_keep(x, w, 1, ss, off)
-    assert torch.equal(h[:, 0], up) and torch.equal(h[:, N], gate)
-    _check(act, up, gate, dtype)
-    _check(ops.swiglu_forward(h), up, gate, dtype)
+    for cfg in (-1, 8, 14, 15, 16, 18):  # (so few tiles are two launches by themselves)
+        act, h = ops.up_swiglu_keep(x, w, 1, ss, off, cfg=cfg)
+        assert torch.equal(h[:, 0], up) and torch.equal(h[:, N], gate)
+        _check(act, up, gate, dtype)
+        _check(ops.swiglu_forward(h), up, gate, dtype)
 
 
-@pytest.mark.parametrize("cfg", [7, 1, 111])
+@pytest.mark.parametrize("cfg", [7, 8, 1, 111])
 def test_swiglu_split_and_non_finite(device, cfg):
     """Infinities and NaN come through the gate's own product: a row's only non-zero value is the gate's, and up is a sum of
     the same value (up == gate), so that no zero weight meets an infinity."""
@@ -110,8 +111,8 @@ def test_swiglu_of_large_operands_split_k(device):
     w[0, N:, 1] = 1
     ss = torch.arange(L, dtype=torch.int32, device=device)
     off = torch.full((1,), L, dtype=torch.int32, device=device)
-    act = ops.up_swiglu(x, w, 1, ss, off, cfg=7)
-    assert torch.equal(act, ops.up_swiglu(x, w, 1, ss, off, cfg=7, split_k=False))
+    act = ops.up_swiglu(x, w, 1, ss, off, cfg=9)
+    assert torch.equal(act, ops.up_swiglu(x, w, 1, ss, off, cfg=9, split_k=False))
     _check(act[:, ::509], up, gate, dtype)
 
 
