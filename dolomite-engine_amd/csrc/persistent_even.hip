@@ -44,10 +44,10 @@ static double tile_cost(const GemmArgs& a, int form, int nb, int bm, bool even, 
   const int cols = mi_ceil_div(a.N, (glu ? 16 : 32) * nb);
   const double all = a.E * row_tiles * cols / cus;
   double rounds = std::ceil(all);
-  if (!even && a.ws != nullptr && mi_gemm_persistent_splits(a.K) && form != PG_SWIGLU_KEEP && rounds > all) {
-    const double parts = std::floor(1.0 / (all - std::floor(all)));
-    rounds += 1.0 / std::fmin(std::fmax(parts, 1.0), (double)PERSIST_SPLIT_MAX) - 1.0;
-  }
+  // (a last round that the plan cuts along K: 8 experts, 5120 -> 4096, 1000 tokens, whose two halves it refuses, 102.6 us with the
+  // credit for them, 76.4 without)
+  if (!even && a.ws != nullptr && mi_gemm_persistent_splits(a.K) && form != PG_SWIGLU_KEEP && rounds > all)
+    rounds += 1.0 / persist_parts(cus, (int)std::ceil((all - std::floor(all)) * cus), mi_ceil_div(a.K, PG_BK)) - 1.0;
   double pairs = bm / 32;
   if (even) pairs = std::fmax(4.0, std::fmin(pairs, std::ceil((avg + 0.5 * sd) / row_tiles / 32.0)));
   const int slices = mi_ceil_div(a.K, PG_BK) < 2 ? 2 : mi_ceil_div(a.K, PG_BK);
@@ -82,9 +82,13 @@ int mi_gemm_even(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s
   return mi_gemm_even_train(a, dtype, form, tile, s);
 }
 
-extern "C" int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form) {
+static int tile_choice(int L, int K, int N, int E, int form, bool ws) {
   if (L < 1 || K < 1 || N < 1 || E < 1 || E > PERSIST_MAX_E || form < PG_PLAIN || form > PG_WEIGHT_KN) return MI_MOE_ESHAPE;
   GemmArgs a = {};
   a.L = L; a.K = K; a.N = N; a.E = E;
+  a.ws = ws ? &a : nullptr;  // (whether there is one)
   return mi_gemm_even_pick(a, form);
 }
+
+extern "C" int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, false); }
+extern "C" int mi_moe_grouped_gemm_tile_choice_ws(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, true); }

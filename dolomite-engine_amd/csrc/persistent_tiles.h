@@ -33,6 +33,13 @@ struct SplitPlan {
   int ws_base;       // first partial-tile slot of the last round's tiles in the workspace
 };
 
+// K ranges that each of the `rem` tiles of a last round is cut into, on `cap` slots
+__host__ __device__ inline int persist_parts(int cap, int rem, int nk) {
+  int p = cap / rem;
+  if (p > PERSIST_SPLIT_MAX) p = PERSIST_SPLIT_MAX;
+  return p >= 2 && nk / p >= PERSIST_SPLIT_MIN_SLICES && nk - nk / p >= PERSIST_SPLIT_MIN_SAVED ? p : 1;
+}
+
 // xcd / slot of the workgroup (slot < nslot); for the finishing kernel, slot is the tile of the last round it adds up
 __device__ __forceinline__ SplitPlan persist_split_plan(int total, int xcd, int slot, int nslot, int nk, bool have_ws,
                                                         bool interleave) {
@@ -60,15 +67,9 @@ __device__ __forceinline__ SplitPlan persist_split_plan(int total, int xcd, int 
     sp.rem_base = xcd * per + sp.full_rounds * nslot;
     sp.ws_base = xcd * nslot;
   }
-  sp.parts = 1;
-  if (have_ws && sp.rem > 0) {
-    int p = cap / sp.rem;
-    if (p > PERSIST_SPLIT_MAX) p = PERSIST_SPLIT_MAX;
-    if (p >= 2 && nk / p >= PERSIST_SPLIT_MIN_SLICES && nk - nk / p >= PERSIST_SPLIT_MIN_SAVED) sp.parts = p;
-  }
+  sp.parts = have_ws && sp.rem > 0 ? persist_parts(cap, sp.rem, nk) : 1;
   return sp;
 }
-
 
 
 struct PgTile {

@@ -227,6 +227,7 @@ int mi_moe_grouped_gemm_choice(int L, int K, int N, int E, int glu, int dtype);
 /* Which tiles configuration 7 takes on the current device for a problem without a workspace: 14, 15, 16 or 18 as above, 0 for
  * its own 256x256.  form: 0 plain, 1 SwiGLU, 2 SwiGLU with the pre-activation, 3 transposed weights. */
 int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form);
+int mi_moe_grouped_gemm_tile_choice_ws(int L, int K, int N, int E, int form);  /* ... for a call with a workspace */
 int mi_moe_scattered_gemm_cfg(const void* in, const void* w, void* out, const int32_t* sorted_scattered,
                               const int32_t* expert_offsets, int L, int K, int N, int E, int k,
                               int grouped_in, int grouped_out, int dtype, int cfg, mi_moe_stream_t stream);
