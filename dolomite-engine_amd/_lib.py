@@ -48,6 +48,7 @@ SIGNATURES: dict[str, tuple] = {
     "mi_moe_grouped_gemm_choice": (_i, [_i, _i, _i, _i, _i, _i]),
     "mi_moe_grouped_gemm_tile_choice": (_i, [_i, _i, _i, _i, _i]),
     "mi_moe_grouped_gemm_tile_choice_ws": (_i, [_i, _i, _i, _i, _i]),
+    "mi_moe_grouped_gemm_tile_choice_load": (_i, [_vp, _i, _i, _i, _i, _i]),
     "mi_moe_grouped_gemm_splits": (_i, [_i, _i]),
     "mi_moe_scattered_gemm_ws": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
     "mi_moe_scattered_gemm_wt_ws": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),

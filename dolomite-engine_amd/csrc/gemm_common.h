@@ -45,11 +45,16 @@ bool mi_gemm_persistent_splits(int K);
 int mi_gemm_persistent(const GemmArgs& a, int dtype, int form, hipStream_t s);
 
 // ---- persistent_even.hip: the same with an expert's row tiles equally high, and other tiles (rows x columns) -----------------
-enum { EVEN_NONE = 0, EVEN_256x128 = 14, EVEN_160x256 = 15, EVEN_224x192 = 16, EVEN_256x256 = 18 };
-// the form that is faster than 256 x 256 tiles for this problem, or EVEN_NONE
-int mi_gemm_even_pick(const GemmArgs& a, int form);
+enum { EVEN_NONE = 0, EVEN_256x128 = 14, EVEN_160x256 = 15, EVEN_224x192 = 16, EVEN_256x256 = 18, EVEN_BY_LOAD = 19 };
+// the tiles that are the fastest for this problem whatever its load, 256 x 256 (EVEN_NONE) or these, or EVEN_BY_LOAD: as it is
+int mi_gemm_tiles_of_any_load(const GemmArgs& a, int form);
 int mi_gemm_even(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s);
 int mi_gemm_even_train(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s);
+// ---- persistent_load.hip: those tiles or 256 x 256 ones, by the experts' rows --------------------------------------------
+int mi_gemm_by_load(const GemmArgs& a, int dtype, int form, hipStream_t s);
+int mi_gemm_by_load_train(const GemmArgs& a, int dtype, int form, hipStream_t s);
+// the launch that adds the parts of tiles cut along K: of 8 nslot workgroups; by_load: unless even tiles were picked
+int mi_gemm_split_finish(const GemmArgs& a, int dtype, int form, int nslot, bool by_load, hipStream_t s);
 
 // ---- persistent_fp8.hip: fp8 weights (wscale, w_tiled); K % 16 == 0, K > 256, N % 8 == 0, at most PERSIST_MAX_E experts,
 // 16-byte aligned output ----------------------------------------------------------------------------------------------

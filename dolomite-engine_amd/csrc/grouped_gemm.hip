@@ -872,6 +872,7 @@ static int launch_naive(GemmArgs a, hipStream_t s) {
 //   7          the persistent kernel (persistent_gemm.hip; K % 8 == 0, N % 8 == 0), tiles by its rule
 //   8 / 9      its 256x256 tiles with their order fixed
 //   14 / 15 / 16 / 18  its even tiles (persistent_even.hip)
+//   19         whichever of these the load on hand wants (persistent_load.h)
 static int run_persistent(GemmArgs a, int dtype, int form, int cfg, hipStream_t s) {
   switch (cfg) {
     case 7: return mi_gemm_persistent(a, dtype, form, s);
@@ -883,6 +884,7 @@ static int run_persistent(GemmArgs a, int dtype, int form, int cfg, hipStream_t 
     case EVEN_160x256:
     case EVEN_224x192:
     case EVEN_256x256: return mi_gemm_even(a, dtype, form, cfg, s);
+    case EVEN_BY_LOAD: return mi_gemm_persistent_ok(a) ? mi_gemm_by_load(a, dtype, form, s) : MI_MOE_EUNSUPPORTED;
     default: return MI_MOE_EUNSUPPORTED;
   }
 }

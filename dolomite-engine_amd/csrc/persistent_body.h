@@ -1,5 +1,5 @@
-// The body of the persistent grouped GEMMs (persistent_gemm.hip: what it is and why; persistent_even.hip: the form for middling
-// loads).
+// The body of the persistent grouped GEMMs (persistent_gemm.hip: what it is and why; persistent_even.hip: the forms for middling
+// loads; persistent_load.h: the one that the load on hand wants).
 #pragma once
 
 #include "gemm_common.h"
@@ -14,7 +14,7 @@
 // NB: blocks of 16 weight rows of a wave (a tile has 4 NB).  EVEN: an expert's row tiles are equally high, in steps of 32 rows, and
 // a low tile costs what it has (pg_locate, half)
 template <typename T, bool GLU, bool WT, bool KEEP, bool NT, int NB = 8, bool EVEN = false, int BM = 256>
-__device__ __forceinline__ void persistent_body(const GemmArgs& a) {
+__device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows& experts) {
   static_assert(!KEEP || GLU, "the pre-activation belongs to the SwiGLU form");
   static_assert(!WT || !GLU, "transposed-weight form");
   static_assert(NB == 8 || !WT, "the image of transposed weights has 256 columns");
@@ -43,7 +43,7 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a) {
 
   // ---- which tiles -----------------------------------------------------------------------------------------------
   PgTable tb;
-  pg_table<BM>(a.expert_offsets, a.L, a.E, tb);
+  pg_table<BM>(experts, a.E, tb);
   const int total = tb.total * a.n_tiles;
   const int nfull = a.K / PG_BK;                    // whole slices; a partial one is padded with zeros
   int nk = (a.K + PG_BK - 1) / PG_BK;
@@ -556,18 +556,39 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a) {
   __builtin_amdgcn_s_waitcnt(pg_wait(0, 0));  // surplus DMA must not outlive the workgroup's LDS
 }
 
+// column tiles of BN columns, and the order that goes with their number (persistent_tiles.h), unless the caller fixed one
+__host__ __device__ inline void persistent_columns(GemmArgs& a, int BN) {
+  a.n_tiles = (a.N + BN - 1) / BN;
+  if (a.remap & PERSIST_REMAP_FIXED) return;
+  a.remap = a.n_tiles >= 8 ? a.remap | PERSIST_REMAP_INTERLEAVE : a.remap & ~PERSIST_REMAP_INTERLEAVE;
+}
+
 // Host side: what a launch with tiles of BM rows and BN columns needs, and its grid.
+static inline int persistent_grid(const GemmArgs& a, int cus, int BM, int BN) {
+  const long max_tiles = ((long)a.L / BM + (a.E < a.L ? a.E : a.L)) * ((a.N + BN - 1) / BN);
+  return ((int)(cus < max_tiles ? cus : max_tiles) + 7) / 8 * 8;
+}
 static inline int persistent_prepare(GemmArgs& a, int BM, int BN, int* grid) {
-  a.n_tiles = mi_ceil_div(a.N, BN);
+  persistent_columns(a, BN);
   a.out_window = PG_OOB / ((uint32_t)a.N * 2u);
   a.kshift = -1;
   if (a.kdiv > 0 && (a.kdiv & (a.kdiv - 1)) == 0)
     for (a.kshift = 0; (1 << a.kshift) < a.kdiv;) ++a.kshift;
-  if (!(a.remap & PERSIST_REMAP_FIXED) && a.n_tiles >= 8) a.remap |= PERSIST_REMAP_INTERLEAVE;  // (see there)
   int cus = 0;
   const int rc = mi_cu_count(&cus);
-  if (rc != MI_MOE_OK) return rc;
-  const long max_tiles = ((long)a.L / BM + (a.E < a.L ? a.E : a.L)) * a.n_tiles;
-  *grid = ((int)(cus < max_tiles ? cus : max_tiles) + 7) / 8 * 8;
+  if (rc == MI_MOE_OK) *grid = persistent_grid(a, cus, BM, BN);
+  return rc;
+}
+// ... and what one needs that picks among the forms: as many workgroups as the one with the most tiles can use, the first form's
+// columns, and the workspace only if a contraction of this length is cut at all
+static inline int by_load_prepare(GemmArgs& a, int form, int* grid) {
+  const int unit = form == PG_SWIGLU || form == PG_SWIGLU_KEEP ? 16 : 32;
+  int cus = 0, rc = persistent_prepare(a, persist_form_rows(0), unit * persist_form_blocks(0), grid);
+  if (rc != MI_MOE_OK || (rc = mi_cu_count(&cus)) != MI_MOE_OK) return rc;
+  for (int i = 1; i < PERSIST_FORMS; ++i) {
+    const int slots = persistent_grid(a, cus, persist_form_rows(i), unit * persist_form_blocks(i));
+    if (slots > *grid) *grid = slots;
+  }
+  if (!mi_gemm_persistent_splits(a.K) || *grid < 16 || form == PG_SWIGLU_KEEP) a.ws = nullptr;
   return MI_MOE_OK;
 }

@@ -3,10 +3,14 @@
 
 #include "persistent_body.h"
 
+template <typename T, int FORM, int NB, int BM> __device__ __forceinline__ void even_body(const GemmArgs& a, const PgRows& experts) {
+  constexpr bool GLU = FORM == PG_SWIGLU || FORM == PG_SWIGLU_KEEP;
+  persistent_body<T, GLU, FORM == PG_WEIGHT_KN, FORM == PG_SWIGLU_KEEP, !GLU, NB, true, BM>(a, experts);
+}
+
 template <typename T, int FORM, int NB, int BM>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_even_kernel(GemmArgs a) {
-  constexpr bool GLU = FORM == PG_SWIGLU || FORM == PG_SWIGLU_KEEP;
-  persistent_body<T, GLU, FORM == PG_WEIGHT_KN, FORM == PG_SWIGLU_KEEP, !GLU, NB, true, BM>(a);
+  even_body<T, FORM, NB, BM>(a, pg_rows(a.expert_offsets, a.L, a.E));
 }
 
 template <typename T, int FORM, int NB, int BM> static int launch_even(GemmArgs a, hipStream_t s) {

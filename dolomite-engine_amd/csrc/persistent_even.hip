@@ -13,7 +13,7 @@
 // them one more (8 experts, 14336 -> 4096, 1000 tokens 299 -> 247 us, 32 experts, 1024 -> 512 SwiGLU, 2048 tokens 46.5 -> 40.8).
 // It fits the LDS for tiles of up to 416 rows and columns together.
 //
-// 256 x 256 tiles / the form the rule picks, us, cold weights (SwiGLU up, then down): 40 experts, 1536 / 512: 500 tokens 37.6 ->
+// 256 x 256 tiles / the fastest form, us, cold weights, experts with about as many rows each (SwiGLU up, then down): 40 experts, 1536 / 512: 500 tokens 37.6 ->
 // 31.6 and 19.7 -> 17.9, 1000 tokens 40.5 -> 36.8 and 21.3 -> 21.2, 2048 tokens 68.6 -> 58.8 and 34.5 -> 34.1, 4096 tokens 103.8 ->
 // 99.8 and 61.5 -> 59.5; 32 experts, 1024 / 512: 509 tokens 25.8 -> 20.1 and 15.5 -> 11.8, 2048 tokens 47.5 -> 40.8 and 29.0 -> 22.2;
 // 8 experts, 14336 -> 4096, 1000 tokens 307 -> 247.
@@ -34,41 +34,105 @@ static double normal_row_tiles(double avg, int bm) {
   return n;
 }
 
-// Time of a launch by the model below, us.  A round is a tile on every CU; a slice takes 0.35 us and 0.013 us for each 16 x 16
-// block of a wave, a tile's ends 1.5 us and 0.035 us for each.  The model orders the forms above as they were measured, and is
-// within a fifth of most times.  What is known here of the experts' rows is their average.
-static double tile_cost(const GemmArgs& a, int form, int nb, int bm, bool even, int cus) {
-  const bool glu = form == PG_SWIGLU || form == PG_SWIGLU_KEEP;
-  const double avg = (double)a.L / a.E, sd = a.E > 1 ? std::sqrt(avg) : 0.0;
-  const double row_tiles = a.E > 1 ? normal_row_tiles(avg, bm) : std::ceil(avg / bm);
-  const int cols = mi_ceil_div(a.N, (glu ? 16 : 32) * nb);
-  const double all = a.E * row_tiles * cols / cus;
-  double rounds = std::ceil(all);
-  // (a last round that the plan cuts along K: 8 experts, 5120 -> 4096, 1000 tokens, whose two halves it refuses, 102.6 us with the
-  // credit for them, 76.4 without)
-  if (!even && a.ws != nullptr && mi_gemm_persistent_splits(a.K) && form != PG_SWIGLU_KEEP && rounds > all)
-    rounds += 1.0 / persist_parts(cus, (int)std::ceil((all - std::floor(all)) * cus), mi_ceil_div(a.K, PG_BK)) - 1.0;
-  double pairs = bm / 32;
-  if (even) pairs = std::fmax(4.0, std::fmin(pairs, std::ceil((avg + 0.5 * sd) / row_tiles / 32.0)));
-  const int slices = mi_ceil_div(a.K, PG_BK) < 2 ? 2 : mi_ceil_div(a.K, PG_BK);
-  return rounds * (slices * (0.35 + 0.013 * pairs * nb) + 1.5 + (form == PG_SWIGLU_KEEP ? 0.07 : 0.035) * pairs * nb);
-}
-
-int mi_gemm_even_pick(const GemmArgs& a, int form) {
-  int cus = 0;
-  if (mi_cu_count(&cus) != MI_MOE_OK) return EVEN_NONE;
-  const struct { int tile, nb, bm; } forms[] = {{EVEN_160x256, 8, 160}, {EVEN_256x256, 8, 256}, {EVEN_224x192, 6, 224}, {EVEN_256x128, 4, 256}};
-  int best = EVEN_NONE;
-  double least = 0.97 * tile_cost(a, form, 8, 256, false, cus);  // (the plain form's loop has no branches)
-  for (const auto& f : forms) {
-    if (form == PG_WEIGHT_KN && f.nb != 8) continue;
-    const double c = tile_cost(a, form, f.nb, f.bm, true, cus);
-    if (c < least) {
-      least = c;
-      best = f.tile;
+// Loads in the shape of a power law, rows of an expert ~ (place in the order)^-p: the relative rows at sixteen places.
+struct LoadShapes {
+  static constexpr int N = 4, PLACES = 16;
+  double rows[N][PLACES];
+  LoadShapes() {
+    for (int n = 0; n < N; ++n) {
+      double sum = 0.0;
+      for (int i = 0; i < PLACES; ++i) sum += rows[n][i] = std::pow((i + 0.5) / PLACES, -0.2 * (n + 1));
+      for (double& r : rows[n]) r *= PLACES / sum;
     }
   }
+};
+static const LoadShapes load_shapes;
+
+// Row tiles of 160, 224 and 256 rows where L rows are spread in shape n over a.E experts (-1: normally around their average)
+struct RowTiles {
+  uint32_t n[3];
+  uint32_t of(int i) const { return n[persist_form_rows(i) == 160 ? 0 : (persist_form_rows(i) == 224 ? 1 : 2)]; }
+};
+static RowTiles row_tiles_of(const GemmArgs& a, int n) {
+  const double avg = (double)a.L / a.E;
+  RowTiles r;
+  for (int b = 0; b < 3; ++b) {
+    const int bm = b == 0 ? 160 : (b == 1 ? 224 : 256);
+    if (a.E == 1) {
+      r.n[b] = (uint32_t)mi_ceil_div(a.L, bm);
+    } else if (n < 0) {
+      r.n[b] = (uint32_t)std::lround(a.E * normal_row_tiles(avg, bm));
+    } else {
+      long tiles = 0;
+      const double per = avg / bm;
+      for (const double rows : load_shapes.rows[n]) {
+        const long whole = (long)(per * rows);
+        tiles += whole + (per * rows > (double)whole);
+      }
+      r.n[b] = (uint32_t)((tiles * a.E + LoadShapes::PLACES / 2) / LoadShapes::PLACES);
+    }
+  }
+  return r;
+}
+// The fastest form for so many row tiles; t: time of each
+static int form_of(const GemmArgs& a, int form, int slots, const RowTiles& r, float (&t)[PERSIST_FORMS]) {
+  int best = 0;
+  for (int i = 0; i < PERSIST_FORMS; ++i) {
+    if (form == PG_WEIGHT_KN && persist_form_blocks(i) != 8) continue;
+    t[i] = persist_time(a, form, i, a.L, r.of(i), persist_cols(a.N, form, persist_form_blocks(i)), slots);
+    if (t[i] < t[best]) best = i;
+  }
   return best;
+}
+
+// The tiles that are the fastest whatever the load, as far as the model goes: 584 of 976 problems of 64 to 6000 tokens in 8 to 64
+// experts, among them all loads of many rounds.  For the others there is pg_tiles_by_load, which costs a launch 0.3 us.
+int mi_gemm_tiles_of_any_load(const GemmArgs& args, int form) {
+  GemmArgs a = args;
+  int cus = 0;
+  if (mi_cu_count(&cus) != MI_MOE_OK) return EVEN_NONE;
+  if (!mi_gemm_persistent_splits(a.K)) a.ws = nullptr;
+  float t[PERSIST_FORMS];
+  const int best = form_of(a, form, cus, row_tiles_of(a, -1), t);
+  for (int n = 0; a.E > 1 && n < LoadShapes::N; ++n) {
+    const int other = form_of(a, form, cus, row_tiles_of(a, n), t);
+    if (t[best] > 1.02f * t[other]) return EVEN_BY_LOAD;
+  }
+  return persist_form_tile(best);
+}
+
+static int tile_choice(int L, int K, int N, int E, int form, bool ws) {
+  if (L < 1 || K < 1 || N < 1 || E < 1 || E > PERSIST_MAX_E || form < PG_PLAIN || form > PG_WEIGHT_KN) return MI_MOE_ESHAPE;
+  GemmArgs a = {};
+  a.L = L; a.K = K; a.N = N; a.E = E;
+  a.ws = ws && mi_gemm_persistent_splits(K) ? &a : nullptr;  // (whether there is one)
+  int cus = 0;
+  float t[PERSIST_FORMS];
+  return mi_cu_count(&cus) != MI_MOE_OK ? EVEN_NONE : persist_form_tile(form_of(a, form, cus, row_tiles_of(a, -1), t));
+}
+
+extern "C" int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, false); }
+extern "C" int mi_moe_grouped_gemm_tile_choice_ws(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, true); }
+
+extern "C" int mi_moe_grouped_gemm_tile_choice_load(const int32_t* ends, int K, int N, int E, int form, int ws) {
+  if (K < 1 || N < 1 || E < 1 || E > PERSIST_MAX_E || form < PG_PLAIN || form > PG_WEIGHT_KN) return MI_MOE_ESHAPE;
+  if (!ends) return MI_MOE_ENULL;
+  GemmArgs a = {};
+  a.L = ends[E - 1]; a.K = K; a.N = N; a.E = E;
+  if (a.L < 1) return MI_MOE_ESHAPE;
+  a.ws = ws ? &a : nullptr;
+  int slots = 0;
+  const int rc = by_load_prepare(a, form, &slots);
+  if (rc != MI_MOE_OK) return rc;
+  RowTiles r = {};
+  for (int e = 0; e < E; ++e) {
+    const int rows = ends[e] - (e > 0 ? ends[e - 1] : 0);
+    r.n[0] += (uint32_t)mi_ceil_div(rows, 160);
+    r.n[1] += (uint32_t)mi_ceil_div(rows, 224);
+    r.n[2] += (uint32_t)mi_ceil_div(rows, 256);
+  }
+  float t[PERSIST_FORMS];
+  return persist_form_tile(form_of(a, form, slots, r, t));
 }
 
 int mi_gemm_even(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s) {
@@ -81,14 +145,3 @@ int mi_gemm_even(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s
   }
   return mi_gemm_even_train(a, dtype, form, tile, s);
 }
-
-static int tile_choice(int L, int K, int N, int E, int form, bool ws) {
-  if (L < 1 || K < 1 || N < 1 || E < 1 || E > PERSIST_MAX_E || form < PG_PLAIN || form > PG_WEIGHT_KN) return MI_MOE_ESHAPE;
-  GemmArgs a = {};
-  a.L = L; a.K = K; a.N = N; a.E = E;
-  a.ws = ws ? &a : nullptr;  // (whether there is one)
-  return mi_gemm_even_pick(a, form);
-}
-
-extern "C" int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, false); }
-extern "C" int mi_moe_grouped_gemm_tile_choice_ws(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, true); }

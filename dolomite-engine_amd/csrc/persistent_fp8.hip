@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_fp8_persistent_kernel(Gem
 
   // ---- which tiles -----------------------------------------------------------------------------------------------
   PgTable tb;
-  pg_table<PF_BM>(a.expert_offsets, a.L, a.E, tb);
+  pg_table<PF_BM>(pg_rows(a.expert_offsets, a.L, a.E), a.E, tb);
   const int nd = (a.K + 127) / 128;                 // weight slices (at least 3); two activation slices each
   const SplitPlan sp = persist_split_plan(tb.total * a.n_tiles, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, 2 * nd, false,
                                           (a.remap & PERSIST_REMAP_INTERLEAVE) != 0);

@@ -53,13 +53,14 @@ static bool persistent_may_split(int K) {
 
 template <typename T, bool GLU, bool WT, bool KEEP>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArgs a) {
+  const PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
   if constexpr (!GLU) {
-    persistent_body<T, GLU, WT, KEEP, true>(a);
+    persistent_body<T, GLU, WT, KEEP, true>(a, experts);
   } else if constexpr (KEEP) {
-    persistent_body<T, GLU, WT, KEEP, false>(a);    // (the backward reads both again)
+    persistent_body<T, GLU, WT, KEEP, false>(a, experts);  // (the backward reads both again)
   } else {
-    if (a.out_nt) persistent_body<T, GLU, WT, KEEP, true>(a);
-    else persistent_body<T, GLU, WT, KEEP, false>(a);
+    if (a.out_nt) persistent_body<T, GLU, WT, KEEP, true>(a, experts);
+    else persistent_body<T, GLU, WT, KEEP, false>(a, experts);
   }
 }
 
@@ -68,11 +69,13 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArg
 // and writes them the way the persistent kernel's epilogue does (same arithmetic, same rounding; thread t holds what
 // thread t of a part held).  Workgroups whose tile does not exist or was not split return at once.
 template <typename T, bool GLU>
-__global__ __launch_bounds__(256) void grouped_gemm_split_finish_kernel(GemmArgs a, int nslot) {
+__global__ __launch_bounds__(256) void grouped_gemm_split_finish_kernel(GemmArgs a, int nslot, int by_load_form) {
   constexpr int BM = 256, BN = GLU ? 128 : 256;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
+  const PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
+  if (by_load_form >= 0 && pg_tiles_by_load(a, experts, by_load_form, 8 * nslot) != EVEN_NONE) return;
   PgTable tb;
-  pg_table<BM>(a.expert_offsets, a.L, a.E, tb);
+  pg_table<BM>(experts, a.E, tb);
   // contiguous: workgroup b adds up tile b / 8 of XCD b % 8's last round; interleaved: tile b of the chip's last round
   const bool interleave = (a.remap & PERSIST_REMAP_INTERLEAVE) != 0;
   const int xcd = interleave ? 0 : (int)(blockIdx.x & 7), j = interleave ? (int)blockIdx.x : (int)(blockIdx.x >> 3);
@@ -138,11 +141,15 @@ static int launch_persistent(GemmArgs a, hipStream_t s) {
   if (!mi_gemm_persistent_splits(a.K) || grid < 16 || a.pre != nullptr) a.ws = nullptr;  // (the finishing launch writes the result only)
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), PG_LDS, s, a);
   if ((rc = mi_launch_status()) != MI_MOE_OK || a.ws == nullptr) return rc;
+  return mi_gemm_split_finish(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, grid / 8, false, s);
+}
+
+int mi_gemm_split_finish(const GemmArgs& a, int dtype, int form, int nslot, bool by_load, hipStream_t s) {
+  auto kern = form == PG_SWIGLU ? (dtype == MI_MOE_BF16 ? grouped_gemm_split_finish_kernel<bf16_t, true> : grouped_gemm_split_finish_kernel<f16_t, true>)
+                                : (dtype == MI_MOE_BF16 ? grouped_gemm_split_finish_kernel<bf16_t, false> : grouped_gemm_split_finish_kernel<f16_t, false>);
   // the tiles that were cut: at most half of the slots of a round that was split hold tiles (rounded up: an odd
   // number of slots per XCD)
-  const int nslot = grid / 8;
-  hipLaunchKernelGGL((grouped_gemm_split_finish_kernel<T, GLU>), dim3(8u * (unsigned)((nslot + 1) / 2), 4), dim3(256), 0, s, a,
-                     nslot);
+  hipLaunchKernelGGL(kern, dim3(8u * (unsigned)((nslot + 1) / 2), 4), dim3(256), 0, s, a, nslot, by_load ? form : -1);
   return mi_launch_status();
 }
 
@@ -155,7 +162,8 @@ bool mi_gemm_persistent_ok(const GemmArgs& a) {
 int mi_gemm_persistent(const GemmArgs& a, int dtype, int form, hipStream_t s) {
   if (!mi_gemm_persistent_ok(a)) return MI_MOE_EUNSUPPORTED;
   if (!(a.remap & PERSIST_REMAP_FIXED)) {
-    const int tile = mi_gemm_even_pick(a, form);
+    const int tile = mi_gemm_tiles_of_any_load(a, form);
+    if (tile == EVEN_BY_LOAD) return mi_gemm_by_load(a, dtype, form, s);
     if (tile != EVEN_NONE) return mi_gemm_even(a, dtype, form, tile, s);
   }
   if (dtype == MI_MOE_BF16) {

@@ -72,6 +72,46 @@ __device__ __forceinline__ SplitPlan persist_split_plan(int total, int xcd, int 
 }
 
 
+// The forms of tiles of the persistent kernel (persistent_even.hip), in the order in which equally fast ones are preferred; all but
+// the first are EVEN.  (Shifts of a constant: lane i of a wave asks for form i.)
+#define PERSIST_FORMS 5
+__host__ __device__ constexpr int persist_form_blocks(int i) { return (0x46888 >> (4 * i)) & 15; }        // nb
+__host__ __device__ constexpr int persist_form_rows(int i) { return ((0x87858 >> (4 * i)) & 15) * 32; }  // bm
+__host__ __device__ constexpr int persist_form_tile(int i) {
+  return i == 0 ? EVEN_NONE : i == 1 ? EVEN_160x256 : i == 2 ? EVEN_256x256 : i == 3 ? EVEN_224x192 : EVEN_256x128;
+}
+// Time of a launch of form i with `row_tiles` row tiles of L rows together and `cols` column tiles, ns.  A round is a tile on every one
+// of the `slots`; a slice takes 0.35 us and 0.013 us for each 16 x 16 block of a wave, a tile's ends 1.5 us and 0.035 us for each;
+// the last round is as long as the plan's cut along K leaves it.  The model orders the forms as they were measured, and is within a
+// fifth of most times.  Every workgroup of a launch, and the one that finishes its cut tiles, has to come to the same result: one
+// rounding for each operation.
+__host__ __device__ inline float persist_time(const GemmArgs& a, int form, int i, uint32_t L, uint32_t row_tiles, uint32_t cols,
+                                              uint32_t slots) {
+#pragma clang fp contract(off)
+  const uint32_t slices = ((uint32_t)a.K + 63) / 64;
+  const float nk = slices < 2 ? 2.0f : (float)slices, blocks_of_a_pair = (float)persist_form_blocks(i);
+  const float ends = nk * 350.0f + 1500.0f, pair = (nk * 13.0f + (form == PG_SWIGLU_KEEP ? 70.0f : 35.0f)) * blocks_of_a_pair;
+  const float loop = i == 0 ? 0.97f : 1.0f;  // (the first form's loop has no branches)
+  const float per_slot = 0.9999995f / (float)slots;  // (a quotient that is whole but for its rounding is whole)
+  // ---- so far what the experts' rows have no part in: computed while they are fetched
+  const float all = (float)row_tiles * (float)cols * per_slot;
+  float rounds = ceilf(all);
+  if (a.ws != nullptr && i == 0 && form != PG_SWIGLU_KEEP) {
+    const uint32_t tiles = row_tiles * cols, rem = tiles % slots, p = rem > 0 ? persist_parts((int)slots, (int)rem, (int)slices) : 1;
+    if (p > 1) rounds = rounds - 1.0f + 1.0f / (float)p;
+  }
+  // pairs of row blocks of an even tile of average height, four at least
+  const uint32_t most = (uint32_t)persist_form_rows(i) / 32, m = 32 * row_tiles;
+  uint32_t pairs = 4 + (L > 4 * m) + (L > 5 * m) + (L > 6 * m) + (L > 7 * m);
+  pairs = i == 0 || pairs > most ? most : pairs;
+  return rounds * ((ends + pair * (float)pairs) * loop);
+}
+// column tiles of tiles of 4 nb blocks
+__host__ __device__ inline uint32_t persist_cols(int N, int form, int nb) {
+  const uint32_t n = (uint32_t)N * (form == PG_SWIGLU || form == PG_SWIGLU_KEEP ? 2 : 1);
+  return nb == 8 ? (n + 255) / 256 : nb == 6 ? (n + 191) / 192 : (n + 127) / 128;
+}
+
 struct PgTile {
   int expert, nt, row_begin, row_end;
 };
@@ -96,28 +136,42 @@ __device__ __forceinline__ int pg_wave_scan(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31: into rows 2 and 3
   return v;
 }
-template <int BM> __device__ __forceinline__ void pg_table(const int32_t* __restrict__ off, int L, int E, PgTable& tb) {
+// Where an expert's rows begin and end, an expert to a lane of four registers
+struct PgRows {
+  int begin[4], end[4];
+};
+__device__ __forceinline__ PgRows pg_rows(const int32_t* __restrict__ off, int L, int E) {
   const int lane = threadIdx.x & 63;
-  int prev[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    tb.incl[c] = 0;
-    tb.end[c] = 0;
-    prev[c] = 0;
-    if (c * 64 >= E) continue;
+  PgRows r;
+  auto load = [&](int c) {
     const int e = c * 64 + lane;
-    if (e < E) tb.end[c] = mi_expert_end(off, L, e);
-    if (e < E && e > 0) prev[c] = off[e - 1];
+    if (e < E) r.end[c] = mi_expert_end(off, L, e);
+    if (e < E && e > 0) r.begin[c] = off[e - 1];
+  };
+#pragma unroll
+  for (int c = 0; c < 4; ++c) r.begin[c] = r.end[c] = 0;
+  load(0);
+  if (E > 64) {
+#pragma unroll
+    for (int c = 1; c < 4; ++c) load(c);
   }
-  int carry = 0;
+  return r;
+}
+template <int BM> __device__ __forceinline__ void pg_table(const PgRows& r, int E, PgTable& tb) {
+  auto tiles = [&](int c) { return pg_wave_scan((int)((uint32_t)(r.end[c] - r.begin[c] + BM - 1) / BM)); };
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    if (c * 64 >= E) continue;
-    const int n = c * 64 + lane < E ? (tb.end[c] - prev[c] + BM - 1) / BM : 0;
-    tb.incl[c] = pg_wave_scan(n) + carry;
-    carry = __builtin_amdgcn_readlane(tb.incl[c], 63);
+    tb.incl[c] = c == 0 ? tiles(0) : 0;
+    tb.end[c] = r.end[c];
   }
-  tb.total = carry;
+  tb.total = __builtin_amdgcn_readlane(tb.incl[0], 63);
+  if (E > 64) {
+#pragma unroll
+    for (int c = 1; c < 4; ++c) {
+      tb.incl[c] = tiles(c) + tb.total;
+      tb.total = __builtin_amdgcn_readlane(tb.incl[c], 63);
+    }
+  }
 }
 // The expert of a lane's row tile by binary search over the table's lanes: six exchanges, where the walk over the experts
 // that this replaces took 2.2 us of a launch with 40 of them (both projections of 40 experts, 1536 / 512, 2048 tokens 112 ->
@@ -174,6 +228,40 @@ template <int BM, bool EVEN = false> __device__ __forceinline__ PgTile pg_locate
     t.row_end = rend;
   }
   return t;
+}
+// The tiles that are the fastest for the experts' rows as they are: lane i has form i.  This is a chain in front of the launch's
+// first load: no division, no branch, 0.3 us of a launch (with whole numbers of 64 bits and a branch for every choice 0.8).
+__device__ __forceinline__ int pg_tiles_by_load(const GemmArgs& a, const PgRows& r, int form, int slots) {
+  const int lane = threadIdx.x & 63;
+  auto add = [&](int c, uint32_t (&n)[3]) {
+    const uint32_t rows = (uint32_t)(r.end[c] - r.begin[c]);
+    n[0] += (rows + 159) / 160;
+    n[1] += (rows + 223) / 224;
+    n[2] += (rows + 255) / 256;
+  };
+  uint32_t n[3] = {0, 0, 0};
+  add(0, n);
+  if (a.E > 64) {
+#pragma unroll
+    for (int c = 1; c < 4; ++c) add(c, n);
+  }
+#pragma unroll
+  for (int b = 0; b < 3; ++b) n[b] = (uint32_t)__builtin_amdgcn_readlane(pg_wave_scan((int)n[b]), 63);
+  const int i = lane < PERSIST_FORMS ? lane : 0, bm = persist_form_rows(i), nb = persist_form_blocks(i);
+  const uint32_t c8 = persist_cols(a.N, form, 8), c6 = persist_cols(a.N, form, 6), c4 = persist_cols(a.N, form, 4);
+  const float t = persist_time(a, form, i, a.L, bm == 160 ? n[0] : (bm == 224 ? n[1] : n[2]), nb == 8 ? c8 : (nb == 6 ? c6 : c4), slots);
+  int best = 0;
+  uint32_t least = 0;  // (positive floats are ordered as their bits)
+#pragma unroll
+  for (int j = 0; j < PERSIST_FORMS; ++j) {
+    if (form == PG_WEIGHT_KN && persist_form_blocks(j) != 8) continue;
+    const uint32_t tj = (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(t), j);
+    if (j == 0 || tj < least) {
+      least = tj;
+      best = j;
+    }
+  }
+  return persist_form_tile(best);
 }
 // pairs of 16-row blocks of a tile
 __device__ __forceinline__ int pg_row_pairs(const PgTile& t) { return (t.row_end - t.row_begin + 31) >> 5; }

@@ -363,7 +363,7 @@ def _gemm_workspace(device: torch.device, K: int, dtype: torch.dtype, enabled: b
 
 
 # forms of the persistent kernel (mi_moe_scattered_gemm_cfg)
-_PERSISTENT_CFGS = (7, 8, 9, 14, 15, 16, 18)
+_PERSISTENT_CFGS = (7, 8, 9, 14, 15, 16, 18, 19)
 
 
 def scattered_gemm(inputs: torch.Tensor, weight: torch.Tensor, k: int, sorted_scattered_idxs: torch.Tensor,
@@ -720,7 +720,7 @@ def up_swiglu_keep(x: torch.Tensor, w_fc: torch.Tensor, k: int, sorted_scattered
     """Up-projection for training: (act (L, I), h (L, 2I)) -- the activation and the pre-activation the backward
     needs.  One launch (mi_moe_up_swiglu_keep) where the persistent tile kernel takes the problem, else the grouped
     GEMM followed by the element-wise SwiGLU on the stored h; either way act is formed from the rounded h.
-    ``cfg``: that launch with the tiles named (7, 8, 9, 14, 15, 16 or 18 as in scattered_gemm), whatever the load."""
+    ``cfg``: that launch with the tiles named (7, 8, 9, 14, 15, 16, 18 or 19: mi_moe_scattered_gemm_cfg), whatever the load."""
     _dev(x, w_fc, sorted_scattered_idxs, expert_offsets)
     _no_grad(x, w_fc)
     x = x.contiguous()

@@ -215,8 +215,10 @@ int mi_moe_scattered_gemm_wt(const void* in, const void* w_kn, void* out, const 
  * with the tiles that its rule picks by the rows per expert; 8 / 9 = its 256x256 tiles with the order in which the XCDs
  * take them fixed to "each XCD a contiguous eighth of the tile list" / "consecutive 32-tile blocks of one chip-wide round"
  * (7 takes the second from 8 column tiles on); 14 / 15 / 16 / 18 = an expert's row tiles equally high and tiles of
- * 256x128 / 160x256 / 224x192 / 256x256.  7 .. 18 give the same bits, except where a call with a workspace cuts tiles along K
- * (mi_moe_scattered_gemm_ws; only 256x256 tiles of 7, 8 and 9): those add in another order.  4, 7 .. 9 and 14 .. 18 are
+ * 256x128 / 160x256 / 224x192 / 256x256; 19 = whichever of the last four or of 256x256 is the fastest for the experts' rows
+ * of the call, which the kernel finds out itself (7 leaves it to it, unless one is the fastest for any load of that size).
+ * 7 .. 19 give the same bits, except where a call with a workspace cuts tiles along K (mi_moe_scattered_gemm_ws; only the
+ * 256x256 tiles of 7, 8, 9 and 19): those add in another order.  4, 7 .. 9 and 14 .. 19 are
  * F16 / BF16 only.  100 + 10 r + w = the weight
  * stream for a few rows per expert (all three element types) with chunks of 16 r rows (r = 1, 2, 4) and w waves that
  * split the contraction (w = 1, 2, 4; r = 4: 1, 2); 100 = the stream in the form its own rule picks.  A configuration that
@@ -224,10 +226,12 @@ int mi_moe_scattered_gemm_wt(const void* in, const void* w_kn, void* out, const 
  * mi_moe_grouped_gemm_choice tells which of these numbers cfg -1 is for a problem with 16-byte aligned operands (glu: the
  * up-projection with SwiGLU, N = I), or returns the error code of a problem that none of them takes. */
 int mi_moe_grouped_gemm_choice(int L, int K, int N, int E, int glu, int dtype);
-/* Which tiles configuration 7 takes on the current device for a problem without a workspace: 14, 15, 16 or 18 as above, 0 for
- * its own 256x256.  form: 0 plain, 1 SwiGLU, 2 SwiGLU with the pre-activation, 3 transposed weights. */
+/* Which tiles are the fastest on the current device for L rows that scatter normally around L / E an expert, in a call without / with
+ * a workspace: 14, 15, 16 or 18 as above, 0 for 256x256.  form: 0 plain, 1 SwiGLU, 2 SwiGLU with the pre-activation, 3 transposed
+ * weights.  _load: what configuration 19 takes for the experts' rows that end at ends[e] (in host memory), ws: with a workspace. */
 int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form);
-int mi_moe_grouped_gemm_tile_choice_ws(int L, int K, int N, int E, int form);  /* ... for a call with a workspace */
+int mi_moe_grouped_gemm_tile_choice_ws(int L, int K, int N, int E, int form);
+int mi_moe_grouped_gemm_tile_choice_load(const int32_t* ends, int K, int N, int E, int form, int ws);
 int mi_moe_scattered_gemm_cfg(const void* in, const void* w, void* out, const int32_t* sorted_scattered,
                               const int32_t* expert_offsets, int L, int K, int N, int E, int k,
                               int grouped_in, int grouped_out, int dtype, int cfg, mi_moe_stream_t stream);
@@ -255,7 +259,7 @@ int mi_moe_scattered_gemm_ws(const void* in, const void* w, void* out, const int
 int mi_moe_scattered_gemm_wt_ws(const void* in, const void* w_kn, void* out, const int32_t* sorted_scattered,
                                 const int32_t* expert_offsets, int L, int K, int N, int E, int k, int grouped_in,
                                 int grouped_out, int dtype, void* ws, size_t ws_bytes, mi_moe_stream_t stream);
-/* ... with the tiles named: cfg 7 (-1: the same), 8, 9, 15 or 18 as above; MI_MOE_EUNSUPPORTED otherwise */
+/* ... with the tiles named: cfg 7 (-1: the same), 8, 9, 15, 18 or 19 as above; MI_MOE_EUNSUPPORTED otherwise */
 int mi_moe_scattered_gemm_wt_cfg(const void* in, const void* w_kn, void* out, const int32_t* sorted_scattered,
                                  const int32_t* expert_offsets, int L, int K, int N, int E, int k, int grouped_in,
                                  int grouped_out, int dtype, int cfg, void* ws, size_t ws_bytes, mi_moe_stream_t stream);
@@ -292,7 +296,7 @@ int mi_moe_up_swiglu_ws(const void* x, const void* w_fc, void* act_out, const in
 int mi_moe_up_swiglu_keep(const void* x, const void* w_fc, void* act_out, void* h_out, const int32_t* sorted_scattered,
                           const int32_t* expert_offsets, int L, int H, int I, int E, int k, int dtype,
                           mi_moe_stream_t stream);
-/* ... always the one launch, with the tiles named: cfg 7, 8, 9, 14, 15, 16 or 18 as above (-1: mi_moe_up_swiglu_keep), for any
+/* ... always the one launch, with the tiles named: cfg 7, 8, 9, 14, 15, 16, 18 or 19 as above (-1: mi_moe_up_swiglu_keep), for any
  * number of rows per expert and I < 2^22; MI_MOE_EUNSUPPORTED otherwise */
 int mi_moe_up_swiglu_keep_cfg(const void* x, const void* w_fc, void* act_out, void* h_out, const int32_t* sorted_scattered,
                               const int32_t* expert_offsets, int L, int H, int I, int E, int k, int dtype, int cfg,
