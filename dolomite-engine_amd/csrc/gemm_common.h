@@ -22,7 +22,7 @@ struct GemmArgs {
   int remap;    // XCD-aware tile order
   void* ws;     // persistent kernel: workspace for splitting the last round of tiles along K (or null)
   void* pre;    // persistent SwiGLU kernel: (L, 2N) pre-activation output next to the activation (or null)
-  int out_nt;   // persistent kernel: store the output non-temporal (set in run_gemm)
+  int out_nt;   // SwiGLU on 256 x 256 tiles, fp8 persistent tiles: store the output non-temporal (persistent_out_nt)
   uint32_t out_window;  // persistent kernel: rows of the output that 32-bit byte offsets reach (set by the launch)
   // fp8 weights (register-staged kernel, W8 form): w holds e4m3fn bytes, row-major (E, rows, K) or in the streamed-tile
   // layout of decode_fp8.hip; wscale (E, rows) fp32 is applied to the accumulators in the epilogue

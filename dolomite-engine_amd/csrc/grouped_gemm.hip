@@ -794,7 +794,7 @@ static int launch_dma(GemmArgs a, hipStream_t s) {
 // next to the weights it stays cached; beyond that it would not survive until it is read and only evicts the operands
 // on its way.  It matters little: up + down + combine 134 MB (32 experts, 16384 tokens) 426 / 431, 134 MB (40 experts) 603 / 605,
 // 235 MB (8 experts, I 14336) 2118 / 2135; 268 MB (16 experts, I 1024) 1358 / 1338, 268 MB (40 experts, 32768 tokens) 1154 / 1151,
-// 470 MB 4086 / 4073.
+// 470 MB 4086 / 4073.  Read by the 256 x 256 tiles' SwiGLU form and the fp8 tiles; the other forms have theirs compiled in.
 static int persistent_out_nt(const GemmArgs& a, bool glu, int elt) {
   if (!glu) return 1;
   return (double)a.L * a.N * elt > 192.0 * 1024 * 1024;
@@ -1063,7 +1063,6 @@ extern "C" int mi_moe_scattered_gemm_wt_cfg(const void* in, const void* w_kn, vo
   a.sorted_scattered = sorted_scattered; a.expert_offsets = expert_offsets;
   a.L = L; a.K = K; a.N = N; a.E = E; a.kdiv = k; a.n_tiles = 0;
   a.gather = !grouped_in; a.scatter = !grouped_out; a.remap = 1; a.ws = ws; a.pre = nullptr;
-  a.out_nt = persistent_out_nt(a, false, 2);
   if (!tiled_shape_ok(a, L, false, 2) || !mi_gemm_persistent_ok(a)) return MI_MOE_EUNSUPPORTED;
   if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
   return run_persistent(a, dtype, PG_WEIGHT_KN, cfg < 0 ? 7 : cfg, static_cast<hipStream_t>(stream));
@@ -1135,7 +1134,6 @@ extern "C" int mi_moe_up_swiglu_keep_cfg(const void* x, const void* w_fc, void* 
     if ((rc = run_gemm(a, dtype, false, -1, L, static_cast<hipStream_t>(stream))) != MI_MOE_OK) return rc;
     return mi_moe_swiglu_forward(pre_out, act_out, L, I, dtype, stream);
   }
-  a.out_nt = 0;
   return run_persistent(a, dtype, PG_SWIGLU_KEEP, cfg < 0 ? 7 : cfg, static_cast<hipStream_t>(stream));
 }
 

@@ -205,7 +205,7 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
 
   // One half slice: NB matrix instructions for each of the tile's 8 row blocks of a wave (EVEN: `pairs`).  B = 0: values [0, 32)
   // of slice k out of the registers read before, while values [32, 64) are read and W_k+2 is fetched; B = 1: those, while slice
-  // k + 1 is read and X_k+2 is fetched.  `hook` has two parts, the ring's rotation and
+  // k + 1 is read and X_k+2 (RING3: X_k+3) is fetched.  `hook` has two parts, the ring's rotation and
   // the next half's addresses: near the half's end, apart; EVEN, whose end a low tile leaves out: both behind the last read,
   // which is more than the issue slots that one matrix instruction leaves (with the plain form's there too, a layer of 8 experts,
   // 4096 / 14336, 8192 tokens: 4076 -> 4104 us).
