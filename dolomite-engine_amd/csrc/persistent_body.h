@@ -379,6 +379,8 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
     const auto srd = __builtin_amdgcn_make_buffer_rsrc(dst, (short)0, (int)((left < window ? left : window) * ld), 0x00020000);
     const uint32_t s0 = dma0 + p4;
     const int col0 = t.nt * BN + wn * WN;
+    uint32_t scr = scr_w;
+    asm volatile("" : "+v"(scr));                   // (or the addresses that it gives are kept in registers from the first tile on)
     // byte offsets of the wave's rows lane and 64 + lane, and of the lane's columns in store it (% CP); saturating sums keep what
     // does not exist past the buffer
     constexpr int CP = GLU ? 2 : 4;
@@ -416,7 +418,7 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
               v[i] = pg_acc(blk * 4 + i);
             }
           }
-          *(wp_t)(size_t)(s0 + (scr_w ^ (nb * 32)) + mbp * (16 / RPP) * 4096) =
+          *(wp_t)(size_t)(s0 + (scr ^ (nb * 32)) + mbp * (16 / RPP) * 4096) =
               (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
         }
       pg_own_agprs();
