@@ -4,6 +4,14 @@
 
 #include "common.h"
 
+// Tiles picked by the load: what the experts' rows have no part in (persist_cost)
+struct PersistCost {
+  float ends, pair;  // ns of a tile without its matrix instructions, and for a pair of row blocks and one of columns
+  float per_slot;    // rounds for a tile
+  int slots;
+  uint32_t cols8, cols6, cols4;  // column tiles of tiles of 32 x so many weight rows
+};
+
 struct GemmArgs {
   const void* in;
   const void* w;
@@ -28,6 +36,7 @@ struct GemmArgs {
   // layout of decode_fp8.hip; wscale (E, rows) fp32 is applied to the accumulators in the epilogue
   const float* wscale;
   int w_tiled;
+  PersistCost cost;
 };
 
 // ---- persistent_gemm.hip ---------------------------------------------------------------------------------------------

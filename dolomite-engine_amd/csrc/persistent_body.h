@@ -13,7 +13,8 @@
 // NT: results are stored non-temporal
 // NB: blocks of 16 weight rows of a wave (a tile has 4 NB).  EVEN: an expert's row tiles are equally high, in steps of 32 rows, and
 // a low tile costs what it has (pg_locate, half)
-template <typename T, bool GLU, bool WT, bool KEEP, bool NT, int NB = 8, bool EVEN = false, int BM = 256>
+// SCANNED: pg_form_by_load has summed up the row tiles
+template <typename T, bool GLU, bool WT, bool KEEP, bool NT, int NB = 8, bool EVEN = false, int BM = 256, bool SCANNED = false>
 __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows& experts) {
   static_assert(!KEEP || GLU, "the pre-activation belongs to the SwiGLU form");
   static_assert(!WT || !GLU, "transposed-weight form");
@@ -43,7 +44,7 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
 
   // ---- which tiles -----------------------------------------------------------------------------------------------
   PgTable tb;
-  pg_table<BM>(experts, a.E, tb);
+  pg_table<BM, SCANNED>(experts, a.E, tb);
   const int total = tb.total * a.n_tiles;
   const int nfull = a.K / PG_BK;                    // whole slices; a partial one is padded with zeros
   int nk = (a.K + PG_BK - 1) / PG_BK;
@@ -361,8 +362,9 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
   // forms the result from the ROUNDED halves, as the separate activation kernel forms it from the stored h.
   // Every tile issues the same number of stores on one path; what does not exist is a lane past the buffer.  With a branch for
   // edge tiles the compiler, which counts stores along the shortest way it can construct, waited for all of them wherever it
-  // needed the next tile's rows, and again in the next tile's first slice: 40 experts, 512 -> 1536, 32768 tokens 401 -> 390 us,
-  // 32 experts, 512 -> 1024, 16384 tokens 142 -> 139, 1536 -> 512 SwiGLU, 32768 tokens 613 -> 608.
+  // needed the next tile's rows, and again in the next tile's first slice: 40 experts, 512 -> 1536, 32768 tokens 389 -> 384 us (389
+  // again with the body as it is now), 32 experts, 512 -> 1024, 16384 tokens 139 -> 136, 1536 ->
+  // 512 SwiGLU, 32768 tokens 639 -> 622.
   // WHAT 0 writes the rows [row0, row0 + out_window) of the output: all of them, unless it has more than 4 GiB.
   auto epilogue_as = [&](auto what_tag, const PgTile& t, uint32_t row0) __attribute__((always_inline)) {
     constexpr int WHAT = decltype(what_tag)::value;
@@ -592,5 +594,6 @@ static inline int by_load_prepare(GemmArgs& a, int form, int* grid) {
     if (slots > *grid) *grid = slots;
   }
   if (!mi_gemm_persistent_splits(a.K) || *grid < 16 || form == PG_SWIGLU_KEEP) a.ws = nullptr;
+  a.cost = persist_cost(a, form, *grid);
   return MI_MOE_OK;
 }

@@ -6,9 +6,9 @@
 // (results stored non-temporal without the SwiGLU, cached with it, whatever their size: the 256 x 256 tiles store results beyond
 // 192 MB non-temporal, here it is the same within 0.3 %: 8 experts, 4096 / 14336, layer of 3600 / 4250 / 5000 tokens cached 1984 / 2423 /
 // 2571 us, non-temporal 1981 / 2418 / 2566)
-template <typename T, int FORM, int NB, int BM> __device__ __forceinline__ void even_body(const GemmArgs& a, const PgRows& experts) {
+template <typename T, int FORM, int NB, int BM, bool SCANNED = false> __device__ __forceinline__ void even_body(const GemmArgs& a, const PgRows& experts) {
   constexpr bool GLU = FORM == PG_SWIGLU || FORM == PG_SWIGLU_KEEP;
-  persistent_body<T, GLU, FORM == PG_WEIGHT_KN, FORM == PG_SWIGLU_KEEP, !GLU, NB, true, BM>(a, experts);
+  persistent_body<T, GLU, FORM == PG_WEIGHT_KN, FORM == PG_SWIGLU_KEEP, !GLU, NB, true, BM, SCANNED>(a, experts);
 }
 
 template <typename T, int FORM, int NB, int BM>

@@ -75,28 +75,34 @@ static RowTiles row_tiles_of(const GemmArgs& a, int n) {
   return r;
 }
 // The fastest form for so many row tiles; t: time of each
-static int form_of(const GemmArgs& a, int form, int slots, const RowTiles& r, float (&t)[PERSIST_FORMS]) {
+static int form_of(const GemmArgs& a, int form, const RowTiles& r, float (&t)[PERSIST_FORMS]) {
   int best = 0;
   for (int i = 0; i < PERSIST_FORMS; ++i) {
     if (form == PG_WEIGHT_KN && persist_form_blocks(i) != 8) continue;
-    t[i] = persist_time(a, form, i, a.L, r.of(i), persist_cols(a.N, form, persist_form_blocks(i)), slots);
+    t[i] = persist_time(a, form, i, r.of(i));
     if (t[i] < t[best]) best = i;
   }
   return best;
 }
 
-// The tiles that are the fastest whatever the load, as far as the model goes: 584 of 976 problems of 64 to 6000 tokens in 8 to 64
-// experts, among them all loads of many rounds.  For the others there is pg_tiles_by_load, which costs a launch 0.3 us.
+// The tiles that are the fastest, or hardly less, whatever the load, as far as the model goes: 732 of 976 problems of 64 to 6000 tokens
+// in 8 to 64 experts, among them all loads of many rounds.  For the others there is pg_form_by_load, which costs a launch 0.2 us, and
+// 1 us where its instructions come from memory: that is worth a loss of more than a twentieth over the loads or a fifth in one of
+// them (lines at 2 % in each: 584 problems, and 0.1 % faster as far as the pick itself goes; at 12 %: 708).
 int mi_gemm_tiles_of_any_load(const GemmArgs& args, int form) {
   GemmArgs a = args;
   int cus = 0;
   if (mi_cu_count(&cus) != MI_MOE_OK) return EVEN_NONE;
   if (!mi_gemm_persistent_splits(a.K)) a.ws = nullptr;
+  a.cost = persist_cost(a, form, cus);
   float t[PERSIST_FORMS];
-  const int best = form_of(a, form, cus, row_tiles_of(a, -1), t);
+  const int best = form_of(a, form, row_tiles_of(a, -1), t);
+  float loss = 0.0f;
   for (int n = 0; a.E > 1 && n < LoadShapes::N; ++n) {
-    const int other = form_of(a, form, cus, row_tiles_of(a, n), t);
-    if (t[best] > 1.02f * t[other]) return EVEN_BY_LOAD;
+    const int other = form_of(a, form, row_tiles_of(a, n), t);
+    const float more = t[best] / t[other] - 1.0f;
+    loss += more;
+    if (more > 0.2f || loss > 0.05f * (LoadShapes::N + 1)) return EVEN_BY_LOAD;
   }
   return persist_form_tile(best);
 }
@@ -107,8 +113,10 @@ static int tile_choice(int L, int K, int N, int E, int form, bool ws) {
   a.L = L; a.K = K; a.N = N; a.E = E;
   a.ws = ws && mi_gemm_persistent_splits(K) ? &a : nullptr;  // (whether there is one)
   int cus = 0;
+  if (mi_cu_count(&cus) != MI_MOE_OK) return EVEN_NONE;
+  a.cost = persist_cost(a, form, cus);
   float t[PERSIST_FORMS];
-  return mi_cu_count(&cus) != MI_MOE_OK ? EVEN_NONE : persist_form_tile(form_of(a, form, cus, row_tiles_of(a, -1), t));
+  return persist_form_tile(form_of(a, form, row_tiles_of(a, -1), t));
 }
 
 extern "C" int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, false); }
@@ -132,7 +140,7 @@ extern "C" int mi_moe_grouped_gemm_tile_choice_load(const int32_t* ends, int K, 
     r.n[2] += (uint32_t)mi_ceil_div(rows, 256);
   }
   float t[PERSIST_FORMS];
-  return persist_form_tile(form_of(a, form, slots, r, t));
+  return persist_form_tile(form_of(a, form, r, t));
 }
 
 int mi_gemm_even(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s) {

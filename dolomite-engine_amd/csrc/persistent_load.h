@@ -1,5 +1,5 @@
 // The persistent grouped GEMM with the tiles that the load on hand wants: every workgroup counts the row tiles that each form would
-// have, out of the experts' ends, and runs the form that persist_time finds the fastest (pg_tiles_by_load).  The host knows the
+// have, out of the experts' ends, and runs the form that persist_time finds the fastest (pg_form_by_load).  The host knows the
 // average of the experts' rows only, and that says little about how many tiles there are: a form picked for rows that scatter
 // around it goes into a second, nearly empty round as soon as a few experts have more of them.
 //
@@ -22,14 +22,14 @@
 
 template <typename T, int FORM, bool NT> __device__ __forceinline__ void whole_body(const GemmArgs& a, const PgRows& experts) {
   constexpr bool GLU = FORM == PG_SWIGLU || FORM == PG_SWIGLU_KEEP;
-  persistent_body<T, GLU, FORM == PG_WEIGHT_KN, FORM == PG_SWIGLU_KEEP, NT>(a, experts);
+  persistent_body<T, GLU, FORM == PG_WEIGHT_KN, FORM == PG_SWIGLU_KEEP, NT, 8, false, 256, true>(a, experts);
 }
 
 template <typename T, int FORM> __global__ __launch_bounds__(256, 1) void grouped_gemm_by_load_kernel(GemmArgs a) {
   constexpr bool GLU = FORM == PG_SWIGLU || FORM == PG_SWIGLU_KEEP;
-  const PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
-  const int tile = pg_tiles_by_load(a, experts, FORM, gridDim.x);
-  if (tile == EVEN_NONE) {
+  PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
+  const int i = pg_form_by_load(a, experts, FORM);
+  if (i == 0) {
     if constexpr (FORM == PG_SWIGLU) {
       if (a.out_nt) whole_body<T, FORM, true>(a, experts);
       else whole_body<T, FORM, false>(a, experts);
@@ -39,19 +39,17 @@ template <typename T, int FORM> __global__ __launch_bounds__(256, 1) void groupe
     return;
   }
   a.ws = nullptr;
-  auto as = [&](auto nb_tag, auto bm_tag) __attribute__((always_inline)) {
-    constexpr int NB = decltype(nb_tag)::value, BM = decltype(bm_tag)::value;
-    persistent_columns(a, (GLU ? 16 : 32) * NB);
-    even_body<T, FORM, NB, BM>(a, experts);
+  auto as = [&](auto itag) __attribute__((always_inline)) {
+    constexpr int I = decltype(itag)::value, NB = persist_form_blocks(I);
+    if constexpr (FORM != PG_WEIGHT_KN || NB == 8) {
+      persistent_columns(a, (GLU ? 16 : 32) * NB);
+      even_body<T, FORM, NB, persist_form_rows(I), true>(a, experts);
+    }
   };
-#define PG_C(v) std::integral_constant<int, (v)>{}
-  if (tile == EVEN_160x256) as(PG_C(8), PG_C(160));
-  if (tile == EVEN_256x256) as(PG_C(8), PG_C(256));
-  if constexpr (FORM != PG_WEIGHT_KN) {
-    if (tile == EVEN_224x192) as(PG_C(6), PG_C(224));
-    if (tile == EVEN_256x128) as(PG_C(4), PG_C(256));
-  }
-#undef PG_C
+  if (i == 1) as(std::integral_constant<int, 1>{});
+  else if (i == 2) as(std::integral_constant<int, 2>{});
+  else if (i == 3) as(std::integral_constant<int, 3>{});
+  else as(std::integral_constant<int, 4>{});
 }
 
 template <typename T, int FORM> static int launch_by_load(GemmArgs a, hipStream_t s) {

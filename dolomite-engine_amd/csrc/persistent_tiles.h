@@ -80,36 +80,44 @@ __host__ __device__ constexpr int persist_form_rows(int i) { return ((0x87858 >>
 __host__ __device__ constexpr int persist_form_tile(int i) {
   return i == 0 ? EVEN_NONE : i == 1 ? EVEN_160x256 : i == 2 ? EVEN_256x256 : i == 3 ? EVEN_224x192 : EVEN_256x128;
 }
-// Time of a launch of form i with `row_tiles` row tiles of L rows together and `cols` column tiles, ns.  A round is a tile on every one
-// of the `slots`; a slice takes 0.35 us and 0.013 us for each 16 x 16 block of a wave, a tile's ends 1.5 us and 0.035 us for each;
-// the last round is as long as the plan's cut along K leaves it.  The model orders the forms as they were measured, and is within a
-// fifth of most times.  Every workgroup of a launch, and the one that finishes its cut tiles, has to come to the same result: one
-// rounding for each operation.
-__host__ __device__ inline float persist_time(const GemmArgs& a, int form, int i, uint32_t L, uint32_t row_tiles, uint32_t cols,
-                                              uint32_t slots) {
+// Time of a launch of form i with `row_tiles` row tiles of a.L rows together, ns.  A round is a tile on every slot; a slice takes
+// 0.35 us and 0.013 us for each 16 x 16 block of a wave, a tile's ends 1.5 us and 0.035 us for each; the last round is as long as the
+// plan's cut along K leaves it.  The model orders the forms as they were measured, and is within a fifth of most times.  Every
+// workgroup of a launch, and the one that finishes its cut tiles, has to come to the same result: one rounding for each operation.
+inline PersistCost persist_cost(const GemmArgs& a, int form, int slots) {
 #pragma clang fp contract(off)
-  const uint32_t slices = ((uint32_t)a.K + 63) / 64;
-  const float nk = slices < 2 ? 2.0f : (float)slices, blocks_of_a_pair = (float)persist_form_blocks(i);
-  const float ends = nk * 350.0f + 1500.0f, pair = (nk * 13.0f + (form == PG_SWIGLU_KEEP ? 70.0f : 35.0f)) * blocks_of_a_pair;
-  const float loop = i == 0 ? 0.97f : 1.0f;  // (the first form's loop has no branches)
-  const float per_slot = 0.9999995f / (float)slots;  // (a quotient that is whole but for its rounding is whole)
-  // ---- so far what the experts' rows have no part in: computed while they are fetched
-  const float all = (float)row_tiles * (float)cols * per_slot;
-  float rounds = ceilf(all);
-  if (a.ws != nullptr && i == 0 && form != PG_SWIGLU_KEEP) {
-    const uint32_t tiles = row_tiles * cols, rem = tiles % slots, p = rem > 0 ? persist_parts((int)slots, (int)rem, (int)slices) : 1;
-    if (p > 1) rounds = rounds - 1.0f + 1.0f / (float)p;
+  PersistCost c;
+  const float nk = a.K <= 2 * 64 ? 2.0f : (float)((a.K + 63) / 64);
+  c.ends = nk * 350.0f + 1500.0f;
+  c.pair = nk * 13.0f + (form == PG_SWIGLU_KEEP ? 70.0f : 35.0f);
+  c.slots = slots;
+  c.per_slot = 0.9999995f / (float)slots;  // (a quotient that is whole but for its rounding is whole)
+  const uint32_t n = (uint32_t)a.N * (form == PG_SWIGLU || form == PG_SWIGLU_KEEP ? 2 : 1);
+  c.cols8 = (n + 255) / 256;
+  c.cols6 = (n + 191) / 192;
+  c.cols4 = (n + 127) / 128;
+  return c;
+}
+__host__ __device__ inline float persist_time(const GemmArgs& a, int form, int i, uint32_t row_tiles) {
+#pragma clang fp contract(off)
+  const PersistCost c = a.cost;
+  const int nb = persist_form_blocks(i);
+  const uint32_t cols8 = c.cols8, cols6 = c.cols6, cols4 = c.cols4, L = (uint32_t)a.L;
+  const uint32_t cols = nb == 8 ? cols8 : (nb == 6 ? cols6 : cols4);
+  float rounds = ceilf((float)row_tiles * (float)cols * c.per_slot);
+  if (__builtin_expect(a.ws != nullptr, 0)) {
+    if (i == 0 && form != PG_SWIGLU_KEEP) {
+      const uint32_t rem = row_tiles * cols % (uint32_t)c.slots;
+      const int p = rem > 0 ? persist_parts(c.slots, (int)rem, (a.K + 63) / 64) : 1;
+      if (p > 1) rounds = rounds - 1.0f + 1.0f / (float)p;
+    }
   }
   // pairs of row blocks of an even tile of average height, four at least
   const uint32_t most = (uint32_t)persist_form_rows(i) / 32, m = 32 * row_tiles;
   uint32_t pairs = 4 + (L > 4 * m) + (L > 5 * m) + (L > 6 * m) + (L > 7 * m);
   pairs = i == 0 || pairs > most ? most : pairs;
-  return rounds * ((ends + pair * (float)pairs) * loop);
-}
-// column tiles of tiles of 4 nb blocks
-__host__ __device__ inline uint32_t persist_cols(int N, int form, int nb) {
-  const uint32_t n = (uint32_t)N * (form == PG_SWIGLU || form == PG_SWIGLU_KEEP ? 2 : 1);
-  return nb == 8 ? (n + 255) / 256 : nb == 6 ? (n + 191) / 192 : (n + 127) / 128;
+  const float loop = i == 0 ? 0.97f : 1.0f;  // (the first form's loop has no branches)
+  return rounds * ((c.ends + c.pair * (float)(pairs * (uint32_t)nb)) * loop);
 }
 
 struct PgTile {
@@ -139,6 +147,7 @@ __device__ __forceinline__ int pg_wave_scan(int v) {
 // Where an expert's rows begin and end, an expert to a lane of four registers
 struct PgRows {
   int begin[4], end[4];
+  int scan[3];  // pg_form_by_load: row tiles of 160, 224 and 256 rows of the first 64 experts, summed up to the lane's
 };
 __device__ __forceinline__ PgRows pg_rows(const int32_t* __restrict__ off, int L, int E) {
   const int lane = threadIdx.x & 63;
@@ -157,13 +166,14 @@ __device__ __forceinline__ PgRows pg_rows(const int32_t* __restrict__ off, int L
   }
   return r;
 }
-template <int BM> __device__ __forceinline__ void pg_table(const PgRows& r, int E, PgTable& tb) {
+template <int BM, bool SCANNED = false> __device__ __forceinline__ void pg_table(const PgRows& r, int E, PgTable& tb) {
   auto tiles = [&](int c) { return pg_wave_scan((int)((uint32_t)(r.end[c] - r.begin[c] + BM - 1) / BM)); };
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    tb.incl[c] = c == 0 ? tiles(0) : 0;
+    tb.incl[c] = 0;
     tb.end[c] = r.end[c];
   }
+  tb.incl[0] = SCANNED ? r.scan[BM == 160 ? 0 : (BM == 224 ? 1 : 2)] : tiles(0);
   tb.total = __builtin_amdgcn_readlane(tb.incl[0], 63);
   if (E > 64) {
 #pragma unroll
@@ -229,27 +239,30 @@ template <int BM, bool EVEN = false> __device__ __forceinline__ PgTile pg_locate
   }
   return t;
 }
-// The tiles that are the fastest for the experts' rows as they are: lane i has form i.  This is a chain in front of the launch's
-// first load: no division, no branch, 0.3 us of a launch (with whole numbers of 64 bits and a branch for every choice 0.8).
-__device__ __forceinline__ int pg_tiles_by_load(const GemmArgs& a, const PgRows& r, int form, int slots) {
+// The form that is the fastest for the experts' rows as they are: lane i has form i.  This is a chain in front of the launch's
+// first load, and its instructions come from memory where a layer's weights have gone through the caches, so it is kept short: no
+// division, no branch, what is the load's only, and the sums are the tile table's too.  Whole numbers of 64 bits and a branch for every
+// choice took 0.8 us of a launch, floats with the host's part among them 0.4, this 0.2; with cold caches the last two 1.1 - 1.5 and
+// 0 - 1.6.
+__device__ __forceinline__ int pg_form_by_load(const GemmArgs& a, PgRows& r, int form) {
   const int lane = threadIdx.x & 63;
-  auto add = [&](int c, uint32_t (&n)[3]) {
+  uint32_t n[3];
+  auto tiles = [&](int c, int b) {
     const uint32_t rows = (uint32_t)(r.end[c] - r.begin[c]);
-    n[0] += (rows + 159) / 160;
-    n[1] += (rows + 223) / 224;
-    n[2] += (rows + 255) / 256;
+    return b == 0 ? (rows + 159) / 160 : (b == 1 ? (rows + 223) / 224 : (rows + 255) / 256);
   };
-  uint32_t n[3] = {0, 0, 0};
-  add(0, n);
-  if (a.E > 64) {
 #pragma unroll
-    for (int c = 1; c < 4; ++c) add(c, n);
+  for (int b = 0; b < 3; ++b) {
+    r.scan[b] = pg_wave_scan((int)tiles(0, b));
+    n[b] = (uint32_t)__builtin_amdgcn_readlane(r.scan[b], 63);
   }
+  if (__builtin_expect(a.E > 64, 0)) {
 #pragma unroll
-  for (int b = 0; b < 3; ++b) n[b] = (uint32_t)__builtin_amdgcn_readlane(pg_wave_scan((int)n[b]), 63);
-  const int i = lane < PERSIST_FORMS ? lane : 0, bm = persist_form_rows(i), nb = persist_form_blocks(i);
-  const uint32_t c8 = persist_cols(a.N, form, 8), c6 = persist_cols(a.N, form, 6), c4 = persist_cols(a.N, form, 4);
-  const float t = persist_time(a, form, i, a.L, bm == 160 ? n[0] : (bm == 224 ? n[1] : n[2]), nb == 8 ? c8 : (nb == 6 ? c6 : c4), slots);
+    for (int b = 0; b < 3; ++b)
+      n[b] += (uint32_t)__builtin_amdgcn_readlane(pg_wave_scan((int)(tiles(1, b) + tiles(2, b) + tiles(3, b))), 63);
+  }
+  const int i = lane < PERSIST_FORMS ? lane : 0, bm = persist_form_rows(i);
+  const float t = persist_time(a, form, i, bm == 160 ? n[0] : (bm == 224 ? n[1] : n[2]));
   int best = 0;
   uint32_t least = 0;  // (positive floats are ordered as their bits)
 #pragma unroll
@@ -261,7 +274,7 @@ __device__ __forceinline__ int pg_tiles_by_load(const GemmArgs& a, const PgRows&
       best = j;
     }
   }
-  return persist_form_tile(best);
+  return __builtin_amdgcn_readfirstlane(best);
 }
 // pairs of 16-row blocks of a tile
 __device__ __forceinline__ int pg_row_pairs(const PgTile& t) { return (t.row_end - t.row_begin + 31) >> 5; }

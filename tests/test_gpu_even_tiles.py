@@ -79,13 +79,15 @@ def test_even_training_forms(device, dtype, rows, E, K, N, tile, tile_kn):
     choice = _lib.load().mi_moe_grouped_gemm_tile_choice
     print(f"even training rows={rows} E={E} K={K} N={N}: {choice(L, K, N, E, KEEP)}, {choice(L, K, 2 * N, E, WEIGHT_KN)}", flush=True)
     assert (choice(L, K, N, E, KEEP), choice(L, K, 2 * N, E, WEIGHT_KN)) == (tile, tile_kn)
-    act, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off)
     plain = ops.scattered_gemm(by_slot, w, 1, ss, off, False, True, cfg=8)
-    assert torch.equal(h, plain)
-    torch.testing.assert_close(h.float(), ref, **TOL[dtype])
-    want = h.float()[:, :N] * torch.nn.functional.silu(h.float()[:, N:])  # (one rounding, and the rounded halves are exact)
-    torch.testing.assert_close(act.float(), want, rtol=TOL[dtype]["rtol"], atol=TOL[dtype]["atol"])
-    assert torch.equal(ops.scattered_gemm(x, w.transpose(1, 2).contiguous(), 1, ss, off, True, True, weight_kn=True), plain)
+    torch.testing.assert_close(plain.float(), ref, **TOL[dtype])
+    want = plain.float()[:, :N] * torch.nn.functional.silu(plain.float()[:, N:])  # (one rounding, and the rounded halves are exact)
+    w_kn = w.transpose(1, 2).contiguous()
+    for cfg, cfg_kn in ((-1, -1), (tile, tile_kn)):  # by the rule, and the tiles that it names for an even load
+        act, h = ops.up_swiglu_keep(by_slot, w, 1, ss, off, cfg=cfg)
+        assert torch.equal(h, plain)
+        torch.testing.assert_close(act.float(), want, rtol=TOL[dtype]["rtol"], atol=TOL[dtype]["atol"])
+        assert torch.equal(ops.scattered_gemm(x, w_kn, 1, ss, off, True, True, cfg=cfg_kn, weight_kn=True), plain)
 
 
 def test_tile_choice_takes_no_time(device):
