@@ -4,12 +4,11 @@
 
 #include "common.h"
 
-// Tiles picked by the load: what the experts' rows have no part in (persist_cost)
+// Tiles picked by the load: what the experts' rows have no part in (persist_cost; with it goes n_tiles, of the first form)
 struct PersistCost {
   float ends, pair;  // ns of a tile without its matrix instructions, and for a pair of row blocks and one of columns
   float per_slot;    // rounds for a tile
-  int slots;
-  uint32_t cols8, cols6, cols4;  // column tiles of tiles of 32 x so many weight rows
+  uint32_t cols6;    // column tiles of tiles of 192 weight rows
 };
 
 struct GemmArgs {
@@ -34,9 +33,15 @@ struct GemmArgs {
   uint32_t out_window;  // persistent kernel: rows of the output that 32-bit byte offsets reach (set by the launch)
   // fp8 weights (register-staged kernel, W8 form): w holds e4m3fn bytes, row-major (E, rows, K) or in the streamed-tile
   // layout of decode_fp8.hip; wscale (E, rows) fp32 is applied to the accumulators in the epilogue
-  const float* wscale;
-  int w_tiled;
-  PersistCost cost;
+  // (16-bit weights: the costs in their place.  The arguments fill two lines of 64 bytes with what the compiler adds to them; a third,
+  // fetched by every launch, cost 0.2 us of it)
+  union {
+    struct {
+      const float* wscale;
+      int w_tiled;
+    };
+    PersistCost cost;
+  };
 };
 
 // ---- persistent_gemm.hip ---------------------------------------------------------------------------------------------

@@ -594,6 +594,6 @@ static inline int by_load_prepare(GemmArgs& a, int form, int* grid) {
     if (slots > *grid) *grid = slots;
   }
   if (!mi_gemm_persistent_splits(a.K) || *grid < 16 || form == PG_SWIGLU_KEEP) a.ws = nullptr;
-  a.cost = persist_cost(a, form, *grid);
+  persist_cost(a, form, *grid);
   return MI_MOE_OK;
 }

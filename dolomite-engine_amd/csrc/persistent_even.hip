@@ -75,11 +75,11 @@ static RowTiles row_tiles_of(const GemmArgs& a, int n) {
   return r;
 }
 // The fastest form for so many row tiles; t: time of each
-static int form_of(const GemmArgs& a, int form, const RowTiles& r, float (&t)[PERSIST_FORMS]) {
+static int form_of(const GemmArgs& a, int form, int slots, const RowTiles& r, float (&t)[PERSIST_FORMS]) {
   int best = 0;
   for (int i = 0; i < PERSIST_FORMS; ++i) {
     if (form == PG_WEIGHT_KN && persist_form_blocks(i) != 8) continue;
-    t[i] = persist_time(a, form, i, r.of(i));
+    t[i] = persist_time(a, form, i, r.of(i), slots);
     if (t[i] < t[best]) best = i;
   }
   return best;
@@ -94,12 +94,12 @@ int mi_gemm_tiles_of_any_load(const GemmArgs& args, int form) {
   int cus = 0;
   if (mi_cu_count(&cus) != MI_MOE_OK) return EVEN_NONE;
   if (!mi_gemm_persistent_splits(a.K)) a.ws = nullptr;
-  a.cost = persist_cost(a, form, cus);
+  persist_cost(a, form, cus);
   float t[PERSIST_FORMS];
-  const int best = form_of(a, form, row_tiles_of(a, -1), t);
+  const int best = form_of(a, form, cus, row_tiles_of(a, -1), t);
   float loss = 0.0f;
   for (int n = 0; a.E > 1 && n < LoadShapes::N; ++n) {
-    const int other = form_of(a, form, row_tiles_of(a, n), t);
+    const int other = form_of(a, form, cus, row_tiles_of(a, n), t);
     const float more = t[best] / t[other] - 1.0f;
     loss += more;
     if (more > 0.2f || loss > 0.05f * (LoadShapes::N + 1)) return EVEN_BY_LOAD;
@@ -114,9 +114,9 @@ static int tile_choice(int L, int K, int N, int E, int form, bool ws) {
   a.ws = ws && mi_gemm_persistent_splits(K) ? &a : nullptr;  // (whether there is one)
   int cus = 0;
   if (mi_cu_count(&cus) != MI_MOE_OK) return EVEN_NONE;
-  a.cost = persist_cost(a, form, cus);
+  persist_cost(a, form, cus);
   float t[PERSIST_FORMS];
-  return persist_form_tile(form_of(a, form, row_tiles_of(a, -1), t));
+  return persist_form_tile(form_of(a, form, cus, row_tiles_of(a, -1), t));
 }
 
 extern "C" int mi_moe_grouped_gemm_tile_choice(int L, int K, int N, int E, int form) { return tile_choice(L, K, N, E, form, false); }
@@ -140,7 +140,7 @@ extern "C" int mi_moe_grouped_gemm_tile_choice_load(const int32_t* ends, int K, 
     r.n[2] += (uint32_t)mi_ceil_div(rows, 256);
   }
   float t[PERSIST_FORMS];
-  return persist_form_tile(form_of(a, form, r, t));
+  return persist_form_tile(form_of(a, form, slots, r, t));
 }
 
 int mi_gemm_even(const GemmArgs& a, int dtype, int form, int tile, hipStream_t s) {

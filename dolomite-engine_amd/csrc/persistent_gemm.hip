@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_split_finish_kernel(GemmArgs
   constexpr int BM = 256, BN = GLU ? 128 : 256;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
   PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
-  if (by_load_form >= 0 && pg_form_by_load(a, experts, by_load_form) != 0) return;
+  if (by_load_form >= 0 && pg_form_by_load(a, experts, by_load_form, 8 * nslot) != 0) return;
   PgTable tb;
   pg_table<BM>(experts, a.E, tb);
   // contiguous: workgroup b adds up tile b / 8 of XCD b % 8's last round; interleaved: tile b of the chip's last round

@@ -28,7 +28,7 @@ template <typename T, int FORM, bool NT> __device__ __forceinline__ void whole_b
 template <typename T, int FORM> __global__ __launch_bounds__(256, 1) void grouped_gemm_by_load_kernel(GemmArgs a) {
   constexpr bool GLU = FORM == PG_SWIGLU || FORM == PG_SWIGLU_KEEP;
   PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
-  const int i = pg_form_by_load(a, experts, FORM);
+  const int i = pg_form_by_load(a, experts, FORM, gridDim.x);
   if (i == 0) {
     if constexpr (FORM == PG_SWIGLU) {
       if (a.out_nt) whole_body<T, FORM, true>(a, experts);

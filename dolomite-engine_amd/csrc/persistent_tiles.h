@@ -84,31 +84,28 @@ __host__ __device__ constexpr int persist_form_tile(int i) {
 // 0.35 us and 0.013 us for each 16 x 16 block of a wave, a tile's ends 1.5 us and 0.035 us for each; the last round is as long as the
 // plan's cut along K leaves it.  The model orders the forms as they were measured, and is within a fifth of most times.  Every
 // workgroup of a launch, and the one that finishes its cut tiles, has to come to the same result: one rounding for each operation.
-inline PersistCost persist_cost(const GemmArgs& a, int form, int slots) {
+inline void persist_cost(GemmArgs& a, int form, int slots) {
 #pragma clang fp contract(off)
-  PersistCost c;
   const float nk = a.K <= 2 * 64 ? 2.0f : (float)((a.K + 63) / 64);
-  c.ends = nk * 350.0f + 1500.0f;
-  c.pair = nk * 13.0f + (form == PG_SWIGLU_KEEP ? 70.0f : 35.0f);
-  c.slots = slots;
-  c.per_slot = 0.9999995f / (float)slots;  // (a quotient that is whole but for its rounding is whole)
   const uint32_t n = (uint32_t)a.N * (form == PG_SWIGLU || form == PG_SWIGLU_KEEP ? 2 : 1);
-  c.cols8 = (n + 255) / 256;
-  c.cols6 = (n + 191) / 192;
-  c.cols4 = (n + 127) / 128;
-  return c;
+  a.n_tiles = (int)((n + 255) / 256);
+  a.cost.ends = nk * 350.0f + 1500.0f;
+  a.cost.pair = nk * 13.0f + (form == PG_SWIGLU_KEEP ? 70.0f : 35.0f);
+  a.cost.per_slot = 0.9999995f / (float)slots;  // (a quotient that is whole but for its rounding is whole)
+  a.cost.cols6 = (n + 191) / 192;
 }
-__host__ __device__ inline float persist_time(const GemmArgs& a, int form, int i, uint32_t row_tiles) {
+__host__ __device__ inline float persist_time(const GemmArgs& a, int form, int i, uint32_t row_tiles, int slots) {
 #pragma clang fp contract(off)
-  const PersistCost c = a.cost;
   const int nb = persist_form_blocks(i);
-  const uint32_t cols8 = c.cols8, cols6 = c.cols6, cols4 = c.cols4, L = (uint32_t)a.L;
+  const uint32_t n = (uint32_t)a.N * (form == PG_SWIGLU || form == PG_SWIGLU_KEEP ? 2 : 1), L = (uint32_t)a.L;
+  const uint32_t cols8 = (uint32_t)a.n_tiles, cols6 = a.cost.cols6, cols4 = (n + 127) / 128;
   const uint32_t cols = nb == 8 ? cols8 : (nb == 6 ? cols6 : cols4);
-  float rounds = ceilf((float)row_tiles * (float)cols * c.per_slot);
+  const float ends = a.cost.ends, pair = a.cost.pair, per_slot = a.cost.per_slot;
+  float rounds = ceilf((float)row_tiles * (float)cols * per_slot);
   if (__builtin_expect(a.ws != nullptr, 0)) {
     if (i == 0 && form != PG_SWIGLU_KEEP) {
-      const uint32_t rem = row_tiles * cols % (uint32_t)c.slots;
-      const int p = rem > 0 ? persist_parts(c.slots, (int)rem, (a.K + 63) / 64) : 1;
+      const uint32_t rem = row_tiles * cols % (uint32_t)slots;
+      const int p = rem > 0 ? persist_parts(slots, (int)rem, (a.K + 63) / 64) : 1;
       if (p > 1) rounds = rounds - 1.0f + 1.0f / (float)p;
     }
   }
@@ -117,7 +114,7 @@ __host__ __device__ inline float persist_time(const GemmArgs& a, int form, int i
   uint32_t pairs = 4 + (L > 4 * m) + (L > 5 * m) + (L > 6 * m) + (L > 7 * m);
   pairs = i == 0 || pairs > most ? most : pairs;
   const float loop = i == 0 ? 0.97f : 1.0f;  // (the first form's loop has no branches)
-  return rounds * ((c.ends + c.pair * (float)(pairs * (uint32_t)nb)) * loop);
+  return rounds * ((ends + pair * (float)(pairs * (uint32_t)nb)) * loop);
 }
 
 struct PgTile {
@@ -244,7 +241,7 @@ template <int BM, bool EVEN = false> __device__ __forceinline__ PgTile pg_locate
 // division, no branch, what is the load's only, and the sums are the tile table's too.  Whole numbers of 64 bits and a branch for every
 // choice took 0.8 us of a launch, floats with the host's part among them 0.4, this 0.2; with cold caches the last two 1.1 - 1.5 and
 // 0 - 1.6.
-__device__ __forceinline__ int pg_form_by_load(const GemmArgs& a, PgRows& r, int form) {
+__device__ __forceinline__ int pg_form_by_load(const GemmArgs& a, PgRows& r, int form, int slots) {
   const int lane = threadIdx.x & 63;
   uint32_t n[3];
   auto tiles = [&](int c, int b) {
@@ -262,7 +259,7 @@ __device__ __forceinline__ int pg_form_by_load(const GemmArgs& a, PgRows& r, int
       n[b] += (uint32_t)__builtin_amdgcn_readlane(pg_wave_scan((int)(tiles(1, b) + tiles(2, b) + tiles(3, b))), 63);
   }
   const int i = lane < PERSIST_FORMS ? lane : 0, bm = persist_form_rows(i);
-  const float t = persist_time(a, form, i, bm == 160 ? n[0] : (bm == 224 ? n[1] : n[2]));
+  const float t = persist_time(a, form, i, bm == 160 ? n[0] : (bm == 224 ? n[1] : n[2]), slots);
   int best = 0;
   uint32_t least = 0;  // (positive floats are ordered as their bits)
 #pragma unroll
