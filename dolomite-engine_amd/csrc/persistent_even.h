@@ -13,6 +13,7 @@ template <typename T, int FORM, int NB, int BM, bool SCANNED = false> __device__
 
 template <typename T, int FORM, int NB, int BM>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_even_kernel(GemmArgs a) {
+  pg_fetch_arguments(a);
   even_body<T, FORM, NB, BM>(a, pg_rows(a.expert_offsets, a.L, a.E));
 }
 

@@ -53,6 +53,7 @@ static bool persistent_may_split(int K) {
 
 template <typename T, bool GLU, bool WT, bool KEEP>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_persistent_kernel(GemmArgs a) {
+  pg_fetch_arguments(a);
   const PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
   if constexpr (!GLU) {
     persistent_body<T, GLU, WT, KEEP, true>(a, experts);

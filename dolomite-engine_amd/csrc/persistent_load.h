@@ -27,6 +27,7 @@ template <typename T, int FORM, bool NT> __device__ __forceinline__ void whole_b
 
 template <typename T, int FORM> __global__ __launch_bounds__(256, 1) void grouped_gemm_by_load_kernel(GemmArgs a) {
   constexpr bool GLU = FORM == PG_SWIGLU || FORM == PG_SWIGLU_KEEP;
+  pg_fetch_arguments(a);
   PgRows experts = pg_rows(a.expert_offsets, a.L, a.E);
   const int i = pg_form_by_load(a, experts, FORM, gridDim.x);
   if (i == 0) {

@@ -141,6 +141,12 @@ __device__ __forceinline__ int pg_wave_scan(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31: into rows 2 and 3
   return v;
 }
+// A launch's arguments requested at once.  Otherwise the compiler asks for each line of them where it first needs it, one trip after
+// the other: 40 experts, 1536 -> 512 SwiGLU, 2048 tokens, 160 x 256 tiles 59.5 -> 59.0 us.
+__device__ __forceinline__ void pg_fetch_arguments(const GemmArgs& a) {
+  asm volatile("" : : "s"(a.in), "s"(a.n_tiles), "s"(a.kdiv), "s"(a.scatter), "s"(a.out_window));
+}
+
 // Where an expert's rows begin and end, an expert to a lane of four registers
 struct PgRows {
   int begin[4], end[4];
