@@ -52,7 +52,7 @@ CUT = [([400, 401, 399, 400], 18), ([576, 406, 331, 287], 0), ([10, 20, 30, 1540
 
 
 @pytest.mark.parametrize("counts,pick", CUT)
-@pytest.mark.parametrize("form", [PLAIN, WEIGHT_KN])
+@pytest.mark.parametrize("form", [PLAIN, SWIGLU, WEIGHT_KN])
 def test_load_and_not_average_picks(device, counts, pick, form):
     """Four experts with 400 rows on average, 8192 -> 8192: where they all have about as many, the even tiles are one round; where two
     have more, 256 x 256 tiles whose second round is cut along K.  On average (what the host knows) it is the former."""
@@ -60,7 +60,8 @@ def test_load_and_not_average_picks(device, counts, pick, form):
 
     if torch.cuda.get_device_properties(device).multi_processor_count != 256:
         pytest.skip("the numbers are those of 256 CUs")
-    K = N = 8192
+    K = rows = 8192  # weight rows
+    N = rows // 2 if form == SWIGLU else rows
     L = sum(counts)
     assert _lib.load().mi_moe_grouped_gemm_tile_choice_ws(L, K, N, 4, form) == 18
     assert _pick(counts, K, N, form, 1) == pick
@@ -69,10 +70,15 @@ def test_load_and_not_average_picks(device, counts, pick, form):
     off = torch.tensor(counts).cumsum(0).int().to(device)
     ss = torch.randperm(L, generator=g, device=device).int()
     x = torch.empty(L, K, device=device, dtype=torch.bfloat16).normal_(generator=g)
-    w = torch.empty(4, N, K, device=device, dtype=torch.bfloat16).normal_(0.0, 0.02, generator=g)
+    w = torch.empty(4, rows, K, device=device, dtype=torch.bfloat16).normal_(0.0, 0.02, generator=g)
     if form == WEIGHT_KN:
         w = w.transpose(1, 2).contiguous()
-    run = lambda cfg: ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=cfg, weight_kn=form == WEIGHT_KN)
+
+    def run(cfg):
+        if form == SWIGLU:
+            return ops.up_swiglu(x, w, 1, ss, off, cfg=cfg)
+        return ops.scattered_gemm(x, w, 1, ss, off, True, False, cfg=cfg, weight_kn=form == WEIGHT_KN)
+
     whole, cut = run(18), run(9)
     assert torch.equal(whole, cut) == (pick == 18)
     for cfg in (7, 19):
