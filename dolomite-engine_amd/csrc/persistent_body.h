@@ -26,9 +26,9 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
   constexpr uint32_t XU = BM * 128, WU = NB * 4096;
   constexpr bool RING3 = 3 * (XU + WU) <= PG_LDS;
   static_assert(RING3 || BM == 256, "");
-  constexpr int PIECES = NB == 8 ? 8 : 4;           // pieces of a unit of weights that the epilogue uses as scratch
-  constexpr int PASS_ROWS = PIECES * (GLU ? 8 : 4), NPASS = (16 * NX + PASS_ROWS - 1) / PASS_ROWS;
-  constexpr int NSTORE = (KEEP ? 3 : 1) * NPASS * PIECES;  // stores of a wave in the epilogue
+  constexpr int PIECES = NB == 8 ? 8 : 4;           // plain form: pieces of a unit of weights that the epilogue uses as scratch
+  constexpr int NSTORE = GLU ? (KEEP ? 3 : 1) * NX * ((NB / 2 + 1) / 2) : (16 * NX + 4 * PIECES - 1) / (4 * PIECES) * PIECES;  // stores of a wave in the epilogue
+  static_assert(NB + (RING3 ? NX : 0) + NSTORE < 64, "a wait counts them all");
   constexpr int MINK = RING3 ? 3 : 2;               // slices of a tile at least
   constexpr int WN = BN / 2, HB = NB / 2;           // ... per wave; SwiGLU: blocks of up, then as many of gate
   typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
@@ -83,6 +83,16 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
   // order, so the swizzle is applied on the global side: lane l fetches chunk (l % 8) ^ ((r >> 1) & 7).
   const int drow = wave * 8 + (lane >> 3);          // row of instruction 0 (instruction j: + 32 j)
   const int lchunk = (lane & 7) ^ ((wave & 1) * 4 + (lane >> 4));
+  // SwiGLU weights: row 8 g + 4 wn + i of the 32 of group nb is what wave column wn multiplies as row 4 g + i of its block nb, and
+  // the blocks share out the wave's columns so that the accumulators of blocks 2 p and 2 p + 1 are eight neighbours of a row (w_row):
+  // results go from registers to memory in 16-byte stores.  Chunks at chunk ^ ((r >> 1) & 1 | (r >> 3) << 1), which again serves
+  // the 16 rows x 4 chunks of a fragment without bank conflicts.
+  const int wchunk = GLU ? (lane & 7) ^ ((wave << 1) | ((lane >> 4) & 1)) : lchunk;
+  auto w_row = [&](int nb) {                        // of the tile's up or gate half, for group nb's row 8 wave + lane / 8
+    const int h = nb % HB, i = (lane >> 3) & 3;
+    const bool paired = h + 1 < HB || h % 2 == 1;
+    return (lane >> 5) * WN + (paired ? 32 * (h / 2) + 8 * wave + 4 * (h % 2) : 16 * h + 4 * wave) + i;
+  };
   const uint32_t row_bytes = (uint32_t)a.K * 2u;
   const u32x4 xsrd = pg_srd(a.in, (uint64_t)(a.gather ? a.L / a.kdiv : a.L) * row_bytes);
   const uint64_t w_bytes = (uint64_t)a.E * (GLU ? 2 : 1) * a.N * row_bytes;
@@ -127,31 +137,34 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
         const int r = 8 * j + 2 * wave + (lane >> 5), f = (r & 3) | ((j & 3) << 2);
         woff[j] = ((uint32_t)r * a.N + ((((lane & 31) >> 1) ^ f) << 4) + (lane & 1) * 8) * 2u;
       } else {
-        const int r = GLU ? 32 * (j % HB) + (j >= HB ? a.N : 0) : 32 * j;
-        woff[j] = (uint32_t)(r + drow) * row_bytes + lchunk * 16u;
+        const int r = GLU ? w_row(j) + (j >= HB ? a.N : 0) : 32 * j + drow;
+        woff[j] = (uint32_t)r * row_bytes + wchunk * 16u;
       }
     }
   };
   const uint32_t w_step = WT ? (uint32_t)a.N * (2u * PG_BK) : 2u * PG_BK;  // bytes from slice to slice
   // a slice with fewer than 64 values: the lanes past them fetch zeros
-  auto mask_x = [&](auto& off, int k) {
-    const bool gone = lchunk * 8 >= a.K - k * PG_BK;
+  auto mask = [&](auto& off, int chunk, int k) {
+    const bool gone = chunk * 8 >= a.K - k * PG_BK;
     for (uint32_t& o : off) o = gone ? PG_OOB : o;
   };
+  auto mask_x = [&](auto& off, int k) { mask(off, lchunk, k); };
   auto mask_w = [&](int k) {
     if constexpr (WT) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) woff[j] = 8 * j + 2 * wave + (lane >> 5) >= a.K - k * PG_BK ? PG_OOB : woff[j];
     } else {
-      mask_x(woff, k);
+      mask(woff, wchunk, k);
     }
   };
 
   // ---- fragment reads ------------------------------------------------------------------------------------------------
   const uint32_t fswz = (frow >> 1) & 7;
   // (EVEN: the two waves of a column take row blocks in turn, so that they share a low tile)
-  const uint32_t fx = (wm * (EVEN ? 16 : 128) + frow) * 128, fw = (wn * WN + frow) * 128;
+  const uint32_t fx = (wm * (EVEN ? 16 : 128) + frow) * 128, fw = (GLU ? 8 * (frow >> 2) + 4 * wn + (frow & 3) : wn * WN + frow) * 128;
   const uint32_t fc0 = lds0 + ((fq ^ fswz) * 16), fc1 = lds0 + (((fq + 4) ^ fswz) * 16);
+  const uint32_t fwswz = GLU ? ((frow >> 1) & 1) | ((frow >> 2) << 1) : fswz;
+  const uint32_t fcw0 = lds0 + ((fq ^ fwswz) * 16), fcw1 = lds0 + (((fq + 4) ^ fwswz) * 16);
   // WT: ds_read_b64_tr_b16 transposes 4 rows x 16 columns across 16 lanes: lane i of the group supplies the address of
   // (row i / 4, columns 4 (i % 4) ..) and receives column i of the four rows.  Lane group q reads rows 8q .. 8q + 3 and,
   // 2 KiB further, 8q + 4 .. 8q + 7: together the 8 contraction values the matrix instruction wants.
@@ -165,7 +178,7 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
       return __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     } else {
       typedef __attribute__((address_space(3))) const u32x4* p;
-      return *(p)(size_t)(base + (GLU && nb >= HB ? HB * 4096 + (nb - HB) * 2048 : nb * 2048));
+      return *(p)(size_t)(base + nb * (GLU ? 4096 : 2048));
     }
   };
   auto read_x = [&](uint32_t base, int mb) -> u32x4 {
@@ -294,7 +307,7 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
 #undef PG_C
   };
   auto read_bases = [&](int ks, uint32_t ps_w, uint32_t ps_x) {
-    rw = WT ? lds0 + ps_w : (ks ? fc1 : fc0) + fw + ps_w;
+    rw = WT ? lds0 + ps_w : (ks ? fcw1 : fcw0) + fw + ps_w;
     rx = (ks ? fc1 : fc0) + fx + ps_x;
     asm volatile("" : "+v"(rx));
     if constexpr (!WT) asm volatile("" : "+v"(rw));
@@ -333,18 +346,8 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
     });
   };
 
-  // ---- epilogue: accumulators -> (SwiGLU) -> the wave's pieces of the free ring unit -> 16-byte stores ------------------
-  // Plain: four passes of 32 rows x 128 columns (256-byte rows, 4 to a piece); SwiGLU: two of 64 rows x 64 columns.
-  // Chunk c of scratch row r lies at slot c ^ (r % 16) (SwiGLU: c ^ (r / 2 % 8)): writes and reads free of conflicts,
-  // and the read-back is linear in the lane.
+  // ---- epilogue: accumulators -> (SwiGLU) -> 16-byte stores --------------------------------------------------------------
   T* __restrict__ out = static_cast<T*>(a.out);
-  constexpr int SB = GLU ? 128 : 256;               // bytes of a scratch row
-  constexpr int RPP = 1024 / SB;                    // scratch rows per piece and per store instruction
-  constexpr int MBP = PASS_ROWS / 16, NBO = GLU ? HB : NB;
-  const uint32_t scr_swz = GLU ? (frow >> 1) & 7 : frow;
-  const uint32_t scr_w = (frow / RPP) * 4096 + (frow % RPP) * SB + (((fq >> 1) ^ scr_swz) * 16) + (fq & 1) * 8;
-  const int srow = lane / (SB / 16), sslot = lane % (SB / 16);
-  const int scc0 = GLU ? sslot ^ ((srow >> 1) & 7) : sslot ^ (srow & 15);  // chunk of store 0; store it: ^ 4 (it % ..)
   // rows lane and 64 + lane of the wave's 128 in the tile
   constexpr int TILE_64 = EVEN ? 128 : 64;
   const int tile_row0 = EVEN ? (lane >> 4) * 32 + wm * 16 + (lane & 15) : wm * 128 + lane;
@@ -358,41 +361,154 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
       hi = a.sorted_scattered[hi < t.row_end ? hi : t.row_end - 1];
     }
   };
-  // WHAT: 0 the kernel's result (SwiGLU: up * silu(gate)); 1 / 2 (KEEP): the up / the gate half of h, into a.pre.  KEEP
-  // forms the result from the ROUNDED halves, as the separate activation kernel forms it from the stored h.
   // Every tile issues the same number of stores on one path; what does not exist is a lane past the buffer.  With a branch for
   // edge tiles the compiler, which counts stores along the shortest way it can construct, waited for all of them wherever it
   // needed the next tile's rows, and again in the next tile's first slice: 40 experts, 512 -> 1536, 32768 tokens 389 -> 384 us (389
   // again with the body as it is now), 32 experts, 512 -> 1024, 16384 tokens 139 -> 136, 1536 ->
   // 512 SwiGLU, 32768 tokens 639 -> 622.
-  // WHAT 0 writes the rows [row0, row0 + out_window) of the output: all of them, unless it has more than 4 GiB.
-  auto epilogue_as = [&](auto what_tag, const PgTile& t, uint32_t row0) __attribute__((always_inline)) {
-    constexpr int WHAT = decltype(what_tag)::value;
-    typedef __attribute__((address_space(3))) u32x2* wp_t;
-    typedef __attribute__((address_space(3))) const u32x4* rp_t;
-    const uint32_t ld = (WHAT == 0 ? a.N : 2 * a.N) * 2u;
+  // Writes the rows [row0, row0 + out_window) of the output: all of them, unless it has more than 4 GiB.
+  // SwiGLU: a lane holds eight neighbouring columns of row lane % 16 of a row block (see w_row), four lanes 64 bytes of it.  KEEP:
+  // the result is formed from the ROUNDED halves of the pre-activation, as the separate activation kernel forms it from the stored
+  // h, and both halves are stored in the same pass.
+  auto epilogue_direct = [&](const PgTile& t, uint32_t row0) __attribute__((always_inline)) {
+    const uint32_t ld = a.N * 2u;
+    const int behind = t.row_end - t.row_begin, rows = behind < BM ? behind : BM;
+    const uint32_t left = a.L - row0;
+    const auto srd = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char*>(out) + (uint64_t)row0 * ld, (short)0,
+                                                       (int)((left < a.out_window ? left : a.out_window) * ld), 0x00020000);
     // (rows of the pre-activation are the sorted order's: addressed from the tile's first, as the whole can exceed 4 GiB -- and so
     // can what an expert has behind a tile that is not EVEN, whose end is the expert's)
+    const auto pre = __builtin_amdgcn_make_buffer_rsrc(KEEP ? static_cast<unsigned char*>(a.pre) + (uint64_t)t.row_begin * (2 * ld) : nullptr,
+                                                       (short)0, KEEP && row0 == 0 ? (int)(rows * (2 * ld)) : 0, 0x00020000);
+    const uint32_t lo = (uint32_t)orow_lo - row0, hi = (uint32_t)orow_hi - row0;
+    const uint32_t rlo = tile_row0 < rows && lo < a.out_window ? lo * ld : PG_OOB;
+    const uint32_t rhi = tile_row0 + TILE_64 < rows && hi < a.out_window ? hi * ld : PG_OOB;
+    // Two pairs: lanes 8 .. 15 of a row block give their first eight columns to lanes 0 .. 7 for those lanes' second eight, so that a
+    // store instruction writes whole 128-byte lines of eight rows, and the next one those of the other eight.
+    // Byte offsets of the lane's columns in pair p (two pairs: in either store), and in the block without a partner; saturating
+    // sums keep what does not exist past the buffer
+    const int col0 = t.nt * BN + wn * WN;
+    constexpr int PAIRS = HB / 2, QUADS = EVEN ? 0 : PAIRS / 2, STORES = PAIRS + HB % 2;
+    uint32_t coff[STORES];
+#pragma unroll
+    for (int p = 0; p < STORES; ++p) {
+      const int col = col0 + (p < 2 * QUADS ? 64 * (p / 2) + 32 * (frow >> 3) : 32 * p) + (p < PAIRS ? 8 : 4) * fq;
+      coff[p] = col < a.N ? (uint32_t)col * 2u : PG_OOB;
+    }
+#pragma unroll
+    for (int mb = 0; mb < NX; ++mb) {
+      if (EVEN && mb * 32 >= rows) break;
+      // where the row block's rows go: lane's own row, and rows frow % 8 and 8 + frow % 8
+      auto row_of = [&](int r) { return (uint32_t)__builtin_amdgcn_ds_bpermute((((mb * 16) & 63) + r) * 4, (int)(mb < 4 ? rlo : rhi)); };
+      auto pre_of = [&](int r) {
+        const int prow = EVEN ? 32 * mb + 16 * wm + r : 128 * wm + 16 * mb + r;
+        return KEEP && prow < rows ? (uint32_t)prow * (2 * ld) : PG_OOB;
+      };
+      uint32_t roff[3] = {}, poff[3] = {};
+      if (QUADS > 0) {
+        roff[0] = row_of(frow & 7);
+        roff[1] = row_of(8 + (frow & 7));
+        poff[0] = pre_of(frow & 7);
+        poff[1] = pre_of(8 + (frow & 7));
+      }
+      if (STORES > 2 * QUADS) {
+        roff[2] = row_of(frow);
+        poff[2] = pre_of(frow);
+      }
+      struct Values { uint32_t r[4], u[4], g[4]; };  // two values each
+      auto values = [&](int p) __attribute__((always_inline)) {
+        Values v;
+#pragma unroll
+        for (int i = 0; i < (p < PAIRS ? 4 : 2); ++i) {
+          const int acc = (mb * 8 + 2 * p + i / 2) * 4 + 2 * (i % 2);
+          float v0 = pg_acc(acc), v1 = pg_acc(acc + 1);
+          {
+            float g0 = pg_acc(acc + 4 * HB), g1 = pg_acc(acc + 4 * HB + 1);
+            if constexpr (KEEP) {
+              v.u[i] = pack2<T>(v0, v1);
+              v.g[i] = pack2<T>(g0, g1);
+              v0 = unpack_lo<T>(v.u[i]);
+              v1 = unpack_hi<T>(v.u[i]);
+              g0 = unpack_lo<T>(v.g[i]);
+              g1 = unpack_hi<T>(v.g[i]);
+            }
+            v0 *= silu_rcp_f32(g0);
+            v1 *= silu_rcp_f32(g1);
+          }
+          v.r[i] = pack2<T>(v0, v1);
+        }
+        return v;
+      };
+      auto store4 = [&](const uint32_t (&v)[4], auto rsrc, uint32_t row, uint32_t col) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_buffer_store_b128((u32x4){v[0], v[1], v[2], v[3]}, rsrc, (int)__builtin_elementwise_add_sat(row, col), 0, NT ? 2 : 0);
+      };
+      auto store2 = [&](const uint32_t (&v)[4], auto rsrc, uint32_t row, uint32_t col) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_buffer_store_b64((u32x2){v[0], v[1]}, rsrc, (int)__builtin_elementwise_add_sat(row, col), 0, NT ? 2 : 0);
+      };
+      auto store_quad = [&](const uint32_t (&v)[4], const uint32_t (&w)[4], auto rsrc, const uint32_t (&row)[3], uint32_t col) __attribute__((always_inline)) {
+        uint32_t x[4], y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)v[i], (int)w[i], 0x128, 0xf, 0xc, false);  // (row_ror:8)
+          y[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)w[i], (int)v[i], 0x128, 0xf, 0x3, false);
+        }
+        store4(x, rsrc, row[0], col);
+        store4(y, rsrc, row[1], col);
+      };
+#pragma unroll
+      for (int p = 0; p < 2 * QUADS; p += 2) {
+        const Values v = values(p), w = values(p + 1);
+        store_quad(v.r, w.r, srd, roff, coff[p]);
+        if constexpr (KEEP) {
+          store_quad(v.u, w.u, pre, poff, coff[p]);
+          store_quad(v.g, w.g, pre, poff, (uint32_t)__builtin_elementwise_add_sat(coff[p], ld));
+        }
+      }
+#pragma unroll
+      for (int p = 2 * QUADS; p < STORES; ++p) {
+        const Values v = values(p);
+        auto store = [&](const uint32_t (&x)[4], auto rsrc, uint32_t row, uint32_t col) __attribute__((always_inline)) {
+          if (p < PAIRS) store4(x, rsrc, row, col);
+          else store2(x, rsrc, row, col);
+        };
+        store(v.r, srd, roff[2], coff[p]);
+        if constexpr (KEEP) {
+          store(v.u, pre, poff[2], coff[p]);
+          store(v.g, pre, poff[2], (uint32_t)__builtin_elementwise_add_sat(coff[p], ld));
+        }
+      }
+      pg_own_agprs();
+    }
+  };
+  // Plain: staged through the wave's pieces of the free ring unit, four passes of 32 rows x 128 columns (256-byte rows, 4 to a
+  // piece), so that a store writes 256 bytes of a row: rows go to scattered places here, and in 128-byte pieces from the registers
+  // they take longer than the staging saves (40 experts, 512 -> 1536, 32768 tokens 392 us; 403, and 490 in 64-byte pieces).
+  // Chunk c of scratch row r lies at slot c ^ (r % 16): writes and reads free of conflicts, and the read-back is linear in the lane.
+  constexpr int PASS_ROWS = 4 * PIECES, MBP = PASS_ROWS / 16, NPASS = (16 * NX + PASS_ROWS - 1) / PASS_ROWS;
+  const uint32_t scr_w = (frow / 4) * 4096 + (frow % 4) * 256 + (((fq >> 1) ^ frow) * 16) + (fq & 1) * 8;
+  const int srow = lane / 16, scc0 = (lane % 16) ^ srow;  // chunk of store 0; store it: ^ 4 (it % 4)
+  auto epilogue_staged = [&](const PgTile& t, uint32_t row0) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) u32x2* wp_t;
+    typedef __attribute__((address_space(3))) const u32x4* rp_t;
+    const uint32_t ld = a.N * 2u;
     const int behind = t.row_end - t.row_begin;
     const int r0 = tile_row0, rows = behind < BM ? behind : BM;
-    const uint32_t window = WHAT == 0 ? a.out_window : (uint32_t)rows, left = WHAT == 0 ? a.L - row0 : (uint32_t)rows;
-    unsigned char* dst = WHAT == 0 ? reinterpret_cast<unsigned char*>(out) + (uint64_t)row0 * ld
-                                   : static_cast<unsigned char*>(a.pre) + (uint64_t)t.row_begin * ld;
-    const auto srd = __builtin_amdgcn_make_buffer_rsrc(dst, (short)0, (int)((left < window ? left : window) * ld), 0x00020000);
+    const uint32_t window = a.out_window, left = a.L - row0;
+    const auto srd = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char*>(out) + (uint64_t)row0 * ld, (short)0,
+                                                       (int)((left < window ? left : window) * ld), 0x00020000);
     const uint32_t s0 = dma0 + p4;
     const int col0 = t.nt * BN + wn * WN;
     uint32_t scr = scr_w;
     asm volatile("" : "+v"(scr));                   // (or the addresses that it gives are kept in registers from the first tile on)
-    // byte offsets of the wave's rows lane and 64 + lane, and of the lane's columns in store it (% CP); saturating sums keep what
-    // does not exist past the buffer
-    constexpr int CP = GLU ? 2 : 4;
-    const uint32_t lo = WHAT == 0 ? (uint32_t)orow_lo - row0 : r0, hi = WHAT == 0 ? (uint32_t)orow_hi - row0 : r0 + TILE_64;
+    // byte offsets of the wave's rows lane and 64 + lane, and of the lane's columns in store it (% 4); saturating sums keep
+    // what does not exist past the buffer
+    const uint32_t lo = (uint32_t)orow_lo - row0, hi = (uint32_t)orow_hi - row0;
     const uint32_t rlo = r0 < rows && lo < window ? lo * ld : PG_OOB, rhi = r0 + TILE_64 < rows && hi < window ? hi * ld : PG_OOB;
-    uint32_t coff[CP];
+    uint32_t coff[4];
 #pragma unroll
-    for (int c = 0; c < CP; ++c) {
+    for (int c = 0; c < 4; ++c) {
       const int col = col0 + (scc0 ^ (4 * c)) * 8;
-      coff[c] = col < a.N && (scc0 ^ (4 * c)) * 8 < WN ? (uint32_t)((WHAT == 2 ? a.N : 0) + col) * 2u : PG_OOB;
+      coff[c] = col < a.N && (scc0 ^ (4 * c)) * 8 < WN ? (uint32_t)col * 2u : PG_OOB;
     }
 #pragma unroll
     for (int p = 0; p < NPASS; ++p) {
@@ -400,28 +516,10 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
 #pragma unroll
       for (int mbp = 0; mbp < MBP; ++mbp)
 #pragma unroll
-        for (int nb = 0; nb < NBO; ++nb) {
-          const int blk = (p * MBP + mbp) * 8 + nb;
-          float v[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (WHAT == 1) {
-              v[i] = pg_acc(blk * 4 + i);
-            } else if (WHAT == 2) {
-              v[i] = pg_acc((blk + HB) * 4 + i);
-            } else if (GLU) {
-              float up = pg_acc(blk * 4 + i), gt = pg_acc((blk + HB) * 4 + i);
-              if (KEEP) {
-                up = Elt<T>::round(up);
-                gt = Elt<T>::round(gt);
-              }
-              v[i] = up * silu_rcp_f32(gt);
-            } else {
-              v[i] = pg_acc(blk * 4 + i);
-            }
-          }
-          *(wp_t)(size_t)(s0 + (scr ^ (nb * 32)) + mbp * (16 / RPP) * 4096) =
-              (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+        for (int nb = 0; nb < NB; ++nb) {
+          const int acc = ((p * MBP + mbp) * 8 + nb) * 4;
+          const float v0 = pg_acc(acc), v1 = pg_acc(acc + 1), v2 = pg_acc(acc + 2), v3 = pg_acc(acc + 3);
+          *(wp_t)(size_t)(s0 + (scr ^ (nb * 32)) + mbp * 4 * 4096) = (u32x2){pack2<T>(v0, v1), pack2<T>(v2, v3)};
         }
       pg_own_agprs();
       // (four at a time: one LDS latency for all of them)
@@ -431,13 +529,13 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
         uint32_t roff[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const int r = p * PASS_ROWS + (it0 + j) * RPP;  // + srow: row of the wave's 128
+          const int r = p * PASS_ROWS + (it0 + j) * 4;  // + srow: row of the wave's 128
           val[j] = *(rp_t)(size_t)(s0 + (it0 + j) * 4096 + lane * 16);
           roff[j] = (uint32_t)__builtin_amdgcn_ds_bpermute(((r & 63) + srow) * 4, (int)(r < 64 ? rlo : rhi));
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          __builtin_amdgcn_raw_buffer_store_b128(val[j], srd, (int)__builtin_elementwise_add_sat(roff[j], coff[(it0 + j) % CP]), 0, NT ? 2 : 0);
+          __builtin_amdgcn_raw_buffer_store_b128(val[j], srd, (int)__builtin_elementwise_add_sat(roff[j], coff[(it0 + j) % 4]), 0, NT ? 2 : 0);
       }
       pg_own_agprs();
     }
@@ -445,14 +543,10 @@ __device__ __forceinline__ void persistent_body(const GemmArgs& a, const PgRows&
   auto epilogue = [&](const PgTile& t) __attribute__((always_inline)) {
     uint32_t row0 = 0;
     do {
-      epilogue_as(std::integral_constant<int, 0>{}, t, row0);
+      if constexpr (GLU) epilogue_direct(t, row0);
+      else epilogue_staged(t, row0);
       row0 += a.out_window;
     } while (row0 < (uint32_t)a.L);
-    if constexpr (KEEP) {
-      // both halves of the pre-activation next to the activation
-      epilogue_as(std::integral_constant<int, 1>{}, t, 0);
-      epilogue_as(std::integral_constant<int, 2>{}, t, 0);
-    }
   };
   // a part of a split tile: accumulators -> workspace, block b of thread t at [b][t]
   auto store_part = [&]() {

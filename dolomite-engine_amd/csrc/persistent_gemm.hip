@@ -24,9 +24,16 @@
 //   * Fragments are read one half slice ahead into a second register set; every LDS read, DMA instruction and scalar
 //     step sits alone between two matrix instructions (a matrix instruction leaves three free issue slots).
 //   * The accumulators are addressed by number (mfma_core.h).
-//   * A tile boundary has no barrier: a wave stages its results through the eight 1 KB pieces of the free ring unit
-//     that its own DMA fills next.  The stores stay in flight under the next tile's first slice (they are counted,
-//     vmcnt retires in issue order).  The tile list of a workgroup is decoded once, a lane per tile.
+//   * A tile boundary has no barrier.  SwiGLU results go from registers to memory: the weight rows are dealt to the matrix
+//     instruction so that a lane ends up with eight neighbouring columns of a row (the staging before, per half of a training
+//     tile once more, and its waits: 40 experts, 1536 -> 512, 2048 tokens 55.4 -> 53 us, with the pre-activation 63 -> 57.5;
+//     32 experts, 1024 -> 512, 16384 tokens 219 -> 214 and 268 -> 255; 32768 tokens, which the stores bound, 690 -> 683 with the
+//     pre-activation).  The plain form stages them through the eight 1 KB pieces of the free ring unit that the wave's own DMA
+//     fills next.  The stores stay in flight under the next tile's first slice (they are counted, vmcnt retires in issue
+//     order).  The tile list of a workgroup is decoded once, a lane per tile.
+//   * What a boundary costs (40 experts, 32768 tokens, uneven; without the stores' traffic / without the epilogue): SwiGLU 1536 ->
+//     512 629 us (602 / 563), plain 512 -> 1536 396 (338 / 286), pre-activation kept 703 (632 / 535).  Starting the workgroups
+//     of an XCD a half or a quarter of a tile apart changes nothing: they are out of step by themselves.
 // Measured (8192 x 8192 x 8192, one expert): the loop runs at 0.94 of the matrix pipe's cycles without DMA; the form it
 // replaces -- eight waves in two groups that alternated between a memory and a matrix phase, 64-byte rows -- reached
 // 0.80 with DMA.
@@ -109,7 +116,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_split_finish_kernel(GemmArgs
     const int orow = a.scatter ? a.sorted_scattered[row] : row;
 #pragma unroll
     for (int nb = 0; nb < (GLU ? 4 : 8); ++nb) {
-      const int col = t.nt * BN + wn * (GLU ? 64 : 128) + nb * 16 + fq * 4;
+      const int col = t.nt * BN + (GLU ? wn * 64 + 32 * (nb / 2) + 8 * fq + 4 * (nb % 2) : wn * 128 + nb * 16 + fq * 4);
       if (col >= a.N) continue;
       float v[4];
 #pragma unroll
