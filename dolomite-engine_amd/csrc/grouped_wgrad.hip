@@ -23,7 +23,8 @@
 //     equal ranges instead leaves the XCDs up to one group apart and costs 10 - 20 % under skewed loads.)
 //     An item of an expert with several groups writes an fp32 partial tile and a second kernel sums the partials
 //     of the expert in group order and rounds once (deterministic); an expert with one group is written directly,
-//     one without rows gets zeros from the second kernel.
+//     one without rows gets zeros from the second kernel.  With few rows per expert none of that pays: whole experts, dealt
+//     round by round (wgrad_whole_experts).
 //   * One wave per SIMD with 128 x 128 accumulators in the AGPR half of the register file, 64-row slices, and the
 //     five-unit DMA ring of persistent_gemm.hip (see there for why): one barrier per slice, one LDS read or DMA
 //     instruction between any two matrix instructions.  A lane loads the indices of its eight rows of a gathered
@@ -89,8 +90,10 @@ __device__ __forceinline__ int wgrad_group_rows(int n, int groups) { return ((n 
 #define WG_LDS (5 * WG_U)
 
 // GA / GB: operand a / b is gathered through its index array
-template <typename T, bool GA, bool GB>
-__global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
+// PLAN: groups and their order come from wgrad_plan_kernel.  Else (wgrad_whole_experts) an item is a tile of a whole expert, round r of
+// the chip the items [r grid, (r + 1) grid), of which XCD x takes the x-th eighth; every tile is written here.
+template <typename T, bool GA, bool GB, bool PLAN>
+__device__ __forceinline__ void wgrad_body(const WgradArgs& a) {
   constexpr int TILE = 256;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   int* item_slot = reinterpret_cast<int*>(smem_raw);  // (between items, when the ring is drained)
@@ -102,14 +105,14 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
   const int upper = lane >> 5;
 
   WgradTable tb;
-  wgrad_table(a.expert_offsets, a.E, a.chunk, tb);
+  if constexpr (PLAN) wgrad_table(a.expert_offsets, a.E, a.chunk, tb);
   const int tiles = a.m_tiles * a.n_tiles;
   const int xcd = blockIdx.x & 7;
   // this XCD's groups: slots [xfirst, xfirst + xgroups) of the planned list
-  const int xfirst = a.next_item[8 + xcd];
-  const int xgroups = a.next_item[8 + xcd + 1] - xfirst;
+  const int xfirst = PLAN ? a.next_item[8 + xcd] : 0;
+  const int xgroups = PLAN ? a.next_item[8 + xcd + 1] - xfirst : 0;
   const int* __restrict__ xlist = a.next_item + 32 + xfirst;
-  const int items_x = xgroups * tiles;
+  const int items_x = PLAN ? xgroups * tiles : a.E * tiles;
 
   // ---- DMA: wave w fetches rows 16 w .. 16 w + 15 of a slice, instruction j the rows j (lanes 0-31) and 8 + j: a lane
   // then needs the indices of eight consecutive rows of a gathered operand, two loads of 16 bytes per slice.  (The two
@@ -144,19 +147,24 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
   // over when it ends, late enough that a workgroup does not hold an item another one could start.
   constexpr int DRAW_AHEAD = 3;
   int drawn = 0;
-  if (threadIdx.x == 0) drawn = atomicAdd(a.next_item + xcd, 1);
-  for (;;) {
+  if (PLAN && threadIdx.x == 0) drawn = atomicAdd(a.next_item + xcd, 1);
+  for (int round = 0;; ++round) {
+    int item = round * (int)gridDim.x + xcd * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
     // (bare barriers: a fence would also wait for the last item's stores)
-    if (threadIdx.x == 0) *item_slot = drawn;
-    __builtin_amdgcn_s_waitcnt(pg_wait(63, 0));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    const int item = __builtin_amdgcn_readfirstlane(*item_slot);
-    __builtin_amdgcn_s_waitcnt(pg_wait(63, 0));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    if constexpr (PLAN) {
+      if (threadIdx.x == 0) *item_slot = drawn;
+      __builtin_amdgcn_s_waitcnt(pg_wait(63, 0));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      item = __builtin_amdgcn_readfirstlane(*item_slot);
+    }
+    if (PLAN || round > 0) {                        // (the last item's results are out of the LDS)
+      __builtin_amdgcn_s_waitcnt(pg_wait(63, 0));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
     if (item >= items_x) break;
-    const int grp = __builtin_amdgcn_readfirstlane(xlist[item / tiles]);
+    const int grp = PLAN ? __builtin_amdgcn_readfirstlane(xlist[item / tiles]) : 0;
     // A group's tiles are numbered in bands of 8 row tiles, column tile slowest inside a band: the 32 workgroups
     // of the XCD, which hold 32 consecutive items, then cover 8 x 4 tiles -- 12 operand slabs for 32 tiles.  (Row
     // tile fastest over all of them would re-read every A slab once per column tile: with 112 x 16 tiles that is
@@ -171,7 +179,18 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
 
     // group -> expert and its row range (wave-uniform)
     int r0 = 0, r1 = 1, expert = 0, expert_groups = 1;
-    {
+    if constexpr (!PLAN) {
+      expert = item / tiles;
+      r0 = expert > 0 ? a.expert_offsets[expert - 1] : 0;
+      r1 = a.expert_offsets[expert];
+      if (r1 <= r0) {                               // no rows: zeros
+        T* __restrict__ out = static_cast<T*>(a.dw) + (size_t)expert * a.M * a.N;
+        const int n = nt * TILE + (threadIdx.x & 31) * 8;
+        for (int m = mt * TILE + (threadIdx.x >> 5); m < a.M && m < (mt + 1) * TILE; m += 8)
+          if (n < a.N) *reinterpret_cast<u32x4*>(out + (size_t)m * a.N + n) = (u32x4){0u, 0u, 0u, 0u};
+        continue;
+      }
+    } else {
       int first = 0, prev = 0;
       bool found = false;
 #pragma unroll
@@ -380,7 +399,7 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
     step(std::true_type{});
     int k = 1;
     for (; k < nk - DRAW_AHEAD; ++k) step(std::false_type{});
-    if (threadIdx.x == 0) drawn = atomicAdd(a.next_item + xcd, 1);
+    if (PLAN && threadIdx.x == 0) drawn = atomicAdd(a.next_item + xcd, 1);
     for (; k < nk; ++k) step(std::false_type{});
     pg_acc_settle();
     // surplus DMA (two slices of zeros) has to land before the ring is used again
@@ -392,7 +411,7 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
     // An expert with one group is final: rounded, staged through 8 KB of LDS per wave (32 rows x 128 columns at a time,
     // 16-byte chunk c of row r at slot c ^ (r % 16)) and stored as whole 256-byte rows.  Otherwise the fp32
     // accumulators go to the group's partial slab as they are: [row block][column block][lane].
-    if (expert_groups == 1) {
+    if (!PLAN || expert_groups == 1) {
       T* __restrict__ out = static_cast<T*>(a.dw) + (size_t)expert * a.M * a.N;
       unsigned char* scratch = smem_raw + 1024 + wave * 8192;  // (past the item slot)
       const bool interior = (mt + 1) * TILE <= a.M && (nt + 1) * TILE <= a.N;
@@ -434,6 +453,13 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
       }
     }
   }
+}
+
+template <typename T, bool GA, bool GB> __global__ __launch_bounds__(256, 1) void grouped_wgrad_kernel(WgradArgs a) {
+  wgrad_body<T, GA, GB, true>(a);
+}
+template <typename T, bool GA, bool GB> __global__ __launch_bounds__(256, 1) void grouped_wgrad_whole_kernel(WgradArgs a) {
+  wgrad_body<T, GA, GB, false>(a);
 }
 
 // Plan of one launch (one workgroup, in front of the main kernel): zero the eight work counters, rank the
@@ -579,6 +605,15 @@ static int wgrad_chunk(int L, int E, int M, int N) {
   return (int)(chunk / 32 * 32);
 }
 
+// Few rows per expert: every expert whole, the items dealt without a plan, which saves two launches and, in the main one, the trips to
+// the plan and to the counters.  What it costs is the balance: the most loaded expert is one item a tile however many rows it has.
+// Planned / whole, us (the load's unevenness in brackets, in ln(rank) of the logits): 40 experts, 1024 x 1536, 1600 tokens of 8 slots
+// 74 / 60 (0), 83 / 67 (0.49), 3000 tokens 96 / 86 and 107 / 98, 5000 tokens 138 / 135 (0.3); 1536 x 512, 2048 tokens 61 / 44 (0.3), 5000
+// tokens 94 / 98 (0.49); 32 experts, 1024 x 1024, 509 tokens 36 / 25 (0); 8 experts, 28672 x 4096, 1000 tokens of 2 slots 873 / 759
+// (0.3).  One expert, which always wants its rows cut: 32 x 1024, 509 rows 17.1 / 15.6, 640 rows 17.5 / 17.8, 40 x 1536, 768 rows 18.1 /
+// 19.9.  (The second bound is for loads that collapse on one expert.)
+static bool wgrad_whole_experts(int L, int E) { return (long)L <= (E == 1 ? 640L : 768L * E) && L <= 32768; }
+
 static long wgrad_max_groups(int L, int E, int chunk) { return (long)L / chunk + (E < L ? E : L); }
 static size_t wgrad_plan_bytes(long groups, int E) { return ((size_t)(32 + groups + 3 * (long)E) * sizeof(int) + 255) / 256 * 256; }
 
@@ -595,8 +630,8 @@ extern "C" size_t mi_moe_grouped_wgrad_workspace_bytes(int L, int E, int M, int 
   return wgrad_slab_bytes(groups, M, N) + wgrad_plan_bytes(groups, E);
 }
 
-template <typename T, bool GA, bool GB> static int launch_wgrad_as(const WgradArgs& g, int grid, hipStream_t s) {
-  auto kern = grouped_wgrad_kernel<T, GA, GB>;
+template <typename T, bool GA, bool GB, bool PLAN> static int launch_wgrad_as(const WgradArgs& g, int grid, hipStream_t s) {
+  auto kern = PLAN ? grouped_wgrad_kernel<T, GA, GB> : grouped_wgrad_whole_kernel<T, GA, GB>;
   static std::atomic<uint64_t> lds_ok{0};
   const int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), WG_LDS, lds_ok);
   if (rc != MI_MOE_OK) return rc;
@@ -604,10 +639,15 @@ template <typename T, bool GA, bool GB> static int launch_wgrad_as(const WgradAr
   return mi_launch_status();
 }
 
+template <typename T, bool PLAN> static int launch_wgrad_main(const WgradArgs& g, int grid, hipStream_t s) {
+  if (g.a_idx != nullptr) return g.b_idx != nullptr ? launch_wgrad_as<T, true, true, PLAN>(g, grid, s) : launch_wgrad_as<T, true, false, PLAN>(g, grid, s);
+  return g.b_idx != nullptr ? launch_wgrad_as<T, false, true, PLAN>(g, grid, s) : launch_wgrad_as<T, false, false, PLAN>(g, grid, s);
+}
+
 template <typename T> static int launch_wgrad(const WgradArgs& g, int grid, int red_at, hipStream_t s) {
   if (g.L > 0) {
-    const int rc = g.a_idx != nullptr ? (g.b_idx != nullptr ? launch_wgrad_as<T, true, true>(g, grid, s) : launch_wgrad_as<T, true, false>(g, grid, s))
-                                      : (g.b_idx != nullptr ? launch_wgrad_as<T, false, true>(g, grid, s) : launch_wgrad_as<T, false, false>(g, grid, s));
+    if (g.next_item == nullptr) return launch_wgrad_main<T, false>(g, grid, s);
+    const int rc = launch_wgrad_main<T, true>(g, grid, s);
     if (rc != MI_MOE_OK) return rc;
   }
   const int m_blocks = mi_ceil_div(g.M, 16), n_blocks = mi_ceil_div(g.N, 16);
@@ -643,7 +683,8 @@ extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const v
   g.chunk = wgrad_chunk(L, E, M, N);
   const long max_groups = wgrad_max_groups(L, E, g.chunk);
   const int red_at = (int)(32 + max_groups);
-  if (L > 0) {
+  const bool whole = wgrad_whole_experts(L, E);
+  if (L > 0 && !whole) {
     g.next_item = reinterpret_cast<int*>(static_cast<unsigned char*>(workspace) + wgrad_slab_bytes(max_groups, M, N));
     hipLaunchKernelGGL(wgrad_plan_kernel, dim3(1), dim3(1024), 0, s, expert_offsets, E, g.chunk, g.next_item, red_at);
   }
@@ -652,9 +693,11 @@ extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const v
   int cus = 0;
   int rc = mi_cu_count(&cus);
   if (rc != MI_MOE_OK) return rc;
-  const long max_items = max_groups * g.m_tiles * g.n_tiles;
-  long grid = cus < max_items ? cus : max_items;
-  grid = (grid + 7) / 8 * 8;
+  // (an XCD can be dealt an eighth of the groups, rounded up: with as many workgroups as items alone, two groups of a router's
+  // gradient, 509 rows, 32 x 1024, were the work of one workgroup each, 33 us)
+  const long tiles = (long)g.m_tiles * g.n_tiles;
+  const long per_xcd = whole ? ((long)E * tiles + 7) / 8 : (max_groups + 7) / 8 * tiles;
+  const long grid = 8 * (per_xcd < cus / 8 ? per_xcd : (cus + 7) / 8);
   return dtype == MI_MOE_BF16 ? launch_wgrad<bf16_t>(g, (int)grid, red_at, s) : launch_wgrad<f16_t>(g, (int)grid, red_at, s);
 }
 

@@ -1,0 +1,70 @@
+"""Weight gradients of few rows per expert, which run without a plan: whole experts, one item a tile.  The sizes sit on both sides of
+the lines that choose (640 rows of one expert, 768 rows per expert on average), with experts that have no rows, fewer than a
+slice of 64, and whole slices.
+
+Against a product in 64 bits: operands are exact, the sums are fp32 (relative error far below the rounding of the result), one
+rounding of at most 2^-8 (bf16, 8 significant bits) or 2^-11 (fp16, 11) of the value, and an absolute term for results that cancel: fp32 partial sums
+err by at most rows * 2^-24 of the sum of the magnitudes, which is below 0.64 rows for products of two unit normals."""
+
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+import torch
+
+from test_built_kernels import _early_uses, _foreign, _objdump
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("gather", ["none", "a", "b"])
+@pytest.mark.parametrize("counts,M,N", [
+    ([1], 8, 8), ([640], 32, 1024), ([641], 40, 264), ([0, 0, 5], 264, 24), ([64, 0, 63, 65, 128, 0, 300], 520, 248),
+    ([1535, 1], 136, 520), ([1535, 2], 136, 520), ([127] * 30 + [0, 2], 264, 264), ([0, 0], 256, 256),
+])
+def test_whole_experts(device, dtype, gather, counts, M, N):
+    from dolomite_engine_amd import ops
+
+    g = torch.Generator().manual_seed(M * 17 + N + len(counts))
+    L, E = sum(counts), len(counts)
+    print(f"wgrad whole {counts[:8]} {M}x{N} {dtype} {gather}", flush=True)
+    rows = max(L, 1)
+    a, b = torch.randn(rows, M, generator=g).to(dtype), torch.randn(rows, N, generator=g).to(dtype)
+    idx = torch.randint(0, rows, (L,), generator=g)
+    ai = idx if gather == "a" else torch.arange(L)
+    bi = idx if gather == "b" else torch.arange(L)
+    off = torch.tensor(counts).cumsum(0)
+    want = torch.zeros(E, M, N, dtype=torch.float64)
+    for e, n in enumerate(counts):
+        r = slice(int(off[e]) - n, int(off[e]))
+        want[e] = a[ai[r]].double().t() @ b[bi[r]].double()
+    dev = lambda t: t.to(torch.int32).to(device)
+    got = ops.grouped_wgrad(a[:L].to(device) if gather != "a" else a.to(device), b[:L].to(device) if gather != "b" else b.to(device),
+                            dev(off), dev(idx) if gather == "a" else None, dev(idx) if gather == "b" else None)
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = eps * want.abs() + max(counts) * 0.64 * max(counts) * 2.0 ** -24 + 2.0 ** -24
+    assert ((got.cpu().double() - want).abs() <= bound).all()
+
+
+def test_built_code(tmp_path):
+    """The accumulators and row indices of these kernels are used as test_built_kernels.py says of the planned ones."""
+    from dolomite_engine_amd import _lib, build, is_built
+
+    if not is_built():
+        build()
+    shutil.copy(os.path.realpath(_lib.load()._name), tmp_path / "lib.so")
+    subprocess.run([_objdump(), "--offloading", str(tmp_path / "lib.so")], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    found = 0
+    for image in sorted(p for p in tmp_path.iterdir() if "gfx950" in p.name):
+        text = subprocess.run([_objdump(), "-d", "--no-show-raw-insn", "--no-leading-addr", str(image)], check=True,
+                              capture_output=True, text=True).stdout
+        for label, body in re.findall(r"^(?:[0-9a-f]+ )?<(\w+)>:\n((?:(?!^(?:[0-9a-f]+ )?<).*\n?)*)", text, re.M):
+            if "grouped_wgrad_whole_kernelI" not in label:
+                continue
+            found += 1
+            code = [line.split("//")[0].strip() for line in body.splitlines()]
+            assert sum("v_mfma" in i for i in code) >= 128
+            assert _foreign(code) == [] and _early_uses(code) == []
+    assert found == 8
