@@ -12,6 +12,7 @@
 // All arithmetic in fp32 from the logits as stored; the eager module rounds its intermediates to the model
 // dtype instead, so the two agree to that dtype's rounding, not bit for bit.
 #include "common.h"
+#include "topk_row.h"
 
 #define AUX_MAX_E 256
 #define AUX_ROWS_PER_BLOCK 32
@@ -135,16 +136,21 @@ __global__ __launch_bounds__(256) void aux_loss_colsum_kernel(const float* __res
   if (lane == 0) colsum[c] = s;
 }
 
-// loss_w[0] = loss, loss_w[1 + e] = d loss / d A_e
-__global__ __launch_bounds__(256) void aux_loss_finish_kernel(const float* __restrict__ colsum, float* __restrict__ loss_w,
-                                                              int Trows, int E) {
+// loss_w[0] = loss, loss_w[1 + e] = d loss / d A_e; loss_out (or null): the loss in the logits' type.  The column sums are taken here,
+// as aux_loss_colsum_kernel takes them, while a column is few blocks; else `partial` holds them already (nblocks = 1).
+template <typename T>
+__global__ __launch_bounds__(1024) void aux_loss_finish_kernel(const float* __restrict__ partial, int nblocks,
+                                                               float* __restrict__ loss_w, T* __restrict__ loss_out, int Trows, int E) {
   __shared__ float A[AUX_MAX_E], F[AUX_MAX_E];
   __shared__ float scal[4];
-  for (int e = threadIdx.x; e < E; e += 256) {
-    A[e] = colsum[e];
-    F[e] = colsum[E + e];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll 4
+  for (int c = wave; c < 2 * E + 1; c += 16) {
+    float v = lane < nblocks ? partial[(size_t)c * nblocks + lane] : 0.f;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, MI_WAVE);
+    if (lane == 0) (c < E ? A[c] : c < 2 * E ? F[c - E] : scal[3]) = v;
   }
-  if (threadIdx.x == 0) scal[3] = colsum[2 * E];
   __syncthreads();
   if (threadIdx.x == 0) {
     float sa = 0.f, sf = 0.f, dot = 0.f;
@@ -159,11 +165,13 @@ __global__ __launch_bounds__(256) void aux_loss_finish_kernel(const float* __res
     scal[0] = sa;
     scal[1] = sf;
     scal[2] = sw;
-    loss_w[0] = sw + 0.1f * (scal[3] / (float)Trows);
+    const float loss = sw + 0.1f * (scal[3] / (float)Trows);
+    loss_w[0] = loss;
+    if (loss_out != nullptr) Elt<T>::store(loss_out, loss);
   }
   __syncthreads();
   // d/dA_e [ sum_e' A_e' c_e' / S ] = (c_e - switch) / S  with c_e = E f_e / sum f  (S = sum A above its floor)
-  for (int e = threadIdx.x; e < E; e += 256) loss_w[1 + e] = ((float)E * F[e] / scal[1] - scal[2]) / scal[0];
+  for (int e = threadIdx.x; e < E; e += 1024) loss_w[1 + e] = ((float)E * F[e] / scal[1] - scal[2]) / scal[0];
 }
 
 template <typename T>
@@ -201,19 +209,21 @@ extern "C" size_t mi_moe_aux_loss_workspace_bytes(int T, int E) {
 }
 
 template <typename T>
-static void aux_forward_launch(const void* logits, const int32_t* idx, float* ws, float* loss_w, int Trows, int E, int k,
-                               hipStream_t s) {
+static void aux_forward_launch(const void* logits, const int32_t* idx, float* ws, float* loss_w, void* loss_out, int Trows, int E,
+                               int k, hipStream_t s) {
   const int nb = aux_blocks(Trows);
   auto kern = E <= 64 ? aux_loss_partial_kernel<T, 1> : aux_loss_partial_kernel<T, AUX_MAX_E / 64>;
   hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, s, static_cast<const T*>(logits), idx, ws, Trows, E, k);
   const int ncols = 2 * E + 1;
   float* colsum = ws + (size_t)nb * ncols;
-  hipLaunchKernelGGL(aux_loss_colsum_kernel, dim3(mi_ceil_div(ncols, 4)), dim3(256), 0, s, ws, colsum, nb, ncols);
-  hipLaunchKernelGGL(aux_loss_finish_kernel, dim3(1), dim3(256), 0, s, colsum, loss_w, Trows, E);
+  if (nb > 64) hipLaunchKernelGGL(aux_loss_colsum_kernel, dim3(mi_ceil_div(ncols, 4)), dim3(256), 0, s, ws, colsum, nb, ncols);
+  hipLaunchKernelGGL((aux_loss_finish_kernel<T>), dim3(1), dim3(1024), 0, s, nb > 64 ? colsum : ws, nb > 64 ? 1 : nb, loss_w,
+                     static_cast<T*>(loss_out), Trows, E);
 }
 
-extern "C" int mi_moe_aux_loss(const void* logits, const int32_t* topk_idx, float* loss_w, void* workspace,
-                               size_t workspace_bytes, int T, int E, int k, int dtype, mi_moe_stream_t stream) {
+// loss_out (or null): the loss in `dtype` as well
+int mi_aux_loss(const void* logits, const int32_t* topk_idx, float* loss_w, void* loss_out, void* workspace, size_t workspace_bytes,
+                int T, int E, int k, int dtype, mi_moe_stream_t stream) {
   if (T < 1 || E < 1 || k < 1) return MI_MOE_ESHAPE;
   if (E > AUX_MAX_E) return MI_MOE_EUNSUPPORTED;
   if (!logits || !topk_idx || !loss_w) return MI_MOE_ENULL;
@@ -221,12 +231,17 @@ extern "C" int mi_moe_aux_loss(const void* logits, const int32_t* topk_idx, floa
   hipStream_t s = static_cast<hipStream_t>(stream);
   float* ws = static_cast<float*>(workspace);
   switch (dtype) {
-    case MI_MOE_F32: aux_forward_launch<float>(logits, topk_idx, ws, loss_w, T, E, k, s); break;
-    case MI_MOE_F16: aux_forward_launch<f16_t>(logits, topk_idx, ws, loss_w, T, E, k, s); break;
-    case MI_MOE_BF16: aux_forward_launch<bf16_t>(logits, topk_idx, ws, loss_w, T, E, k, s); break;
+    case MI_MOE_F32: aux_forward_launch<float>(logits, topk_idx, ws, loss_w, loss_out, T, E, k, s); break;
+    case MI_MOE_F16: aux_forward_launch<f16_t>(logits, topk_idx, ws, loss_w, loss_out, T, E, k, s); break;
+    case MI_MOE_BF16: aux_forward_launch<bf16_t>(logits, topk_idx, ws, loss_w, loss_out, T, E, k, s); break;
     default: return MI_MOE_EDTYPE;
   }
   return mi_launch_status();
+}
+
+extern "C" int mi_moe_aux_loss(const void* logits, const int32_t* topk_idx, float* loss_w, void* workspace,
+                               size_t workspace_bytes, int T, int E, int k, int dtype, mi_moe_stream_t stream) {
+  return mi_aux_loss(logits, topk_idx, loss_w, nullptr, workspace, workspace_bytes, T, E, k, dtype, stream);
 }
 
 extern "C" int mi_moe_aux_loss_backward(const void* logits, const float* loss_w, const float* grad, void* d_logits, int T,
@@ -252,5 +267,80 @@ extern "C" int mi_moe_aux_loss_backward(const void* logits, const float* loss_w,
       break;
     default: return MI_MOE_EDTYPE;
   }
+  return mi_launch_status();
+}
+
+// d logits of a training step in one pass: the auxiliary loss's part as above, rounded, and the gates' part of
+// router_dlogits_kernel (router_general.hip) on top of it, with the same roundings.  grad (or null: no such part) is the loss's
+// upstream gradient in the logits' type, d_gates (or null) the gates'.
+template <typename T>
+__global__ __launch_bounds__(256) void router_dlogits_aux_kernel(const T* __restrict__ logits, const int32_t* __restrict__ idx,
+                                                                 const T* __restrict__ d_gates, const float* __restrict__ loss_w,
+                                                                 const T* __restrict__ grad, T* __restrict__ d_logits, int Trows, int E,
+                                                                 int k) {
+  const int lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= Trows) return;
+  const float gl = grad != nullptr ? Elt<T>::load(grad) : 0.f;
+  const float zc = 0.2f / (float)Trows;
+  float w[4], base[4] = {};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = grad != nullptr && lane + 64 * i < E ? loss_w[1 + lane + 64 * i] : 0.f;
+  // picked logit, its expert and the incoming gradient of slot j = lane (k <= 64)
+  int e_j = 0;
+  float z = -INFINITY, g = 0.f;
+  if (d_gates != nullptr && lane < k) {
+    e_j = idx[(size_t)t * k + lane];
+    z = Elt<T>::load(logits + (size_t)t * E + e_j);
+    g = Elt<T>::load(d_gates + (size_t)t * k + lane);
+  }
+  if (grad != nullptr) {
+    float p[4];
+    const float lse = aux_row_softmax<T>(logits + (size_t)t * E, E, lane, p);
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s = fmaf(p[i], w[i], s);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, MI_WAVE);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) base[i] = Elt<T>::round(gl * p[i] * ((w[i] - s) + zc * lse));
+  }
+  float dz = 0.f;
+  if (d_gates != nullptr) {
+    float zmax = z;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) zmax = fmaxf(zmax, __shfl_xor(zmax, off, MI_WAVE));
+    float p = lane < k ? expf(z - zmax) : 0.f;
+    p /= wave_sum_f32(p);
+    const float dot = wave_sum_f32(p * g);
+    dz = Elt<T>::round(p * (g - dot));
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = lane + 64 * i;
+    if (64 * i >= E) break;
+    float val = base[i];
+    if (d_gates != nullptr) {
+      for (int j = 0; j < k; ++j) {
+        const int ej = __shfl(e_j, j, MI_WAVE);
+        const float dzj = __shfl(dz, j, MI_WAVE);
+        if (ej == e) val = grad != nullptr ? Elt<T>::round(dzj + base[i]) : dzj;
+      }
+    }
+    if (e < E) Elt<T>::store(d_logits + (size_t)t * E + e, val);
+  }
+}
+
+int mi_router_dlogits_aux(const void* logits, const int32_t* idx, const void* d_gates, const float* loss_w, const void* grad,
+                          void* d_logits, int T, int E, int k, int dtype, hipStream_t s) {
+  const dim3 grid(mi_ceil_div(T, 4)), block(256);
+  if (E > AUX_MAX_E || k > 64) return MI_MOE_EUNSUPPORTED;
+  if (dtype == MI_MOE_BF16)
+    hipLaunchKernelGGL((router_dlogits_aux_kernel<bf16_t>), grid, block, 0, s, static_cast<const bf16_t*>(logits), idx,
+                       static_cast<const bf16_t*>(d_gates), loss_w, static_cast<const bf16_t*>(grad), static_cast<bf16_t*>(d_logits), T, E, k);
+  else if (dtype == MI_MOE_F16)
+    hipLaunchKernelGGL((router_dlogits_aux_kernel<f16_t>), grid, block, 0, s, static_cast<const f16_t*>(logits), idx,
+                       static_cast<const f16_t*>(d_gates), loss_w, static_cast<const f16_t*>(grad), static_cast<f16_t*>(d_logits), T, E, k);
+  else return MI_MOE_EDTYPE;
   return mi_launch_status();
 }

@@ -49,7 +49,8 @@ __global__ __launch_bounds__(256) void swiglu_backward_kernel(const T* __restric
                                                               const T* __restrict__ gates,
                                                               const int32_t* __restrict__ sorted_scattered,
                                                               T* __restrict__ d_h, T* __restrict__ act_g,
-                                                              T* __restrict__ d_gates, int L, int I) {
+                                                              T* __restrict__ d_gates, int32_t* __restrict__ tokens,
+                                                              int L, int I, int k) {
   constexpr int CE = Chunk<T>::N;
   const int lane = threadIdx.x & 63;
   const int cpr = I / CE;
@@ -78,6 +79,7 @@ __global__ __launch_bounds__(256) void swiglu_backward_kernel(const T* __restric
       *reinterpret_cast<u32x4*>(dr + I + c * CE) = Chunk<T>::pack(dg);
       if (act_g != nullptr) *reinterpret_cast<u32x4*>(act_g + (size_t)row * I + c * CE) = Chunk<T>::pack(ag);
     }
+    if (tokens != nullptr && lane == 0) tokens[row] = slot / k;
     if (d_gates != nullptr) {
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, MI_WAVE);
@@ -132,6 +134,9 @@ __global__ __launch_bounds__(256) void swiglu_forward_kernel(const T* __restrict
   }
 }
 
+int mi_swiglu_backward(const void* h, const void* d_act, const void* gates, const int32_t* sorted_scattered, void* d_h, void* act_g,
+                       void* d_gates, int32_t* tokens, int L, int I, int k, int dtype, mi_moe_stream_t stream);
+
 extern "C" int mi_moe_swiglu_forward(const void* h, void* act_out, int L, int I, int dtype, mi_moe_stream_t stream) {
   if (L < 0 || I < 1) return MI_MOE_ESHAPE;
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16 && dtype != MI_MOE_F32) return MI_MOE_EDTYPE;
@@ -159,6 +164,12 @@ extern "C" int mi_moe_swiglu_forward(const void* h, void* act_out, int L, int I,
 extern "C" int mi_moe_swiglu_backward(const void* h, const void* d_act, const void* gates,
                                       const int32_t* sorted_scattered, void* d_h, void* act_g, void* d_gates, int L,
                                       int I, int dtype, mi_moe_stream_t stream) {
+  return mi_swiglu_backward(h, d_act, gates, sorted_scattered, d_h, act_g, d_gates, nullptr, L, I, 1, dtype, stream);
+}
+
+// tokens (or null): the token of every row, its slot / k
+int mi_swiglu_backward(const void* h, const void* d_act, const void* gates, const int32_t* sorted_scattered, void* d_h, void* act_g,
+                       void* d_gates, int32_t* tokens, int L, int I, int k, int dtype, mi_moe_stream_t stream) {
   if (L < 0 || I < 1) return MI_MOE_ESHAPE;
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16 && dtype != MI_MOE_F32) return MI_MOE_EDTYPE;
   if (I % (dtype == MI_MOE_F32 ? 4 : 8) != 0) return MI_MOE_EUNSUPPORTED;
@@ -172,17 +183,17 @@ extern "C" int mi_moe_swiglu_backward(const void* h, const void* d_act, const vo
     hipLaunchKernelGGL((swiglu_backward_kernel<bf16_t>), dim3((unsigned)blocks), dim3(256), 0, s,
                        static_cast<const bf16_t*>(h), static_cast<const bf16_t*>(d_act),
                        static_cast<const bf16_t*>(gates), sorted_scattered, static_cast<bf16_t*>(d_h),
-                       static_cast<bf16_t*>(act_g), static_cast<bf16_t*>(d_gates), L, I);
+                       static_cast<bf16_t*>(act_g), static_cast<bf16_t*>(d_gates), tokens, L, I, k);
   else if (dtype == MI_MOE_F16)
     hipLaunchKernelGGL((swiglu_backward_kernel<f16_t>), dim3((unsigned)blocks), dim3(256), 0, s,
                        static_cast<const f16_t*>(h), static_cast<const f16_t*>(d_act), static_cast<const f16_t*>(gates),
                        sorted_scattered, static_cast<f16_t*>(d_h), static_cast<f16_t*>(act_g),
-                       static_cast<f16_t*>(d_gates), L, I);
+                       static_cast<f16_t*>(d_gates), tokens, L, I, k);
   else
     hipLaunchKernelGGL((swiglu_backward_kernel<float>), dim3((unsigned)blocks), dim3(256), 0, s,
                        static_cast<const float*>(h), static_cast<const float*>(d_act), static_cast<const float*>(gates),
                        sorted_scattered, static_cast<float*>(d_h), static_cast<float*>(act_g),
-                       static_cast<float*>(d_gates), L, I);
+                       static_cast<float*>(d_gates), tokens, L, I, k);
   return mi_launch_status();
 }
 

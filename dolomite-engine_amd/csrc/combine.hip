@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const T* __restrict__ 
   const int k = K > 0 ? K : k_rt;
   const int cpr = H / V;  // chunks per row
   for (int t = blockIdx.x; t < Trows; t += gridDim.x) {
-    const T* g = gates + (size_t)t * k;
+    const T* g = gates == nullptr ? nullptr : gates + (size_t)t * k;  // (none: the plain sum)
     const T* row = o + ((size_t)t * k) * H;
     for (int c = threadIdx.x; c < cpr; c += blockDim.x) {
       float acc[V];
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const T* __restrict__ 
         for (int j = 0; j < K; ++j) v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + (size_t)j * H));
 #pragma unroll
         for (int j = 0; j < K; ++j) {
-          const float gj = Elt<T>::load(g + j);
+          const float gj = g == nullptr ? 1.f : Elt<T>::load(g + j);
           float f[V];
           Chunk<T>::unpack(v[j], f);
 #pragma unroll
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const T* __restrict__ 
       } else {
 #pragma unroll 4
         for (int j = 0; j < k; ++j) {
-          const float gj = Elt<T>::load(g + j);
+          const float gj = g == nullptr ? 1.f : Elt<T>::load(g + j);
           const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + (size_t)j * H));
           float f[V];
           Chunk<T>::unpack(v, f);
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void combine_scalar_kernel(const T* __restrict
     const int h = (int)(id - (long)t * H);
     float acc = 0.f;
     for (int j = 0; j < k; ++j)
-      acc = fmaf(Elt<T>::load(gates + (size_t)t * k + j), Elt<T>::load(o + ((size_t)t * k + j) * H + h), acc);
+      acc = fmaf(gates == nullptr ? 1.f : Elt<T>::load(gates + (size_t)t * k + j), Elt<T>::load(o + ((size_t)t * k + j) * H + h), acc);
     if (tail.shared != nullptr || tail.residual != nullptr || tail.has_scale) {
       acc = Elt<T>::round(acc);
       if (tail.shared != nullptr) acc = Elt<T>::round(acc + Elt<T>::load(static_cast<const T*>(tail.shared) + id));
@@ -178,11 +178,11 @@ static int launch_combine(const void* o, const void* gates, void* y, int T_, int
 }
 
 static int combine_entry(const void* o, const void* gates, void* y, int T, int k, int H, int dtype, CombineTail tail,
-                         mi_moe_stream_t stream) {
+                         mi_moe_stream_t stream, bool gated = true) {
   if (T < 0 || k < 1 || H < 1) return MI_MOE_ESHAPE;
   if ((double)T * k * H >= 9.0e18) return MI_MOE_ESHAPE;
   if (T == 0) return MI_MOE_OK;
-  if (!o || !gates || !y) return MI_MOE_ENULL;
+  if (!o || (gated && !gates) || !y) return MI_MOE_ENULL;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {
     case MI_MOE_F32: return launch_combine<float>(o, gates, y, T, k, H, tail, s);
@@ -203,4 +203,10 @@ extern "C" int mi_moe_combine_block_tail(const void* o, const void* gates, const
                                          int dtype, mi_moe_stream_t stream) {
   const CombineTail tail = {shared, residual, residual_scale, has_scale != 0};
   return combine_entry(o, gates, y, T, k, H, dtype, tail, stream);
+}
+
+// y[t] = round(sum of token t's k rows) [+ add[t], rounded again]
+int mi_combine_sum(const void* o, const void* add, void* y, int T, int k, int H, int dtype, mi_moe_stream_t stream) {
+  const CombineTail tail = {nullptr, add, 1.0f, 0};
+  return combine_entry(o, nullptr, y, T, k, H, dtype, tail, stream, false);
 }

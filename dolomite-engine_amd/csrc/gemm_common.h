@@ -87,6 +87,7 @@ int mi_gemm_stream_form(const GemmArgs& a, bool glu, int elt);
 int mi_gemm_stream(const GemmArgs& a, int dtype, bool glu, int form, hipStream_t s);
 
 // ---- grouped_gemm.hip: one expert that owns every row, rows in place (no index arrays): out = in @ W^T, or with SwiGLU ------
+int mi_gemm_one_expert_wt(const void* in, const void* w_kn, void* out, int L, int K, int N, int dtype, mi_moe_stream_t stream);
 int mi_gemm_one_expert(const void* in, const void* w, void* out, int L, int K, int N, bool glu, int dtype, mi_moe_stream_t stream);
 
 // end of expert e's rows

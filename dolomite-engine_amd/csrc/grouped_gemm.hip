@@ -1068,6 +1068,18 @@ extern "C" int mi_moe_scattered_gemm_wt_cfg(const void* in, const void* w_kn, vo
   return run_persistent(a, dtype, PG_WEIGHT_KN, cfg < 0 ? 7 : cfg, static_cast<hipStream_t>(stream));
 }
 
+// one expert that owns every row, in place; w_kn is (K, N)
+int mi_gemm_one_expert_wt(const void* in, const void* w_kn, void* out, int L, int K, int N, int dtype, mi_moe_stream_t stream) {
+  GemmArgs a;
+  a.in = in; a.w = w_kn; a.out = out;
+  a.sorted_scattered = nullptr; a.expert_offsets = nullptr;
+  a.L = L; a.K = K; a.N = N; a.E = 1; a.kdiv = 1; a.n_tiles = 0;
+  a.gather = 0; a.scatter = 0; a.remap = 1; a.ws = nullptr; a.pre = nullptr;
+  if (!tiled_shape_ok(a, L, false, 2) || !mi_gemm_persistent_ok(a)) return MI_MOE_EUNSUPPORTED;
+  if (!tiled_aligned(a, 2)) return MI_MOE_EALIGN;
+  return run_persistent(a, dtype, PG_WEIGHT_KN, 7, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int mi_moe_scattered_gemm_wt_ws(const void* in, const void* w_kn, void* out,
                                            const int32_t* sorted_scattered, const int32_t* expert_offsets, int L,
                                            int K, int N, int E, int k, int grouped_in, int grouped_out, int dtype,

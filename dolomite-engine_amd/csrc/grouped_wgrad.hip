@@ -45,7 +45,7 @@ struct WgradArgs {
   const void* b;                  // (rows_b, N)
   const int32_t* a_idx;           // (L,) row of `a` for sorted row r, or null: r itself
   const int32_t* b_idx;           // same for `b`
-  const int32_t* expert_offsets;  // (E,) inclusive ends of the experts' row ranges
+  const int32_t* expert_offsets;  // (E,) inclusive ends of the experts' row ranges (null: one expert owns all rows)
   float* partial;                 // [group][row block][column block][lane]: blocks of 16 x 16, four values a lane
   void* dw;                       // (E, M, N): written directly for an expert with a single group
   int* next_item;                 // plan: [0..8) per-XCD work counters, zero on entry; [8..17) first slot of each XCD
@@ -58,7 +58,7 @@ struct WgradArgs {
 struct WgradTable {
   int groups[4], end[4];
 };
-__device__ __forceinline__ void wgrad_table(const int32_t* __restrict__ off, int E, int chunk, WgradTable& tb) {
+__device__ __forceinline__ void wgrad_table(const int32_t* __restrict__ off, int L, int E, int chunk, WgradTable& tb) {
   const int lane = threadIdx.x & 63;
   int carry = 0;
 #pragma unroll
@@ -67,7 +67,7 @@ __device__ __forceinline__ void wgrad_table(const int32_t* __restrict__ off, int
     tb.end[c] = 0;
     if (c * 64 >= E) continue;
     const int e = c * 64 + lane;
-    const int end = e < E ? off[e] : 0;
+    const int end = e < E ? (off != nullptr ? off[e] : L) : 0;
     const int prev = (e < E && e > 0) ? off[e - 1] : 0;
     int incl = e < E ? (end - prev + chunk - 1) / chunk : 0;
 #pragma unroll
@@ -105,7 +105,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a) {
   const int upper = lane >> 5;
 
   WgradTable tb;
-  if constexpr (PLAN) wgrad_table(a.expert_offsets, a.E, a.chunk, tb);
+  if constexpr (PLAN) wgrad_table(a.expert_offsets, a.L, a.E, a.chunk, tb);
   const int tiles = a.m_tiles * a.n_tiles;
   const int xcd = blockIdx.x & 7;
   // this XCD's groups: slots [xfirst, xfirst + xgroups) of the planned list
@@ -182,7 +182,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a) {
     if constexpr (!PLAN) {
       expert = item / tiles;
       r0 = expert > 0 ? a.expert_offsets[expert - 1] : 0;
-      r1 = a.expert_offsets[expert];
+      r1 = a.expert_offsets != nullptr ? a.expert_offsets[expert] : a.L;
       if (r1 <= r0) {                               // no rows: zeros
         T* __restrict__ out = static_cast<T*>(a.dw) + (size_t)expert * a.M * a.N;
         const int n = nt * TILE + (threadIdx.x & 31) * 8;
@@ -471,7 +471,7 @@ template <typename T, bool GA, bool GB> __global__ __launch_bounds__(256, 1) voi
 //   plan[red_at..)  (expert, first group, groups) of each of those experts, in expert order
 // Up to WGRAD_PLAN_SORT groups are ranked; beyond that the groups are dealt in row order.
 #define WGRAD_PLAN_SORT 8192
-__global__ __launch_bounds__(1024) void wgrad_plan_kernel(const int32_t* __restrict__ offsets, int E, int chunk,
+__global__ __launch_bounds__(1024) void wgrad_plan_kernel(const int32_t* __restrict__ offsets, int L, int E, int chunk,
                                                           int* __restrict__ plan, int red_at) {
   __shared__ int first[WGRAD_MAX_E + 1];  // groups in front of expert e
   __shared__ int ends[WGRAD_MAX_E];       // the offsets (one round trip to memory for all of them)
@@ -479,7 +479,7 @@ __global__ __launch_bounds__(1024) void wgrad_plan_kernel(const int32_t* __restr
   __shared__ int rows[WGRAD_PLAN_SORT];
   const int tid = threadIdx.x;
   if (tid < 8) plan[tid] = 0;
-  for (int e = tid; e < E; e += blockDim.x) ends[e] = offsets[e];
+  for (int e = tid; e < E; e += blockDim.x) ends[e] = offsets != nullptr ? offsets[e] : L;
   __syncthreads();
   // groups of expert e, then every expert adds up the ones in front of it by itself (E <= 256: no scan needed)
   for (int e = tid; e < E; e += blockDim.x) {
@@ -658,16 +658,17 @@ template <typename T> static int launch_wgrad(const WgradArgs& g, int grid, int 
   return mi_launch_status();
 }
 
-extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx,
-                                    const int32_t* expert_offsets, void* dw, void* workspace, size_t workspace_bytes,
-                                    int L, int a_rows, int b_rows, int M, int N, int E, int dtype, mi_moe_stream_t stream) {
+// (no expert_offsets: one expert owns all rows)
+int mi_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx, const int32_t* expert_offsets, void* dw,
+                     void* workspace, size_t workspace_bytes, int L, int a_rows, int b_rows, int M, int N, int E, int dtype,
+                     mi_moe_stream_t stream, bool need_offsets) {
   if (L < 0 || M < 1 || N < 1 || E < 1) return MI_MOE_ESHAPE;
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16) return MI_MOE_EDTYPE;
   if (M % 8 != 0 || N % 8 != 0 || E > WGRAD_MAX_E) return MI_MOE_EUNSUPPORTED;
   if (a_rows < 0 || b_rows < 0) return MI_MOE_ESHAPE;
   // rows are addressed with 32-bit byte offsets
   if ((uint64_t)a_rows * M * 2 >= (1ull << 32) || (uint64_t)b_rows * N * 2 >= (1ull << 32)) return MI_MOE_EUNSUPPORTED;
-  if (!dw || !expert_offsets) return MI_MOE_ENULL;
+  if (!dw || (!expert_offsets && (need_offsets || E != 1))) return MI_MOE_ENULL;
   if (L > 0 && (!a || !b)) return MI_MOE_ENULL;
   if (!mi_aligned(a, 16) || !mi_aligned(b, 16) || !mi_aligned(dw, 16) || !mi_aligned(workspace, 16)) return MI_MOE_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -686,7 +687,7 @@ extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const v
   const bool whole = wgrad_whole_experts(L, E);
   if (L > 0 && !whole) {
     g.next_item = reinterpret_cast<int*>(static_cast<unsigned char*>(workspace) + wgrad_slab_bytes(max_groups, M, N));
-    hipLaunchKernelGGL(wgrad_plan_kernel, dim3(1), dim3(1024), 0, s, expert_offsets, E, g.chunk, g.next_item, red_at);
+    hipLaunchKernelGGL(wgrad_plan_kernel, dim3(1), dim3(1024), 0, s, expert_offsets, L, E, g.chunk, g.next_item, red_at);
   }
   g.m_tiles = mi_ceil_div(M, 256);
   g.n_tiles = mi_ceil_div(N, 256);
@@ -699,6 +700,12 @@ extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const v
   const long per_xcd = whole ? ((long)E * tiles + 7) / 8 : (max_groups + 7) / 8 * tiles;
   const long grid = 8 * (per_xcd < cus / 8 ? per_xcd : (cus + 7) / 8);
   return dtype == MI_MOE_BF16 ? launch_wgrad<bf16_t>(g, (int)grid, red_at, s) : launch_wgrad<f16_t>(g, (int)grid, red_at, s);
+}
+
+extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx,
+                                    const int32_t* expert_offsets, void* dw, void* workspace, size_t workspace_bytes,
+                                    int L, int a_rows, int b_rows, int M, int N, int E, int dtype, mi_moe_stream_t stream) {
+  return mi_grouped_wgrad(a, a_idx, b, b_idx, expert_offsets, dw, workspace, workspace_bytes, L, a_rows, b_rows, M, N, E, dtype, stream, true);
 }
 
 // ---- fp32 weight gradient on the matrix cores ----------------------------------------------------------------

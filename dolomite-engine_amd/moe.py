@@ -29,7 +29,7 @@ import torch.nn.functional as F
 
 from . import ops
 from .activations import GLUActivation, get_activation_function, is_glu
-from .autograd import FusedRouter, ScatteredSwiGLUExperts, SwitchAuxLoss, one_expert_rows
+from .autograd import FusedRouter, RoutedExperts, ScatteredSwiGLUExperts, SwitchAuxLoss, one_expert_rows
 from .enums import Kernel
 from .kernels import is_kernel_allowed
 from .linear import ParameterizedLinear
@@ -254,6 +254,22 @@ class MoE(nn.Module):
                 add_aux_loss(0)
                 return y if self.use_padding_free_transformer else y.reshape(batch_size, sequence_length, self.hidden_size)
 
+        if self.training and pre_norm is None and self._fused_swiglu and self.keep_preactivation:
+            # training: router, routed experts and auxiliary loss behind one library call in either direction (None: as above)
+            trained = self._train_native(hidden_states)
+            if trained is not None:
+                moe_output, aux_loss = trained
+                if self.shared_intermediate_size is not None:
+                    moe_output = moe_output + self._compute_shared_experts(hidden_states)
+                if not self.use_padding_free_transformer:
+                    moe_output = moe_output.reshape(batch_size, sequence_length, self.hidden_size)
+                if residual_scale is not None:
+                    moe_output = moe_output * residual_scale
+                if residual is not None:
+                    moe_output = moe_output + residual.reshape(moe_output.shape)
+                add_aux_loss(aux_loss)
+                return moe_output
+
         routed = None
         presorted = None
         if pre_norm is None and self._use_fused_router(hidden_states) and ops.router_fused_sort_supported(
@@ -371,6 +387,23 @@ class MoE(nn.Module):
             logits = self._unfused_logits(hidden_states)
         return ops.layer_forward(hidden_states, gate_weight, self.router_logit_bias, self.top_k, *weights,
                                  shared_fc, shared_proj, residual, residual_scale, pre_norm, logits), logits
+
+    def _train_native(self, hidden_states: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor] | None:
+        """(expert output, auxiliary loss) through autograd.RoutedExperts, None where it does not take the call."""
+        if not (is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda and torch.is_grad_enabled()
+                and ops._TIMER is None and self._stages_as_written()):
+            return None
+        fc, proj, gate = self._modules_by_name("c_fc", "c_proj", "gate")
+        if fc.weight_q is not None or proj.weight_q is not None or fc.bias is not None or proj.bias is not None:
+            return None
+        gate_weight, bias = gate.weight, self.router_logit_bias
+        # (with a router that has no gradient the loss has none either)
+        if not (hidden_states.requires_grad or gate_weight.requires_grad):
+            return None
+        sizes = ops.layer_train_sizes(hidden_states, gate_weight, bias, fc.weight, proj.weight, self.top_k)
+        if sizes is None:
+            return None
+        return RoutedExperts.apply(hidden_states, gate_weight, fc.weight, proj.weight, bias, self.top_k, sizes)
 
     def _unfused_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         """Router logits of shapes the router kernel does not take (more than 256 experts, a hidden size that is not a

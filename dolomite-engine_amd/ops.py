@@ -13,6 +13,7 @@ compositions are in ``autograd.py``).
 
 from __future__ import annotations
 
+import ctypes
 import functools
 
 import torch
@@ -1022,3 +1023,85 @@ def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor
         return None
     check(rc)
     return y
+
+
+# ------------------------------------------------------------------------------------------------
+# a training step's routed experts
+# ------------------------------------------------------------------------------------------------
+
+
+@functools.lru_cache(maxsize=256)
+def _layer_train_sizes(dev: int, T: int, H: int, E: int, k: int, I: int, code: int) -> tuple[int, int, int, int] | None:
+    """Bytes of what the forward keeps and of either direction's workspace, and a contraction length that may use the split-K
+    workspace (or 0): functions of the sizes and of the current device's compute units alone.  None: not a shape of the calls."""
+    lib = _lib.load()
+    sizes = [ctypes.c_size_t() for _ in range(3)]
+    if lib.mi_moe_layer_train_sizes(T, H, E, k, I, code, *(ctypes.byref(s) for s in sizes)) != 0:
+        return None
+    splits = next((K for K in (H, I, 2 * I) if lib.mi_moe_grouped_gemm_splits(K, code)), 0)
+    return (*(s.value for s in sizes), splits)
+
+
+def layer_train_sizes(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor | None, w_fc: torch.Tensor,
+                      w_proj: torch.Tensor, k: int) -> tuple[int, int, int, int] | None:
+    """What :func:`layer_train_forward` needs to know, or None for anything the stages' own wrappers have to look at."""
+    dev, dtype = x.get_device(), x.dtype
+    code = _DTYPE_CODE.get(dtype)
+    if code is None or code == F32 or dev < 0 or dev != _current_device() or x.dim() != 2 or w_fc.dim() != 3:
+        return None
+    T, H = x.shape
+    E, I2, _ = w_fc.shape
+    I = I2 // 2
+    if I2 % 2 or gate_weight.shape != (E, H) or w_fc.shape != (E, I2, H) or w_proj.shape != (E, H, I):
+        return None
+    for t in (x, gate_weight, w_fc, w_proj):
+        if t.dtype != dtype or t.get_device() != dev or not t.is_contiguous() or t.data_ptr() % 16:
+            return None
+    if bias is not None and (bias.shape != (E,) or bias.dtype != torch.float32 or bias.get_device() != dev
+                             or not bias.is_contiguous() or bias.requires_grad):
+        return None
+    return _layer_train_sizes(dev, T, H, E, k, I, code)
+
+
+def layer_train_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor | None, w_fc: torch.Tensor,
+                        w_proj: torch.Tensor, k: int, sizes: tuple[int, int, int, int]):
+    """(y (T, H), auxiliary loss (0-d, x's dtype), what the backward needs) of a training step's routed experts in one library
+    call: the launches of autograd.FusedRouter, SwitchAuxLoss and ScatteredSwiGLUExperts."""
+    T, H = x.shape
+    E, I2, _ = w_fc.shape
+    saved_bytes, ws_bytes, _, splits = sizes
+    dev = x.device
+    y = torch.empty_like(x)
+    aux = torch.empty((), dtype=x.dtype, device=dev)
+    saved = torch.empty(saved_bytes, dtype=torch.uint8, device=dev)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    gemm_ws, gemm_bytes = _gemm_workspace(dev, splits, x.dtype) if splits else (None, 0)
+    check(_lib.load().mi_moe_layer_train_forward(
+        x.data_ptr(), gate_weight.data_ptr(), _ptr(bias), w_fc.data_ptr(), w_proj.data_ptr(), y.data_ptr(), aux.data_ptr(),
+        saved.data_ptr(), saved_bytes, T, H, E, k, I2 // 2, _code(x.dtype), ws.data_ptr(), ws_bytes, _ptr(gemm_ws), gemm_bytes,
+        _stream()))
+    return y, aux, saved
+
+
+def layer_train_backward(x: torch.Tensor, gate_weight: torch.Tensor, w_fc: torch.Tensor, w_proj: torch.Tensor,
+                         saved: torch.Tensor, dy: torch.Tensor | None, d_aux: torch.Tensor | None, k: int,
+                         wanted: tuple[bool, bool, bool, bool], sizes: tuple[int, int, int, int]):
+    """Gradients of x, the gate, the up- and the down-projection (None where not ``wanted``, or where nothing arrives)."""
+    _dev(x, gate_weight, w_fc, w_proj, saved, dy, d_aux)
+    _no_grad(x, gate_weight, w_fc, w_proj, dy, d_aux)
+    T, H = x.shape
+    E, I2, _ = w_fc.shape
+    if dy is not None:
+        dy = dy.contiguous()
+        if dy.data_ptr() % 16:
+            dy = dy.clone()
+    saved_bytes, _, ws_bytes, splits = sizes
+    # (the experts' weights get no gradient from the auxiliary loss alone)
+    grads = [torch.empty_like(t) if want and (i < 2 or dy is not None) else None
+             for i, (t, want) in enumerate(zip((x, gate_weight, w_fc, w_proj), wanted))]
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+    gemm_ws, gemm_bytes = _gemm_workspace(x.device, splits, x.dtype) if splits else (None, 0)
+    check(_lib.load().mi_moe_layer_train_backward(
+        x.data_ptr(), gate_weight.data_ptr(), w_fc.data_ptr(), w_proj.data_ptr(), saved.data_ptr(), saved_bytes, _ptr(dy), _ptr(d_aux),
+        *(_ptr(g) for g in grads), T, H, E, k, I2 // 2, _code(x.dtype), ws.data_ptr(), ws_bytes, _ptr(gemm_ws), gemm_bytes, _stream()))
+    return grads

@@ -455,6 +455,24 @@ int mi_moe_layer_forward(const void* x, const void* norm_w, float norm_eps, int 
                          int T, int H, int E, int k, int I, int S, int dtype, void* ws, size_t ws_bytes, void* gemm_ws,
                          size_t gemm_ws_bytes, mi_moe_stream_t stream);
 
+/* ---- a training step's routed experts -----------------------------------------------------------------------------------
+ * MoE.forward in training mode with a SwiGLU activation (moe.py:212-290, the auxiliary loss of moe.py:346-369) and its backward, one
+ * call each: F16 / BF16, E <= 64 and a multiple of 8, k <= 8, H % 16 == 0, I % 8 == 0, operands under 2^31 elements
+ * (MI_MOE_EUNSUPPORTED otherwise), all pointers 16-byte aligned.  mi_moe_layer_train_sizes gives the bytes of `saved` (the pre-activation,
+ * routing and loss terms that the forward leaves for the backward) and of either call's workspace.
+ *   forward: y (T, H), aux_loss one value of `dtype`.
+ *   backward: dy (T, H) or NULL (no gradient reached y), d_aux one value of `dtype` or NULL; dx (T, H), d_gate_w (E, H), d_w_fc
+ *   (E, 2I, H), d_w_proj (E, H, I), each NULL where it is not wanted (the last two without dy: refused).
+ * gemm_ws: as in the _ws calls (or NULL). */
+int mi_moe_layer_train_sizes(int T, int H, int E, int k, int I, int dtype, size_t* saved, size_t* forward_ws, size_t* backward_ws);
+int mi_moe_layer_train_forward(const void* x, const void* gate_w, const float* gate_bias, const void* w_fc, const void* w_proj,
+                               void* y, void* aux_loss, void* saved, size_t saved_bytes, int T, int H, int E, int k, int I, int dtype,
+                               void* ws, size_t ws_bytes, void* gemm_ws, size_t gemm_ws_bytes, mi_moe_stream_t stream);
+int mi_moe_layer_train_backward(const void* x, const void* gate_w, const void* w_fc, const void* w_proj, const void* saved,
+                                size_t saved_bytes, const void* dy, const void* d_aux, void* dx, void* d_gate_w, void* d_w_fc, void* d_w_proj,
+                                int T, int H, int E, int k, int I, int dtype, void* ws, size_t ws_bytes, void* gemm_ws,
+                                size_t gemm_ws_bytes, mi_moe_stream_t stream);
+
 /*
  * Diagnostics (no counterpart in the reference; nothing in the layer calls them): the pieces of the persistent grouped GEMM's
  * inner loop in isolation, for a benchmark that wants measured rates beside the grouped GEMM's own figure.  One workgroup

@@ -1,0 +1,123 @@
+"""A training step's routed experts behind one library call in either direction against the stage-by-stage functions that it
+stands for.  The same kernels in the same order on the same operands: results are the same bits, but for d logits, whose two parts
+one kernel forms (the compiler may contract its products otherwise: at most one rounding step of the model dtype, 2^-8 in bf16
+and 2^-11 in fp16, on what the gate and the router's part of dx are made of)."""
+
+import pytest
+import torch
+
+from dolomite_engine_amd import Kernel, MoE, enable_kernels
+from dolomite_engine_amd.loss import clear_aux_loss, get_aux_loss
+
+pytestmark = pytest.mark.gpu
+
+SIZES = {"even": (512, 256, 16, 4, 264), "wide": (96, 1024, 8, 2, 520), "small": (5, 128, 8, 8, 64), "one": (1, 64, 8, 1, 8),
+         "large": (3000, 256, 40, 8, 128), "blocks": (2049, 128, 64, 6, 64)}
+
+
+def _layer(device, dtype, sizes, shared=None):
+    T, H, E, k, I = sizes
+    torch.manual_seed(T)
+    layer = MoE(hidden_size=H, intermediate_size=I, shared_intermediate_size=shared, num_experts=E, num_experts_per_tok=k,
+                activation_function="swiglu", add_bias=False, dropout=0.0, init_method="normal", initializer_range=0.1,
+                m_width=None, num_layers=1, use_padding_free_transformer=True).to(device).to(dtype).train()
+    return layer, torch.randn(T, H, device=device).to(dtype)
+
+
+def _step(layer, x, parts="both", x_grad=True, dy_form="plain", scale=None):
+    layer.zero_grad(set_to_none=True)
+    x = x.detach().clone().requires_grad_(x_grad)
+    clear_aux_loss()
+    with enable_kernels([Kernel.scattermoe]):
+        y = layer(x, **({} if scale is None else dict(residual=x, residual_scale=scale)))
+        aux = get_aux_loss()
+        torch.manual_seed(7)
+        dy = torch.randn(*y.shape, device=y.device).to(y.dtype)
+        if dy_form == "strided":
+            dy = torch.stack([dy, dy], dim=-1)[..., 0]
+        elif dy_form == "misaligned":
+            dy = torch.cat([dy.reshape(-1)[:1], dy.reshape(-1)])[1:].view_as(dy)
+        wanted = [(y, dy), (aux, torch.full_like(aux, 0.3))]
+        if parts != "both":
+            wanted = wanted[:1] if parts == "y" else wanted[1:]
+        torch.autograd.backward(*zip(*wanted))
+    out = {"y": y.detach(), "aux": aux.detach(), "x": x.grad}
+    return out | {n: p.grad for n, p in layer.named_parameters()}
+
+
+def _check(monkeypatch, dtype, layer, x, **how):
+    taken = []
+    native = MoE._train_native
+    monkeypatch.setattr(MoE, "_train_native", lambda self, h: taken.append(native(self, h)) or taken[-1])
+    got = _step(layer, x, **how)
+    assert taken and taken[-1] is not None, "the one-call form did not run"
+    monkeypatch.setattr(MoE, "_train_native", lambda self, h: None)
+    want = _step(layer, x, **how)
+    monkeypatch.undo()
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for name, w in want.items():
+        g = got[name]
+        assert (g is None) == (w is None), name
+        if w is None:
+            continue
+        assert g.dtype == w.dtype and g.shape == w.shape, name
+        if name in ("x", "gate.weight"):
+            # an entry is a sum over tokens or experts of terms that are each off by a rounding step at most
+            assert (g.float() - w.float()).norm() <= 2 * eps * w.float().norm(), name
+        else:
+            assert torch.equal(g, w), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("name", list(SIZES))
+def test_equals_stages(device, monkeypatch, name, dtype):
+    layer, x = _layer(device, dtype, SIZES[name])
+    print(f"train native {name} {dtype}", flush=True)
+    _check(monkeypatch, dtype, layer, x)
+
+
+@pytest.mark.parametrize("how", [dict(parts="y"), dict(parts="aux"), dict(x_grad=False), dict(parts="aux", x_grad=False),
+                                 dict(dy_form="strided"), dict(scale=0.25)])
+def test_parts_and_forms(device, monkeypatch, how):
+    layer, x = _layer(device, torch.bfloat16, SIZES["even"])
+    print(f"train native {how}", flush=True)
+    _check(monkeypatch, torch.bfloat16, layer, x, **how)
+
+
+def test_misaligned_gradient(device):
+    """(The stages refuse an upstream gradient that does not start on 16 bytes.)"""
+    layer, x = _layer(device, torch.bfloat16, SIZES["even"])
+    want, got = _step(layer, x), _step(layer, x, dy_form="misaligned")
+    assert all(torch.equal(got[n], w) for n, w in want.items())
+
+
+@pytest.mark.parametrize("frozen", [("gate",), ("c_fc",), ("c_proj",), ("c_fc", "c_proj"), ("gate", "c_fc", "c_proj")])
+def test_frozen_parameters_get_no_gradient(device, frozen):
+    layer, x = _layer(device, torch.bfloat16, SIZES["even"], shared=64)
+    full = _step(layer, x)
+    for name in frozen:
+        getattr(layer, name).weight.requires_grad_(False)
+    part = _step(layer, x)
+    for name, g in part.items():
+        if name.split(".")[0] in frozen:
+            assert g is None, name
+        else:
+            assert torch.equal(g, full[name]), name
+
+
+def test_router_without_a_gradient_leaves_the_loss_without_one(device):
+    layer, x = _layer(device, torch.bfloat16, SIZES["even"])
+    layer.gate.weight.requires_grad_(False)
+    clear_aux_loss()
+    with enable_kernels([Kernel.scattermoe]):
+        y = layer(x)
+    assert y.requires_grad and not get_aux_loss().requires_grad
+
+
+def test_replaced_stage_is_called(device):
+    layer, x = _layer(device, torch.bfloat16, SIZES["even"])
+    calls = []
+    compute = layer._compute_experts
+    layer._compute_experts = lambda *a, **k: calls.append(1) or compute(*a, **k)
+    _step(layer, x)
+    assert calls
