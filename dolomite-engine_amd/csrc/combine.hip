@@ -72,7 +72,9 @@ __device__ __forceinline__ void combine_tail(float (&acc)[V], const CombineTail&
   }
 }
 
-template <typename T, int K>
+// GATED: rows are weighted with the token's gates (else: the plain sum.  A test of the pointer in place of the parameter costs the
+// weighted form 1 us: 385 tokens of 32 experts, 1024 / 512, layer 82.0 -> 82.9 us.)
+template <typename T, int K, bool GATED = true>
 __global__ __launch_bounds__(256) void combine_vec_kernel(const T* __restrict__ o, const T* __restrict__ gates,
                                                           T* __restrict__ y, int Trows, int k_rt, int H,
                                                           CombineTail tail) {
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const T* __restrict__ 
   const int k = K > 0 ? K : k_rt;
   const int cpr = H / V;  // chunks per row
   for (int t = blockIdx.x; t < Trows; t += gridDim.x) {
-    const T* g = gates == nullptr ? nullptr : gates + (size_t)t * k;  // (none: the plain sum)
+    const T* g = GATED ? gates + (size_t)t * k : nullptr;
     const T* row = o + ((size_t)t * k) * H;
     for (int c = threadIdx.x; c < cpr; c += blockDim.x) {
       float acc[V];
@@ -93,7 +95,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const T* __restrict__ 
         for (int j = 0; j < K; ++j) v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + (size_t)j * H));
 #pragma unroll
         for (int j = 0; j < K; ++j) {
-          const float gj = g == nullptr ? 1.f : Elt<T>::load(g + j);
+          const float gj = GATED ? Elt<T>::load(g + j) : 1.f;
           float f[V];
           Chunk<T>::unpack(v[j], f);
 #pragma unroll
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const T* __restrict__ 
       } else {
 #pragma unroll 4
         for (int j = 0; j < k; ++j) {
-          const float gj = g == nullptr ? 1.f : Elt<T>::load(g + j);
+          const float gj = GATED ? Elt<T>::load(g + j) : 1.f;
           const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + (size_t)j * H));
           float f[V];
           Chunk<T>::unpack(v, f);
@@ -147,7 +149,8 @@ static void launch_combine_vec(const void* o, const void* gates, void* y, int T_
   // one workgroup per token row as long as the grid allows: handed out one by one as workgroups retire, the rows
   // stream faster than with a fixed share of rows per workgroup (32768 tokens of 1536: 0.163 -> 0.156 ms)
   if (blocks > (1L << 20)) blocks = 1L << 20;
-  hipLaunchKernelGGL((combine_vec_kernel<T, K>), dim3((unsigned)blocks), dim3(threads), 0, s,
+  auto kern = gates != nullptr ? combine_vec_kernel<T, K, true> : combine_vec_kernel<T, K, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(threads), 0, s,
                      static_cast<const T*>(o), static_cast<const T*>(gates), static_cast<T*>(y), T_, k, H, tail);
 }
 
