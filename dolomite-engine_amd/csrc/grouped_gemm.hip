@@ -493,6 +493,8 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_kernel(GemmArgs a) {
 //       s_barrier                  : tile kt+1 complete, stage cur free
 //       B: MFMA(step 1, buf1)      | ds_read step 0 of tile kt+1 -> buf0 | DMA tile kt+4 -> stage cur
 // The waits are explicit (s_waitcnt immediates); a fence-carrying __syncthreads would drain all DMA.
+// (Eight stages where a CU has one workgroup: one expert of 509 rows, 1024 -> 512 SwiGLU, 12.5 -> 12.9 us.)
+// KTAIL: the last slice has fewer than 32 values of k.  Lanes past them fetch the row's last chunk, and their fragments are zeros.
 // ------------------------------------------------------------------------------------------------
 
 __device__ __forceinline__ constexpr int waitcnt_imm(int vm, int lgkm) {
@@ -520,7 +522,7 @@ __device__ __forceinline__ void dma16_to_lds(const void* base, uint32_t byte_off
                  : "memory", "m0");
 }
 
-template <typename T, int BM, int BNW, int WM, int WN, bool GLU>
+template <typename T, int BM, int BNW, int WM, int WN, bool GLU, bool KTAIL>
 __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GemmArgs a) {
   constexpr int BK = 32;
   constexpr int NSTAGE = 4;
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GemmArgs 
   constexpr int LD_PER = (NLD + NMFMA - 1) / NMFMA;
   static_assert(ROWS % (16 * NW) == 0 && BM % 16 == 0, "tile/wave shape");
   static_assert(!GLU || NB % 2 == 0, "SwiGLU needs an even number of column blocks per wave");
-  static_assert(3 * NLD <= 63, "vmcnt range");
+  static_assert((NSTAGE - 1) * NLD <= 63 && (NSTAGE & (NSTAGE - 1)) == 0, "vmcnt range");
   typedef typename Mfma32<T>::vec frag_t;
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   typedef const __attribute__((address_space(1))) void* glb_ptr_t;
@@ -580,9 +582,11 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GemmArgs 
       src[j] = wbase + ((size_t)half * a.N + col) * a.K + lchunk * 8;
     }
   }
-  const int nk = a.K / BK;
+  const int nk = KTAIL ? (a.K + BK - 1) / BK : a.K / BK;
+  const int k_last = KTAIL ? a.K - 8 - lchunk * 8 : 0;  // where the lane's last chunk of a row begins, less its place in a slice
   auto dma_tile = [&](int kt, int stage) {
-    const int k0 = (kt < nk ? kt : nk - 1) * BK;  // surplus rounds re-fetch the last tile; never consumed
+    int k0 = (kt < nk ? kt : nk - 1) * BK;  // surplus rounds re-fetch the last tile; never consumed
+    if (KTAIL && k0 > k_last) k0 = k_last;
 #pragma unroll
     for (int j = 0; j < NLD; ++j) {
       unsigned char* dst = smem_raw + stage * STAGE_BYTES + (j * NW + wave) * 1024;
@@ -635,19 +639,26 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GemmArgs 
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = Mfma32<T>::run(wf[buf][nb], xf[buf][mb], acc[nb][mb]);
   };
+  auto trim = [&](int kt, int kk) {                 // values past K: zeros in both operands
+    const bool in = kt * BK + kk * 16 + fhalf * 8 < a.K;
+    const frag_t none = {};
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) wf[kk][nb] = in ? wf[kk][nb] : none;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) xf[kk][mb] = in ? xf[kk][mb] : none;
+  };
 
   // ---- pipeline ----------------------------------------------------------------------------------------
-  dma_tile(0, 0);
-  dma_tile(1, 1);
-  dma_tile(2, 2);
-  dma_tile(3, 3);
-  __builtin_amdgcn_s_waitcnt(waitcnt_imm(3 * NLD, 0));
+#pragma unroll
+  for (int kt = 0; kt < NSTAGE; ++kt) dma_tile(kt, kt);
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm((NSTAGE - 1) * NLD, 0));
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   read_frags(0, 0, 0);
 
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & (NSTAGE - 1), nxt = (kt + 1) & (NSTAGE - 1);
+    if (KTAIL && kt == nk - 1) trim(kt, 0);
     read_frags(cur, 1, 1);
     mfma_step(0);
 #pragma unroll
@@ -657,13 +668,14 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GemmArgs 
     }
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * NLD, 0));
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm((NSTAGE - 2) * NLD, 0));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 
+    if (KTAIL && kt == nk - 1) trim(kt, 1);
     read_frags(nxt, 0, 0);
-    dma_tile(kt + 4, cur);
+    dma_tile(kt + NSTAGE, cur);
     mfma_step(1);
 #pragma unroll
     for (int i = 0; i < NMFMA; ++i) {
@@ -767,11 +779,11 @@ static int launch_tiled_w8(GemmArgs a, hipStream_t s) {
   return launch_tiled_k<T, BM, BNW, WM, WN, GLU, true, true>(a, s);
 }
 
-template <typename T, int BM, int BNW, int WM, int WN, bool GLU>
+template <typename T, int BM, int BNW, int WM, int WN, bool GLU, bool KTAIL>
 static int launch_dma(GemmArgs a, hipStream_t s) {
   constexpr int BN = GLU ? BNW / 2 : BNW;
   constexpr size_t lds = 4ull * (BM + BNW) * 32 * sizeof(T);
-  auto kern = grouped_gemm_dma_kernel<T, BM, BNW, WM, WN, GLU>;
+  auto kern = grouped_gemm_dma_kernel<T, BM, BNW, WM, WN, GLU, KTAIL>;
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> lds_ok{0};
     const int rc = mi_allow_lds_once(reinterpret_cast<const void*>(kern), (int)lds, lds_ok);
@@ -784,6 +796,20 @@ static int launch_dma(GemmArgs a, hipStream_t s) {
   if (grid > 0x7fffffffL) return MI_MOE_ESHAPE;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(WM * WN * 64), lds, s, a);
   return mi_launch_status();
+}
+
+// 128 x 128 tiles of an experts' average load
+static double small_tiles(const GemmArgs& a, bool glu) {
+  return (double)a.E * mi_ceil_div(mi_ceil_div(a.L, a.E), 128) * mi_ceil_div(a.N, glu ? 64 : 128);
+}
+
+// The 128 x 128 tiles of a contraction that is no multiple of 32 come by DMA as well while there is at most one to a CU.  Staged through
+// registers / by DMA, us: one expert of 3001 rows, 920 -> 344 SwiGLU fp16 17.4 / 15.6 (144 tiles); 8 experts of 375, 1000 -> 392 18.3 / 16.2
+// (168); 7 of 171, 472 -> 200 11.1 / 10.1 (56); but 8 of 750, 1000 -> 392 29.3 / 31.6 (336) and 17 of 188, 920 -> 520 27.5 / 28.6 (306).
+template <typename T, bool GLU>
+static int launch_128x128(const GemmArgs& a, hipStream_t s) {
+  if (a.K % 32 != 0 && small_tiles(a, GLU) <= 256) return launch_dma<T, 128, 128, 2, 2, GLU, true>(a, s);
+  return launch_tiled<T, 128, 128, 2, 2, GLU>(a, s);
 }
 
 // Cache policy of the persistent kernel's output stores.  The plain form's output -- the (slots, hidden) rows the
@@ -893,10 +919,10 @@ template <typename T, bool GLU>
 static int dispatch_cfg(GemmArgs a, int cfg, hipStream_t s) {
   switch (cfg) {
     case 0: return launch_tiled<T, 256, 256, 2, 2, GLU>(a, s);
-    case 1: return launch_tiled<T, 128, 128, 2, 2, GLU>(a, s);
+    case 1: return launch_128x128<T, GLU>(a, s);
     case 2: return launch_tiled<T, 32, 256, 1, 4, GLU>(a, s);
     case 5: return launch_tiled<T, 32, 128, 1, 2, GLU>(a, s);
-    case 4: return a.K % 32 == 0 ? launch_dma<T, 128, 128, 2, 2, GLU>(a, s) : MI_MOE_EUNSUPPORTED;
+    case 4: return a.K % 32 == 0 ? launch_dma<T, 128, 128, 2, 2, GLU, false>(a, s) : MI_MOE_EUNSUPPORTED;
     default: return run_persistent(a, std::is_same<T, bf16_t>::value ? MI_MOE_BF16 : MI_MOE_F16, GLU ? PG_SWIGLU : PG_PLAIN, cfg, s);
   }
 }
@@ -932,14 +958,15 @@ static bool tiled_aligned(const GemmArgs& a, int elt_bytes) {
 // Beyond that the 128 x 128 tiles win while they are at most one to a CU (experts chosen by random logits, cold weights, up
 // projection: 24 experts of 120 rows, 1024 -> 512 (240 of them) 28.9 / 20.9; 12 experts, 2048 -> 1024 (240) 47.2 / 36.4; 6 experts,
 // 4096 -> 1792 (210) 81.8 / 63.6; but 32 experts, 1024 -> 512 (320) 29.3 / 32.8 and 24 of 150 rows (384) 29.2 / 27.0, with their
-// down-projections 48.2 / 46.3), and where K is ragged, which costs the 256 x 256 tiles' DMA half lines, while they are
-// all resident, two to a CU (920 -> 520: 24 experts of 240 rows (432) 35.2 / 32.8, 17 of 300 (459) 32.2 / 29.3, 20 of 300 (540) 33.0 /
-// 46.7, 24 of 300 (648) 34.6 / 49.1).
+// down-projections 48.2 / 46.3).  Where K is ragged, which costs the persistent tiles' DMA half lines, up to 256 of them (17.3 / 16.2,
+// 16.8 / 14.7; but 17 of 188 rows, 920 -> 520 (306) 20.9 / 27.5 and back (272) 14.6 / 17.9, 8 of 750, 1000 -> 392 (336) 20.2 / 29.3 and
+// back (384) 14.8 / 16.7), and for contractions below 256 while they are all resident, two to a CU.
 static bool few_large_tiles(const GemmArgs& a, bool glu) {
   const int avg = (a.L + a.E - 1) / a.E;
+  if (a.K % 32 != 0 && a.K >= 256) return small_tiles(a, glu) <= 256;
   if ((double)a.E * mi_ceil_div(avg, 256) * mi_ceil_div(a.N, glu ? 128 : 256) <= 72) return true;
   // (a quarter of the experts has a row tile more than the average one)
-  const double small = (double)a.E * mi_ceil_div(avg, 128) * mi_ceil_div(a.N, glu ? 64 : 128);
+  const double small = small_tiles(a, glu);
   return a.K % 32 == 0 ? 1.25 * small <= 256 : small <= 512;
 }
 
