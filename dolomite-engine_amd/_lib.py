@@ -71,6 +71,7 @@ SIGNATURES: dict[str, tuple] = {
     "mi_moe_layer_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i, _i, _i]),
     "mi_moe_layer_forward": (_i, [_vp, _vp, ctypes.c_float, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp,
                                   ctypes.c_float, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp, _sz, _vp]),
+    "mi_moe_router_ragged": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "mi_moe_layer_train_sizes": (_i, [_i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "mi_moe_layer_train_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp, _sz, _vp]),
     "mi_moe_layer_train_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _sz,

@@ -106,7 +106,9 @@ extern "C" int mi_moe_layer_forward(const void* x, const void* norm_w, float nor
   } else {
     const bool streaming = dtype != MI_MOE_F32 && E <= 64 && k <= 8 && H % 16 == 0;
     const size_t need = streaming ? mi_moe_router_fused_sort_workspace_bytes(T, H, E, k) : 0;
-    if (need > 0) {
+    if (dtype != MI_MOE_F32 && H % 16 != 0) {
+      rc = mi_moe_router_ragged(x, gate_w, gate_bias, T, H, E, k, dtype, nullptr, gates, experts, stream);
+    } else if (need > 0) {
       rc = mi_moe_router_fused_sort(x, gate_w, gate_bias, T, H, E, k, dtype, nullptr, gates, experts, se, ss, off, rws, need, stream);
       sorted = true;
     } else {

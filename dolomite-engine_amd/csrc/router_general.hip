@@ -137,11 +137,12 @@ __global__ __launch_bounds__(256) void router_general_kernel(const T* __restrict
   for (int st = first + wave; st < last; st += 4) {
     const int k0 = st * KSTEP;
     const int kpos = k0 + q * LPL;
-    const bool valid = kpos < H;  // the matrix instruction runs on all lanes: out-of-range k contributes zeros
+    // the matrix instruction runs on all lanes: out-of-range k contributes zeros (a row may end in the middle of a lane's step)
+    const bool valid = kpos < H, both = sizeof(T) == 4 || kpos + HALF < H;  // (fp32: a multiple of 8, a lane's step)
     u32x4 xa[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
     if (valid) {
       xa[0] = *reinterpret_cast<const u32x4*>(xrow + kpos);
-      xa[1] = *reinterpret_cast<const u32x4*>(xrow + kpos + HALF);
+      if (both) xa[1] = *reinterpret_cast<const u32x4*>(xrow + kpos + HALF);
     }
 #pragma unroll
     for (int eb = 0; eb < NEB; ++eb) {
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(256) void router_general_kernel(const T* __restrict
         if (valid) {
           const T* wrow = gw + (size_t)e * H + kpos;
           wa[0] = *reinterpret_cast<const u32x4*>(wrow);
-          wa[1] = *reinterpret_cast<const u32x4*>(wrow + HALF);
+          if (both) wa[1] = *reinterpret_cast<const u32x4*>(wrow + HALF);
         }
         GMfma<T>::run(wa, xa, acc[eb]);
       }
@@ -302,6 +303,19 @@ int mi_router_general(const void* x, const void* gw, const float* bias, int T_, 
       return router_general_by_blocks<bf16_t>(x, gw, bias, T_, H, E, k, logits_out, gates, idx, ws, splits, s);
     default: return MI_MOE_EDTYPE;
   }
+}
+
+// 16-bit rows that are a multiple of 8 long, up to 64 experts: one launch in place of torch's linear and the top-k kernel (3001 rows
+// of 920, 17 experts, fp16: 13.3 -> 9.8 us, and a launch and torch's dispatch less: a layer of 8 experts, 59 -> 38 us).
+extern "C" int mi_moe_router_ragged(const void* x, const void* gate_w, const float* bias, int T, int H, int E, int k, int dtype,
+                                    void* logits_out, void* gates_out, int32_t* idx_out, mi_moe_stream_t stream) {
+  if (T < 0 || H < 1 || E < 1 || k < 1 || k > E) return MI_MOE_ESHAPE;
+  if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16) return MI_MOE_EDTYPE;
+  if (H % 8 != 0 || E > 64) return MI_MOE_EUNSUPPORTED;
+  if (T == 0) return MI_MOE_OK;
+  if (!x || !gate_w || !gates_out || !idx_out) return MI_MOE_ENULL;
+  if (!mi_aligned(x, 16) || !mi_aligned(gate_w, 16)) return MI_MOE_EALIGN;
+  return mi_router_general(x, gate_w, bias, T, H, E, k, dtype, logits_out, gates_out, idx_out, nullptr, static_cast<hipStream_t>(stream));
 }
 
 // ------------------------------------------------------------------------------------------------

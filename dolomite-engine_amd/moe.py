@@ -383,7 +383,8 @@ class MoE(nn.Module):
             return None, None
         gate_weight = gate.weight
         logits = None
-        if pre_norm is None and not ops.router_fused_supported(hidden_states, self.num_experts, self.top_k):
+        if (pre_norm is None and not ops.router_fused_supported(hidden_states, self.num_experts, self.top_k)
+                and not self._routes_ragged(hidden_states, gate)):
             logits = self._unfused_logits(hidden_states)
         return ops.layer_forward(hidden_states, gate_weight, self.router_logit_bias, self.top_k, *weights,
                                  shared_fc, shared_proj, residual, residual_scale, pre_norm, logits), logits
@@ -405,9 +406,20 @@ class MoE(nn.Module):
             return None
         return RoutedExperts.apply(hidden_states, gate_weight, fc.weight, proj.weight, bias, self.top_k, sizes)
 
+    def _routes_ragged(self, hidden_states: torch.Tensor, gate: nn.Module) -> bool:
+        """Whether the router's own kernel takes rows that the fused forms do not, without a gradient (its backward would want
+        multiples of 8 experts) and where the gate is only its weight."""
+        if not (ops.router_ragged_supported(hidden_states, self.num_experts, self.top_k)
+                and _called_as_written(gate, ParameterizedLinear, _LINEAR_FORWARD)):
+            return False
+        weight = gate.weight
+        return (gate.bias is None and weight.dtype == hidden_states.dtype and hidden_states.shape[0] > 0
+                and weight.shape == (self.num_experts, hidden_states.shape[-1])
+                and hidden_states.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
     def _unfused_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         """Router logits of shapes the router kernel does not take (more than 256 experts, a hidden size that is not a
-        multiple of 16): they come from torch, the selection still follows the kernel's tie rule (value descending,
+        multiple of 8, or with a gradient of 16): they come from torch, the selection still follows the kernel's tie rule (value descending,
         expert index ascending) in training and in inference alike."""
         ops._warn_once(("router_unfused", self.num_experts, self.hidden_size, hidden_states.dtype),
                        f"MoE router with {self.num_experts} experts, hidden size {self.hidden_size}, "
@@ -454,6 +466,12 @@ class MoE(nn.Module):
                 return logits, weights, experts, (srt if srt[0] is not None else None)
             return (*ops.router_fused(hidden_states, self.gate.weight, self.top_k, bias=self.router_logit_bias,
                                       return_logits=self.training), None)
+
+        if (is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda and logits is None
+                and not self._needs_grad(hidden_states) and not _HOOKS._global_forward_hooks
+                and not _HOOKS._global_forward_pre_hooks and self._routes_ragged(hidden_states, self.gate)):
+            return (*ops.router_ragged(hidden_states, self.gate.weight, self.top_k, bias=self.router_logit_bias,
+                                       return_logits=True), None)
 
         if is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda:
             router_logits = self._unfused_logits(hidden_states) if logits is None else logits
@@ -650,6 +668,7 @@ class MoE(nn.Module):
 _ROUTE, _USE_FUSED_ROUTER = MoE._route, MoE._use_fused_router
 _COMPUTE_EXPERTS, _COMPUTE_SHARED_EXPERTS = MoE._compute_experts, MoE._compute_shared_experts
 _EXPERTS_FORWARD = ParameterizedExperts.forward
+_LINEAR_FORWARD = ParameterizedLinear.forward
 _IDENTITY_FORWARD = nn.Identity.forward
 _HOOKS = torch.nn.modules.module
 

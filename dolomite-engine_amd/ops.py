@@ -163,6 +163,33 @@ def router_fused_supported(x: torch.Tensor, num_experts: int, k: int) -> bool:
     return x.dtype in (torch.bfloat16, torch.float16) and x.shape[-1] % 16 == 0
 
 
+def router_ragged_supported(x: torch.Tensor, num_experts: int, k: int) -> bool:
+    """What :func:`router_ragged` takes that :func:`router_fused` does not: 16-bit rows that are a multiple of 8 long."""
+    return (x.dtype in (torch.bfloat16, torch.float16) and x.shape[-1] % 16 == 8 and 1 <= k <= num_experts <= 64)
+
+
+def router_ragged(x: torch.Tensor, gate_weight: torch.Tensor, k: int, bias: torch.Tensor | None = None,
+                  return_logits: bool = False):
+    """:func:`router_fused` for the shapes of :func:`router_ragged_supported`, in one launch."""
+    _dev(x, gate_weight, bias)
+    _no_grad(x, gate_weight)
+    x = x.contiguous()
+    gate_weight = gate_weight.contiguous()
+    T, H = x.shape
+    E = gate_weight.shape[0]
+    if gate_weight.dtype != x.dtype or gate_weight.shape[1] != H:
+        raise ValueError("gate weight must be (E, H) in the dtype of x")
+    if bias is not None:
+        bias = bias.to(torch.float32).contiguous()
+    logits = torch.empty((T, E), dtype=x.dtype, device=x.device) if return_logits else None
+    gates = torch.empty((T, k), dtype=x.dtype, device=x.device)
+    idx = torch.empty((T, k), dtype=torch.int32, device=x.device)
+    with _stage("router_fused"):
+        check(_lib.load().mi_moe_router_ragged(_ptr(x), _ptr(gate_weight), _ptr(bias), T, H, E, k, _code(x.dtype), _ptr(logits),
+                                               _ptr(gates), _ptr(idx), _stream()))
+    return logits, gates, idx
+
+
 def router_fused(x: torch.Tensor, gate_weight: torch.Tensor, k: int, bias: torch.Tensor | None = None,
                  return_logits: bool = False, split_k: bool = True):
     """logits = x @ gate_weight^T (+bias) in x.dtype, top-k, softmax: one pass over x.
@@ -1007,7 +1034,7 @@ def layer_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.Tensor
     if pre_norm is not None:
         if not rmsnorm_router_fused_supported(x, E, k) or (norm_w is not None and norm_w.shape != (H,)):
             return None
-    elif logits is None and not router_fused_supported(x, E, k):
+    elif logits is None and not (router_fused_supported(x, E, k) or router_ragged_supported(x, E, k)):
         return None
     ws_bytes, splits = _layer_sizes(dev, T, H, E, k, I, S, code, pre_norm is not None)
     y = torch.empty_like(x)

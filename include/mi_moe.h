@@ -107,6 +107,11 @@ int mi_moe_router_fused(const void* x, const void* gate_w, const float* bias, in
 int mi_moe_router_dlogits(const void* logits, const int32_t* idx, const void* d_gates, const void* d_logits_extra,
                           int T, int E, int k, int dtype, void* d_logits_out, mi_moe_stream_t stream);
 
+/* mi_moe_router_fused for 16-bit rows that are a multiple of 8 long (its own forms take multiples of 16), up to 64 experts and any
+ * k; logits_out (T, E) or NULL. */
+int mi_moe_router_ragged(const void* x, const void* gate_w, const float* bias, int T, int H, int E, int k, int dtype,
+                         void* logits_out, void* gates_out, int32_t* idx_out, mi_moe_stream_t stream);
+
 /*
  * Fused router followed by the expert sort / bin of mi_moe_sort_bin, with the seam between them removed.
  * Replaces: MoE._compute_routing_weights + the sort / bincount / cumsum of the scatter branch
