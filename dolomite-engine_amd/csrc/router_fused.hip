@@ -12,6 +12,7 @@
 //     per-lane maximum of 64-bit keys (ordered value << 32 | ~expert) and a 2-step butterfly.
 #include "common.h"
 #include "sort_block.h"
+#include "topk_row.h"
 
 template <typename T> struct RMfma;
 template <> struct RMfma<bf16_t> {
@@ -127,6 +128,65 @@ __device__ __forceinline__ void router_epilogue(const f32x4 (&acc)[4], int t, bo
         if (hist != nullptr) atomicAdd(&hist[wi[j]], 1);
       }
     }
+  }
+}
+
+// The same where the parts of a group's logits meet in LDS and other waves have nothing to do: `quarter` 0 .. 3 takes tokens
+// 4 quarter .. + 3 of the group, 16 lanes a token (lane j of them has experts j, 16 + j, ...).  A round of the selection is then three
+// maxima in the lane and four DPP moves, and four waves share the group: the epilogue above, a thousand instructions of one wave, is
+// 2 us of a launch that few tokens wait for.  Parts are added in part order, the terms of a softmax in slot order: the same bits.
+// red: part p's accumulators at red + 4096 p bytes, [block of 16 experts][lane].
+template <typename T, int PARTS>
+__device__ __forceinline__ void router_epilogue_rows(const f32x4* red, int parts, int quarter, int tok0, int Trows,
+                                                     const float* __restrict__ bias, int E, int k, T* __restrict__ logits_out,
+                                                     T* __restrict__ gates, int32_t* __restrict__ idx, int* hist = nullptr) {
+  const int lane = threadIdx.x & 63, j = lane & 15, row = 4 * quarter + (lane >> 4);
+  const int t = tok0 + row;
+  const bool tvalid = t < Trows;
+  const float* src = reinterpret_cast<const float*>(red) + ((j >> 2) * 16 + row) * 4 + (j & 3);
+  uint32_t keys[4];
+#pragma unroll
+  for (int eb = 0; eb < 4; ++eb) {
+    keys[eb] = 0u;
+    if (eb * 16 >= E) continue;
+    const int e = eb * 16 + j;
+    float v = src[eb * 256];
+    if constexpr (PARTS > 0) {
+#pragma unroll
+      for (int p = 1; p < PARTS; ++p) v += src[(p * 4 + eb) * 256];
+    } else {
+      for (int p = 1; p < parts; ++p) v += src[(p * 4 + eb) * 256];
+    }
+    v = Elt<T>::round(v);
+    if (e >= E) continue;
+    if (bias != nullptr) v = Elt<T>::round(v + bias[e]);
+    keys[eb] = (router_ordered16<T>(Bits16<T>::of(v)) << 16) | (0xffffu - (uint32_t)e);
+    if (logits_out != nullptr && tvalid) Elt<T>::store(logits_out + (size_t)t * E + e, v);
+  }
+  uint32_t first = 0u, mine = 0u;
+#pragma unroll
+  for (int n = 0; n < ROUTER_KMAX; ++n) {
+    if (n >= k) break;
+    auto larger = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+    uint32_t best = larger(larger(keys[0], keys[1]), larger(keys[2], keys[3]));
+    best = larger(best, dpp_row_u32<0xB1>(best));   // quad_perm [1, 0, 3, 2]
+    best = larger(best, dpp_row_u32<0x4E>(best));   // quad_perm [2, 3, 0, 1]
+    best = larger(best, dpp_row_u32<0x141>(best));  // row_half_mirror
+    best = larger(best, dpp_row_u32<0x140>(best));  // row_mirror
+#pragma unroll
+    for (int eb = 0; eb < 4; ++eb) keys[eb] = keys[eb] == best ? 0u : keys[eb];
+    if (n == 0) first = best;
+    mine = j == n ? best : mine;
+  }
+  const float p = j < k ? expf(router_value_of_key<T>(mine) - router_value_of_key<T>(first)) : 0.f;
+  float denom = 0.f;
+#pragma unroll
+  for (int n = 0; n < ROUTER_KMAX; ++n) denom += __shfl(p, (lane & 48) + n, MI_WAVE);
+  if (tvalid && j < k) {
+    const int e = (int)(0xffffu - (mine & 0xffffu));
+    Elt<T>::store(gates + (size_t)t * k + j, p / denom);
+    idx[(size_t)t * k + j] = e;
+    if (hist != nullptr) atomicAdd(&hist[e], 1);
   }
 }
 
@@ -345,25 +405,22 @@ __global__ __launch_bounds__(ROUTER_LDS_WAVES * 64) void router_fused_lds_kernel
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       f32x4* red = reinterpret_cast<f32x4*>(wlds + red_at);
-      if (part != 0) {
 #pragma unroll
-        for (int eb = 0; eb < 4; ++eb) red[(wave * 4 + eb) * 64 + lane] = acc[eb];
-      }
+      for (int eb = 0; eb < 4; ++eb) red[(wave * 4 + eb) * 64 + lane] = acc[eb];
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_waitcnt(0xc07f);
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (part == 0) {
-        for (int p = 1; p < ksplit; ++p) {
-#pragma unroll
-          for (int eb = 0; eb < 4; ++eb) acc[eb] += red[((wave + p) * 4 + eb) * 64 + lane];
-        }
+      if (active) {
+        for (int quarter = part; quarter < 4; quarter += ksplit)
+          router_epilogue_rows<T, 0>(red + slot * ksplit * 256, ksplit, quarter, grp * 16, Trows, bias, E, k, logits_out, gates, idx,
+                                     chunk_hist != nullptr ? whist : nullptr);
       }
-    }
-    if (active && part == 0) {
+      grp += stride;
+    } else if (active) {
       const int t = grp * 16 + r;
       grp += stride;
-      if (!KS && grp < ngroups) open_group(grp);
+      if (grp < ngroups) open_group(grp);
       router_epilogue<T>(acc, t, t < Trows, q, bias, E, k, logits_out, gates, idx,
                          chunk_hist != nullptr ? whist : nullptr);
     } else {
@@ -408,7 +465,7 @@ __global__ __launch_bounds__(ROUTER_LDS_WAVES * 64) void router_fused_direct_ker
     int32_t* __restrict__ chunk_hist, int nchunks, RouterSort sort) {
   typedef typename RMfma<T>::vec frag_t;
   constexpr int S = ROUTER_DIRECT_STEPS, W = ROUTER_LDS_WAVES;
-  __shared__ f32x4 red[(W - 1) * 4 * 64];
+  __shared__ f32x4 red[W * 4 * 64];
   __shared__ float ssred[W * 16];
   __shared__ int whist[64];
   const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
@@ -515,19 +572,11 @@ __global__ __launch_bounds__(ROUTER_LDS_WAVES * 64) void router_fused_direct_ker
           acc[eb] = RMfma<T>::run(__builtin_bit_cast(frag_t, wr[s][eb][1]), __builtin_bit_cast(frag_t, xr[s][1]), acc[eb]);
         }
     }
-  if (part != 0) {
 #pragma unroll
-    for (int eb = 0; eb < 4; ++eb) red[((part - 1) * 4 + eb) * 64 + lane] = acc[eb];
-  }
+  for (int eb = 0; eb < 4; ++eb) red[(part * 4 + eb) * 64 + lane] = acc[eb];
   __syncthreads();
-  if (part == 0) {
-#pragma unroll
-    for (int p = 0; p < W - 1; ++p) {
-#pragma unroll
-      for (int eb = 0; eb < 4; ++eb) acc[eb] += red[(p * 4 + eb) * 64 + lane];
-    }
-    router_epilogue<T>(acc, t, t < Trows, q, bias, E, k, logits_out, gates, idx, chunk_hist != nullptr ? whist : nullptr);
-  }
+  if (part < 4)
+    router_epilogue_rows<T, W>(red, W, part, blockIdx.x * 16, Trows, bias, E, k, logits_out, gates, idx, chunk_hist != nullptr ? whist : nullptr);
   if constexpr (SORT) {
     __syncthreads();
     sort_single_block<W>(idx, Trows * k, E, sort.nbits, sort.sorted_expert, sort.sorted_scattered, sort.expert_offsets,
@@ -767,8 +816,8 @@ __global__ __launch_bounds__(ROUTER_SPLIT_WAVES * 64) void router_splitk_partial
   }
 }
 
-// Four waves per token group: wave w adds splits w, w + 4, ... (all of its loads in flight at once), wave 0 adds
-// the four sums in wave order and runs the epilogue.  The order of additions is fixed by the launch shape alone.
+// Four waves per token group: wave w adds splits w, w + 4, ... (all of its loads in flight at once) and runs the epilogue of a
+// quarter of the tokens, on the four sums in wave order.  The order of additions is fixed by the launch shape alone.
 template <typename T>
 __global__ __launch_bounds__(256) void router_splitk_finish_kernel(const f32x4* __restrict__ partial, int splits,
                                                                    const float* __restrict__ bias, int Trows, int E, int k,
@@ -776,9 +825,7 @@ __global__ __launch_bounds__(256) void router_splitk_finish_kernel(const f32x4* 
                                                                    int32_t* __restrict__ idx) {
   __shared__ f32x4 red[4][4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, q = lane >> 4;
   const int tg = blockIdx.x;
-  const int t = tg * 16 + r;
   f32x4 acc[4];
 #pragma unroll
   for (int eb = 0; eb < 4; ++eb) acc[eb] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -791,15 +838,7 @@ __global__ __launch_bounds__(256) void router_splitk_finish_kernel(const f32x4* 
 #pragma unroll
   for (int eb = 0; eb < 4; ++eb) red[wave][eb][lane] = acc[eb];
   __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int eb = 0; eb < 4; ++eb) {
-    f32x4 sum = red[0][eb][lane];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) sum += red[w][eb][lane];
-    acc[eb] = sum;
-  }
-  router_epilogue<T>(acc, t, t < Trows, q, bias, E, k, logits_out, gates, idx);
+  router_epilogue_rows<T, 4>(&red[0][0][0], 4, wave, tg * 16, Trows, bias, E, k, logits_out, gates, idx);
 }
 
 // The finish kernel with the expert sort folded in (few tokens, T * k <= SORT_SINGLE_BLOCK_MAX): every workgroup
@@ -815,9 +854,7 @@ __global__ __launch_bounds__(WAVES * 64) void router_splitk_finish_sort_kernel(
   __shared__ f32x4 red[4][4][64];
   __shared__ int is_last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, q = lane >> 4;
   const int tg = blockIdx.x;
-  const int t = tg * 16 + r;
   f32x4 acc[4];
 #pragma unroll
   for (int eb = 0; eb < 4; ++eb) acc[eb] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -832,18 +869,12 @@ __global__ __launch_bounds__(WAVES * 64) void router_splitk_finish_sort_kernel(
     for (int eb = 0; eb < 4; ++eb) red[wave][eb][lane] = acc[eb];
   }
   __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int eb = 0; eb < 4; ++eb) {
-      f32x4 sum = red[0][eb][lane];
-#pragma unroll
-      for (int w = 1; w < 4; ++w) sum += red[w][eb][lane];
-      acc[eb] = sum;
-    }
-    router_epilogue<T>(acc, t, t < Trows, q, bias, E, k, logits_out, gates, idx);
+  if (wave < 4) {
+    router_epilogue_rows<T, 4>(&red[0][0][0], 4, wave, tg * 16, Trows, bias, E, k, logits_out, gates, idx);
     __threadfence();  // this workgroup's experts are visible device-wide before its ticket is
-    if (lane == 0) is_last = atomicAdd(ticket, 1u) == gridDim.x - 1;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) is_last = atomicAdd(ticket, 1u) == gridDim.x - 1;
   __syncthreads();
   if (!is_last) return;
   __threadfence();  // ... and the last workgroup reads what the others published
