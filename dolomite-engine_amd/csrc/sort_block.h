@@ -19,6 +19,17 @@ __device__ __forceinline__ int wave_incl_scan_i32(int v, int lane) {
   return v;
 }
 
+// sum over the lanes of a wave, in scalar registers
+__device__ __forceinline__ int wave_total_i32(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr 1, 2, 4, 8: rows of 16
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15: into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31: into rows 2 and 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // One step of the stable scatter: a wave's 64 slots from `slot - lane` on, lane l holding slot's expert e (ok: a valid one).
 // mybase[e]: output position of the wave's next slot of expert e.
 __device__ __forceinline__ void sort_scatter_step(int slot, int e, bool ok, int nbits, int* mybase,
