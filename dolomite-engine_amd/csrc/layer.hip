@@ -12,7 +12,9 @@
 bool mi_rmsnorm_router_sorts(int T, int H, int E);
 int mi_rmsnorm_router(const void* h, const void* ln_weight, float eps, const void* gate_w, const float* bias, int T, int H, int E,
                       int k, int dtype, void* x_norm_out, void* logits_out, void* gates_out, int32_t* idx_out,
-                      int32_t* sorted_expert, int32_t* sorted_scattered, int32_t* expert_offsets, mi_moe_stream_t stream);
+                      int32_t* sorted_expert, int32_t* sorted_scattered, int32_t* expert_offsets, int32_t* hist,
+                      mi_moe_stream_t stream);
+size_t mi_rmsnorm_router_sort_bytes(int T, int H, int E, int k);
 
 // combine.hip, backward.hip, aux_loss.hip, grouped_wgrad.hip
 int mi_combine_sum(const void* o, const void* add, void* y, int T, int k, int H, int dtype, mi_moe_stream_t stream);
@@ -52,6 +54,8 @@ LayerSpace layer_space(int T, int H, int E, int k, int I, int S, int elt, bool n
   const size_t r1 = mi_moe_router_fused_workspace_bytes(T, H, E), r2 = mi_moe_sort_bin_workspace_bytes((int)L, E);
   r = r > r1 ? r : r1;
   r = r > r2 ? r : r2;
+  const size_t r3 = norm ? mi_rmsnorm_router_sort_bytes(T, H, E, k) : 0;
+  r = r > r3 ? r : r3;
   w.router = take(at, r + 16);
   w.x_norm = take(at, norm ? (size_t)T * H * elt : 0);
   w.act = take(at, L * I * elt);
@@ -96,9 +100,10 @@ extern "C" int mi_moe_layer_forward(const void* x, const void* norm_w, float nor
   if (has_norm) {
     if (logits) return MI_MOE_EUNSUPPORTED;
     void* xn = b + w.x_norm;
-    sorted = mi_rmsnorm_router_sorts(T, H, E);
+    const bool counts = mi_rmsnorm_router_sort_bytes(T, H, E, k) > 0;
+    sorted = counts || mi_rmsnorm_router_sorts(T, H, E);
     if ((rc = mi_rmsnorm_router(x, norm_w, norm_eps, gate_w, gate_bias, T, H, E, k, dtype, xn, nullptr, gates, experts,
-                                sorted ? se : nullptr, ss, off, stream)) != MI_MOE_OK)
+                                sorted ? se : nullptr, ss, off, counts ? static_cast<int32_t*>(rws) : nullptr, stream)) != MI_MOE_OK)
       return rc;
     x = xn;
   } else if (logits) {

@@ -1206,10 +1206,20 @@ extern "C" int mi_moe_rmsnorm_router_fused_supported(int H, int E, int k, int dt
 
 bool mi_rmsnorm_router_sorts(int T, int H, int E) { return T >= 1 && router_norm_one_group(T, H, E); }
 
-// sorted_expert (mi_rmsnorm_router_sorts) or null: the sort in the same launch
+// Bytes with which the RMSNorm router counts the experts of its chunks for the sort, as the plain form does: that saves the sort a
+// launch beyond its one-block form, and most of that form's time from about 2048 slots on (0: not a shape of that).
+size_t mi_rmsnorm_router_sort_bytes(int T, int H, int E, int k) {
+  int blocks = 0, waves = 0;
+  if (T < 1 || router_norm_one_group(T, H, E) || (long)T * k <= 2048 || (long)T * k > 0x7fffffffL - 8192) return 0;
+  if (E > 64 || k > ROUTER_KMAX || H % 16 != 0 || !router_lds_fits(H, E) || router_lds_shape(T, &blocks, &waves) != MI_MOE_OK) return 0;
+  return ((size_t)E * mi_ceil_div(T, waves * 16) + (size_t)E) * sizeof(int32_t);
+}
+
+// sorted_expert or null: the sort in the same launch (mi_rmsnorm_router_sorts) or, with `hist` of mi_rmsnorm_router_sort_bytes, behind it
 int mi_rmsnorm_router(const void* h, const void* ln_weight, float eps, const void* gate_w, const float* bias, int T, int H, int E,
                       int k, int dtype, void* x_norm_out, void* logits_out, void* gates_out, int32_t* idx_out,
-                      int32_t* sorted_expert, int32_t* sorted_scattered, int32_t* expert_offsets, mi_moe_stream_t stream) {
+                      int32_t* sorted_expert, int32_t* sorted_scattered, int32_t* expert_offsets, int32_t* hist,
+                      mi_moe_stream_t stream) {
   if (T < 0 || H < 1 || E < 1 || k < 1 || k > E) return MI_MOE_ESHAPE;
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16) return MI_MOE_EDTYPE;
   if (!mi_moe_rmsnorm_router_fused_supported(H, E, k, dtype)) return MI_MOE_EUNSUPPORTED;
@@ -1226,9 +1236,15 @@ int mi_rmsnorm_router(const void* h, const void* ln_weight, float eps, const voi
                                                 sorted_scattered, expert_offsets, s);
   }
   const size_t lds = rmsnorm_router_lds_bytes(H, E, 2);
-  if (dtype == MI_MOE_BF16)
-    return launch_router_lds<bf16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, lds, s);
-  return launch_router_lds<f16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, lds, s);
+  int blocks = 0, waves = 0, rc = MI_MOE_OK;
+  if (sorted_expert == nullptr) hist = nullptr;
+  if (hist != nullptr && (rc = router_lds_shape(T, &blocks, &waves)) != MI_MOE_OK) return rc;
+  const int nchunks = hist != nullptr ? mi_ceil_div(T, waves * 16) : 0;
+  rc = dtype == MI_MOE_BF16
+           ? launch_router_lds<bf16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, lds, s, hist, nchunks)
+           : launch_router_lds<f16_t, true>(h, gate_w, bias, T, H, E, k, logits_out, gates_out, idx_out, norm, lds, s, hist, nchunks);
+  if (rc != MI_MOE_OK || hist == nullptr) return rc;
+  return mi_sort_after_hist(idx_out, T * k, E, waves * 16 * k, sorted_expert, sorted_scattered, expert_offsets, hist, s);
 }
 
 extern "C" int mi_moe_rmsnorm_router_fused(const void* h, const void* ln_weight, float eps, const void* gate_w,
@@ -1236,5 +1252,5 @@ extern "C" int mi_moe_rmsnorm_router_fused(const void* h, const void* ln_weight,
                                            void* x_norm_out, void* logits_out, void* gates_out, int32_t* idx_out,
                                            mi_moe_stream_t stream) {
   return mi_rmsnorm_router(h, ln_weight, eps, gate_w, bias, T, H, E, k, dtype, x_norm_out, logits_out, gates_out, idx_out, nullptr,
-                           nullptr, nullptr, stream);
+                           nullptr, nullptr, nullptr, stream);
 }

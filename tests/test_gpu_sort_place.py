@@ -34,3 +34,22 @@ def test_behind_the_router(device, T, E, k):
         assert torch.equal(got, want)
     order = np.argsort(idx.cpu().numpy().reshape(-1), kind="stable")
     assert np.array_equal(ss.cpu().numpy(), order)
+
+
+@pytest.mark.parametrize("T,H,E,k", [(256, 128, 40, 8), (257, 128, 40, 8), (1025, 1024, 32, 2), (4097, 256, 40, 8), (9000, 64, 64, 1),
+                                     (16400, 128, 8, 2), (33000, 64, 17, 3)])
+def test_behind_the_norm(device, T, H, E, k):
+    """The layer's one-call forward, whose RMSNorm router counts for the sort, against the stages, which sort by themselves."""
+    from dolomite_engine_amd import Kernel, MoE, enable_kernels
+
+    torch.manual_seed(T)
+    m = MoE(hidden_size=H, intermediate_size=64, shared_intermediate_size=None, num_experts=E, num_experts_per_tok=k,
+            activation_function="swiglu", add_bias=False, dropout=0.0, init_method="normal", initializer_range=0.1, m_width=None,
+            num_layers=1, use_padding_free_transformer=True).to(device).bfloat16().eval()
+    x = torch.randn(T, H, device=device).bfloat16()
+    norm = (1 + 0.1 * torch.randn(H, device=device)).bfloat16()
+    with torch.no_grad(), enable_kernels([Kernel.scattermoe]):
+        got = m(x, pre_norm=(norm, 1e-5))
+        stage, m._route = m._route, lambda *a, **kw: stage(*a, **kw)  # (a replaced stage: stage by stage)
+        want = m(x, pre_norm=(norm, 1e-5))
+    assert torch.equal(got, want)
