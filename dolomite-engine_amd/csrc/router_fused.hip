@@ -822,10 +822,12 @@ template <typename T>
 __global__ __launch_bounds__(256) void router_splitk_finish_kernel(const f32x4* __restrict__ partial, int splits,
                                                                    const float* __restrict__ bias, int Trows, int E, int k,
                                                                    T* __restrict__ logits_out, T* __restrict__ gates,
-                                                                   int32_t* __restrict__ idx) {
+                                                                   int32_t* __restrict__ idx, int32_t* __restrict__ chunk_hist) {
   __shared__ f32x4 red[4][4][64];
+  __shared__ int whist[64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tg = blockIdx.x;
+  if (threadIdx.x < 64) whist[threadIdx.x] = 0;
   f32x4 acc[4];
 #pragma unroll
   for (int eb = 0; eb < 4; ++eb) acc[eb] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -838,7 +840,11 @@ __global__ __launch_bounds__(256) void router_splitk_finish_kernel(const f32x4* 
 #pragma unroll
   for (int eb = 0; eb < 4; ++eb) red[wave][eb][lane] = acc[eb];
   __syncthreads();
-  router_epilogue_rows<T, 4>(&red[0][0][0], 4, wave, tg * 16, Trows, bias, E, k, logits_out, gates, idx);
+  router_epilogue_rows<T, 4>(&red[0][0][0], 4, wave, tg * 16, Trows, bias, E, k, logits_out, gates, idx,
+                             chunk_hist != nullptr ? whist : nullptr);
+  if (chunk_hist == nullptr) return;
+  __syncthreads();
+  if (threadIdx.x < E) chunk_hist[(size_t)threadIdx.x * gridDim.x + tg] = whist[threadIdx.x];
 }
 
 // The finish kernel with the expert sort folded in (few tokens, T * k <= SORT_SINGLE_BLOCK_MAX): every workgroup
@@ -919,7 +925,7 @@ static int launch_router_splitk(const void* x, const void* gw, const float* bias
   int rc = mi_launch_status();
   if (rc != MI_MOE_OK) return rc;
   hipLaunchKernelGGL((router_splitk_finish_kernel<T>), dim3(groups), dim3(256), 0, s, static_cast<const f32x4*>(ws),
-                     splits, bias, T_, E, k, static_cast<T*>(logits_out), static_cast<T*>(gates), idx);
+                     splits, bias, T_, E, k, static_cast<T*>(logits_out), static_cast<T*>(gates), idx, static_cast<int32_t*>(nullptr));
   return mi_launch_status();
 }
 
@@ -1023,12 +1029,19 @@ static int launch_router(const void* x, const void* gw, const float* bias, int T
 }
 
 // Router + sort in two launches (split K, the finishing launch sorts in its last workgroup).
-// [partial logits][ticket, padded to 256 bytes]
+// [partial logits][ticket, padded to 256 bytes; or the table of the groups' counts]
+// Beyond ROUTER_TICKET_SLOTS the finishing launch counts its group's experts and the sort's placing launch follows: its last
+// workgroup alone takes longer to sort them (router + sort, us: 64 experts, hidden 4096, 6 a token, 1024 tokens 25.7 -> 16.4, 350 19.4 ->
+// 14.4; 40 experts, hidden 1536, 8 a token, 300 tokens 17.6 -> 11.6; 64 tokens of 32 experts 10.4 either way).
+#define ROUTER_TICKET_SLOTS 1024
 static size_t router_sort_ws_bytes(int T_, int H, int E, int k) {
   const size_t base = router_ws_bytes(T_, H, E);
   if (base == 0 || (long)T_ * k > SORT_SINGLE_BLOCK_MAX) return 0;
-  return base + 256;
+  return base + 256 + ((long)T_ * k > ROUTER_TICKET_SLOTS ? ((size_t)E * mi_ceil_div(T_, 16) + E) * sizeof(int32_t) : 0);
 }
+
+int mi_sort_after_hist(const int32_t* topk_idx, int L, int E, int chunk, int32_t* sorted_expert,
+                       int32_t* sorted_scattered, int32_t* expert_offsets, int32_t* ws, hipStream_t s);  // routing.hip
 
 template <typename T>
 static int launch_router_splitk_sort(const void* x, const void* gw, const float* bias, int T_, int H, int E, int k,
@@ -1046,6 +1059,13 @@ static int launch_router_splitk_sort(const void* x, const void* gw, const float*
                      static_cast<f32x4*>(ws), ticket);
   int rc = mi_launch_status();
   if (rc != MI_MOE_OK) return rc;
+  if ((long)T_ * k > ROUTER_TICKET_SLOTS) {
+    int32_t* table = reinterpret_cast<int32_t*>(ticket + 64);
+    hipLaunchKernelGGL((router_splitk_finish_kernel<T>), dim3(groups), dim3(256), 0, s, static_cast<const f32x4*>(ws), splits, bias, T_, E,
+                       k, static_cast<T*>(logits_out), static_cast<T*>(gates), idx, table);
+    if ((rc = mi_launch_status()) != MI_MOE_OK) return rc;
+    return mi_sort_after_hist(idx, T_ * k, E, 16 * k, sorted_expert, sorted_scattered, expert_offsets, table, s);
+  }
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   const bool few = (long)T_ * k <= SORT_WAVES * 64 * SORT_ID_STEPS;  // (sixteen waves cost the adding part: 13 -> 15 us at 1256 ids)
@@ -1058,9 +1078,6 @@ static int launch_router_splitk_sort(const void* x, const void* gw, const float*
 
 // Many tokens: router (LDS-resident gate weights) with the sort's histogram pass folded in, then the sort's scan
 // and scatter passes (routing.hip) on chunks of waves * 16 tokens.
-int mi_sort_after_hist(const int32_t* topk_idx, int L, int E, int chunk, int32_t* sorted_expert,
-                       int32_t* sorted_scattered, int32_t* expert_offsets, int32_t* ws, hipStream_t s);
-
 static bool router_hist_shape(int T_, int H, int E, int k, int* chunk_tokens, int* nchunks) {
   if (router_few_tokens(T_, H, E) || (long)T_ * k > 0x7fffffffL - 8192) return false;
   if (!router_lds_fits(H, E)) return false;
