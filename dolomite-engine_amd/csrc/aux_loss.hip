@@ -152,22 +152,30 @@ __global__ __launch_bounds__(1024) void aux_loss_finish_kernel(const float* __re
     if (lane == 0) (c < E ? A[c] : c < 2 * E ? F[c - E] : scal[3]) = v;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float sa = 0.f, sf = 0.f, dot = 0.f;
-    for (int e = 0; e < E; ++e) {
-      sa += A[e];
-      sf += F[e];
+  if (wave == 0) {
+    // lane l has experts l, 64 + l, ...; fixed butterflies (one thread's walk over 32 experts and its divisions took 3 us)
+    float av[AUX_MAX_E / 64], fv[AUX_MAX_E / 64], sa = 0.f, sf = 0.f, dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < AUX_MAX_E / 64; ++i) {
+      const int e = lane + 64 * i;
+      av[i] = e < E ? A[e] : 0.f;
+      fv[i] = e < E ? F[e] : 0.f;
+      sa += av[i];
+      sf += fv[i];
     }
-    sa = fmaxf(sa, 1e-12f);
-    sf = fmaxf(sf, 1e-12f);
-    for (int e = 0; e < E; ++e) dot = fmaf(A[e] / sa, F[e] / sf, dot);
-    const float sw = (float)E * dot;
-    scal[0] = sa;
-    scal[1] = sf;
-    scal[2] = sw;
-    const float loss = sw + 0.1f * (scal[3] / (float)Trows);
-    loss_w[0] = loss;
-    if (loss_out != nullptr) Elt<T>::store(loss_out, loss);
+    sa = fmaxf(wave_sum_f32(sa), 1e-12f);
+    sf = fmaxf(wave_sum_f32(sf), 1e-12f);
+#pragma unroll
+    for (int i = 0; i < AUX_MAX_E / 64; ++i) dot = fmaf(av[i] / sa, fv[i] / sf, dot);
+    const float sw = (float)E * wave_sum_f32(dot);
+    if (lane == 0) {
+      scal[0] = sa;
+      scal[1] = sf;
+      scal[2] = sw;
+      const float loss = sw + 0.1f * (scal[3] / (float)Trows);
+      loss_w[0] = loss;
+      if (loss_out != nullptr) Elt<T>::store(loss_out, loss);
+    }
   }
   __syncthreads();
   // d/dA_e [ sum_e' A_e' c_e' / S ] = (c_e - switch) / S  with c_e = E f_e / sum f  (S = sum A above its floor)
