@@ -163,7 +163,7 @@ namespace {
 struct TrainSpace {
   size_t h, logits, gates, experts, sorted_scattered, offsets, loss_w, saved;  // kept for the backward
   size_t router, aux, sorted_expert, act, o, forward;                          // the forward's workspace
-  size_t a, d_h, act_g, d_gates, tokens, d_logits, dx_router, backward;        // the backward's
+  size_t a, act_g, d_h, d_gates, tokens, d_logits, dx_router, backward;        // the backward's
 };
 
 size_t larger(size_t a, size_t b) { return a > b ? a : b; }
@@ -189,12 +189,13 @@ TrainSpace train_space(int T, int H, int E, int k, int I) {
   w.o = take(at, L * H * elt);
   w.forward = at;
   at = 0;
-  // one after the other: the gradient of the activation, the slots' gradient of x, the weight gradients' workspace
-  const size_t wg = larger(larger(mi_moe_grouped_wgrad_workspace_bytes((int)L, E, 2 * I, H), mi_moe_grouped_wgrad_workspace_bytes((int)L, E, H, I)),
-                           mi_moe_grouped_wgrad_workspace_bytes(T, 1, E, H));
-  w.a = take(at, larger(larger(L * I * elt, L * H * elt), wg + 16));
+  // one after the other: the gradient of the activation with the gated activation behind it, the workspace of the down-projection's
+  // weight gradient in place of the former, the slots' gradient of x, the other weight gradients' workspace
+  const size_t wg = larger(mi_moe_grouped_wgrad_workspace_bytes((int)L, E, 2 * I, H), mi_moe_grouped_wgrad_workspace_bytes(T, 1, E, H)) + 16;
+  const size_t front = (larger(L * I * elt, mi_moe_grouped_wgrad_workspace_bytes((int)L, E, H, I) + 16) + 255) / 256 * 256;
+  w.a = take(at, larger(larger(front + L * I * elt, L * H * elt), wg));
+  w.act_g = w.a + front;
   w.d_h = take(at, L * 2 * I * elt);
-  w.act_g = take(at, L * I * elt);
   w.d_gates = take(at, L * elt);
   w.tokens = take(at, L * 4);
   w.d_logits = take(at, (size_t)T * E * elt);
@@ -291,11 +292,17 @@ extern "C" int mi_moe_layer_train_backward(const void* x, const void* gate_w, co
   int32_t* tokens = reinterpret_cast<int32_t*>(b + w.tokens);
   const bool router = dx || d_gate_w;
   auto split = [&](int K) { return gemm_ws && mi_moe_grouped_gemm_splits(K, dtype) ? gemm_ws : nullptr; };
+  auto wgrad = [&](const void* ga, const int32_t* ai, const void* gb, const int32_t* bi, const int32_t* offsets, void* dw, int rows, int a_rows,
+                   int b_rows, int M, int N, int experts_) {
+    return mi_grouped_wgrad(ga, ai, gb, bi, offsets, dw, a, mi_moe_grouped_wgrad_workspace_bytes(rows, experts_, M, N), rows, a_rows, b_rows, M, N,
+                            experts_, dtype, stream, false);
+  };
   int rc;
   if (dy) {
     // gradient of the activation, in sorted order and before the router weight; then d h, gate times activation, and d gates
     if ((rc = mi_moe_scattered_gemm_wt_ws(dy, w_proj, a, ss, off, L, H, I, E, k, 0, 1, dtype, split(H), gemm_ws_bytes, stream)) != MI_MOE_OK) return rc;
     if ((rc = mi_swiglu_backward(h, a, gates, ss, d_h, act_g, d_gates, tokens, L, I, k, dtype, stream)) != MI_MOE_OK) return rc;
+    if (d_w_proj && (rc = wgrad(dy, tokens, act_g, nullptr, off, d_w_proj, L, T, L, H, I, E)) != MI_MOE_OK) return rc;
   }
   if (router) {
     if ((rc = mi_router_dlogits_aux(logits, experts, d_gates, loss_w, d_aux, d_logits, T, E, k, dtype, static_cast<hipStream_t>(stream))) != MI_MOE_OK)
@@ -307,13 +314,7 @@ extern "C" int mi_moe_layer_train_backward(const void* x, const void* gate_w, co
       return rc;
     if ((rc = mi_combine_sum(a, dx_router, dx, T, k, H, dtype, stream)) != MI_MOE_OK) return rc;
   }
-  auto wgrad = [&](const void* ga, const int32_t* ai, const void* gb, const int32_t* bi, const int32_t* offsets, void* dw, int rows, int a_rows,
-                   int b_rows, int M, int N, int experts_) {
-    return mi_grouped_wgrad(ga, ai, gb, bi, offsets, dw, a, mi_moe_grouped_wgrad_workspace_bytes(rows, experts_, M, N), rows, a_rows, b_rows, M, N,
-                            experts_, dtype, stream, false);
-  };
   if (d_w_fc && (rc = wgrad(d_h, nullptr, x, tokens, off, d_w_fc, L, L, T, 2 * I, H, E)) != MI_MOE_OK) return rc;
-  if (d_w_proj && (rc = wgrad(dy, tokens, act_g, nullptr, off, d_w_proj, L, T, L, H, I, E)) != MI_MOE_OK) return rc;
   if (d_gate_w && (rc = wgrad(d_logits, nullptr, x, nullptr, nullptr, d_gate_w, T, T, T, E, H, 1)) != MI_MOE_OK) return rc;
   return MI_MOE_OK;
 }
