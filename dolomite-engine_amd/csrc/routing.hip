@@ -252,10 +252,10 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(const int32_
 // Passes 2 and 3 in one launch, for a table of up to 256 chunks and 64 experts: every block reads the whole table,
 // 40 KB at most, and adds up for itself what of each expert lies before its slots, and in all.  The launch in front of the scatter, a
 // third of the sort's time, is gone; in exchange a block has one trip to the table, on which its own ids ride along.  A block has
-// `per` consecutive chunks, up to 2048 slots; a wave keeps its ids, up to 256, for both passes over them.
-// Three launches / two (four waves a block 8.7 / 12.0), us: 16384 slots of 40 experts 9.0 / 7.0, 131072 of 32 10.5 / 7.5, 262144 of 40
-// 14.8 / 9.6, 12004 of 17 8.4 / 6.5.
-#define SORT_PLACE_WAVES 8
+// `per` consecutive chunks, up to 2048 slots; a wave keeps its ids, up to 128, for both passes over them.
+// Three launches / two, us: 16384 slots of 40 experts 9.0 / 6.5 (eight waves a block 7.1, four 8.7), 131072 of 32 10.5 / 7.1, 262144 of 40
+// 14.8 / 9.3, 12004 of 17 8.4 / 6.2.
+#define SORT_PLACE_WAVES 16
 #define SORT_PLACE_CHUNKS 256
 #define SORT_PLACE_E 64
 #define SORT_PLACE_SLOTS 512  // a block has as many chunks as this holds
@@ -275,7 +275,7 @@ __global__ __launch_bounds__((SORT_PLACE_WAVES * 64)) void sort_place_kernel(con
     const int at = wave * per_wave + j * 64 + lane, slot = first + at;
     id[j] = j * 64 < per_wave && at < slots && slot < L ? ids[slot] : -1;
   }
-  // wave w: experts w, w + 8, ...; lane l: chunks l, 64 + l, ...
+  // wave w: experts w, w + 16, ...; lane l: chunks l, 64 + l, ...
   const int mine = blockIdx.x * per, ncol = mi_ceil_div_dev(nblk, 64);
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
