@@ -891,7 +891,8 @@ static int launch_naive(GemmArgs a, hipStream_t s) {
 }
 
 // tile configurations
-//   0 / 1 / 2 / 5  register-staged 256x256 / 128x128 / 32x256 / 32x128 (any K % 8 == 0)
+//   0 / 1 / 2 / 5  register-staged 256x256 / 128x128 / 32x256 / 32x128 (any K % 8 == 0; 1 comes by DMA where K % 32 != 0 and the tiles
+//              are few, see launch_128x128)
 //   3          one thread per output element (any shape, any dtype)
 //   4          DMA-staged 128x128, one tile per workgroup (K % 32 == 0)
 //   100 + 10 rb + nw  weight stream (stream_gemm.hip): row blocks of 16 per unit, waves that split the contraction

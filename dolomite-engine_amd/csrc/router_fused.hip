@@ -1028,7 +1028,7 @@ static int launch_router(const void* x, const void* gw, const float* bias, int T
   return mi_launch_status();
 }
 
-// Router + sort in two launches (split K, the finishing launch sorts in its last workgroup).
+// Router + sort in two launches (split K, the finishing launch sorts in its last workgroup), or three.
 // [partial logits][ticket, padded to 256 bytes; or the table of the groups' counts]
 // Beyond ROUTER_TICKET_SLOTS the finishing launch counts its group's experts and the sort's placing launch follows: its last
 // workgroup alone takes longer to sort them (router + sort, us: 64 experts, hidden 4096, 6 a token, 1024 tokens 25.7 -> 16.4, 350 19.4 ->

@@ -232,8 +232,8 @@ def router_fused_sort_supported(x: torch.Tensor, num_experts: int, k: int) -> bo
 
 def router_fused_sort(x: torch.Tensor, gate_weight: torch.Tensor, k: int, bias: torch.Tensor | None = None,
                       return_logits: bool = False):
-    """:func:`router_fused` and :func:`sort_bin` in two launches instead of three (the router's finishing launch
-    sorts as well).  Returns (logits or None, gates (T, k), experts (T, k) int32, sorted_expert_idxs (L,),
+    """:func:`router_fused` and :func:`sort_bin` with the seam between them removed (the router's finishing launch
+    sorts as well, or counts the experts for the sort's last pass).  Returns (logits or None, gates (T, k), experts (T, k) int32, sorted_expert_idxs (L,),
     sorted_scattered_idxs (L,), expert_offsets (E,)), identical to the separate calls."""
     _dev(x, gate_weight, bias)
     _no_grad(x, gate_weight)
