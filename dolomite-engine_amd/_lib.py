@@ -76,6 +76,8 @@ SIGNATURES: dict[str, tuple] = {
     "mi_moe_layer_train_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp, _sz, _vp]),
     "mi_moe_layer_train_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _sz,
                                          _vp, _sz, _vp]),
+    "mi_moe_layer_train_backward_parts": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i,
+                                               _vp, _sz, _vp, _sz, _vp]),
     "mi_moe_probe_sink_bytes": (_sz, []),
     "mi_moe_probe_kloop": (_i, [_i, _vp, _sz, _i, _vp, _sz, _vp]),
     "mi_moe_fp8_tiled_bytes": (_sz, [_i, _i, _i, _i]),

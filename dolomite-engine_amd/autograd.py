@@ -262,10 +262,14 @@ class RoutedExperts(torch.autograd.Function):
     """(y, auxiliary loss) of a training step's router, routed experts and loss as one function: FusedRouter, SwitchAuxLoss and
     ScatteredSwiGLUExperts with their launches behind one library call in either direction (ops.layer_train_forward).  A small
     batch is bound by the host: 17 calls with their own argument checks and allocations, and three functions' bookkeeping,
-    took 300 to 450 us a step whatever the kernels did."""
+    took 300 to 450 us a step whatever the kernels did.
+
+    ``x_router``: None, or x once more.  Then the experts' and the router's gradient of x are handed back one after the other,
+    as the three functions do, and not as their sum: with a third gradient of x (the shared experts', which autograd has by
+    then) the order of the additions, each rounded, is part of the result."""
 
     @staticmethod
-    def forward(ctx, x, gate_w, w_fc, w_proj, bias, k, sizes):
+    def forward(ctx, x, x_router, gate_w, w_fc, w_proj, bias, k, sizes):
         y, aux, saved = ops.layer_train_forward(x, gate_w, bias, w_fc, w_proj, k, sizes)
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(x, gate_w, w_fc, w_proj, saved)
@@ -275,6 +279,6 @@ class RoutedExperts(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy, d_aux):
         if dy is None and d_aux is None:
-            return (None,) * 7
-        grads = ops.layer_train_backward(*ctx.saved_tensors, dy, d_aux, ctx.k, ctx.needs_input_grad[:4], ctx.sizes)
+            return (None,) * 8
+        grads = ops.layer_train_backward(*ctx.saved_tensors, dy, d_aux, ctx.k, ctx.needs_input_grad[:5], ctx.sizes)
         return (*grads, None, None, None)

@@ -268,13 +268,13 @@ extern "C" int mi_moe_layer_train_forward(const void* x, const void* gate_w, con
   return rc != MI_MOE_OK ? rc : mi_moe_combine(o, gates, y, T, k, H, dtype, stream);
 }
 
-extern "C" int mi_moe_layer_train_backward(const void* x, const void* gate_w, const void* w_fc, const void* w_proj, const void* saved,
-                                           size_t saved_bytes, const void* dy, const void* d_aux, void* dx, void* d_gate_w, void* d_w_fc,
-                                           void* d_w_proj, int T, int H, int E, int k, int I, int dtype, void* ws, size_t ws_bytes,
-                                           void* gemm_ws, size_t gemm_ws_bytes, mi_moe_stream_t stream) {
+extern "C" int mi_moe_layer_train_backward_parts(const void* x, const void* gate_w, const void* w_fc, const void* w_proj, const void* saved,
+                                                 size_t saved_bytes, const void* dy, const void* d_aux, void* dx, void* dx_router_out,
+                                                 void* d_gate_w, void* d_w_fc, void* d_w_proj, int T, int H, int E, int k, int I, int dtype,
+                                                 void* ws, size_t ws_bytes, void* gemm_ws, size_t gemm_ws_bytes, mi_moe_stream_t stream) {
   if (!train_ok(T, H, E, k, I, dtype)) return MI_MOE_EUNSUPPORTED;
-  if (!x || !gate_w || !w_fc || !w_proj || !saved || !ws || (!dy && !d_aux) || (!dy && (d_w_fc || d_w_proj))) return MI_MOE_ENULL;
-  for (const void* p : {x, gate_w, w_fc, w_proj, saved, dy, static_cast<const void*>(dx), static_cast<const void*>(d_gate_w),
+  if (!x || !gate_w || !w_fc || !w_proj || !saved || !ws || (!dy && !d_aux) || (!dy && (d_w_fc || d_w_proj || (dx && dx_router_out)))) return MI_MOE_ENULL;
+  for (const void* p : {x, gate_w, w_fc, w_proj, saved, dy, static_cast<const void*>(dx), static_cast<const void*>(dx_router_out), static_cast<const void*>(d_gate_w),
                         static_cast<const void*>(d_w_fc), static_cast<const void*>(d_w_proj), static_cast<const void*>(ws)})
     if (!mi_aligned(p, 16)) return MI_MOE_EALIGN;
   const TrainSpace w = train_space(T, H, E, k, I);
@@ -287,10 +287,12 @@ extern "C" int mi_moe_layer_train_backward(const void* x, const void* gate_w, co
   const int32_t* ss = reinterpret_cast<const int32_t*>(k0 + w.sorted_scattered);
   const int32_t* off = reinterpret_cast<const int32_t*>(k0 + w.offsets);
   const float* loss_w = reinterpret_cast<const float*>(k0 + w.loss_w);
-  void *a = b + w.a, *d_h = b + w.d_h, *act_g = b + w.act_g, *d_logits = b + w.d_logits, *dx_router = b + w.dx_router;
+  void *a = b + w.a, *d_h = b + w.d_h, *act_g = b + w.act_g, *d_logits = b + w.d_logits;
   void* d_gates = dy ? b + w.d_gates : nullptr;
   int32_t* tokens = reinterpret_cast<int32_t*>(b + w.tokens);
-  const bool router = dx || d_gate_w;
+  // the router's gradient of x: on its own, or all of dx, or what the sum over a token's rows adds
+  void* dx_router = dx_router_out ? dx_router_out : !dx ? nullptr : dy ? b + w.dx_router : dx;
+  const bool router = dx_router || d_gate_w;
   auto split = [&](int K) { return gemm_ws && mi_moe_grouped_gemm_splits(K, dtype) ? gemm_ws : nullptr; };
   auto wgrad = [&](const void* ga, const int32_t* ai, const void* gb, const int32_t* bi, const int32_t* offsets, void* dw, int rows, int a_rows,
                    int b_rows, int M, int N, int experts_) {
@@ -307,14 +309,22 @@ extern "C" int mi_moe_layer_train_backward(const void* x, const void* gate_w, co
   if (router) {
     if ((rc = mi_router_dlogits_aux(logits, experts, d_gates, loss_w, d_aux, d_logits, T, E, k, dtype, static_cast<hipStream_t>(stream))) != MI_MOE_OK)
       return rc;
-    if (dx && (rc = mi_gemm_one_expert_wt(d_logits, gate_w, dy ? dx_router : dx, T, E, H, dtype, stream)) != MI_MOE_OK) return rc;
+    if (dx_router && (rc = mi_gemm_one_expert_wt(d_logits, gate_w, dx_router, T, E, H, dtype, stream)) != MI_MOE_OK) return rc;
   }
   if (dy && dx) {
     if ((rc = mi_moe_scattered_gemm_wt_ws(d_h, w_fc, a, ss, off, L, 2 * I, H, E, 1, 1, 0, dtype, split(2 * I), gemm_ws_bytes, stream)) != MI_MOE_OK)
       return rc;
-    if ((rc = mi_combine_sum(a, dx_router, dx, T, k, H, dtype, stream)) != MI_MOE_OK) return rc;
+    if ((rc = mi_combine_sum(a, dx_router_out ? nullptr : dx_router, dx, T, k, H, dtype, stream)) != MI_MOE_OK) return rc;
   }
   if (d_w_fc && (rc = wgrad(d_h, nullptr, x, tokens, off, d_w_fc, L, L, T, 2 * I, H, E)) != MI_MOE_OK) return rc;
   if (d_gate_w && (rc = wgrad(d_logits, nullptr, x, nullptr, nullptr, d_gate_w, T, T, T, E, H, 1)) != MI_MOE_OK) return rc;
   return MI_MOE_OK;
+}
+
+extern "C" int mi_moe_layer_train_backward(const void* x, const void* gate_w, const void* w_fc, const void* w_proj, const void* saved,
+                                           size_t saved_bytes, const void* dy, const void* d_aux, void* dx, void* d_gate_w, void* d_w_fc,
+                                           void* d_w_proj, int T, int H, int E, int k, int I, int dtype, void* ws, size_t ws_bytes,
+                                           void* gemm_ws, size_t gemm_ws_bytes, mi_moe_stream_t stream) {
+  return mi_moe_layer_train_backward_parts(x, gate_w, w_fc, w_proj, saved, saved_bytes, dy, d_aux, dx, nullptr, d_gate_w, d_w_fc, d_w_proj, T, H,
+                                           E, k, I, dtype, ws, ws_bytes, gemm_ws, gemm_ws_bytes, stream);
 }

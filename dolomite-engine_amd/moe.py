@@ -404,7 +404,8 @@ class MoE(nn.Module):
         sizes = ops.layer_train_sizes(hidden_states, gate_weight, bias, fc.weight, proj.weight, self.top_k)
         if sizes is None:
             return None
-        return RoutedExperts.apply(hidden_states, gate_weight, fc.weight, proj.weight, bias, self.top_k, sizes)
+        x_router = None if self.shared_intermediate_size is None else hidden_states
+        return RoutedExperts.apply(hidden_states, x_router, gate_weight, fc.weight, proj.weight, bias, self.top_k, sizes)
 
     def _routes_ragged(self, hidden_states: torch.Tensor, gate: nn.Module) -> bool:
         """Whether the router's own kernel takes rows that the fused forms do not, without a gradient (its backward would want

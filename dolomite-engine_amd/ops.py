@@ -1112,8 +1112,9 @@ def layer_train_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.
 
 def layer_train_backward(x: torch.Tensor, gate_weight: torch.Tensor, w_fc: torch.Tensor, w_proj: torch.Tensor,
                          saved: torch.Tensor, dy: torch.Tensor | None, d_aux: torch.Tensor | None, k: int,
-                         wanted: tuple[bool, bool, bool, bool], sizes: tuple[int, int, int, int]):
-    """Gradients of x, the gate, the up- and the down-projection (None where not ``wanted``, or where nothing arrives)."""
+                         wanted: tuple[bool, bool, bool, bool, bool], sizes: tuple[int, int, int, int]):
+    """Gradients of x, of x through the router alone, of the gate, the up- and the down-projection (None where not ``wanted``,
+    or where nothing arrives).  The first holds the router's part too unless the second is wanted."""
     _dev(x, gate_weight, w_fc, w_proj, saved, dy, d_aux)
     _no_grad(x, gate_weight, w_fc, w_proj, dy, d_aux)
     T, H = x.shape
@@ -1123,12 +1124,14 @@ def layer_train_backward(x: torch.Tensor, gate_weight: torch.Tensor, w_fc: torch
         if dy.data_ptr() % 16:
             dy = dy.clone()
     saved_bytes, _, ws_bytes, splits = sizes
-    # (the experts' weights get no gradient from the auxiliary loss alone)
-    grads = [torch.empty_like(t) if want and (i < 2 or dy is not None) else None
-             for i, (t, want) in enumerate(zip((x, gate_weight, w_fc, w_proj), wanted))]
+    # (the experts get no gradient from the auxiliary loss alone)
+    experts = dy is not None
+    arrives = (experts or not wanted[1], True, True, experts, experts)
+    grads = [torch.empty_like(t) if want and some else None
+             for t, want, some in zip((x, x, gate_weight, w_fc, w_proj), wanted, arrives)]
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
     gemm_ws, gemm_bytes = _gemm_workspace(x.device, splits, x.dtype) if splits else (None, 0)
-    check(_lib.load().mi_moe_layer_train_backward(
+    check(_lib.load().mi_moe_layer_train_backward_parts(
         x.data_ptr(), gate_weight.data_ptr(), w_fc.data_ptr(), w_proj.data_ptr(), saved.data_ptr(), saved_bytes, _ptr(dy), _ptr(d_aux),
         *(_ptr(g) for g in grads), T, H, E, k, I2 // 2, _code(x.dtype), ws.data_ptr(), ws_bytes, _ptr(gemm_ws), gemm_bytes, _stream()))
     return grads

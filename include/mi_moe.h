@@ -468,7 +468,10 @@ int mi_moe_layer_forward(const void* x, const void* norm_w, float norm_eps, int 
  * routing and loss terms that the forward leaves for the backward) and of either call's workspace.
  *   forward: y (T, H), aux_loss one value of `dtype`.
  *   backward: dy (T, H) or NULL (no gradient reached y), d_aux one value of `dtype` or NULL; dx (T, H), d_gate_w (E, H), d_w_fc
- *   (E, 2I, H), d_w_proj (E, H, I), each NULL where it is not wanted (the last two without dy: refused).
+ *   (E, 2I, H), d_w_proj (E, H, I), each NULL where it is not wanted (the last two without dy: refused).  dx is the sum of the
+ *   experts' part and the router's.
+ *   backward_parts: the two apart, dx (refused without dy) the experts' and dx_router (T, H) the router's, for a caller that adds
+ *   other gradients of x in between; dx_router NULL: as backward.
  * gemm_ws: as in the _ws calls (or NULL). */
 int mi_moe_layer_train_sizes(int T, int H, int E, int k, int I, int dtype, size_t* saved, size_t* forward_ws, size_t* backward_ws);
 int mi_moe_layer_train_forward(const void* x, const void* gate_w, const float* gate_bias, const void* w_fc, const void* w_proj,
@@ -478,6 +481,10 @@ int mi_moe_layer_train_backward(const void* x, const void* gate_w, const void* w
                                 size_t saved_bytes, const void* dy, const void* d_aux, void* dx, void* d_gate_w, void* d_w_fc, void* d_w_proj,
                                 int T, int H, int E, int k, int I, int dtype, void* ws, size_t ws_bytes, void* gemm_ws,
                                 size_t gemm_ws_bytes, mi_moe_stream_t stream);
+int mi_moe_layer_train_backward_parts(const void* x, const void* gate_w, const void* w_fc, const void* w_proj, const void* saved,
+                                      size_t saved_bytes, const void* dy, const void* d_aux, void* dx, void* dx_router, void* d_gate_w,
+                                      void* d_w_fc, void* d_w_proj, int T, int H, int E, int k, int I, int dtype, void* ws, size_t ws_bytes,
+                                      void* gemm_ws, size_t gemm_ws_bytes, mi_moe_stream_t stream);
 
 /*
  * Diagnostics (no counterpart in the reference; nothing in the layer calls them): the pieces of the persistent grouped GEMM's
