@@ -258,6 +258,22 @@ class FusedRouter(torch.autograd.Function):
         return dx, dw, None, None
 
 
+class RaggedLogits(torch.autograd.Function):
+    """logits = x @ gate_w^T (+ bias) in x.dtype from the kernel that routes without a gradient (ops.router_ragged), so that the
+    selection does not depend on whether there is one; the two products of the backward are torch's, as a linear layer's."""
+
+    @staticmethod
+    def forward(ctx, x, gate_w, bias, k):
+        ctx.save_for_backward(x, gate_w)
+        return ops.router_ragged(x, gate_w, k, bias=bias, return_logits=True)[0]
+
+    @staticmethod
+    def backward(ctx, dl):
+        x, gate_w = ctx.saved_tensors
+        dx = dl @ gate_w if ctx.needs_input_grad[0] else None
+        return dx, dl.t() @ x if ctx.needs_input_grad[1] else None, None, None
+
+
 class RoutedExperts(torch.autograd.Function):
     """(y, auxiliary loss) of a training step's router, routed experts and loss as one function: FusedRouter, SwitchAuxLoss and
     ScatteredSwiGLUExperts with their launches behind one library call in either direction (ops.layer_train_forward).  A small

@@ -29,7 +29,7 @@ import torch.nn.functional as F
 
 from . import ops
 from .activations import GLUActivation, get_activation_function, is_glu
-from .autograd import FusedRouter, RoutedExperts, ScatteredSwiGLUExperts, SwitchAuxLoss, one_expert_rows
+from .autograd import FusedRouter, RaggedLogits, RoutedExperts, ScatteredSwiGLUExperts, SwitchAuxLoss, one_expert_rows
 from .enums import Kernel
 from .kernels import is_kernel_allowed
 from .linear import ParameterizedLinear
@@ -408,10 +408,12 @@ class MoE(nn.Module):
         return RoutedExperts.apply(hidden_states, x_router, gate_weight, fc.weight, proj.weight, bias, self.top_k, sizes)
 
     def _routes_ragged(self, hidden_states: torch.Tensor, gate: nn.Module) -> bool:
-        """Whether the router's own kernel takes rows that the fused forms do not, without a gradient (its backward would want
-        multiples of 8 experts) and where the gate is only its weight."""
+        """Whether the router's own kernel forms the logits of rows that the fused forms do not take, where the gate is only its
+        weight.  Nothing here depends on the mode or on a gradient: a forward and its recomputation, training and evaluation
+        choose the same experts at a near-tie, which two orders of summation need not."""
         if not (ops.router_ragged_supported(hidden_states, self.num_experts, self.top_k)
-                and _called_as_written(gate, ParameterizedLinear, _LINEAR_FORWARD)):
+                and _called_as_written(gate, ParameterizedLinear, _LINEAR_FORWARD) and not _backward_hooks(gate)
+                and not _HOOKS._global_forward_hooks and not _HOOKS._global_forward_pre_hooks):
             return False
         weight = gate.weight
         return (gate.bias is None and weight.dtype == hidden_states.dtype and hidden_states.shape[0] > 0
@@ -419,9 +421,9 @@ class MoE(nn.Module):
                 and hidden_states.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
     def _unfused_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
-        """Router logits of shapes the router kernel does not take (more than 256 experts, a hidden size that is not a
-        multiple of 8, or with a gradient of 16): they come from torch, the selection still follows the kernel's tie rule (value descending,
-        expert index ascending) in training and in inference alike."""
+        """Router logits of shapes the router kernel does not take (more than 256 experts, or 64 and a hidden size that is not
+        a multiple of 16, or one that is not a multiple of 8): they come from torch, the selection still follows the kernel's tie
+        rule (value descending, expert index ascending) in training and in inference alike."""
         ops._warn_once(("router_unfused", self.num_experts, self.hidden_size, hidden_states.dtype),
                        f"MoE router with {self.num_experts} experts, hidden size {self.hidden_size}, "
                        f"{hidden_states.dtype}: not a shape of the fused router kernel; the logits are computed "
@@ -468,14 +470,16 @@ class MoE(nn.Module):
             return (*ops.router_fused(hidden_states, self.gate.weight, self.top_k, bias=self.router_logit_bias,
                                       return_logits=self.training), None)
 
-        if (is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda and logits is None
-                and not self._needs_grad(hidden_states) and not _HOOKS._global_forward_hooks
-                and not _HOOKS._global_forward_pre_hooks and self._routes_ragged(hidden_states, self.gate)):
-            return (*ops.router_ragged(hidden_states, self.gate.weight, self.top_k, bias=self.router_logit_bias,
-                                       return_logits=True), None)
-
         if is_kernel_allowed(Kernel.scattermoe) and hidden_states.is_cuda:
-            router_logits = self._unfused_logits(hidden_states) if logits is None else logits
+            if logits is not None:
+                router_logits = logits
+            elif not self._routes_ragged(hidden_states, self.gate):
+                router_logits = self._unfused_logits(hidden_states)
+            elif not self._needs_grad(hidden_states):
+                return (*ops.router_ragged(hidden_states, self.gate.weight, self.top_k, bias=self.router_logit_bias,
+                                           return_logits=True), None)
+            else:
+                router_logits = RaggedLogits.apply(hidden_states, self.gate.weight, self.router_logit_bias, self.top_k)
             with torch.no_grad():
                 router_weights, selected_experts = ops.router_topk_softmax(router_logits.detach(), self.top_k)
             if torch.is_grad_enabled() and router_logits.requires_grad:
@@ -679,3 +683,10 @@ def _called_as_written(module: nn.Module | None, cls: type, forward) -> bool:
         return False
     own = module.__dict__
     return not own["_forward_hooks"] and not own["_forward_pre_hooks"] and "forward" not in own
+
+
+def _backward_hooks(module: nn.Module) -> bool:
+    """Whether calling the module would put a hook into the graph."""
+    own = module.__dict__
+    return bool(own["_backward_hooks"] or own["_backward_pre_hooks"] or _HOOKS._global_backward_hooks
+                or _HOOKS._global_backward_pre_hooks)
