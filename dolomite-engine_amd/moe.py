@@ -415,7 +415,10 @@ class MoE(nn.Module):
                 and _called_as_written(gate, ParameterizedLinear, _LINEAR_FORWARD) and not _backward_hooks(gate)
                 and not _HOOKS._global_forward_hooks and not _HOOKS._global_forward_pre_hooks):
             return False
-        weight = gate.weight
+        weight, bias = gate.weight, self.router_logit_bias
+        # (torch broadcasts a bias of another shape and gives it a gradient; the kernel reads one value an expert)
+        if bias is not None and (bias.shape != (self.num_experts,) or bias.requires_grad):
+            return False
         return (gate.bias is None and weight.dtype == hidden_states.dtype and hidden_states.shape[0] > 0
                 and weight.shape == (self.num_experts, hidden_states.shape[-1])
                 and hidden_states.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)

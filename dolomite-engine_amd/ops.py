@@ -180,6 +180,8 @@ def router_ragged(x: torch.Tensor, gate_weight: torch.Tensor, k: int, bias: torc
     if gate_weight.dtype != x.dtype or gate_weight.shape[1] != H:
         raise ValueError("gate weight must be (E, H) in the dtype of x")
     if bias is not None:
+        if bias.shape != (E,):
+            raise ValueError("bias must be (E,)")
         bias = bias.to(torch.float32).contiguous()
     logits = torch.empty((T, E), dtype=x.dtype, device=x.device) if return_logits else None
     gates = torch.empty((T, k), dtype=x.dtype, device=x.device)

@@ -112,6 +112,36 @@ def test_backward_hook_of_the_gate_is_called(device, which, training):
     assert calls
 
 
+@pytest.mark.parametrize("training", [True, False])
+def test_bias_of_another_shape_is_broadcast(device, training):
+    from dolomite_engine_amd import Kernel, enable_kernels, ops
+
+    m = _layer(device, torch.bfloat16, 136, 5, 2).train(training)
+    x = torch.randn(20, 136, device=device).bfloat16()
+    forms = [torch.tensor(0.5), torch.tensor([0.5], device=device), torch.full((20, 5), 0.5, device=device), torch.full((5,), 0.5, device=device)]
+    with torch.no_grad(), enable_kernels([Kernel.scattermoe]):
+        routed = []
+        for bias in forms:
+            m.router_logit_bias = bias
+            routed.append(m._compute_routing_weights(x))
+            m(x)
+    for got in routed[:2]:
+        assert all(torch.equal(a, b) for a, b in zip(got, routed[2]))
+    torch.testing.assert_close(routed[3][0], routed[2][0], rtol=2.0 ** -7, atol=2.0 ** -7)  # (another order of summation: a rounding step)
+    with pytest.raises(ValueError):
+        ops.router_ragged(x, m.gate.weight.detach(), 2, bias=forms[1])
+
+
+def test_bias_with_a_gradient_gets_one(device):
+    from dolomite_engine_amd import Kernel, enable_kernels
+
+    m = _layer(device, torch.bfloat16, 136, 5, 2).train()
+    m.router_logit_bias = torch.zeros(5, device=device, requires_grad=True)
+    with enable_kernels([Kernel.scattermoe]):
+        m(torch.randn(20, 136, device=device).bfloat16()).sum().backward()
+    assert m.router_logit_bias.grad is not None
+
+
 def test_gate_that_is_more_than_its_weight_is_called(device):
     from dolomite_engine_amd import Kernel, MoE, enable_kernels
 
