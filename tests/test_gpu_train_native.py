@@ -117,6 +117,23 @@ def test_router_without_a_gradient_leaves_the_loss_without_one(device):
     assert y.requires_grad and not get_aux_loss().requires_grad
 
 
+@pytest.mark.parametrize("hook", ["full_backward_hook", "full_backward_pre_hook"])
+@pytest.mark.parametrize("everywhere", [False, True])
+def test_backward_hooks_are_called(device, hook, everywhere):
+    layer, x = _layer(device, torch.bfloat16, SIZES["even"])
+    want = _step(layer, x)
+    calls = []
+    call = lambda mod, *grads: calls.append(mod) if mod is layer.dropout else None
+    handle = (getattr(torch.nn.modules.module, "register_module_" + hook)(call) if everywhere
+              else getattr(layer.dropout, "register_" + hook)(call))
+    try:
+        got = _step(layer, x)
+    finally:
+        handle.remove()
+    assert len(calls) == 2  # behind the experts and in front of the residual
+    assert all(torch.equal(got[n], w) for n, w in want.items())
+
+
 def test_replaced_stage_is_called(device):
     layer, x = _layer(device, torch.bfloat16, SIZES["even"])
     calls = []
