@@ -611,8 +611,24 @@ static int wgrad_chunk(int L, int E, int M, int N) {
 // 74 / 60 (0), 83 / 67 (0.49), 3000 tokens 96 / 86 and 107 / 98, 5000 tokens 138 / 135 (0.3); 1536 x 512, 2048 tokens 61 / 44 (0.3), 5000
 // tokens 94 / 98 (0.49); 32 experts, 1024 x 1024, 509 tokens 36 / 25 (0); 8 experts, 28672 x 4096, 1000 tokens of 2 slots 873 / 759
 // (0.3).  One expert, which always wants its rows cut: 32 x 1024, 509 rows 17.1 / 15.6, 640 rows 17.5 / 17.8, 40 x 1536, 768 rows 18.1 /
-// 19.9.  (The second bound is for loads that collapse on one expert.)
-static bool wgrad_whole_experts(int L, int E) { return (long)L <= (E == 1 ? 640L : 768L * E) && L <= 32768; }
+// 19.9.
+// `most`: rows that one expert can have at most, one a token.  If every token chooses the same experts, L / most of them, their tiles are
+// all the work there is, one item of `most` rows each: the more there are of them, the more rows they may have.  Planned / whole, us, the
+// load even, with half and with all of the tokens on the same experts: 1024 x 1024, top-1 of 8 experts (16 tiles), 1536 tokens 23 / 14, 33 / 26
+// and 39 / 37, 4096 57 / 21, 53 / 51 and 46 / 82; top-1 of 64, 32768 tokens 93 / 82, 126 / 339 and 139 / 618; top-2 of 32 (32), 2048 37 / 26, 52 /
+// 40 and 54 / 53, 8192 54 / 44, 74 / 105 and 87 / 166; 1024 x 512, top-8 of 32 (64), 3072 41 / 31, 51 / 50 and 59 / 69; 1536 x 512, top-8 of 40
+// (96), 3840 64 / 57, 87 / 75 and 98 / 96; 512 x 256, top-2 of 8 (4), 1024 21 / 13, 21 / 20 and 21 / 25; 4096 x 4096, top-1 of 8 (256), 6144
+// 217 / 216, 410 / 217 and 698 / 186.  At the line half of the tokens cost less than planned, all of them up to a fifth more.  (256 CUs)
+static bool wgrad_whole_experts(int L, int E, long most, long tiles) {
+  if (E == 1) return L <= 640;
+  return (long)L <= 768L * E && L <= 32768 && (L == 0 || most <= 1024 + 32 * (L / most * tiles));
+}
+
+// (an operand with fewer rows than there are slots is gathered, and a token chooses an expert once)
+static long wgrad_most_rows(int L, int a_rows, int b_rows) {
+  const int rows = a_rows < b_rows ? a_rows : b_rows;
+  return rows < 1 ? 1 : rows < L ? rows : L;
+}
 
 static long wgrad_max_groups(int L, int E, int chunk) { return (long)L / chunk + (E < L ? E : L); }
 static size_t wgrad_plan_bytes(long groups, int E) { return ((size_t)(32 + groups + 3 * (long)E) * sizeof(int) + 255) / 256 * 256; }
@@ -684,22 +700,27 @@ int mi_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const i
   g.chunk = wgrad_chunk(L, E, M, N);
   const long max_groups = wgrad_max_groups(L, E, g.chunk);
   const int red_at = (int)(32 + max_groups);
-  const bool whole = wgrad_whole_experts(L, E);
+  g.m_tiles = mi_ceil_div(M, 256);
+  g.n_tiles = mi_ceil_div(N, 256);
+  const long tiles = (long)g.m_tiles * g.n_tiles;
+  const bool whole = wgrad_whole_experts(L, E, wgrad_most_rows(L, a_rows, b_rows), tiles);
   if (L > 0 && !whole) {
     g.next_item = reinterpret_cast<int*>(static_cast<unsigned char*>(workspace) + wgrad_slab_bytes(max_groups, M, N));
     hipLaunchKernelGGL(wgrad_plan_kernel, dim3(1), dim3(1024), 0, s, expert_offsets, L, E, g.chunk, g.next_item, red_at);
   }
-  g.m_tiles = mi_ceil_div(M, 256);
-  g.n_tiles = mi_ceil_div(N, 256);
   int cus = 0;
   int rc = mi_cu_count(&cus);
   if (rc != MI_MOE_OK) return rc;
   // (an XCD can be dealt an eighth of the groups, rounded up: with as many workgroups as items alone, two groups of a router's
   // gradient, 509 rows, 32 x 1024, were the work of one workgroup each, 33 us)
-  const long tiles = (long)g.m_tiles * g.n_tiles;
   const long per_xcd = whole ? ((long)E * tiles + 7) / 8 : (max_groups + 7) / 8 * tiles;
   const long grid = 8 * (per_xcd < cus / 8 ? per_xcd : (cus + 7) / 8);
   return dtype == MI_MOE_BF16 ? launch_wgrad<bf16_t>(g, (int)grid, red_at, s) : launch_wgrad<f16_t>(g, (int)grid, red_at, s);
+}
+
+extern "C" int mi_moe_grouped_wgrad_whole(int L, int a_rows, int b_rows, int M, int N, int E) {
+  if (L < 0 || a_rows < 0 || b_rows < 0 || M < 1 || N < 1 || E < 1) return MI_MOE_ESHAPE;
+  return wgrad_whole_experts(L, E, wgrad_most_rows(L, a_rows, b_rows), (long)mi_ceil_div(M, 256) * mi_ceil_div(N, 256));
 }
 
 extern "C" int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx,

@@ -371,6 +371,9 @@ size_t mi_moe_grouped_wgrad_workspace_bytes(int L, int E, int M, int N);
 int mi_moe_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx,
                          const int32_t* expert_offsets, void* dw, void* workspace, size_t workspace_bytes,
                          int L, int a_rows, int b_rows, int M, int N, int E, int dtype, mi_moe_stream_t stream);
+/* 1 where mi_moe_grouped_wgrad adds up every expert's rows in one go (few rows per expert, and none that can have many), 0 where it
+ * cuts them into groups. */
+int mi_moe_grouped_wgrad_whole(int L, int a_rows, int b_rows, int M, int N, int E);
 
 /* The same sums for F32 operands on the fp32 matrix instruction (no counterpart of its own in the reference: its
  * scattermoe backward serves every dtype): one workgroup per (expert, 128 x 128 tile of dw) adds the expert's rows

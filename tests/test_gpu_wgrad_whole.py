@@ -1,6 +1,6 @@
 """Weight gradients of few rows per expert, which run without a plan: whole experts, one item a tile.  The sizes sit on both sides of
-the lines that choose (640 rows of one expert, 768 rows per expert on average), with experts that have no rows, fewer than a
-slice of 64, and whole slices.
+the lines that choose (640 rows of one expert, 768 rows per expert on average, as many as one expert can have), with experts that
+have no rows, fewer than a slice of 64, and whole slices.
 
 Against a product in 64 bits: operands are exact, the sums are fp32 (relative error far below the rounding of the result), one
 rounding of at most 2^-8 (bf16, 8 significant bits) or 2^-11 (fp16, 11) of the value, and an absolute term for results that cancel: fp32 partial sums
@@ -46,6 +46,53 @@ def test_whole_experts(device, dtype, gather, counts, M, N):
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     bound = eps * want.abs() + max(counts) * 0.64 * max(counts) * 2.0 ** -24 + 2.0 ** -24
     assert ((got.cpu().double() - want).abs() <= bound).all()
+
+
+# (tokens, experts, top-k, M, N) at both sides of the bound on what one expert can have: 1024 + 32 rows for each of the k experts' tiles
+HOT = [(1088, 3, 1, 264, 8, 1), (1089, 3, 1, 264, 8, 0), (1409, 8, 2, 520, 264, 0), (1408, 8, 2, 520, 264, 1),
+       (2048, 40, 2, 1024, 1024, 1), (2049, 40, 2, 1024, 1024, 0), (3073, 40, 8, 1024, 512, 0), (3072, 40, 8, 1024, 512, 1), (32768, 64, 1, 1024, 1024, 0), (6000, 8, 1, 4096, 4096, 1),
+       (768, 2, 1, 8, 8, 1), (1057, 2, 1, 8, 8, 0)]
+
+
+@pytest.mark.parametrize("T,E,k,M,N,whole", HOT)
+def test_choice(T, E, k, M, N, whole):
+    from dolomite_engine_amd import _lib
+
+    choose = _lib.load().mi_moe_grouped_wgrad_whole
+    assert choose(T * k, T * k, T, M, N, E) == choose(T * k, T, T * k, M, N, E) == whole
+
+
+def test_choice_by_the_average():
+    from dolomite_engine_amd import _lib
+
+    choose = _lib.load().mi_moe_grouped_wgrad_whole
+    assert choose(640, 640, 640, 32, 1024, 1) == 1 and choose(641, 641, 641, 32, 1024, 1) == 0
+    assert choose(6144, 6144, 768, 256, 256, 8) == 1 and choose(6152, 6152, 769, 256, 256, 8) == 0
+    assert choose(32768, 32768, 4096, 4096, 4096, 64) == 1 and choose(32776, 32776, 4097, 4096, 4096, 64) == 0
+    assert choose(0, 0, 0, 8, 8, 4) == 1 and choose(-1, 0, 0, 8, 8, 1) < 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("load", ["even", "hot"])
+@pytest.mark.parametrize("T,E,k,M,N,whole", [h for h in HOT if h[0] * h[2] * h[3] * h[4] < 1 << 32])
+def test_gathered_by_token(device, load, T, E, k, M, N, whole):
+    from dolomite_engine_amd import ops
+
+    g = torch.Generator().manual_seed(T + M)
+    score = torch.rand(T, E, generator=g)
+    if load == "hot":
+        score[:, E - k:] += 1  # every token chooses the same experts
+    sel, ss = score.topk(k, dim=1).indices.flatten().sort(stable=True)
+    off, tok = torch.bincount(sel, minlength=E).cumsum(0), ss // k
+    print(f"wgrad by token T={T} E={E} k={k} {M}x{N} {load}", flush=True)
+    a, b = torch.randn(T * k, M, generator=g).bfloat16().to(device), torch.randn(T, N, generator=g).bfloat16().to(device)
+    got = ops.grouped_wgrad(a, b, off.int().to(device), None, tok.int().to(device))
+    turned = ops.grouped_wgrad(b, a, off.int().to(device), tok.int().to(device), None)
+    rows = torch.bincount(sel, minlength=E).tolist()
+    want = torch.stack([p.double().t() @ q.double() for p, q in zip(a.split(rows), b[tok.to(device)].split(rows))])
+    bound = 2.0 ** -8 * want.abs() + max(rows) * 0.64 * max(rows) * 2.0 ** -24 + 2.0 ** -24
+    assert ((got.double() - want).abs() <= bound).all()
+    assert ((turned.transpose(1, 2).double() - want).abs() <= bound).all()
 
 
 def test_built_code(tmp_path):
