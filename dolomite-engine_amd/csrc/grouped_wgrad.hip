@@ -646,6 +646,12 @@ extern "C" size_t mi_moe_grouped_wgrad_workspace_bytes(int L, int E, int M, int 
   return wgrad_slab_bytes(groups, M, N) + wgrad_plan_bytes(groups, E);
 }
 
+// what a call inside the library needs: whole experts leave no partial results
+size_t mi_grouped_wgrad_bytes(int L, int a_rows, int b_rows, int M, int N, int E) {
+  const long tiles = (long)mi_ceil_div(M, 256) * mi_ceil_div(N, 256);
+  return wgrad_whole_experts(L, E, wgrad_most_rows(L, a_rows, b_rows), tiles) ? 0 : mi_moe_grouped_wgrad_workspace_bytes(L, E, M, N);
+}
+
 template <typename T, bool GA, bool GB, bool PLAN> static int launch_wgrad_as(const WgradArgs& g, int grid, hipStream_t s) {
   auto kern = PLAN ? grouped_wgrad_kernel<T, GA, GB> : grouped_wgrad_whole_kernel<T, GA, GB>;
   static std::atomic<uint64_t> lds_ok{0};
@@ -674,21 +680,23 @@ template <typename T> static int launch_wgrad(const WgradArgs& g, int grid, int 
   return mi_launch_status();
 }
 
-// (no expert_offsets: one expert owns all rows)
+// `entry`: called through the library's interface, where offsets and the whole workspace are asked for.  Else no expert_offsets: one
+// expert owns all rows; and mi_grouped_wgrad_bytes of workspace, or none.
 int mi_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx, const int32_t* expert_offsets, void* dw,
                      void* workspace, size_t workspace_bytes, int L, int a_rows, int b_rows, int M, int N, int E, int dtype,
-                     mi_moe_stream_t stream, bool need_offsets) {
+                     mi_moe_stream_t stream, bool entry) {
   if (L < 0 || M < 1 || N < 1 || E < 1) return MI_MOE_ESHAPE;
   if (dtype != MI_MOE_BF16 && dtype != MI_MOE_F16) return MI_MOE_EDTYPE;
   if (M % 8 != 0 || N % 8 != 0 || E > WGRAD_MAX_E) return MI_MOE_EUNSUPPORTED;
   if (a_rows < 0 || b_rows < 0) return MI_MOE_ESHAPE;
   // rows are addressed with 32-bit byte offsets
   if ((uint64_t)a_rows * M * 2 >= (1ull << 32) || (uint64_t)b_rows * N * 2 >= (1ull << 32)) return MI_MOE_EUNSUPPORTED;
-  if (!dw || (!expert_offsets && (need_offsets || E != 1))) return MI_MOE_ENULL;
+  if (!dw || (!expert_offsets && (entry || E != 1))) return MI_MOE_ENULL;
   if (L > 0 && (!a || !b)) return MI_MOE_ENULL;
   if (!mi_aligned(a, 16) || !mi_aligned(b, 16) || !mi_aligned(dw, 16) || !mi_aligned(workspace, 16)) return MI_MOE_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (L > 0 && (!workspace || workspace_bytes < mi_moe_grouped_wgrad_workspace_bytes(L, E, M, N))) return MI_MOE_EWORKSPACE;
+  const size_t need = entry ? mi_moe_grouped_wgrad_workspace_bytes(L, E, M, N) : mi_grouped_wgrad_bytes(L, a_rows, b_rows, M, N, E);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return MI_MOE_EWORKSPACE;
 
   WgradArgs g;
   g.a = a; g.b = b; g.a_idx = a_idx; g.b_idx = b_idx; g.expert_offsets = expert_offsets;

@@ -26,7 +26,8 @@ int mi_router_dlogits_aux(const void* logits, const int32_t* idx, const void* d_
                           void* d_logits, int T, int E, int k, int dtype, hipStream_t s);
 int mi_grouped_wgrad(const void* a, const int32_t* a_idx, const void* b, const int32_t* b_idx, const int32_t* expert_offsets, void* dw,
                      void* workspace, size_t workspace_bytes, int L, int a_rows, int b_rows, int M, int N, int E, int dtype,
-                     mi_moe_stream_t stream, bool need_offsets);
+                     mi_moe_stream_t stream, bool entry);
+size_t mi_grouped_wgrad_bytes(int L, int a_rows, int b_rows, int M, int N, int E);
 
 namespace {
 
@@ -191,8 +192,8 @@ TrainSpace train_space(int T, int H, int E, int k, int I) {
   at = 0;
   // one after the other: the gradient of the activation with the gated activation behind it, the workspace of the down-projection's
   // weight gradient in place of the former, the slots' gradient of x, the other weight gradients' workspace
-  const size_t wg = larger(mi_moe_grouped_wgrad_workspace_bytes((int)L, E, 2 * I, H), mi_moe_grouped_wgrad_workspace_bytes(T, 1, E, H)) + 16;
-  const size_t front = (larger(L * I * elt, mi_moe_grouped_wgrad_workspace_bytes((int)L, E, H, I) + 16) + 255) / 256 * 256;
+  const size_t wg = larger(mi_grouped_wgrad_bytes((int)L, (int)L, T, 2 * I, H, E), mi_grouped_wgrad_bytes(T, T, T, E, H, 1));
+  const size_t front = (larger(L * I * elt, mi_grouped_wgrad_bytes((int)L, T, (int)L, H, I, E)) + 255) / 256 * 256;
   w.a = take(at, larger(larger(front + L * I * elt, L * H * elt), wg));
   w.act_g = w.a + front;
   w.d_h = take(at, L * 2 * I * elt);
@@ -296,7 +297,7 @@ extern "C" int mi_moe_layer_train_backward_parts(const void* x, const void* gate
   auto split = [&](int K) { return gemm_ws && mi_moe_grouped_gemm_splits(K, dtype) ? gemm_ws : nullptr; };
   auto wgrad = [&](const void* ga, const int32_t* ai, const void* gb, const int32_t* bi, const int32_t* offsets, void* dw, int rows, int a_rows,
                    int b_rows, int M, int N, int experts_) {
-    return mi_grouped_wgrad(ga, ai, gb, bi, offsets, dw, a, mi_moe_grouped_wgrad_workspace_bytes(rows, experts_, M, N), rows, a_rows, b_rows, M, N,
+    return mi_grouped_wgrad(ga, ai, gb, bi, offsets, dw, a, mi_grouped_wgrad_bytes(rows, a_rows, b_rows, M, N, experts_), rows, a_rows, b_rows, M, N,
                             experts_, dtype, stream, false);
   };
   int rc;

@@ -72,6 +72,26 @@ def test_choice_by_the_average():
     assert choose(0, 0, 0, 8, 8, 4) == 1 and choose(-1, 0, 0, 8, 8, 1) < 0
 
 
+@pytest.mark.parametrize("T,H,E,k,I,whole", [(509, 1024, 32, 8, 512, True), (1000, 4096, 8, 2, 14336, True), (640, 64, 8, 1, 8, True),
+                                             (4097, 256, 8, 2, 520, False)])
+def test_training_call_has_no_room_for_partial_results_that_whole_experts_do_not_leave(T, H, E, k, I, whole):
+    import ctypes
+
+    from dolomite_engine_amd import _lib
+
+    lib = _lib.load()
+    sizes = [ctypes.c_size_t() for _ in range(3)]
+    assert lib.mi_moe_layer_train_sizes(T, H, E, k, I, 2, *(ctypes.byref(s) for s in sizes)) == 0
+    L = T * k
+    # gradient of the activation with the gated activation, or the slots' gradient of x; d h, d gates, tokens, d logits, the router's d x
+    operands = [max(4 * L * I, 2 * L * H), 4 * L * I, 2 * L, 4 * L, 2 * T * E, 2 * T * H]
+    # (the gate's gradient is one expert's: its partial results are counted from 641 rows on)
+    gate = 0 if T <= 640 else lib.mi_moe_grouped_wgrad_workspace_bytes(T, 1, E, H)
+    most = sum(operands) + max(0, gate - operands[0]) + 512 * len(operands)
+    slabs = lib.mi_moe_grouped_wgrad_workspace_bytes(L, E, 2 * I, H)
+    assert sizes[2].value <= most if whole else sizes[2].value >= slabs
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("load", ["even", "hot"])
 @pytest.mark.parametrize("T,E,k,M,N,whole", [h for h in HOT if h[0] * h[2] * h[3] * h[4] < 1 << 32])
