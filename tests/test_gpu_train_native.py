@@ -70,6 +70,27 @@ def test_equals_stages(device, monkeypatch, name, dtype):
     _check(monkeypatch, layer, x)
 
 
+# sizes where the experts' weight gradients are cut into groups, whose partial results lie where the backward's first operands were:
+# both, with H above and below 2 I and I, the down-projection's alone, and more than 32768 slots
+PLANNED = {"both": ((4097, 256, 8, 2, 520), (0, 0)), "tall": ((4097, 512, 8, 2, 136), (0, 0)), "one of them": ((1160, 256, 8, 1, 520), (1, 0)),
+           "long": ((4600, 128, 64, 8, 64), (0, 0))}
+
+
+@pytest.mark.parametrize("load", ["even", "skewed"])
+@pytest.mark.parametrize("name", list(PLANNED))
+def test_planned_weight_gradients(device, monkeypatch, name, load):
+    from dolomite_engine_amd import _lib
+
+    (T, H, E, k, I), whole = PLANNED[name]
+    choose = _lib.load().mi_moe_grouped_wgrad_whole
+    assert (choose(T * k, T * k, T, 2 * I, H, E), choose(T * k, T, T * k, H, I, E)) == whole
+    layer, x = _layer(device, torch.bfloat16, PLANNED[name][0])
+    if load == "skewed":
+        layer.router_logit_bias = -2 * (torch.arange(E, device=device) + 1.0).log()
+    print(f"train native planned {name} {load}", flush=True)
+    _check(monkeypatch, layer, x)
+
+
 @pytest.mark.parametrize("how", [dict(parts="y"), dict(parts="aux"), dict(x_grad=False), dict(parts="aux", x_grad=False),
                                  dict(dy_form="strided"), dict(scale=0.25)])
 def test_parts_and_forms(device, monkeypatch, how):
