@@ -399,15 +399,16 @@ class MoE(nn.Module):
             return None
         if fc.weight_q is not None or proj.weight_q is not None or fc.bias is not None or proj.bias is not None:
             return None
-        gate_weight, bias = gate.weight, self.router_logit_bias
+        # (once each: a parametrized weight is computed where it is read)
+        gate_weight, w_fc, w_proj, bias = gate.weight, fc.weight, proj.weight, self.router_logit_bias
         # (with a router that has no gradient the loss has none either)
         if not (hidden_states.requires_grad or gate_weight.requires_grad):
             return None
-        sizes = ops.layer_train_sizes(hidden_states, gate_weight, bias, fc.weight, proj.weight, self.top_k)
+        sizes = ops.layer_train_sizes(hidden_states, gate_weight, bias, w_fc, w_proj, self.top_k)
         if sizes is None:
             return None
         x_router = None if self.shared_intermediate_size is None else hidden_states
-        return RoutedExperts.apply(hidden_states, x_router, gate_weight, fc.weight, proj.weight, bias, self.top_k, sizes)
+        return RoutedExperts.apply(hidden_states, x_router, gate_weight, w_fc, w_proj, bias, self.top_k, sizes)
 
     def _routes_ragged(self, hidden_states: torch.Tensor, gate: nn.Module) -> bool:
         """Whether the router's own kernel forms the logits of rows that the fused forms do not take, where the gate is only its

@@ -155,6 +155,23 @@ def test_backward_hooks_are_called(device, hook, everywhere):
     assert all(torch.equal(got[n], w) for n, w in want.items())
 
 
+def test_parametrized_weight_is_computed_once(device):
+    layer, x = _layer(device, torch.bfloat16, SIZES["even"])
+    want = _step(layer, x)
+    calls = []
+
+    class Counted(torch.nn.Module):
+        def forward(self, w):
+            calls.append(1)
+            return w * 1
+
+    torch.nn.utils.parametrize.register_parametrization(layer.c_fc, "weight", Counted())
+    calls.clear()
+    got = _step(layer, x)
+    assert len(calls) == 1
+    assert torch.equal(got["y"], want["y"]) and torch.equal(got["c_fc.parametrizations.weight.original"], want["c_fc.weight"])
+
+
 def test_replaced_stage_is_called(device):
     layer, x = _layer(device, torch.bfloat16, SIZES["even"])
     calls = []
