@@ -1112,6 +1112,12 @@ def layer_train_forward(x: torch.Tensor, gate_weight: torch.Tensor, bias: torch.
     return y, aux, saved
 
 
+def _as_laid_out(t: torch.Tensor) -> torch.Tensor:
+    """t, row-major and from 16 bytes on."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 def layer_train_backward(x: torch.Tensor, gate_weight: torch.Tensor, w_fc: torch.Tensor, w_proj: torch.Tensor,
                          saved: torch.Tensor, dy: torch.Tensor | None, d_aux: torch.Tensor | None, k: int,
                          wanted: tuple[bool, bool, bool, bool, bool], sizes: tuple[int, int, int, int]):
@@ -1121,10 +1127,10 @@ def layer_train_backward(x: torch.Tensor, gate_weight: torch.Tensor, w_fc: torch
     _no_grad(x, gate_weight, w_fc, w_proj, dy, d_aux)
     T, H = x.shape
     E, I2, _ = w_fc.shape
+    # (a saved-tensor hook may hand back other strides than it was given; the library sees pointers only)
+    x, gate_weight, w_fc, w_proj, saved = (_as_laid_out(t) for t in (x, gate_weight, w_fc, w_proj, saved))
     if dy is not None:
-        dy = dy.contiguous()
-        if dy.data_ptr() % 16:
-            dy = dy.clone()
+        dy = _as_laid_out(dy)
     saved_bytes, _, ws_bytes, splits = sizes
     # (the experts get no gradient from the auxiliary loss alone)
     experts = dy is not None

@@ -155,6 +155,25 @@ def test_backward_hooks_are_called(device, hook, everywhere):
     assert all(torch.equal(got[n], w) for n, w in want.items())
 
 
+def _strided(t):
+    return torch.stack([t, t], dim=-1)[..., 0]
+
+
+def _shifted(t):
+    return torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("unpack", [_strided, _shifted, lambda t: t.transpose(0, -1).contiguous().transpose(0, -1), lambda t: t.to("cuda:0")])
+def test_saved_tensor_hooks(device, unpack):
+    """What a hook hands back has the values, but not the strides or the alignment of what it was given."""
+    layer, x = _layer(device, torch.bfloat16, SIZES["wide"])
+    want = _step(layer, x)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(1) or t.cpu(), lambda t: unpack(t.to(device))):
+        got = _step(layer, x)
+    assert packed and all(torch.equal(got[n], w) for n, w in want.items())
+
+
 def test_parametrized_weight_is_computed_once(device):
     layer, x = _layer(device, torch.bfloat16, SIZES["even"])
     want = _step(layer, x)
