@@ -847,16 +847,16 @@ __global__ __launch_bounds__(256) void router_splitk_finish_kernel(const f32x4* 
   if (threadIdx.x < E) chunk_hist[(size_t)threadIdx.x * gridDim.x + tg] = whist[threadIdx.x];
 }
 
-// The finish kernel with the expert sort folded in (few tokens, T * k <= SORT_SINGLE_BLOCK_MAX): every workgroup
+// The finish kernel with the expert sort folded in (few tokens, T * k <= ROUTER_TICKET_SLOTS): every workgroup
 // publishes its 16 tokens' experts and takes a ticket; the workgroup that draws the last ticket sorts all T * k ids
 // in the same launch (the single-block counting sort of routing.hip).  One launch boundary less on a path that is a
 // chain of short dependent launches.  `ticket` is a counter in the workspace that the partial kernel has zeroed.
-// WAVES: waves of a workgroup; the first four add the partials, all of them sort.
-template <typename T, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void router_splitk_finish_sort_kernel(
+template <typename T>
+__global__ __launch_bounds__(SORT_THREADS) void router_splitk_finish_sort_kernel(
     const f32x4* __restrict__ partial, int splits, const float* __restrict__ bias, int Trows, int E, int k, int nbits,
     T* __restrict__ logits_out, T* __restrict__ gates, int32_t* __restrict__ idx, unsigned* __restrict__ ticket,
     int32_t* __restrict__ sorted_expert, int32_t* __restrict__ sorted_scattered, int32_t* __restrict__ expert_offsets) {
+  static_assert(SORT_WAVES == 4, "a wave for each quarter of the group, and for the sort");
   __shared__ f32x4 red[4][4][64];
   __shared__ int is_last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -864,28 +864,24 @@ __global__ __launch_bounds__(WAVES * 64) void router_splitk_finish_sort_kernel(
   f32x4 acc[4];
 #pragma unroll
   for (int eb = 0; eb < 4; ++eb) acc[eb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  if (wave < 4) {
 #pragma unroll 4
-    for (int ks = wave; ks < splits; ks += 4) {
-      const f32x4* src = partial + ((size_t)ks * gridDim.x + tg) * 4 * 64;
+  for (int ks = wave; ks < splits; ks += 4) {
+    const f32x4* src = partial + ((size_t)ks * gridDim.x + tg) * 4 * 64;
 #pragma unroll
-      for (int eb = 0; eb < 4; ++eb) acc[eb] += src[eb * 64 + lane];
-    }
-#pragma unroll
-    for (int eb = 0; eb < 4; ++eb) red[wave][eb][lane] = acc[eb];
+    for (int eb = 0; eb < 4; ++eb) acc[eb] += src[eb * 64 + lane];
   }
+#pragma unroll
+  for (int eb = 0; eb < 4; ++eb) red[wave][eb][lane] = acc[eb];
   __syncthreads();
-  if (wave < 4) {
-    router_epilogue_rows<T, 4>(&red[0][0][0], 4, wave, tg * 16, Trows, bias, E, k, logits_out, gates, idx);
-    __threadfence();  // this workgroup's experts are visible device-wide before its ticket is
-  }
+  router_epilogue_rows<T, 4>(&red[0][0][0], 4, wave, tg * 16, Trows, bias, E, k, logits_out, gates, idx);
+  __threadfence();  // this workgroup's experts are visible device-wide before its ticket is
   __syncthreads();
   if (threadIdx.x == 0) is_last = atomicAdd(ticket, 1u) == gridDim.x - 1;
   __syncthreads();
   if (!is_last) return;
   __threadfence();  // ... and the last workgroup reads what the others published
-  sort_single_block<WAVES>(idx, Trows * k, E, nbits, sorted_expert, sorted_scattered, expert_offsets,
-                    reinterpret_cast<int*>(&red[0][0][0]));
+  sort_single_block<SORT_WAVES>(idx, Trows * k, E, nbits, sorted_expert, sorted_scattered, expert_offsets,
+                                reinterpret_cast<int*>(&red[0][0][0]));
 }
 
 // K splits for the few-token path: one 64-wide K step per wave and round, enough workgroups to occupy the chip
@@ -1068,9 +1064,8 @@ static int launch_router_splitk_sort(const void* x, const void* gw, const float*
   }
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
-  const bool few = (long)T_ * k <= SORT_WAVES * 64 * SORT_ID_STEPS;  // (sixteen waves cost the adding part: 13 -> 15 us at 1256 ids)
-  auto kern = few ? router_splitk_finish_sort_kernel<T, SORT_WAVES> : router_splitk_finish_sort_kernel<T, SORT_MANY_WAVES>;
-  hipLaunchKernelGGL(kern, dim3(groups), dim3((few ? SORT_WAVES : SORT_MANY_WAVES) * 64), 0, s, static_cast<const f32x4*>(ws),
+  static_assert(ROUTER_TICKET_SLOTS <= SORT_THREADS * SORT_ID_STEPS, "the last workgroup keeps every id in registers");
+  hipLaunchKernelGGL((router_splitk_finish_sort_kernel<T>), dim3(groups), dim3(SORT_THREADS), 0, s, static_cast<const f32x4*>(ws),
                      splits, bias, T_, E, k, nbits, static_cast<T*>(logits_out), static_cast<T*>(gates), idx, ticket,
                      sorted_expert, sorted_scattered, expert_offsets);
   return mi_launch_status();
