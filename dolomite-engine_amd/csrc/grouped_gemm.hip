@@ -806,6 +806,7 @@ static double small_tiles(const GemmArgs& a, bool glu) {
 // The 128 x 128 tiles of a contraction that is no multiple of 32 come by DMA as well while there is at most one to a CU.  Staged through
 // registers / by DMA, us: one expert of 3001 rows, 920 -> 344 SwiGLU fp16 17.4 / 15.6 (144 tiles); 8 experts of 375, 1000 -> 392 18.3 / 16.2
 // (168); 7 of 171, 472 -> 200 11.1 / 10.1 (56); but 8 of 750, 1000 -> 392 29.3 / 31.6 (336) and 17 of 188, 920 -> 520 27.5 / 28.6 (306).
+// (256: the CUs these were measured on, here and below.  A choice is a function of the sizes, and is asked for without a device.)
 template <typename T, bool GLU>
 static int launch_128x128(const GemmArgs& a, hipStream_t s) {
   if (a.K % 32 != 0 && small_tiles(a, GLU) <= 256) return launch_dma<T, 128, 128, 2, 2, GLU, true>(a, s);

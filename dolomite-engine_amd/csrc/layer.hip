@@ -157,7 +157,7 @@ extern "C" int mi_moe_layer_forward(const void* x, const void* norm_w, float nor
 // ---- a training step's routed experts, forward and backward ----------------------------------------------------------------
 // The launches of autograd.FusedRouter, SwitchAuxLoss and ScatteredSwiGLUExperts (16-bit, pre-activation kept), one call each
 // way.  Behind one call the router's gradient of x is added where the k rows of a token are summed, instead of in a pass of its own
-// over both (32768 tokens of 1536: 46 us), the rows' tokens come out of the SwiGLU's backward, and the loss and its gradient stay
+// over both (32768 tokens of 1536: 46 us; with shared experts it is handed back apart, see autograd.RoutedExperts), the rows' tokens come out of the SwiGLU's backward, and the loss and its gradient stay
 // in the logits' type (three small launches).
 namespace {
 

@@ -399,7 +399,8 @@ __global__ __launch_bounds__(ROUTER_LDS_WAVES * 64) void router_fused_lds_kernel
     }
     }
     if constexpr (KS) {
-      // every wave is done with the weights; the parts of a group meet in LDS and part 0 adds them in part order
+      // every wave is done with the weights; the parts of a group meet in LDS, and each of its waves adds them, in part order, for
+      // the tokens that it selects for
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
       __builtin_amdgcn_s_barrier();

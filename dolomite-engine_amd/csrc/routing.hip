@@ -250,7 +250,7 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(const int32_
 }
 
 // Passes 2 and 3 in one launch, for a table of up to 256 chunks and 64 experts: every block reads the whole table,
-// 40 KB at most, and adds up for itself what of each expert lies before its slots, and in all.  The launch in front of the scatter, a
+// 64 KB at most, and adds up for itself what of each expert lies before its slots, and in all.  The launch in front of the scatter, a
 // third of the sort's time, is gone; in exchange a block has one trip to the table, on which its own ids ride along.  A block has
 // `per` consecutive chunks, up to 2048 slots; a wave keeps its ids, up to 128, for both passes over them.
 // Three launches / two, us: 16384 slots of 40 experts 9.0 / 6.5 (eight waves a block 7.1, four 8.7), 131072 of 32 10.5 / 7.1, 262144 of 40
@@ -480,6 +480,6 @@ extern "C" int mi_moe_sort_bin_static(const int32_t* topk_idx, int T, int k, int
     ws = sort_static_scratch(&rc);
     if (!ws) return rc;
   }
-  // the one-block path (need == 0) touches no workspace; otherwise the same three launches on the library's array
+  // the one-block path (need == 0) touches no workspace; otherwise the same launches on the library's array
   return mi_moe_sort_bin(topk_idx, T, k, E, sorted_expert, sorted_scattered, expert_offsets, ws, need, stream);
 }
